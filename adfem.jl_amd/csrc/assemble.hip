@@ -524,6 +524,8 @@ void launch_assemble_to(const System &s, const double2 *xy, const admfem_problem
 
 void launch_assemble(System &s, const admfem_problem &p, hipStream_t st) {
   SellOut o{s.d_sell_val.p, s.d_diag.p, s.rhs.p};
+  s.a_version++;
+  s.mass = p.mass_coef != 0.0;
   launch_assemble_to(s, s.mesh->xy.p, p, o, st);
 }
 

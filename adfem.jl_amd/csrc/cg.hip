@@ -699,11 +699,12 @@ void launch_graph(System &s, CGWork *w, bool mixed, int max_iter, hipStream_t st
 void cg_solve(System &s, const double *b, double *x_out, const admfem_solve_opts &o,
               admfem_solve_stats &stats, hipStream_t st) {
   auto t0 = std::chrono::steady_clock::now();
-  CGWork *w = ensure_work(s);
-  const int nb = w->nblocks, np = s.npad;
   const bool mixed = o.precision == ADMFEM_PREC_MIXED;
   REQUIRE(o.precision == ADMFEM_PREC_FP64 || mixed, ADMFEM_ERR_ARG, "bad precision");
   REQUIRE(o.rtol > 0 && o.max_iter > 0, ADMFEM_ERR_ARG, "bad rtol/max_iter");
+  if (mg_solve(s, b, x_out, o, stats, st)) return;
+  CGWork *w = ensure_work(s);
+  const int nb = w->nblocks, np = s.npad;
   CGScalars init{};
   init.rtol2 = o.rtol * o.rtol;
   const double delta = o.replace_delta > 0 ? o.replace_delta : REPLACE_DELTA;

@@ -186,6 +186,8 @@ void mesh_user_pattern(Mesh &m);
 
 // ------------------------------------------------------------------ system
 struct CGWork;
+struct MgPlan;
+struct MgWork;
 struct System {
   Mesh *mesh = nullptr;
   int degree = 1;  // the mesh's element degree
@@ -235,6 +237,12 @@ struct System {
   DevBuf<int> d_vrow;
   DevBuf<int2> d_dof_ends;
   CGWork *work = nullptr;
+  // multigrid (mg.hip): the topology's grids and the solver's arrays, made on
+  // first use; a_version counts the matrices assembled into d_sell_val
+  MgPlan *mg_plan = nullptr;
+  MgWork *mg_work = nullptr;
+  uint64_t a_version = 1;
+  bool mass = false;  // the assembled matrix has a mass term
   size_t device_bytes() const;
   // user node / dof id -> internal row, and back (mesh systems)
   const std::vector<int> &uperm() const { return degree == 2 ? perm2 : mesh->perm; }
@@ -367,6 +375,11 @@ void cg_solve(System &s, const double *b_int, double *x_int,
               const admfem_solve_opts &o, admfem_solve_stats &stats,
               hipStream_t st);
 void cg_work_free(CGWork *w);
+// mg.hip
+void mg_plan_free(MgPlan *p);
+void mg_work_free(MgWork *w);
+bool mg_solve(System &s, const double *b_int, double *x_int, const admfem_solve_opts &o,
+              admfem_solve_stats &stats, hipStream_t st);
 void spmv_repeat(System &s, int precision, int repeat, hipStream_t st);
 // sparse_op.hip
 void sparse_solve(const long long *ind, const double *vv, int64_t nnz, int n, const double *rhs,

@@ -504,6 +504,8 @@ System *system_from_device_csr(int n, DevBuf<int> &rp, DevBuf<int> &col, int64_t
 void system_free(System *s) {
   if (!s) return;
   if (s->work) cg_work_free(s->work);
+  if (s->mg_work) mg_work_free(s->mg_work);
+  if (s->mg_plan) mg_plan_free(s->mg_plan);
   delete s;
 }
 

@@ -655,6 +655,8 @@ struct Server {
   void serve_seq(Req &q, System &s) {
     inputs(q);
     admfem_problem p = problem(q);
+    s.a_version++;
+    s.mass = p.mass_coef != 0.0;
     launch_assemble_to(s, q.xy, p, SellOut{s.d_sell_val.p, s.d_diag.p, s.rhs.p},
                        st);
     admfem_solve_opts so{ADMFEM_PREC_FP64, o.max_iter, o.rtol, 0, 0.0};
