@@ -54,6 +54,12 @@ _SIGS = {
     "admfem_sparse_solve_grad": (c_int, [c_vp, c_vp, c_i64, c_int, c_vp, c_vp, c_vp, c_vp,
                                          ctypes.POINTER(SolveOpts), ctypes.POINTER(SolveStats),
                                          c_vp]),
+    "admfem_sparse_solve_on": (c_int, [c_vp, c_vp, c_vp, c_i64, c_int, c_vp, c_vp,
+                                       ctypes.POINTER(SolveOpts), ctypes.POINTER(SolveStats),
+                                       c_vp]),
+    "admfem_sparse_solve_grad_on": (c_int, [c_vp, c_vp, c_vp, c_i64, c_int, c_vp, c_vp, c_vp,
+                                            c_vp, ctypes.POINTER(SolveOpts),
+                                            ctypes.POINTER(SolveStats), c_vp]),
     "admfem_sparse_solve_info": (c_int, [c_vp]),
     # A. reference-named
     "init_nnfem_mesh": (c_ll_p, [c_vp, c_int, c_vp, c_int, c_int, c_int, c_int, c_vp]),

@@ -30,7 +30,11 @@ _DEV = "cuda"
 
 class SparseTensor:
     """n x n matrix as COO triplets: ``indices`` [nnz, 2] int64 (0-based) and
-    differentiable ``values`` [nnz] float64, both on the GPU."""
+    differentiable ``values`` [nnz] float64, both on the GPU.  ``mesh``: the
+    mesh whose dofs the rows are, when an operator of that mesh made the matrix
+    (``solve`` then works on grids laid over it); None otherwise."""
+
+    mesh = None
 
     def __init__(self, indices, values, n):
         # the reference converts indices to Int64 and values to Float64
@@ -46,11 +50,12 @@ class SparseTensor:
     def __add__(self, other):
         if not isinstance(other, SparseTensor) or other.n != self.n:
             raise TypeError("SparseTensor + SparseTensor of the same size")
-        return SparseTensor(torch.cat([self.indices, other.indices]),
-                            torch.cat([self.values, other.values]), self.n)
+        return _on(self.mesh if self.mesh is other.mesh else None,
+                   SparseTensor(torch.cat([self.indices, other.indices]),
+                                torch.cat([self.values, other.values]), self.n))
 
     def __mul__(self, a):
-        return SparseTensor(self.indices, self.values * a, self.n)
+        return _on(self.mesh, SparseTensor(self.indices, self.values * a, self.n))
 
     __rmul__ = __mul__
 
@@ -69,6 +74,11 @@ class SparseTensor:
 
     def __truediv__(self, rhs):  # not Julia's \, kept explicit: use solve()
         raise TypeError("use admfem.ops.solve(A, rhs) for A \\ rhs")
+
+
+def _on(mesh, A):
+    A.mesh = mesh
+    return A
 
 
 def _dev(t, dtype=torch.float64):
@@ -109,7 +119,7 @@ def compute_fem_laplace_matrix1(kappa, mesh=None):
         return SparseTensor(ind, vv, mesh.ndof).to_scipy().tocsc()
     ind, vv = _LaplaceCOO.apply(kappa, mesh, L.admfem_fem_laplace_scalar,
                                 L.admfem_fem_laplace_scalar_grad)
-    return SparseTensor(ind, vv, mesh.ndof)
+    return _on(mesh, SparseTensor(ind, vv, mesh.ndof))
 
 
 def compute_fem_mass_matrix1(rho, mesh=None):
@@ -122,7 +132,7 @@ def compute_fem_mass_matrix1(rho, mesh=None):
     L = _lib.lib()
     r = torch.as_tensor(rho) if isinstance(rho, np.ndarray) else rho
     ind, vv = _LaplaceCOO.apply(r, mesh, L.admfem_fem_mass_matrix, L.admfem_fem_mass_matrix_grad)
-    return SparseTensor(ind, vv, mesh.ndof)
+    return _on(mesh, SparseTensor(ind, vv, mesh.ndof))
 
 
 class _Source(torch.autograd.Function):
@@ -324,21 +334,21 @@ def impose_Dirichlet_boundary_conditions(A, rhs, bdnode=None, bdval=None):
     if not torch.is_tensor(bdval):
         bdval = torch.as_tensor(np.asarray(bdval, dtype=np.float64))
     oi, ov, orhs = _Dirichlet.apply(A.values, rhs, bdval, A.indices.contiguous(), bd, A.n)
-    B = SparseTensor(oi, ov, A.n)
+    B = _on(A.mesh, SparseTensor(oi, ov, A.n))
     return B if homogeneous else (B, orhs)
 
 
 class _Solve(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, vv, rhs, ind, n, opts):
+    def forward(ctx, vv, rhs, ind, n, opts, mesh):
         vv, rhs = _dev(vv), _dev(rhs)
         u = torch.empty(n, dtype=torch.float64, device=_DEV)
         st = _lib.SolveStats()
-        _lib.check(_lib.lib().admfem_sparse_solve(
-            _lib.ptr(ind), _lib.ptr(vv), ind.shape[0], n, _lib.ptr(rhs), _lib.ptr(u),
+        _lib.check(_lib.lib().admfem_sparse_solve_on(
+            mesh.handle if mesh is not None else None, _lib.ptr(ind), _lib.ptr(vv), ind.shape[0], n, _lib.ptr(rhs), _lib.ptr(u),
             ctypes.byref(opts), ctypes.byref(st), _lib.stream_ptr()))
         ctx.save_for_backward(vv, ind, u)
-        ctx.n, ctx.opts = n, opts
+        ctx.n, ctx.opts, ctx.mesh = n, opts, mesh
         return u
 
     @staticmethod
@@ -348,18 +358,18 @@ class _Solve(torch.autograd.Function):
         gv = torch.empty_like(vv)
         gr = torch.empty(ctx.n, dtype=torch.float64, device=_DEV)
         st = _lib.SolveStats()
-        _lib.check(_lib.lib().admfem_sparse_solve_grad(
-            _lib.ptr(ind), _lib.ptr(vv), ind.shape[0], ctx.n, _lib.ptr(u), _lib.ptr(g_u),
+        _lib.check(_lib.lib().admfem_sparse_solve_grad_on(
+            ctx.mesh.handle if ctx.mesh is not None else None, _lib.ptr(ind), _lib.ptr(vv), ind.shape[0], ctx.n, _lib.ptr(u), _lib.ptr(g_u),
             _lib.ptr(gv), _lib.ptr(gr), ctypes.byref(ctx.opts), ctypes.byref(st),
             _lib.stream_ptr()))
-        return gv, gr, None, None, None
+        return gv, gr, None, None, None, None
 
 
 def solve(A, rhs, precision="fp64", rtol=1e-12, max_iter=1000000):
     """``A \\ rhs`` for an SPD SparseTensor (ADCME SparseSolver, with its
     gradient SparseSolverGrad)."""
     opts = solve_opts(precision, rtol, max_iter)
-    return _Solve.apply(A.values, rhs, A.indices.contiguous(), A.n, opts)
+    return _Solve.apply(A.values, rhs, A.indices.contiguous(), A.n, opts, A.mesh)
 
 
 def solve_pattern_info():

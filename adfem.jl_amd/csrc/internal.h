@@ -138,6 +138,7 @@ constexpr int64_t PAR_GRAIN = 16384;  // items per host thread, at least
 
 // --------------------------------------------------------------------- mesh
 struct Mesh {
+  uint64_t serial = 0;     // of the meshes made by this process
   int nnode = 0, nelem = 0, order = 2;
   int degree = 1, nd = 3;  // element degree and dofs per element (3 or 6)
   int64_t ndof = 0;        // nnode (P1) or nnode + nedges (P2)
@@ -242,6 +243,8 @@ struct System {
   MgPlan *mg_plan = nullptr;
   MgWork *mg_work = nullptr;
   uint64_t a_version = 1;
+  bool mg_off = false;      // sparse systems whose mesh is not known
+  uint64_t mg_serial = 0;   // sparse systems: the mesh the grids were laid over
   bool mass = false;  // the assembled matrix has a mass term
   size_t device_bytes() const;
   // user node / dof id -> internal row, and back (mesh systems)
@@ -378,15 +381,16 @@ void cg_work_free(CGWork *w);
 // mg.hip
 void mg_plan_free(MgPlan *p);
 void mg_work_free(MgWork *w);
+void mg_set_mesh(System &s, const Mesh *m, const int *order, hipStream_t st);
 bool mg_solve(System &s, const double *b_int, double *x_int, const admfem_solve_opts &o,
               admfem_solve_stats &stats, hipStream_t st);
 void spmv_repeat(System &s, int precision, int repeat, hipStream_t st);
-// sparse_op.hip
-void sparse_solve(const long long *ind, const double *vv, int64_t nnz, int n, const double *rhs,
+// sparse_op.hip (m: the mesh whose dofs the rows are, or null)
+void sparse_solve(const Mesh *m, const long long *ind, const double *vv, int64_t nnz, int n, const double *rhs,
                   double *u, const admfem_solve_opts &o, admfem_solve_stats &stats,
                   hipStream_t st);
 void sparse_solve_info(int64_t info[4]);
-void sparse_solve_grad(const long long *ind, const double *vv, int64_t nnz, int n,
+void sparse_solve_grad(const Mesh *m, const long long *ind, const double *vv, int64_t nnz, int n,
                        const double *u, const double *grad_u, double *grad_vv,
                        double *grad_rhs, const admfem_solve_opts &o, admfem_solve_stats &stats,
                        hipStream_t st);

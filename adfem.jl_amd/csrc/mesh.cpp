@@ -8,6 +8,7 @@
 // per-element geometry (area, weights, Gauss points) is computed on the GPU
 // (geometry.hip).
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstring>
 #include <numeric>
@@ -154,8 +155,10 @@ Mesh *mesh_build(const double *coords, int nnode, const int *elems, int nelem,
   QuadRule rule;
   REQUIRE(quad_rule(order, rule) > 0, ADMFEM_ERR_UNSUPPORTED,
           "integration order " + std::to_string(order) + " not built (orders 0-4 are)");
+  static std::atomic<uint64_t> serials{0};
   Mesh *m = new Mesh();
   try {
+    m->serial = ++serials;
     m->nnode = nnode;
     m->nelem = nelem;
     m->order = order;
@@ -485,6 +488,7 @@ System *system_from_device_csr(int n, DevBuf<int> &rp, DevBuf<int> &col, int64_t
   System *s = new System();
   try {
     s->mesh = nullptr;
+    s->mg_off = true;
     s->n = n;
     s->npad = (n + 63) / 64 * 64;
     s->row_bd.assign(n, -1);

@@ -825,27 +825,59 @@ __global__ void __launch_bounds__(RT)
 
 // ------------------------------------------------------------------ the plan
 
-// Each row's point: P1 the node, P2 the vertex or the edge's midpoint.
-__device__ __forceinline__ double2 row_point(const double2 *__restrict__ xy,
-                                             const int2 *__restrict__ ends, int i) {
-  if (!ends) return xy[i];
-  const int2 e = ends[i];
-  const double2 a = xy[e.x], b = xy[e.y];
-  return make_double2(0.5 * (a.x + b.x), 0.5 * (a.y + b.y));
+// Each row's point.  Mesh systems: P1 the node (ends null), P2 the vertex or
+// the edge's midpoint (ends: mesh-internal vertices).  Sparse systems whose
+// rows are a mesh's dofs (perm not null): caller's row order[i] (order null:
+// i), a vertex below nnode, else the edge's midpoint.
+__global__ void __launch_bounds__(NT)
+    plan_points(int n, const double2 *__restrict__ xy, const int2 *__restrict__ ends,
+                const int *__restrict__ order, const int *__restrict__ perm, int nnode,
+                const long long *__restrict__ edges, long long nedges,
+                double2 *__restrict__ pt) {
+  const int i = blockIdx.x * NT + threadIdx.x;
+  if (i >= n) return;
+  int a, b;
+  if (perm) {
+    const int u = order ? order[i] : i;
+    if (u < nnode) {
+      a = b = perm[u];
+    } else {
+      a = perm[edges[u - nnode] - 1];
+      b = perm[edges[nedges + u - nnode] - 1];
+    }
+  } else if (ends) {
+    a = ends[i].x;
+    b = ends[i].y;
+  } else {
+    a = b = i;
+  }
+  const double2 p = xy[a], q = xy[b];
+  pt[i] = make_double2(0.5 * (p.x + q.x), 0.5 * (p.y + q.y));
+}
+
+// A row takes part in the grids when it is no Dirichlet row and is coupled
+// to another one.
+__device__ __forceinline__ bool takes_part(int i, const int *__restrict__ row_bd,
+                                           const int *__restrict__ sp,
+                                           const int *__restrict__ sc) {
+  if (row_bd[i] >= 0) return false;
+  const int s0 = sp[i >> 6], w = (sp[(i >> 6) + 1] - s0) >> 6, off = s0 + (i & 63);
+  for (int k = 0; k < w; k++)
+    if (sc[off + 64 * k] != i) return true;
+  return false;
 }
 
 // Per block: the interior rows' bounding box, count and largest coupling
 // extents (|dx|, |dy| over the matrix entries).
 __global__ void __launch_bounds__(NT)
-    plan_extent(int n, const double2 *__restrict__ xy, const int2 *__restrict__ ends,
-                const int *__restrict__ row_bd, const int *__restrict__ sp,
+    plan_extent(int n, const double2 *__restrict__ pt, const int *__restrict__ row_bd, const int *__restrict__ sp,
                 const int *__restrict__ sc, double *__restrict__ out) {
   const int i = blockIdx.x * NT + threadIdx.x;
   // min x, min y, -max x, -max y, -max |dx|, -max |dy|
   double v[6] = {1e300, 1e300, 1e300, 1e300, 0.0, 0.0};
   double cnt = 0.0;
-  if (i < n && row_bd[i] < 0) {
-    const double2 a = row_point(xy, ends, i);
+  if (i < n && takes_part(i, row_bd, sp, sc)) {
+    const double2 a = pt[i];
     v[0] = a.x;
     v[1] = a.y;
     v[2] = -a.x;
@@ -855,7 +887,7 @@ __global__ void __launch_bounds__(NT)
     for (int k = 0; k < w; k++) {
       const int j = sc[off + 64 * k];
       if (j >= n) continue;
-      const double2 b = row_point(xy, ends, j);
+      const double2 b = pt[j];
       v[4] = fmin(v[4], -fabs(a.x - b.x));
       v[5] = fmin(v[5], -fabs(a.y - b.y));
     }
@@ -889,19 +921,19 @@ __global__ void __launch_bounds__(NT)
   if (threadIdx.x == 0) out[blockIdx.x] = s;
 }
 
-// Each row's cell (-1 for Dirichlet rows) and its position in it; key: the
-// cell, Dirichlet rows last.
+// Each row's cell (-1: takes no part) and its position in it; key: the cell,
+// the rows that take no part last.
 __global__ void __launch_bounds__(NT)
-    plan_cells(int n, int npad, const double2 *__restrict__ xy, const int2 *__restrict__ ends,
-               const int *__restrict__ row_bd, double x0, double y0, double hx, double hy,
+    plan_cells(int n, int npad, const double2 *__restrict__ pt, const int *__restrict__ row_bd,
+               const int *__restrict__ sp, const int *__restrict__ sc, double x0, double y0, double hx, double hy,
                int ncx, int ncy, int *__restrict__ cell, float2 *__restrict__ frac,
                int *__restrict__ key, int *__restrict__ row) {
   const int i = blockIdx.x * NT + threadIdx.x;
   if (i >= npad) return;
   int c = -1;
   float2 f = make_float2(0.0f, 0.0f);
-  if (i < n && row_bd[i] < 0) {
-    const double2 a = row_point(xy, ends, i);
+  if (i < n && takes_part(i, row_bd, sp, sc)) {
+    const double2 a = pt[i];
     const double tx = (a.x - x0) / hx, ty = (a.y - y0) / hy;
     const int ix = min(max((int)floor(tx), 0), ncx - 1), iy = min(max((int)floor(ty), 0), ncy - 1);
     f = make_float2(fminf(fmaxf((float)(tx - ix), 0.0f), 1.0f),
@@ -956,16 +988,20 @@ __global__ void __launch_bounds__(NT)
   }
 }
 
-MgPlan *build_plan(System &s, hipStream_t st) {
+// The plan of a mesh system, or of a sparse system whose rows are the dofs
+// of mesh m (row i: the caller's order[i], order null: i).
+MgPlan *build_plan(System &s, const Mesh &m, const int *order, hipStream_t st) {
   MgPlan *pl = new MgPlan();
   try {
-    const Mesh &m = *s.mesh;
     const int n = s.n, np = s.npad;
-    const int2 *ends = s.degree == 2 ? s.d_dof_ends.p : nullptr;
+    const bool own = s.mesh != nullptr;
     const unsigned g = nb(n, NT);
     DevBuf<double> ext((size_t)7 * g), ar(256);
-    plan_extent<<<g, NT, 0, st>>>(n, m.xy.p, ends, s.d_row_bd.p, s.d_slice_ptr.p, s.d_sell_col.p,
-                                  ext.p);
+    DevBuf<double2> pt(n);
+    plan_points<<<g, NT, 0, st>>>(n, m.xy.p, own && s.degree == 2 ? s.d_dof_ends.p : nullptr,
+                                  order, own ? nullptr : m.d_perm.p, m.nnode, m.d_edges.p,
+                                  m.nedges, pt.p);
+    plan_extent<<<g, NT, 0, st>>>(n, pt.p, s.d_row_bd.p, s.d_slice_ptr.p, s.d_sell_col.p, ext.p);
     plan_area<<<256, NT, 0, st>>>(m.nelem, m.area.p, ar.p);
     HIPCHECK(hipGetLastError());
     std::vector<double> he((size_t)7 * g), ha(256);
@@ -996,8 +1032,8 @@ MgPlan *build_plan(System &s, hipStream_t st) {
     pl->frac.alloc(np);
     pl->crow.alloc(n);
     pl->cptr.alloc(ncell + 1);
-    plan_cells<<<nb(np, NT), NT, 0, st>>>(n, np, m.xy.p, ends, s.d_row_bd.p, x0, y0, hx, hy, ncx,
-                                          ncy, pl->cell.p, pl->frac.p, key.p, row.p);
+    plan_cells<<<nb(np, NT), NT, 0, st>>>(n, np, pt.p, s.d_row_bd.p, s.d_slice_ptr.p,
+                                          s.d_sell_col.p, x0, y0, hx, hy, ncx, ncy, pl->cell.p, pl->frac.p, key.p, row.p);
     HIPCHECK(hipGetLastError());
     int bits = 1;
     while (ncell >> bits) bits++;
@@ -1056,8 +1092,8 @@ size_t tail_lds(const MgPlan &pl) {
 void mg_plan_free(MgPlan *p) { delete p; }
 
 const MgPlan *mg_plan(System &s, hipStream_t st) {
-  if (!s.mg_plan) s.mg_plan = build_plan(s, st);
-  return s.mg_plan->ok ? s.mg_plan : nullptr;
+  if (!s.mg_plan && s.mesh) s.mg_plan = build_plan(s, *s.mesh, nullptr, st);
+  return s.mg_plan && s.mg_plan->ok ? s.mg_plan : nullptr;
 }
 
 size_t mg_grid_floats(const MgPlan &pl) {
@@ -1266,11 +1302,25 @@ void launch_graph(const MgPlan &pl, MgWork *w, hipStream_t st) {
 // Systems below this many rows stay with Jacobi-PCG.
 constexpr int MG_MIN_ROWS = 4096;
 
+// A sparse system's rows are the dofs of mesh m (m null: unknown, and it is
+// Jacobi-PCG's); its plan is kept for as long as the mesh stays the same one.
+void mg_set_mesh(System &s, const Mesh *m, const int *order, hipStream_t st) {
+  s.mg_off = !m || m->ndof != s.n || s.n < MG_MIN_ROWS;
+  if (s.mg_off || (s.mg_plan && s.mg_serial == m->serial)) return;
+  if (s.mg_work) mg_work_free(s.mg_work);
+  if (s.mg_plan) mg_plan_free(s.mg_plan);
+  s.mg_work = nullptr;
+  s.mg_plan = nullptr;
+  s.mg_plan = build_plan(s, *m, order, st);
+  s.mg_serial = m->serial;
+  s.mass = true;  // the matrix is the caller's: look before using the grids
+}
+
 // Solves by multigrid CG when that suits the system; false when it is
 // Jacobi-PCG's.
 bool mg_solve(System &s, const double *b, double *x_out, const admfem_solve_opts &o,
               admfem_solve_stats &stats, hipStream_t st) {
-  if (!s.mesh || s.n < MG_MIN_ROWS) return false;
+  if (s.mg_off || s.n < MG_MIN_ROWS) return false;
   auto t0 = std::chrono::steady_clock::now();
   const MgPlan *plan = mg_plan(s, st);
   if (!plan) return false;

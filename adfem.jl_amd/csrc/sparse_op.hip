@@ -267,7 +267,7 @@ void build_pattern(CooPattern &p, const long long *ind, int64_t nnz, int n, int 
 
 // The kept pattern for these indices (rebuilt when they differ), with the
 // values summed into its solver format.  Caller holds g_lock.
-System &pattern_with_values(const long long *ind, const double *vv, int64_t nnz, int n,
+System &pattern_with_values(const Mesh *m, const long long *ind, const double *vv, int64_t nnz, int n,
                             hipStream_t st) {
   REQUIRE(n > 0 && nnz >= 0 && nnz < INT32_MAX, ADMFEM_ERR_ARG, "bad sizes");
   int dev = 0;
@@ -294,6 +294,8 @@ System &pattern_with_values(const long long *ind, const double *vv, int64_t nnz,
                                                p.reordered ? p.pos.p : nullptr, vv, p.s->val.p);
   HIPCHECK(hipGetLastError());
   launch_to_sell(*p.s, st);
+  p.s->a_version++;
+  mg_set_mesh(*p.s, m, p.reordered ? p.order.p : nullptr, st);
   return *p.s;
 }
 
@@ -309,11 +311,11 @@ void solve_kept(CooPattern &p, const double *b, double *x, const admfem_solve_op
 
 }  // namespace
 
-void sparse_solve(const long long *ind, const double *vv, int64_t nnz, int n, const double *rhs,
+void sparse_solve(const Mesh *m, const long long *ind, const double *vv, int64_t nnz, int n, const double *rhs,
                   double *u, const admfem_solve_opts &o, admfem_solve_stats &stats,
                   hipStream_t st) {
   std::lock_guard<std::mutex> g(g_lock);
-  pattern_with_values(ind, vv, nnz, n, st);
+  pattern_with_values(m, ind, vv, nnz, n, st);
   solve_kept(*g_kept, rhs, u, o, stats, st);
 }
 
@@ -325,12 +327,12 @@ void sparse_solve_info(int64_t info[4]) {
   info[3] = g_kept && g_kept->reordered ? 1 : 0;
 }
 
-void sparse_solve_grad(const long long *ind, const double *vv, int64_t nnz, int n,
+void sparse_solve_grad(const Mesh *m, const long long *ind, const double *vv, int64_t nnz, int n,
                        const double *u, const double *grad_u, double *grad_vv,
                        double *grad_rhs, const admfem_solve_opts &o, admfem_solve_stats &stats,
                        hipStream_t st) {
   std::lock_guard<std::mutex> g(g_lock);
-  pattern_with_values(ind, vv, nnz, n, st);
+  pattern_with_values(m, ind, vv, nnz, n, st);
   solve_kept(*g_kept, grad_u, grad_rhs, o, stats, st);  // lambda = A^-1 dL/du = dL/drhs
   if (nnz) coo_grad<<<nb(nnz, 256), 256, 0, st>>>(nnz, ind, grad_rhs, u, grad_vv);
   HIPCHECK(hipGetLastError());

@@ -382,6 +382,19 @@ int admfem_sparse_solve_grad(const long long *indices, const double *vv,
                              double *grad_rhs, const admfem_solve_opts *o,
                              admfem_solve_stats *st, void *stream);
 
+/* The same for a matrix whose rows are the dofs of mesh m (what the operators
+ * of section C return, before or after ImposeDirichlet): the node positions
+ * let the solver lay multigrid grids over the mesh instead of running plain
+ * Jacobi-PCG.  m NULL, or with another number of dofs than n: the functions
+ * above. */
+int admfem_sparse_solve_on(admfem_mesh m, const long long *indices, const double *vv, int64_t nnz,
+                           int n, const double *rhs, double *u, const admfem_solve_opts *o,
+                           admfem_solve_stats *st, void *stream);
+int admfem_sparse_solve_grad_on(admfem_mesh m, const long long *indices, const double *vv,
+                                int64_t nnz, int n, const double *u, const double *grad_u,
+                                double *grad_vv, double *grad_rhs, const admfem_solve_opts *o,
+                                admfem_solve_stats *st, void *stream);
+
 /* Instrumentation (no reference counterpart): the pattern the general
  * sparse solve keeps (the last one built on any device): info[0..3] = n,
  * triplets it was built from, distinct (row, col) slots, and 1 when the

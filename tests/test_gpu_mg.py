@@ -119,3 +119,38 @@ def test_multigrid_reports_matrices_it_cannot_solve():
     assert st["rel_residual"] <= 1e-12
     x1, _ = S.solve(rtol=1e-12, check_every=1)
     assert torch.equal(x0, x1)  # replayed graphs against single launches
+
+
+@pytest.mark.parametrize("degree,m", [(1, 70), (2, 36)])
+def test_operator_chain_with_grids_matches_oracle(degree, m):
+    """A \\ rhs for matrices the mesh's operators made (solved on grids laid
+    over the mesh), for the same matrix without its mesh, and for another
+    mesh's matrix of the same pattern afterwards (its own grids): u and the
+    gradients against the oracle's chain, tolerance as above."""
+    for seed in (1, 2):
+        c, e = meshgen.jittered_square(m, seed=7)
+        if seed == 2:  # same connectivity, other node positions
+            c = c * [1.0, 0.5]
+        om = O.OracleMesh(c, e) if degree == 1 else O.OracleMesh(c, e, degree=2)
+        gm = admfem.Mesh(c, e, degree=degree, zero_based=True)
+        rng = np.random.default_rng(seed)
+        kap, f = np.exp(0.5 * rng.standard_normal(om.ngauss)), rng.uniform(-1, 1, om.ngauss)
+        bd = om.bcnode()
+        bv = rng.standard_normal(bd.size)
+        w = rng.standard_normal(gm.ndof)
+        ref = O.forward_adjoint(om, kap, f, bd, bv, lambda u: w)
+        for with_mesh in (True, False):
+            k = torch.tensor(kap, device="cuda", requires_grad=True)
+            K = admfem.compute_fem_laplace_matrix1(k, gm)
+            F = admfem.compute_fem_source_term1(torch.tensor(f, device="cuda"), gm)
+            A, r = admfem.impose_Dirichlet_boundary_conditions(K, F, bd, bv)
+            assert A.mesh is gm and (2.0 * A).mesh is gm and (A + A).mesh is gm
+            if not with_mesh:
+                A = admfem.SparseTensor(A.indices, A.values, A.n)
+                assert A.mesh is None
+            u = admfem.solve(A, r, rtol=1e-13)
+            (u * torch.tensor(w, device="cuda")).sum().backward()
+            for a, b in ((u.detach(), ref["u"]), (k.grad, ref["grad_kappa"])):
+                d = np.linalg.norm(a.cpu().numpy() - b) / np.linalg.norm(b)
+                print(degree, m, seed, with_mesh, d, flush=True)
+                assert d < 1e-9
