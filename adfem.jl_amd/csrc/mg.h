@@ -8,7 +8,7 @@ namespace admfem {
 constexpr int MG_MAXLEV = 16;    // grid levels at most
 constexpr int MG_HALO = 2;       // zero nodes around a grid (the stencils reach 2)
 constexpr int MG_TAIL = 2048;    // padded nodes of the first level of the tail kernel
-constexpr int MG_DENSE = 64;     // nodes of the last level at most (dense inverse)
+constexpr int MG_DENSE = 49;     // nodes of the last level at most (dense inverse)
 
 // One grid level: nx x ny nodes stored with a halo of MG_HALO zero nodes on
 // every side (pitch px, pn entries in all), node (x, y) at mg_at.
@@ -21,6 +21,12 @@ struct MgLevel {
 };
 __host__ __device__ inline int mg_at(int px, int x, int y) {
   return (y + MG_HALO) * px + x + MG_HALO;
+}
+
+// a grid's nodes along a side on the next one; its padded size
+__host__ __device__ inline int mg_next(int n) { return n / 2 + 1; }
+__host__ __device__ inline int mg_pn(int nx, int ny) {
+  return ((nx + 2 * MG_HALO) * (ny + 2 * MG_HALO) + 63) / 64 * 64;
 }
 
 // One system: its matrix, the plan's arrays (shared by every system of the
@@ -36,22 +42,37 @@ struct MgSys {
   const int *cell;          // grid cell of each row (-1: not interpolated)
   const float2 *frac;       // position inside the cell
   const int *cptr, *crow;   // rows by cell
+  const float2 *cfrac;      // frac in that order
+  const int *pos;           // each row's place in it (-1: none)
   const double *b;          // right-hand side
   double *x, *r, *q, *p[2];
   float *z, *rs, *x0, *t;   // preconditioned residual, scaled residual,
-                            // smoothed correction, residual / corrected
-  double *part;             // 4 x nblk block partials
-  float *cinv;              // dense inverse of the last level
+                            // smoothed correction, corrected
+  float *ts;                // the restriction's input, in the cells' order
+  double *part4, *partz;    // 4 x nblk and nblk block partials
+  double *sum4, *sumz;      // their sums, when one block makes them
+  int gsum;                 // values the wide kernels sum: nblk, or 1
+  float *pack, *cinv;       // the tail's grids below its first, the dense
+                            // inverse of the last one behind them
   int n, npad, nblk;
   int nlev, tail;           // grid levels, first one of the tail kernel
   MgLevel lv[MG_MAXLEV];
 };
 
-struct MgScal {
-  double rtol2, bb, tol2, rr, rz, alpha, beta;
+// One system's solve: the state, in two copies (mk_dir reads a and writes b,
+// mk_update reads b and writes a, every other kernel reads a).
+struct MgState {
+  double rz, rr;
   int status;               // as in cg.hip: 0 run, 1 converged, 2 iterations
                             // spent, 3 NaN, 4 breakdown
-  int it, maxit, apply, first, nrepl;
+  int it, first;
+};
+struct MgScal {
+  double bb, tol2;
+  double rr_true, true_prev;  // |b - A x|^2 when CG last stopped, and before
+  int maxit, nrepl;
+  int checked;              // the final residual is known
+  MgState a, b;
 };
 
 // A topology's grids (made once per system, mg_plan).
@@ -59,9 +80,8 @@ struct MgPlan {
   bool ok = false;          // false: the rows do not suit one uniform grid
   int nlev = 0, tail = 0;
   int nx[MG_MAXLEV], ny[MG_MAXLEV], px[MG_MAXLEV], pn[MG_MAXLEV];
-  DevBuf<int> cell, cptr, crow;
-  DevBuf<float2> frac;
-  size_t bytes() const { return cell.bytes() + cptr.bytes() + crow.bytes() + frac.bytes(); }
+  DevBuf<int> cell, cptr, crow, pos;
+  DevBuf<float2> frac, cfrac;
 };
 
 // The system's plan (built on the first call); null when the solver should
@@ -70,6 +90,8 @@ const MgPlan *mg_plan(System &s, hipStream_t st);
 
 // Device floats of the grid levels of one system, and the level pointers of
 // a descriptor laid out from `base`.
+// (and the partials' pointers: nblk blocks, summed by one block or not)
+void mg_parts(MgSys &d, int nblk, bool reduce, double *part);
 size_t mg_grid_floats(const MgPlan &pl);
 void mg_grid_layout(const MgPlan &pl, float *base, MgSys &d);
 

@@ -28,17 +28,26 @@
 // A solve is converged when the residual recomputed from the FP64 matrix is.
 //
 // One iteration (every kernel returns at once when its system is done):
-//   mk_dir     p = z + beta p, q = A p; partials of p.q, r.q, q.q, r.r
-//   ms_alpha   alpha = r.z / p.q and the new |r|^2 = r.r - 2 alpha r.q +
-//              alpha^2 q.q
-//   mk_update  x += alpha p, r -= alpha q, first smoothing step from zero
-//   mk_res     residual of that, mk_restrict to the first grid (with its
-//              first smoothing step)
-//   gk_*       the grids down to MG_TAIL nodes: residual, restriction
-//   mk_tail    the remaining grids, one workgroup per system, in LDS
-//   gk_*       and up: prolongation, smoothing
-//   mk_prolong, mk_post  the fine level's; z, partials of r.z
-//   ms_beta    beta = r.z / previous r.z
+//   mk_res       residual of the first smoothing step (taken from zero where
+//                the residual itself is written)
+//   mk_restrict  to the first grid, with its first smoothing step
+//   gk_down      the grids down to MG_TAIL nodes: residual and restriction of
+//                a tile in one launch
+//   mk_tail      the remaining grids, one workgroup per system, in LDS
+//   gk_up        and up: prolongation and smoothing of a tile; the first grid
+//                also interpolates its rows
+//   mk_post      the fine level's second smoothing step: z, partials of r.z
+//   mk_dir       beta = r.z / previous r.z, p = z + beta p, q = A p; partials
+//                of p.q, r.q, q.q, r.r
+//   mk_update    alpha = r.z / p.q, the new |r|^2 = r.r - 2 alpha r.q +
+//                alpha^2 q.q, x += alpha p, r -= alpha q, first smoothing
+// When every grid fits the tail, mk_tail also restricts and interpolates: five
+// launches an iteration.  The scalars need no launch of their own: every
+// block of mk_dir and mk_update sums the partials itself, in one order, and
+// block 0 keeps the result for the next kernel (two copies of the state, each
+// kernel reading one and writing the other).  Above MG_SUM partials one
+// block sums them first (ms_reduce): 1,032 blocks reading 1,032 x 4 partials
+// cost less than a launch, 4,104 blocks reading 4,104 would not.
 // No atomics, no fences; every reduction has one order.
 #include <hipcub/hipcub.hpp>
 
@@ -60,6 +69,8 @@ constexpr int ST_RUN = 0, ST_CONV = 1, ST_MAXIT = 2, ST_NAN = 3, ST_BREAK = 4;
 // Smoothing weight: any value below 2 is safe; 1.6 took the fewest
 // iterations over jittered meshes (15 with 4/3, 13 - 14 with 1.5 - 1.7).
 constexpr float OM = 1.6f;
+// Partials that the wide kernels' blocks sum themselves, at most.
+constexpr int MG_SUM = 1280;
 
 inline unsigned nb(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 
@@ -71,8 +82,8 @@ __device__ __forceinline__ int2 where(const int2 *map, int sys) {
 }
 
 typedef float f2_t __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ gptr<f2_t> frac_ptr(const MgSys &d) {
-  return (gptr<f2_t>)reinterpret_cast<const f2_t *>(d.frac);
+__device__ __forceinline__ gptr<f2_t> frac_ptr(const float2 *p) {
+  return (gptr<f2_t>)reinterpret_cast<const f2_t *>(p);
 }
 
 template <int NV>
@@ -91,6 +102,51 @@ __device__ __forceinline__ void put_partials(const double (&v)[NV], double *part
 #pragma unroll
     for (int k = 0; k < NT / 64; k++) t += sh[threadIdx.x][k];
     global_mut(part)[(size_t)threadIdx.x * G + lb] = t;
+  }
+}
+
+// A wide kernel's block's sums of NV arrays of G values (the same in every
+// block); G = 1: already summed.
+template <int NV>
+__device__ __forceinline__ void sum_small(const double *v_, int G, double (&out)[NV]) {
+  const gptr<double> v = global_ptr(v_);
+  if (G == 1) {
+#pragma unroll
+    for (int j = 0; j < NV; j++) out[j] = v[j];
+    return;
+  }
+  __shared__ double sh[NV][NT / 64];
+  double a[NV];
+#pragma unroll
+  for (int j = 0; j < NV; j++) a[j] = 0.0;
+  int k = threadIdx.x;
+  for (; k + 3 * NT < G; k += 4 * NT) {
+    double t[NV][4];
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+#pragma unroll
+      for (int j = 0; j < NV; j++) t[j][u] = v[(size_t)j * G + k + u * NT];
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+#pragma unroll
+      for (int j = 0; j < NV; j++) a[j] += t[j][u];
+  }
+  for (; k < G; k += NT)
+#pragma unroll
+    for (int j = 0; j < NV; j++) a[j] += v[(size_t)j * G + k];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+#pragma unroll
+  for (int j = 0; j < NV; j++) {
+    const double t = wave_sum(a[j]);
+    if (lane == 0) sh[j][wv] = t;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < NV; j++) {
+    double t = 0.0;
+#pragma unroll
+    for (int w = 0; w < NT / 64; w++) t += sh[j][w];
+    out[j] = t;
   }
 }
 
@@ -163,9 +219,11 @@ __global__ void __launch_bounds__(NT)
   global_mut(d.minv)[i] = aii > 0.0 ? (float)(1.0 / sum) : 0.0f;
 }
 
-// The first grid's matrix P^T A P: one thread per grid node, gathering from
-// the rows of its four cells; the 25 sums of a thread live in LDS (they are
-// addressed by the columns' cells).
+// The first grid's matrix P^T A P: four threads per grid node, one for each
+// of its cells, gathering from the cell's rows; a thread's 25 sums live in
+// LDS (they are addressed by the columns' cells).  Bound by the latency of
+// the row -> column -> cell loads: with one thread per node it took 88 us for
+// 4,356 nodes (P1 128^2) and 473 us for 1,000 (P2 40^2).
 constexpr int GT = 128;
 __global__ void __launch_bounds__(GT)
     mk_galerkin(const int2 *__restrict__ map, const MgSys *__restrict__ D, int sys) {
@@ -174,31 +232,33 @@ __global__ void __launch_bounds__(GT)
   if (mb.x < 0) return;
   const MgSys &d = D[mb.x];
   const MgLevel &l = d.lv[0];
-  const int id = mb.y * GT + threadIdx.x, tid = threadIdx.x;
-  if (id >= l.nx * l.ny) return;
+  const int tid = threadIdx.x, id = mb.y * (GT / 4) + (tid >> 2), nn = l.nx * l.ny;
   const int X = id % l.nx, Y = id / l.nx, ncx = l.nx - 1, ncy = l.ny - 1;
 #pragma unroll
   for (int o = 0; o < 25; o++) acc[o][tid] = 0.0;
-  const gptr<int> cptr = global_ptr(d.cptr), crow = global_ptr(d.crow), cell = global_ptr(d.cell);
-  const gptr<int> sc = global_ptr(d.sc), sp = global_ptr(d.sp);
-  const gptr<double> sv = global_ptr(d.sv64), dg = global_ptr(d.diag);
-  const gptr<f2_t> frac = frac_ptr(d);
-  for (int cy = max(Y - 1, 0); cy <= min(Y, ncy - 1); cy++) {
-    const int c0 = cy * ncx + max(X - 1, 0), c1 = cy * ncx + min(X, ncx - 1);
-    for (int k = cptr[c0]; k < cptr[c1 + 1]; k++) {
-      const int i = crow[k], ci = cell[i];
+  const int cx = X - (tid & 1), cy = Y - ((tid >> 1) & 1);
+  if (id < nn && cx >= 0 && cx < ncx && cy >= 0 && cy < ncy) {
+    const gptr<int> cptr = global_ptr(d.cptr), crow = global_ptr(d.crow),
+                    cell = global_ptr(d.cell);
+    const gptr<int> sc = global_ptr(d.sc), sp = global_ptr(d.sp);
+    const gptr<double> sv = global_ptr(d.sv64), dg = global_ptr(d.diag);
+    const gptr<f2_t> frac = frac_ptr(d.frac);
+    const int c = cy * ncx + cx, k1 = cptr[c + 1];
+    for (int k = cptr[c]; k < k1; k++) {
+      const int i = crow[k];
       const f2_t f = frac[i];
-      const double wi = (double)(ci - cy * ncx == X ? 1.0f - f.x : f.x) *
-                        (double)(cy == Y ? 1.0f - f.y : f.y);
+      const double wi =
+          (double)(cx == X ? 1.0f - f.x : f.x) * (double)(cy == Y ? 1.0f - f.y : f.y);
       const int s0 = sp[i >> 6], w = (sp[(i >> 6) + 1] - s0) >> 6, off = s0 + (i & 63);
+#pragma unroll 4
       for (int e = -1; e < w; e++) {
         const int j = e < 0 ? i : sc[off + 64 * e];
         const double v = wi * (e < 0 ? dg[i] : sv[off + 64 * e]);
         const int cj = cell[j];
-        if (cj < 0) continue;
         const f2_t g = frac[j];
-        const int ox = cj % ncx - X + 2, oy = cj / ncx - Y + 2;
-        if (ox < 0 || ox > 3 || oy < 0 || oy > 3) continue;  // (the plan excludes these)
+        const int jy = cj / ncx, ox = cj - jy * ncx - X + 2, oy = jy - Y + 2;
+        // (cj < 0: no part; the plan excludes cells further off)
+        if (cj < 0 || ox < 0 || ox > 3 || oy < 0 || oy > 3) continue;
         acc[oy * 5 + ox][tid] += v * ((1.0 - g.x) * (1.0 - g.y));
         acc[oy * 5 + ox + 1][tid] += v * ((double)g.x * (1.0 - g.y));
         acc[oy * 5 + ox + 5][tid] += v * ((1.0 - g.x) * (double)g.y);
@@ -206,9 +266,13 @@ __global__ void __launch_bounds__(GT)
       }
     }
   }
-  const int at = mg_at(l.px, X, Y);
-#pragma unroll
-  for (int o = 0; o < 25; o++) global_mut(l.a)[(size_t)o * l.pn + at] = (float)acc[o][tid];
+  __syncthreads();
+  for (int t = tid; t < 25 * (GT / 4); t += GT) {
+    const int o = t / (GT / 4), q = t % (GT / 4), node = mb.y * (GT / 4) + q;
+    if (node < nn)
+      global_mut(l.a)[(size_t)o * l.pn + mg_at(l.px, node % l.nx, node / l.nx)] =
+          (float)((acc[o][4 * q] + acc[o][4 * q + 1]) + (acc[o][4 * q + 2] + acc[o][4 * q + 3]));
+  }
 }
 
 // One node's entries of the next grid's matrix: P^T A P with the bilinear
@@ -256,33 +320,28 @@ __device__ __forceinline__ void coarse_node(const MgLevel &f, const MgLevel &c, 
 __device__ __forceinline__ void weight_node(const MgLevel &l, int x, int y) {
   const gptr<float> a = global_ptr(l.a);
   const int at = mg_at(l.px, x, y);
-  const float aii = a[(size_t)12 * l.pn + at];
-  double s = 0.0;
+  float v[25], ajj[25];
 #pragma unroll
   for (int o = 0; o < 25; o++) {
-    const float v = a[(size_t)o * l.pn + at];
-    const float ajj = a[(size_t)12 * l.pn + at + (o / 5 - 2) * l.px + o % 5 - 2];
-    if (ajj > 0.0f) s += fabs((double)v) / sqrt((double)ajj);
+    v[o] = a[(size_t)o * l.pn + at];
+    ajj[o] = a[(size_t)12 * l.pn + at + (o / 5 - 2) * l.px + o % 5 - 2];
   }
-  global_mut(l.minv)[at] = aii > 1e-30f ? (float)(1.0 / (sqrt((double)aii) * s)) : 0.0f;
+  float s = 0.0f;
+#pragma unroll
+  for (int o = 0; o < 25; o++)
+    if (ajj[o] > 1e-30f) s += fabsf(v[o]) * rsqrtf(ajj[o]);
+  global_mut(l.minv)[at] = ajj[12] > 1e-30f ? rsqrtf(ajj[12]) / s : 0.0f;
 }
 
+// Grid k's weights and the matrix of grid k + 1.
 __global__ void __launch_bounds__(GT)
-    gk_galerkin(const int2 *__restrict__ map, const MgSys *__restrict__ D, int sys, int k) {
+    gk_setup(const int2 *__restrict__ map, const MgSys *__restrict__ D, int sys, int k) {
   const int2 mb = where(map, sys);
   if (mb.x < 0) return;
-  const MgLevel &f = D[mb.x].lv[k - 1], &c = D[mb.x].lv[k];
+  const MgLevel &f = D[mb.x].lv[k], &c = D[mb.x].lv[k + 1];
   const int id = mb.y * GT + threadIdx.x;
+  if (id < f.nx * f.ny) weight_node(f, id % f.nx, id / f.nx);
   if (id < c.nx * c.ny) coarse_node(f, c, id % c.nx, id / c.nx);
-}
-
-__global__ void __launch_bounds__(GT)
-    gk_weights(const int2 *__restrict__ map, const MgSys *__restrict__ D, int sys, int k) {
-  const int2 mb = where(map, sys);
-  if (mb.x < 0) return;
-  const MgLevel &l = D[mb.x].lv[k];
-  const int id = mb.y * GT + threadIdx.x;
-  if (id < l.nx * l.ny) weight_node(l, id % l.nx, id / l.nx);
 }
 
 // The tail's grids (from d.tail on, whose matrix is there) and the dense
@@ -305,7 +364,24 @@ __global__ void __launch_bounds__(ST)
     for (int id = threadIdx.x; id < nn; id += ST) weight_node(l, id % l.nx, id / l.nx);
     __syncthreads();
   }
-  __shared__ double A[MG_DENSE][MG_DENSE + 1], sc[MG_DENSE], col[MG_DENSE];
+  // entries and weights of the grids below the first, node by node, as mk_tail
+  // keeps them in LDS
+  {
+    float *pk = d.pack;
+    for (int k = d.tail + 1; k < d.nlev; k++) {
+      const MgLevel &l = d.lv[k];
+      const int nn = l.nx * l.ny;
+      for (int id = threadIdx.x; id < nn; id += ST) {
+        const int at = mg_at(l.px, id % l.nx, id / l.nx);
+#pragma unroll
+        for (int o = 0; o < 25; o++)
+          global_mut(pk)[o * nn + id] = global_ptr(l.a)[(size_t)o * l.pn + at];
+        global_mut(pk)[25 * nn + id] = OM * global_ptr(l.minv)[at];
+      }
+      pk += 26 * nn;
+    }
+  }
+  __shared__ double A[2][MG_DENSE][MG_DENSE + 1], sc[MG_DENSE];
   const MgLevel &l = d.lv[d.nlev - 1];
   const int nn = l.nx * l.ny;
   const gptr<float> a = global_ptr(l.a);
@@ -320,35 +396,26 @@ __global__ void __launch_bounds__(ST)
     double v = 0.0;
     if (abs(dx) <= 2 && abs(dy) <= 2)
       v = (double)a[(size_t)((dy + 2) * 5 + dx + 2) * l.pn + mg_at(l.px, i % l.nx, i / l.nx)];
-    A[i][j] = v * sc[i] * sc[j];
+    A[0][i][j] = v * sc[i] * sc[j];
   }
   __syncthreads();
-  for (int k = 0; k < nn; k++) {
-    const double pv = A[k][k];
-    const bool skip = !(pv > 1e-9);
-    for (int i = threadIdx.x; i < nn; i += ST) col[i] = A[i][k];
-    __syncthreads();
-    if (skip) {  // the variable leaves the system: zero row and column
-      for (int t = threadIdx.x; t < nn; t += ST) {
-        A[t][k] = 0.0;
-        A[k][t] = 0.0;
+  const int gi = threadIdx.x >> 6, gj = threadIdx.x & 63;
+  for (int k = 0; k < nn; k++) {  // step k reads one copy and writes the other
+    const double(*P)[MG_DENSE + 1] = A[k & 1];
+    double(*Q)[MG_DENSE + 1] = A[(k & 1) ^ 1];
+    const double pv = P[k][k];
+    const bool keep = pv > 1e-9;  // else the variable leaves the system
+    const double ip = keep ? 1.0 / pv : 0.0;
+    if (gj < nn)
+      for (int i = gi; i < nn; i += ST / 64) {
+        const double pij = P[i][gj], pik = P[i][k], pkj = P[k][gj] * ip;
+        Q[i][gj] = i == k ? (gj == k ? ip : pkj) : gj == k ? -pik * ip : pij - pik * pkj;
       }
-    } else {
-      for (int t = threadIdx.x; t < nn; t += ST)
-        if (t != k) A[k][t] /= pv;
-      __syncthreads();
-      for (int t = threadIdx.x; t < nn * nn; t += ST) {
-        const int i = t / nn, j = t % nn;
-        if (i != k && j != k) A[i][j] -= col[i] * A[k][j];
-      }
-      __syncthreads();
-      for (int t = threadIdx.x; t < nn; t += ST) A[t][k] = t == k ? 1.0 / pv : -col[t] / pv;
-    }
     __syncthreads();
   }
   for (int t = threadIdx.x; t < nn * nn; t += ST) {
     const int i = t / nn, j = t % nn;
-    global_mut(d.cinv)[t] = (float)(A[i][j] * sc[i] * sc[j]);
+    global_mut(d.cinv)[t] = (float)(A[nn & 1][i][j] * sc[i] * sc[j]);
   }
 }
 
@@ -413,9 +480,8 @@ __device__ __forceinline__ double dot32(const MgSys &d, int i, L load) {
 }
 
 // Start: x = b on identity rows and 0 elsewhere, r = b - A x (0 on those
-// rows, b on the rest), p = 0.  Restart (FRESH false): r = b - A x of the
-// current x.  Partials of r.r and b.b.  (b_ null: the descriptor's b.)
-template <bool FRESH>
+// rows, b on the rest), p = 0; partials of r.r and b.b.  (b_ null: the
+// descriptor's b.)
 __global__ void __launch_bounds__(NT)
     mk_start(const int2 *__restrict__ map, const MgSys *__restrict__ D, int sys,
              const double *b_) {
@@ -426,66 +492,135 @@ __global__ void __launch_bounds__(NT)
   double t[2] = {0.0, 0.0};
   if (i < d.npad) {
     const double bi = i < d.n ? global_ptr(b_ ? b_ : d.b)[i] : 0.0;
-    double ri;
-    if (FRESH) {
-      const bool ident = i >= d.n || global_ptr(d.row_bd)[i] >= 0;
-      ri = ident ? 0.0 : bi;
-      global_mut(d.x)[i] = (ident && i < d.n) ? bi : 0.0;
-      global_mut(d.p[0])[i] = 0.0;
-      global_mut(d.p[1])[i] = 0.0;
-    } else {
-      const gptr<double> x = global_ptr(d.x);
-      const double ax = global_ptr(d.diag)[i] * x[i] +
-                        sell_dot<double>(i, d.sp, d.sc, d.sv64, [&](int c) { return x[c]; });
-      ri = bi - ax;
-    }
+    const bool ident = i >= d.n || global_ptr(d.row_bd)[i] >= 0;
+    const double ri = ident ? 0.0 : bi;
+    global_mut(d.x)[i] = (ident && i < d.n) ? bi : 0.0;
+    global_mut(d.p[0])[i] = 0.0;
+    global_mut(d.p[1])[i] = 0.0;
+    // never written for a row outside the grids, but read (times zero) through
+    // its padding entries
+    if (global_ptr(d.pos)[i] < 0) global_mut(d.t)[i] = 0.0f;
     global_mut(d.r)[i] = ri;
     first_smooth(d, i, ri);
     t[0] = ri * ri;
     t[1] = bi * bi;
   }
-  put_partials<2>(t, d.part, d.nblk, m.y);
+  put_partials<2>(t, d.part4, d.nblk, m.y);
 }
 
 __global__ void __launch_bounds__(RT)
-    ms_start(const MgSys *__restrict__ D, MgScal *S_, int sys, int fresh, double rtol2,
-             int maxit) {
+    ms_start(const MgSys *__restrict__ D, MgScal *S_, int sys, double rtol2, int maxit) {
   const MgSys &d = D[sys];
   MgScal *S = S_ + sys;
   double t[2];
-  sum_partials<2>(d.part, d.nblk, t);
+  sum_partials<2>(d.part4, d.nblk, t);
   if (threadIdx.x != 0) return;
-  if (fresh) {
-    S->rtol2 = rtol2;
-    S->bb = t[1];
-    S->tol2 = rtol2 * t[1];
-    S->it = 0;
-    S->maxit = maxit;
-    S->nrepl = 0;
-  } else {
-    S->nrepl += 1;
+  MgScal s{};
+  s.bb = t[1];
+  s.tol2 = rtol2 * t[1];
+  s.maxit = maxit;
+  s.true_prev = -1.0;
+  s.a.rr = t[0];
+  s.a.first = 1;
+  s.a.status = (!(t[0] == t[0]) || !isfinite(t[0])) ? ST_NAN
+               : t[0] <= s.tol2                     ? ST_CONV
+                                                    : ST_RUN;
+  *S = s;
+}
+
+// The residual recomputed from the FP64 matrix once CG has stopped, in the
+// form a restart continues from; partials of r.r.
+__global__ void __launch_bounds__(NT)
+    mk_check(const int2 *__restrict__ map, const MgSys *__restrict__ D, const MgScal *S, int sys,
+             const double *b_) {
+  const int2 m = where(map, sys);
+  if (m.x < 0 || S[m.x].a.status == ST_RUN || S[m.x].checked) return;
+  const MgSys &d = D[m.x];
+  const int i = m.y * NT + threadIdx.x;
+  double t[1] = {0.0};
+  if (i < d.npad) {
+    const gptr<double> x = global_ptr(d.x);
+    const double bi = i < d.n ? global_ptr(b_ ? b_ : d.b)[i] : 0.0;
+    const double ax = global_ptr(d.diag)[i] * x[i] +
+                      sell_dot<double>(i, d.sp, d.sc, d.sv64, [&](int c) { return x[c]; });
+    const double ri = bi - ax;
+    global_mut(d.r)[i] = ri;
+    first_smooth(d, i, ri);
+    t[0] = ri * ri;
   }
-  S->rr = t[0];
-  S->rz = 0.0;
-  S->alpha = S->beta = 0.0;
-  S->first = 1;
-  S->apply = 0;
-  S->status = (!(t[0] == t[0]) || !isfinite(t[0])) ? ST_NAN
-              : t[0] <= S->tol2                    ? ST_CONV
-              : S->it >= S->maxit                  ? ST_MAXIT
-                                                   : ST_RUN;
+  put_partials<1>(t, d.part4, d.nblk, m.y);
+}
+
+// The recursive residual decides only when the true one agrees; otherwise CG
+// restarts from the true one, until that no longer helps.  host: a pinned
+// copy of the state for the host (null: none).
+__global__ void __launch_bounds__(RT)
+    ms_check(const MgSys *__restrict__ D, MgScal *S_, const int *__restrict__ list, int sys,
+             MgScal *host) {
+  if (list) sys = list[blockIdx.x];
+  if (sys < 0) return;
+  MgScal *S = S_ + sys;
+  if (S->a.status != ST_RUN && !S->checked) {  // (uniform: written at the end only)
+    double t[1];
+    sum_partials<1>(D[sys].part4, D[sys].nblk, t);
+    if (threadIdx.x == 0) {
+      const double rr = t[0];
+      S->rr_true = rr;
+      if (S->a.status == ST_CONV && !(rr <= S->tol2) && S->a.it < S->maxit && S->nrepl < 8 &&
+          rr == rr && !(S->true_prev >= 0.0 && !(rr < 0.25 * S->true_prev))) {
+        S->true_prev = rr;
+        S->nrepl += 1;
+        S->a.rr = rr;
+        S->a.first = 1;
+        S->a.status = ST_RUN;
+      } else {
+        if (S->a.status == ST_CONV && rr != rr) S->a.status = ST_NAN;
+        S->checked = 1;
+      }
+    }
+  }
+  if (host && threadIdx.x == 0) host[sys] = *S;
+}
+
+// sum_small's input for systems with many partials: one block's sums.
+template <int NV>
+__global__ void __launch_bounds__(RT)
+    ms_reduce(const MgSys *__restrict__ D, const MgScal *S, const int *__restrict__ list,
+              int sys) {
+  if (list) sys = list[blockIdx.x];
+  if (sys < 0) return;
+  const MgSys &d = D[sys];
+  if (d.gsum == d.nblk || (NV == 1 ? S[sys].a : S[sys].b).status != ST_RUN) return;
+  double t[NV];
+  sum_partials<NV>(NV == 1 ? d.partz : d.part4, d.nblk, t);
+  if (threadIdx.x == 0)
+#pragma unroll
+    for (int j = 0; j < NV; j++) global_mut(NV == 1 ? d.sumz : d.sum4)[j] = t[j];
 }
 
 // p = z + beta p (into the other buffer), q = A p; partials of p.q, r.q,
 // q.q, r.r.  A neighbour's p is formed on the fly by the same fused
 // multiply-add as its own row forms it.
 __global__ void __launch_bounds__(NT)
-    mk_dir(const int2 *__restrict__ map, const MgSys *__restrict__ D, const MgScal *S, int sys) {
+    mk_dir(const int2 *__restrict__ map, const MgSys *__restrict__ D, MgScal *S_, int sys) {
   const int2 m = where(map, sys);
-  if (m.x < 0 || S[m.x].status != ST_RUN) return;
+  if (m.x < 0) return;
   const MgSys &d = D[m.x];
-  const double beta = S[m.x].beta;
-  const bool odd = S[m.x].it & 1;
+  MgScal *S = S_ + m.x;
+  const bool lead = m.y == 0 && threadIdx.x == 0;
+  MgState st = S->a;
+  if (st.status != ST_RUN) {
+    if (lead) S->b.status = st.status;
+    return;
+  }
+  double rz[1];
+  sum_small<1>(d.gsum == d.nblk ? d.partz : d.sumz, d.gsum, rz);
+  st.status = rz[0] != rz[0] || !isfinite(rz[0]) ? ST_NAN : !(rz[0] > 0.0) ? ST_BREAK : ST_RUN;
+  const double beta = st.first ? 0.0 : rz[0] / st.rz;
+  st.rz = rz[0];
+  if (lead) S->b = st;
+  if (st.status != ST_RUN) return;
+  const bool odd = st.it & 1;
   const gptr<double> p = global_ptr(d.p[odd]);
   const gptr<float> z = global_ptr(d.z);
   const int i = m.y * NT + threadIdx.x;
@@ -495,7 +630,8 @@ __global__ void __launch_bounds__(NT)
     auto load = [&](int c) { return zp{z[c], p[c]}; };
     auto comb = [&](zp v) { return fma(beta, v.p, (double)v.z); };
     const double pi = comb(load(i)), ri = global_ptr(d.r)[i];
-    const double qi = global_ptr(d.diag)[i] * pi + sell_dot<double>(i, d.sp, d.sc, d.sv64, load, comb);
+    const double qi =
+        global_ptr(d.diag)[i] * pi + sell_dot<double>(i, d.sp, d.sc, d.sv64, load, comb);
     global_mut(d.p[!odd])[i] = pi;
     global_mut(d.q)[i] = qi;
     t[0] = pi * qi;
@@ -503,49 +639,40 @@ __global__ void __launch_bounds__(NT)
     t[2] = qi * qi;
     t[3] = ri * ri;
   }
-  put_partials<4>(t, d.part, d.nblk, m.y);
+  put_partials<4>(t, d.part4, d.nblk, m.y);
 }
 
-__global__ void __launch_bounds__(RT)
-    ms_alpha(const MgSys *__restrict__ D, MgScal *S_, const int *__restrict__ list, int sys) {
-  if (list) sys = list[blockIdx.x];
-  MgScal *S = S_ + sys;
-  if (S->status != ST_RUN) {
-    if (threadIdx.x == 0) S->apply = 0;
+// x += alpha p, r -= alpha q (p: the buffer mk_dir wrote), first smoothing
+// step of the next V-cycle
+__global__ void __launch_bounds__(NT)
+    mk_update(const int2 *__restrict__ map, const MgSys *__restrict__ D, MgScal *S_, int sys) {
+  const int2 m = where(map, sys);
+  if (m.x < 0) return;
+  const MgSys &d = D[m.x];
+  MgScal *S = S_ + m.x;
+  const bool lead = m.y == 0 && threadIdx.x == 0;
+  MgState st = S->b;
+  if (st.status != ST_RUN) {
+    if (lead) S->a.status = st.status;
     return;
   }
   double t[4];
-  sum_partials<4>(D[sys].part, D[sys].nblk, t);
-  if (threadIdx.x != 0) return;
+  sum_small<4>(d.gsum == d.nblk ? d.part4 : d.sum4, d.gsum, t);
   const double pq = t[0];
-  S->apply = 0;
-  S->it += 1;
-  if (pq != pq || !isfinite(pq)) {
-    S->status = ST_NAN;
-  } else if (!(pq > 0.0)) {
-    S->status = ST_BREAK;  // not SPD
-  } else {
-    const double alpha = S->rz / pq;
-    S->alpha = alpha;
-    S->rr = fmax(t[3] - 2.0 * alpha * t[1] + alpha * alpha * t[2], 0.0);
-    S->apply = 1;
-    if (S->rr <= S->tol2) S->status = ST_CONV;
-    else if (S->it >= S->maxit) S->status = ST_MAXIT;
-  }
-}
-
-// x += alpha p, r -= alpha q, first smoothing step (p: the buffer mk_dir
-// wrote, after ms_alpha has counted the step)
-__global__ void __launch_bounds__(NT)
-    mk_update(const int2 *__restrict__ map, const MgSys *__restrict__ D, const MgScal *S,
-              int sys) {
-  const int2 m = where(map, sys);
-  if (m.x < 0 || !S[m.x].apply) return;
-  const MgSys &d = D[m.x];
-  const double alpha = S[m.x].alpha;
+  const bool ok = pq > 0.0 && isfinite(pq);  // else NaN, or not SPD
+  const double alpha = ok ? st.rz / pq : 0.0;
+  st.it += 1;
+  st.first = 0;
+  st.rr = ok ? fmax(t[3] - 2.0 * alpha * t[1] + alpha * alpha * t[2], 0.0) : st.rr;
+  st.status = pq != pq || isinf(pq) ? ST_NAN
+              : !ok                 ? ST_BREAK
+              : st.rr <= S->tol2    ? ST_CONV
+              : st.it >= S->maxit   ? ST_MAXIT
+                                    : ST_RUN;
+  if (lead) S->a = st;
   const int i = m.y * NT + threadIdx.x;
-  if (i >= d.npad) return;
-  const double pi = global_ptr(d.p[S[m.x].it & 1])[i];
+  if (!ok || i >= d.npad) return;
+  const double pi = global_ptr(d.p[st.it & 1])[i];
   const double xi = fma(alpha, pi, global_ptr(d.x)[i]);
   const double ri = fma(-alpha, global_ptr(d.q)[i], global_ptr(d.r)[i]);
   global_mut(d.x)[i] = xi;
@@ -553,103 +680,163 @@ __global__ void __launch_bounds__(NT)
   first_smooth(d, i, ri);
 }
 
-// t = the fine residual after the first smoothing step, in the unscaled
-// form's dual times the interpolation's weight: sqrt(a_ii) (rs - Â x0)
+// ts = the fine residual after the first smoothing step, in the unscaled
+// form's dual, sqrt(a_ii) (rs - Â x0), in the order of the cells
 __global__ void __launch_bounds__(NT)
     mk_res(const int2 *__restrict__ map, const MgSys *__restrict__ D, const MgScal *S, int sys) {
   const int2 m = where(map, sys);
-  if (m.x < 0 || S[m.x].status != ST_RUN) return;
+  if (m.x < 0 || S[m.x].a.status != ST_RUN) return;
   const MgSys &d = D[m.x];
   const int i = m.y * NT + threadIdx.x;
   if (i >= d.npad) return;
   const gptr<float> x0 = global_ptr(d.x0);
   const double res = (double)global_ptr(d.rs)[i] - (double)x0[i] -
                      dot32(d, i, [&](int c) { return x0[c]; });
-  global_mut(d.t)[i] = (float)(res * (double)global_ptr(d.sq)[i]);
+  const int k = global_ptr(d.pos)[i];
+  if (k >= 0) global_mut(d.ts)[k] = (float)(res * (double)global_ptr(d.sq)[i]);
 }
 
-// First grid: b = P^T t and the first smoothing step from zero.
+// One cell's share of node (X, Y) of the first grid in P^T t: the sum over
+// the rows of cell (X - (q & 1), Y - (q >> 1)).
+__device__ __forceinline__ double restrict_cell(const MgSys &d, const MgLevel &l, int X, int Y,
+                                                int q) {
+  const int ncx = l.nx - 1, ncy = l.ny - 1, cx = X - (q & 1), cy = Y - (q >> 1);
+  if (cx < 0 || cx >= ncx || cy < 0 || cy >= ncy) return 0.0;
+  const gptr<int> cptr = global_ptr(d.cptr);
+  const gptr<f2_t> cfrac = frac_ptr(d.cfrac);
+  const gptr<float> t = global_ptr(d.ts);
+  const int c = cy * ncx + cx, k1 = cptr[c + 1];
+  double s = 0.0;
+  int k = cptr[c];
+  for (; k + 3 < k1; k += 4) {  // four rows' loads in flight
+    f2_t f[4];
+    float v[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      f[u] = cfrac[k + u];
+      v[u] = t[k + u];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+      s += (double)((q & 1 ? f[u].x : 1.0f - f[u].x) * (q >> 1 ? f[u].y : 1.0f - f[u].y)) *
+           (double)v[u];
+  }
+  for (; k < k1; k++) {
+    const f2_t f = cfrac[k];
+    s += (double)((q & 1 ? f.x : 1.0f - f.x) * (q >> 1 ? f.y : 1.0f - f.y)) * (double)t[k];
+  }
+  return s;
+}
+
+// A cell's shares of its four corners' P^T t.
+__device__ __forceinline__ void cell_shares(const MgSys &d, int c, float (&out)[4]) {
+  const gptr<f2_t> cfrac = frac_ptr(d.cfrac);
+  const gptr<float> t = global_ptr(d.ts);
+  const int k0 = global_ptr(d.cptr)[c], k1 = global_ptr(d.cptr)[c + 1];
+  double s[4] = {0.0, 0.0, 0.0, 0.0};
+  for (int k = k0; k < k1; k += 4) {  // four rows' loads in flight
+    f2_t f[4];
+    float v[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const int j = min(k + u, k1 - 1);
+      f[u] = cfrac[j];
+      v[u] = k + u < k1 ? t[j] : 0.0f;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      s[0] += (double)((1.0f - f[u].x) * (1.0f - f[u].y)) * (double)v[u];
+      s[1] += (double)(f[u].x * (1.0f - f[u].y)) * (double)v[u];
+      s[2] += (double)((1.0f - f[u].x) * f[u].y) * (double)v[u];
+      s[3] += (double)(f[u].x * f[u].y) * (double)v[u];
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < 4; q++) out[q] = (float)s[q];
+}
+
+// First grid: b = P^T t and the first smoothing step from zero; four threads
+// a node, one for each of its cells.
 __global__ void __launch_bounds__(NT)
     mk_restrict(const int2 *__restrict__ map, const MgSys *__restrict__ D, const MgScal *S,
                 int sys) {
   const int2 m = where(map, sys);
-  if (m.x < 0 || S[m.x].status != ST_RUN) return;
+  if (m.x < 0 || S[m.x].a.status != ST_RUN) return;
   const MgSys &d = D[m.x];
   const MgLevel &l = d.lv[0];
-  const int id = m.y * NT + threadIdx.x;
-  if (id >= l.nx * l.ny) return;
-  const int X = id % l.nx, Y = id / l.nx, ncx = l.nx - 1, ncy = l.ny - 1;
-  const gptr<int> cptr = global_ptr(d.cptr), crow = global_ptr(d.crow), cell = global_ptr(d.cell);
-  const gptr<float> t = global_ptr(d.t);
-  const gptr<f2_t> frac = frac_ptr(d);
-  double s = 0.0;
-  for (int cy = max(Y - 1, 0); cy <= min(Y, ncy - 1); cy++) {
-    const int c0 = cy * ncx + max(X - 1, 0), c1 = cy * ncx + min(X, ncx - 1);
-    const int k1 = cptr[c1 + 1];
-    for (int k = cptr[c0]; k < k1; k++) {
-      const int i = crow[k];
-      const f2_t f = frac[i];
-      s += (double)((cell[i] - cy * ncx == X ? 1.0f - f.x : f.x) *
-                    (cy == Y ? 1.0f - f.y : f.y)) * (double)t[i];
-    }
-  }
+  const int id = m.y * (NT / 4) + (threadIdx.x >> 2);
+  const bool in = id < l.nx * l.ny;
+  const int X = id % l.nx, Y = id / l.nx;
+  double s = in ? restrict_cell(d, l, X, Y, threadIdx.x & 3) : 0.0;
+  s += __shfl_xor(s, 1, 64);
+  s += __shfl_xor(s, 2, 64);
+  if (!in || (threadIdx.x & 3)) return;
   const int at = mg_at(l.px, X, Y);
   global_mut(l.b)[at] = (float)s;
   global_mut(l.x)[at] = OM * global_ptr(l.minv)[at] * (float)s;
 }
 
-// A grid node's product with its stencil, v read through `at`.
+// A grid node's product with its stencil; v: the node's value, pv its pitch.
 template <class V>
-__device__ __forceinline__ double stencil(const MgLevel &l, int at, V v) {
+__device__ __forceinline__ double stencil(const MgLevel &l, int at, V v, int pv) {
   const gptr<float> a = global_ptr(l.a);
-  float c[25], x[25];
+  float c[25];
 #pragma unroll
-  for (int o = 0; o < 25; o++) {
-    c[o] = a[(size_t)o * l.pn + at];
-    x[o] = v[at + (o / 5 - 2) * l.px + o % 5 - 2];
-  }
+  for (int o = 0; o < 25; o++) c[o] = a[(size_t)o * l.pn + at];
   double s = 0.0;
 #pragma unroll
-  for (int o = 0; o < 25; o++) s += (double)c[o] * (double)x[o];
+  for (int o = 0; o < 25; o++)
+    s += (double)c[o] * (double)v[(o / 5 - 2) * pv + o % 5 - 2];
   return s;
 }
 
-// t = b - A x on grid k
-__global__ void __launch_bounds__(NT)
-    gk_res(const int2 *__restrict__ map, const MgSys *__restrict__ D, const MgScal *S, int sys,
-           int k) {
+// Tiles of the grids above the tail: TC x TC nodes of the coarser grid, or
+// TF x TF nodes of the finer one.  Both keep a block at one or two rounds of
+// its threads, and the residuals (or corrected values) that neighbouring
+// tiles both need are 13% of a tile's.
+constexpr int TF = 16, TC = TF / 2, TT = 320;
+
+// Grid k -> k + 1: residual b - A x of a tile (in LDS), restricted, with the
+// coarser grid's first smoothing step from zero.
+__global__ void __launch_bounds__(TT)
+    gk_down(const int2 *__restrict__ map, const MgSys *__restrict__ D, const MgScal *S, int sys,
+            int k) {
   const int2 m = where(map, sys);
-  if (m.x < 0 || S[m.x].status != ST_RUN) return;
-  const MgLevel &l = D[m.x].lv[k];
-  const int id = m.y * NT + threadIdx.x;
-  if (id >= l.nx * l.ny) return;
-  const int at = mg_at(l.px, id % l.nx, id / l.nx);
-  global_mut(l.t)[at] = (float)((double)global_ptr(l.b)[at] - stencil(l, at, global_ptr(l.x)));
+  if (m.x < 0 || S[m.x].a.status != ST_RUN) return;
+  const MgLevel &l = D[m.x].lv[k], &c = D[m.x].lv[k + 1];
+  constexpr int W = TF + 1, WX = W + 2 * MG_HALO;  // residuals, values around
+  __shared__ float xs[WX * WX], ts[W * W];
+  const int ntx = (c.nx + TC - 1) / TC;
+  const int X0 = m.y % ntx * TC, Y0 = m.y / ntx * TC;  // coarse corner
+  const int x0 = 2 * X0 - 1, y0 = 2 * Y0 - 1;          // the residuals' corner
+  for (int i = threadIdx.x; i < WX * WX; i += TT) {
+    const int x = x0 - MG_HALO + i % WX, y = y0 - MG_HALO + i / WX;
+    xs[i] = x >= 0 && x < l.nx && y >= 0 && y < l.ny ? global_ptr(l.x)[mg_at(l.px, x, y)] : 0.0f;
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < W * W; i += TT) {
+    const int ix = i % W, iy = i / W, x = x0 + ix, y = y0 + iy;
+    float res = 0.0f;
+    if (x >= 0 && x < l.nx && y >= 0 && y < l.ny) {
+      const int at = mg_at(l.px, x, y);
+      res = (float)((double)global_ptr(l.b)[at] -
+                    stencil(l, at, xs + (iy + MG_HALO) * WX + ix + MG_HALO, WX));
+    }
+    ts[i] = res;
+  }
+  __syncthreads();
+  if (threadIdx.x >= TC * TC) return;
+  const int ix = threadIdx.x % TC, iy = threadIdx.x / TC, X = X0 + ix, Y = Y0 + iy;
+  if (X >= c.nx || Y >= c.ny) return;
+  const float *t = ts + (2 * iy + 1) * W + 2 * ix + 1;
+  const float s = t[0] + 0.5f * ((t[-1] + t[1]) + (t[-W] + t[W])) +
+                  0.25f * ((t[-W - 1] + t[-W + 1]) + (t[W - 1] + t[W + 1]));
+  const int at = mg_at(c.px, X, Y);
+  global_mut(c.b)[at] = s;
+  global_mut(c.x)[at] = OM * global_ptr(c.minv)[at] * s;
 }
 
-template <class V>
-__device__ __forceinline__ float restrict_at(V t, int px, int X, int Y) {
-  const int at = mg_at(px, 2 * X, 2 * Y);
-  return t[at] + 0.5f * ((t[at - 1] + t[at + 1]) + (t[at - px] + t[at + px])) +
-         0.25f * ((t[at - px - 1] + t[at - px + 1]) + (t[at + px - 1] + t[at + px + 1]));
-}
-
-// grid k: b = P^T t of grid k - 1 and the first smoothing step from zero.
-// The nodes just outside grid k - 1 are its halo, where t stays zero.
-__global__ void __launch_bounds__(NT)
-    gk_restrict(const int2 *__restrict__ map, const MgSys *__restrict__ D, const MgScal *S,
-                int sys, int k) {
-  const int2 m = where(map, sys);
-  if (m.x < 0 || S[m.x].status != ST_RUN) return;
-  const MgLevel &f = D[m.x].lv[k - 1], &l = D[m.x].lv[k];
-  const int id = m.y * NT + threadIdx.x;
-  if (id >= l.nx * l.ny) return;
-  const int X = id % l.nx, Y = id / l.nx, at = mg_at(l.px, X, Y);
-  const float s = restrict_at(global_ptr(f.t), f.px, X, Y);
-  global_mut(l.b)[at] = s;
-  global_mut(l.x)[at] = OM * global_ptr(l.minv)[at] * s;
-}
-
+// A grid's correction at node (x, y) of the finer grid.
 template <class V>
 __device__ __forceinline__ float prolong_at(V xc, int px, int x, int y) {
   const int at = mg_at(px, x >> 1, y >> 1), ax = x & 1, ay = y & 1;
@@ -657,170 +844,331 @@ __device__ __forceinline__ float prolong_at(V xc, int px, int x, int y) {
   return 0.25f * ((xc[at] + xc[at + ax]) + (xc[at + ay * px] + xc[at + ay * px + ax]));
 }
 
-// t = x + P x of grid k + 1
-__global__ void __launch_bounds__(NT)
-    gk_prolong(const int2 *__restrict__ map, const MgSys *__restrict__ D, const MgScal *S,
-               int sys, int k) {
-  const int2 m = where(map, sys);
-  if (m.x < 0 || S[m.x].status != ST_RUN) return;
-  const MgLevel &l = D[m.x].lv[k], &c = D[m.x].lv[k + 1];
-  const int id = m.y * NT + threadIdx.x;
-  if (id >= l.nx * l.ny) return;
-  const int x = id % l.nx, y = id / l.nx, at = mg_at(l.px, x, y);
-  global_mut(l.t)[at] = global_ptr(l.x)[at] + prolong_at(global_ptr(c.x), c.px, x, y);
+// Interpolation in a cell (v: its first node, pv the pitch).
+template <class V>
+__device__ __forceinline__ float bilinear(f2_t f, V v, int pv) {
+  return (1.0f - f.x) * (1.0f - f.y) * v[0] + f.x * (1.0f - f.y) * v[1] +
+         (1.0f - f.x) * f.y * v[pv] + f.x * f.y * v[pv + 1];
 }
 
-// x = t + w M^-1 (b - A t)
-__global__ void __launch_bounds__(NT)
-    gk_smooth(const int2 *__restrict__ map, const MgSys *__restrict__ D, const MgScal *S,
-              int sys, int k) {
+// Grid k: a tile's corrected values x + P t of grid k + 1 (in LDS), then
+// t = those + w M^-1 (b - A those).  ROWS (k = 0): the smoothed values stay in LDS and
+// the rows of the tile's cells take theirs, t = x0 + sqrt(a_ii) P x.
+template <bool ROWS>
+__global__ void __launch_bounds__(TT)
+    gk_up(const int2 *__restrict__ map, const MgSys *__restrict__ D, const MgScal *S, int sys,
+          int k) {
   const int2 m = where(map, sys);
-  if (m.x < 0 || S[m.x].status != ST_RUN) return;
-  const MgLevel &l = D[m.x].lv[k];
-  const int id = m.y * NT + threadIdx.x;
-  if (id >= l.nx * l.ny) return;
-  const int at = mg_at(l.px, id % l.nx, id / l.nx);
-  const gptr<float> t = global_ptr(l.t);
-  const float res = (float)((double)global_ptr(l.b)[at] - stencil(l, at, t));
-  global_mut(l.x)[at] = fmaf(OM * global_ptr(l.minv)[at], res, t[at]);
+  if (m.x < 0 || S[m.x].a.status != ST_RUN) return;
+  const MgSys &d = D[m.x];
+  const MgLevel &l = d.lv[k], &c = d.lv[k + 1];
+  constexpr int W = ROWS ? TF + 1 : TF, WX = W + 2 * MG_HALO;
+  __shared__ float ts[WX * WX], xs[ROWS ? W * W : 1];
+  const int ntx = ((ROWS ? l.nx - 1 : l.nx) + TF - 1) / TF;
+  const int x0 = m.y % ntx * TF, y0 = m.y / ntx * TF;
+  for (int i = threadIdx.x; i < WX * WX; i += TT) {
+    const int x = x0 - MG_HALO + i % WX, y = y0 - MG_HALO + i / WX;
+    ts[i] = x >= 0 && x < l.nx && y >= 0 && y < l.ny
+                ? global_ptr(l.x)[mg_at(l.px, x, y)] + prolong_at(global_ptr(c.t), c.px, x, y)
+                : 0.0f;
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < W * W; i += TT) {
+    const int ix = i % W, iy = i / W, x = x0 + ix, y = y0 + iy;
+    if (x >= l.nx || y >= l.ny) continue;
+    const int at = mg_at(l.px, x, y);
+    const float *t = ts + (iy + MG_HALO) * WX + ix + MG_HALO;
+    const float res = (float)((double)global_ptr(l.b)[at] - stencil(l, at, t, WX));
+    const float v = fmaf(OM * global_ptr(l.minv)[at], res, t[0]);
+    // (x of this grid is still read by neighbouring tiles: t takes the result)
+    if (ROWS) xs[i] = v;
+    else global_mut(l.t)[at] = v;
+  }
+  if (!ROWS) return;
+  __syncthreads();
+  const int ncx = l.nx - 1, ncy = l.ny - 1;
+  const gptr<int> cptr = global_ptr(d.cptr), crow = global_ptr(d.crow);
+  const gptr<f2_t> cfrac = frac_ptr(d.cfrac);
+  for (int i = threadIdx.x; i < TF * TF; i += TT) {
+    const int ix = i % TF, iy = i / TF, cx = x0 + ix, cy = y0 + iy;
+    if (cx >= ncx || cy >= ncy) continue;
+    const int cl = cy * ncx + cx, k1 = cptr[cl + 1];
+    for (int q = cptr[cl]; q < k1; q++) {
+      const int r = crow[q];
+      global_mut(d.t)[r] = fmaf(global_ptr(d.sq)[r], bilinear(cfrac[q], xs + iy * W + ix, W),
+                                global_ptr(d.x0)[r]);
+    }
+  }
 }
 
-// The grids from d.tail on, in one workgroup: vectors in LDS, stencils read
-// from the caches.  LDS: x, b and t of every grid of the tail.
+// A tail grid's product with its stencil, FP32 (at most MG_TAIL nodes: the
+// cancellation costs three digits at most): v the node's value, pv its pitch.
+template <class C>
+__device__ __forceinline__ float stencil32(C c, const float *v, int pv) {
+  float s = 0.0f;
+#pragma unroll
+  for (int o = 0; o < 25; o++) s = fmaf(c(o), v[(o / 5 - 2) * pv + o % 5 - 2], s);
+  return s;
+}
+
+// The grids from d.tail on, in one workgroup.  A chain of some fifteen
+// barriers, so latency is all: every stencil entry is requested before the
+// first barrier (the first grid's into registers, TAIL_NODES nodes a thread,
+// the others' into LDS), and the phases then run on LDS alone.  With the
+// entries read in each phase it took 15 us for a first grid of 34 x 34.  When
+// every grid is in the tail it also restricts from the rows and interpolates
+// to them.  LDS: x, b and t of every grid, entries and weights of all but the
+// first, the dense inverse.
+constexpr int TAIL_NODES = MG_TAIL / RT;
+constexpr int TAIL_LEVELS = 10;  // grids of a tail, at most
+static_assert(TAIL_NODES * RT == MG_TAIL, "a thread owns whole nodes");
 __global__ void __launch_bounds__(RT)
     mk_tail(const MgSys *__restrict__ D, const MgScal *S, const int *__restrict__ list, int sys) {
   if (list) sys = list[blockIdx.x];
-  if (S[sys].status != ST_RUN) return;
+  if (sys < 0 || S[sys].a.status != ST_RUN) return;
   extern __shared__ float lds[];
+  __shared__ float part[RT / 64][64];
   const MgSys &d = D[sys];
   const int tid = threadIdx.x, first = d.tail, last = d.nlev - 1;
-  int tot = 0;
-  for (int k = first; k <= last; k++) tot += d.lv[k].pn;
-  for (int i = tid; i < 3 * tot; i += RT) lds[i] = 0.0f;
-  __syncthreads();
-  // x, b, t of grid k at off(k), off(k) + tot, off(k) + 2 tot
-  {
-    const MgLevel &l = d.lv[first];
-    for (int id = tid; id < l.nx * l.ny; id += RT) {
-      const int at = mg_at(l.px, id % l.nx, id / l.nx);
-      lds[at] = global_ptr(l.x)[at];
-      lds[tot + at] = global_ptr(l.b)[at];
+  const MgLevel &F = d.lv[first];
+  const int fx = F.nx, nf = fx * F.ny;
+  // the grids' sizes, kept in LDS: the descriptor's fields would be read from
+  // memory in every phase
+  struct Dim { int nx, ny, px, pn, nn; float inv; };
+  __shared__ Dim dm[TAIL_LEVELS];
+  if (tid <= last - first) {
+    int nx = F.nx, ny = F.ny;
+    for (int u = 0; u < tid; u++) {
+      nx = mg_next(nx);
+      ny = mg_next(ny);
     }
+    dm[tid] = Dim{nx, ny, nx + 2 * MG_HALO, mg_pn(nx, ny), nx * ny, 1.0f / (float)nx};
+  }
+  __syncthreads();
+  // (wave-uniform: scalar registers)
+  auto dims = [&](int u) {
+    const Dim q = dm[u];
+    auto si = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
+    return Dim{si(q.nx), si(q.ny), si(q.px), si(q.pn), si(q.nn),
+               __int_as_float(si(__float_as_int(q.inv)))};
+  };
+  const Dim d0 = dims(0);
+  // node id -> position (exact: ids are far below 2^20)
+  auto split = [](const Dim &q, int id, int &x, int &y) {
+    y = (int)(((float)id + 0.5f) * q.inv);
+    x = id - y * q.nx;
+  };
+  const int nu = last - first;  // the last grid's index in dm
+  int tot = 0;
+  for (int u = 0; u <= nu; u++) tot += dims(u).pn;
+  float *coef = lds + 3 * tot;
+  float ca[TAIL_NODES][25], ma[TAIL_NODES];
+  int fat[TAIL_NODES];
+#pragma unroll
+  for (int u = 0; u < TAIL_NODES; u++) {
+    int x, y;
+    split(d0, min(tid + u * RT, nf - 1), x, y);
+    fat[u] = mg_at(d0.px, x, y);
+    ma[u] = OM * global_ptr(F.minv)[fat[u]];
+#pragma unroll
+    for (int o = 0; o < 25; o++) ca[u][o] = global_ptr(F.a)[(size_t)o * d0.pn + fat[u]];
+  }
+  for (int i = tid; i < 3 * tot; i += RT) lds[i] = 0.0f;
+  int npk = 0;  // the pack: entries and weights of the other grids, the inverse
+  for (int u = 1; u <= nu; u++) npk += 26 * dims(u).nn;
+  const float *cinv = coef + npk;
+  npk += dims(nu).nn * dims(nu).nn;
+  {
+    const gptr<float> pk = global_ptr(d.pack);
+    int i = tid;
+    for (; i + 7 * RT < npk; i += 8 * RT) {
+      float v[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) v[u] = pk[i + u * RT];
+#pragma unroll
+      for (int u = 0; u < 8; u++) coef[i + u * RT] = v[u];
+    }
+    float v[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) v[u] = pk[min(i + u * RT, npk - 1)];
+#pragma unroll
+    for (int u = 0; u < 8; u++)
+      if (i + u * RT < npk) coef[i + u * RT] = v[u];
+  }
+  // the first grid's right-hand side and first smoothing step from zero
+  if (first == 0) {
+    // each cell's rows once, into its corners' shares; then the nodes' sums
+    const int ncx = fx - 1, nc = ncx * (d0.ny - 1);
+    float *share = coef + npk;  // [4][nc]
+    for (int c = tid; c < nc; c += RT) {
+      float s[4];
+      cell_shares(d, c, s);
+#pragma unroll
+      for (int q = 0; q < 4; q++) share[q * nc + c] = s[q];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < TAIL_NODES; u++) {
+      const int id = tid + u * RT;
+      if (id >= nf) continue;
+      int X, Y;
+      split(d0, id, X, Y);
+      float s = 0.0f;
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const int cx = X - (q & 1), cy = Y - (q >> 1);
+        if (cx >= 0 && cx < ncx && cy >= 0 && cy < d0.ny - 1) s += share[q * nc + cy * ncx + cx];
+      }
+      lds[tot + fat[u]] = s;
+      lds[fat[u]] = ma[u] * s;
+    }
+  } else {
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < TAIL_NODES; u++)
+      if (tid + u * RT < nf) {
+        lds[fat[u]] = global_ptr(F.x)[fat[u]];
+        lds[tot + fat[u]] = global_ptr(F.b)[fat[u]];
+      }
   }
   __syncthreads();
   int off = 0;
-  for (int k = first; k < last; k++) {  // down
-    const MgLevel &l = d.lv[k], &c = d.lv[k + 1];
+  const float *cf = coef;  // entries of the grid below the current one
+  for (int u = 0; u < nu; u++) {  // down
+    const Dim l = dims(u), c = dims(u + 1);
     float *x = lds + off, *b = x + tot, *t = b + tot;
-    for (int id = tid; id < l.nx * l.ny; id += RT) {
-      const int at = mg_at(l.px, id % l.nx, id / l.nx);
-      t[at] = (float)((double)b[at] - stencil(l, at, x));
+    if (u == 0) {
+#pragma unroll
+      for (int v = 0; v < TAIL_NODES; v++)
+        if (tid + v * RT < nf)
+          t[fat[v]] = b[fat[v]] - stencil32([&](int o) { return ca[v][o]; }, x + fat[v], l.px);
+    } else {
+      const float *cl = cf - 26 * l.nn;
+      for (int id = tid; id < l.nn; id += RT) {
+        int px, py;
+        split(l, id, px, py);
+        const int at = mg_at(l.px, px, py);
+        t[at] = b[at] - stencil32([&](int o) { return cl[o * l.nn + id]; }, x + at, l.px);
+      }
     }
     __syncthreads();
     float *xc = x + l.pn, *bc = xc + tot;
-    for (int id = tid; id < c.nx * c.ny; id += RT) {
-      const int X = id % c.nx, Y = id / c.nx, at = mg_at(c.px, X, Y);
-      const float s = restrict_at(t, l.px, X, Y);
+    for (int id = tid; id < c.nn; id += RT) {
+      int X, Y;
+      split(c, id, X, Y);
+      const int at = mg_at(c.px, X, Y);
+      const float *v = t + mg_at(l.px, 2 * X, 2 * Y);
+      const float s = v[0] + 0.5f * ((v[-1] + v[1]) + (v[-l.px] + v[l.px])) +
+                      0.25f * ((v[-l.px - 1] + v[-l.px + 1]) + (v[l.px - 1] + v[l.px + 1]));
       bc[at] = s;
-      xc[at] = OM * global_ptr(c.minv)[at] * s;
+      xc[at] = cf[25 * c.nn + id] * s;
     }
     __syncthreads();
     off += l.pn;
+    cf += 26 * c.nn;
   }
-  {  // last grid: the dense inverse
-    const MgLevel &l = d.lv[last];
-    const int nn = l.nx * l.ny;
+  {  // last grid: the dense inverse (symmetric)
+    const Dim q = dims(nu);
+    const int lx = q.nx, nn = q.nn, px = q.px, i = tid & 63, g = tid >> 6;
     float *x = lds + off, *b = x + tot;
-    for (int i = tid; i < nn; i += RT) {
-      float s = 0.0f;
-      for (int j = 0; j < nn; j++)
-        s = fmaf(global_ptr(d.cinv)[j * nn + i], b[mg_at(l.px, j % l.nx, j / l.nx)], s);
-      x[mg_at(l.px, i % l.nx, i / l.nx)] = s;
+    float s = 0.0f;
+    if (i < nn)
+      for (int j = g; j < nn; j += RT / 64)
+        s = fmaf(cinv[j * nn + i], b[mg_at(px, j % lx, j / lx)], s);
+    part[g][i] = s;
+    __syncthreads();
+    if (tid < nn) {
+      s = 0.0f;
+#pragma unroll
+      for (int g2 = 0; g2 < RT / 64; g2++) s += part[g2][tid];
+      x[mg_at(px, tid % lx, tid / lx)] = s;
     }
     __syncthreads();
   }
-  for (int k = last - 1; k >= first; k--) {  // up
-    const MgLevel &l = d.lv[k], &c = d.lv[k + 1];
+  for (int u = nu - 1; u >= 0; u--) {  // up
+    const Dim l = dims(u), c = dims(u + 1);
     off -= l.pn;
+    cf -= 26 * c.nn;  // entries of grid u + 1; grid u's end there
     float *x = lds + off, *b = x + tot, *t = b + tot, *xc = x + l.pn;
-    for (int id = tid; id < l.nx * l.ny; id += RT) {
-      const int px = id % l.nx, py = id / l.nx, at = mg_at(l.px, px, py);
+    for (int id = tid; id < l.nn; id += RT) {
+      int px, py;
+      split(l, id, px, py);
+      const int at = mg_at(l.px, px, py);
       t[at] = x[at] + prolong_at(xc, c.px, px, py);
     }
     __syncthreads();
-    for (int id = tid; id < l.nx * l.ny; id += RT) {
-      const int at = mg_at(l.px, id % l.nx, id / l.nx);
-      const float res = (float)((double)b[at] - stencil(l, at, t));
-      x[at] = fmaf(OM * global_ptr(l.minv)[at], res, t[at]);
+    if (u == 0) {
+#pragma unroll
+      for (int v = 0; v < TAIL_NODES; v++)
+        if (tid + v * RT < nf)
+          x[fat[v]] = fmaf(
+              ma[v],
+              b[fat[v]] - stencil32([&](int o) { return ca[v][o]; }, t + fat[v], l.px), t[fat[v]]);
+    } else {
+      const float *cl = cf - 26 * l.nn;
+      for (int id = tid; id < l.nn; id += RT) {
+        int px, py;
+        split(l, id, px, py);
+        const int at = mg_at(l.px, px, py);
+        x[at] = fmaf(cl[25 * l.nn + id],
+                     b[at] - stencil32([&](int o) { return cl[o * l.nn + id]; }, t + at, l.px),
+                     t[at]);
+      }
     }
     __syncthreads();
   }
-  const MgLevel &l = d.lv[first];
-  for (int id = tid; id < l.nx * l.ny; id += RT) {
-    const int at = mg_at(l.px, id % l.nx, id / l.nx);
-    global_mut(l.x)[at] = lds[at];
+  if (first > 0) {
+#pragma unroll
+    for (int u = 0; u < TAIL_NODES; u++)
+      if (tid + u * RT < nf) global_mut(F.t)[fat[u]] = lds[fat[u]];
+    return;
   }
-}
-
-// t = x0 + sqrt(a_ii) P x of the first grid
-__global__ void __launch_bounds__(NT)
-    mk_prolong(const int2 *__restrict__ map, const MgSys *__restrict__ D, const MgScal *S,
-               int sys) {
-  const int2 m = where(map, sys);
-  if (m.x < 0 || S[m.x].status != ST_RUN) return;
-  const MgSys &d = D[m.x];
-  const MgLevel &l = d.lv[0];
-  const int i = m.y * NT + threadIdx.x;
-  if (i >= d.npad) return;
-  float v = global_ptr(d.x0)[i];
-  const int c = global_ptr(d.cell)[i];
-  if (c >= 0) {
-    const gptr<float> x = global_ptr(l.x);
-    const f2_t f = frac_ptr(d)[i];
-    const int at = mg_at(l.px, c % (l.nx - 1), c / (l.nx - 1));
-    const float s = (1.0f - f.x) * (1.0f - f.y) * x[at] + f.x * (1.0f - f.y) * x[at + 1] +
-                    (1.0f - f.x) * f.y * x[at + l.px] + f.x * f.y * x[at + l.px + 1];
-    v = fmaf(global_ptr(d.sq)[i], s, v);
+  const gptr<int> cell = global_ptr(d.cell);
+  const gptr<f2_t> frac = frac_ptr(d.frac);
+  const gptr<float> sq = global_ptr(d.sq), x0 = global_ptr(d.x0);
+  const float icx = 1.0f / (float)(fx - 1);
+  for (int i = tid; i < d.npad; i += 4 * RT) {  // four rows' loads in flight
+    int c[4];
+    f2_t f[4];
+    float w[4], y[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const int j = min(i + u * RT, d.npad - 1);
+      c[u] = cell[j];
+      f[u] = frac[j];
+      w[u] = sq[j];
+      y[u] = x0[j];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      if (i + u * RT >= d.npad || c[u] < 0) continue;
+      const int cy = (int)(((float)c[u] + 0.5f) * icx);
+      global_mut(d.t)[i + u * RT] =
+          fmaf(w[u], bilinear(f[u], lds + mg_at(d0.px, c[u] - cy * (fx - 1), cy), d0.px), y[u]);
+    }
   }
-  global_mut(d.t)[i] = v;
 }
 
 // z = S (t + w M^-1 (rs - Â t)); partials of r.z
 __global__ void __launch_bounds__(NT)
     mk_post(const int2 *__restrict__ map, const MgSys *__restrict__ D, const MgScal *S, int sys) {
   const int2 m = where(map, sys);
-  if (m.x < 0 || S[m.x].status != ST_RUN) return;
+  if (m.x < 0 || S[m.x].a.status != ST_RUN) return;
   const MgSys &d = D[m.x];
   const int i = m.y * NT + threadIdx.x;
   double v[1] = {0.0};
   if (i < d.npad) {
     const gptr<float> t = global_ptr(d.t);
-    const double res = (double)global_ptr(d.rs)[i] - (double)t[i] -
+    // a row outside the grids (Dirichlet, uncoupled) has no t: its value is x0
+    const float ti = global_ptr(d.pos)[i] < 0 ? global_ptr(d.x0)[i] : t[i];
+    const double res = (double)global_ptr(d.rs)[i] - (double)ti -
                        dot32(d, i, [&](int c) { return t[c]; });
-    const float zi = (float)(fma((double)(OM * global_ptr(d.minv)[i]), res, (double)t[i]) *
+    const float zi = (float)(fma((double)(OM * global_ptr(d.minv)[i]), res, (double)ti) *
                              global_ptr(d.dsq)[i]);
     global_mut(d.z)[i] = zi;
     v[0] = global_ptr(d.r)[i] * (double)zi;
   }
-  put_partials<1>(v, d.part, d.nblk, m.y);
-}
-
-__global__ void __launch_bounds__(RT)
-    ms_beta(const MgSys *__restrict__ D, MgScal *S_, const int *__restrict__ list, int sys) {
-  if (list) sys = list[blockIdx.x];
-  MgScal *S = S_ + sys;
-  if (S->status != ST_RUN) return;
-  double t[1];
-  sum_partials<1>(D[sys].part, D[sys].nblk, t);
-  if (threadIdx.x != 0) return;
-  const double rz = t[0];
-  if (rz != rz || !isfinite(rz)) S->status = ST_NAN;
-  else if (!(rz > 0.0)) S->status = ST_BREAK;
-  else {
-    S->beta = S->first ? 0.0 : rz / S->rz;
-    S->rz = rz;
-    S->first = 0;
-  }
+  put_partials<1>(v, d.partz, d.nblk, m.y);
 }
 
 // ------------------------------------------------------------------ the plan
@@ -962,6 +1310,21 @@ __global__ void __launch_bounds__(NT)
   cptr[c] = lo;
 }
 
+// The rows' positions in the order of their cells.
+__global__ void __launch_bounds__(NT)
+    plan_cfrac(int n, int npad, const int *__restrict__ crow, const int *__restrict__ cell,
+               const float2 *__restrict__ frac, float2 *__restrict__ cfrac,
+               int *__restrict__ pos) {
+  const int k = blockIdx.x * NT + threadIdx.x;
+  if (k < n) {
+    const int i = crow[k];
+    cfrac[k] = frac[i];
+    pos[i] = cell[i] < 0 ? -1 : k;
+  } else if (k < npad) {
+    pos[k] = -1;
+  }
+}
+
 // Per block: occupied cells and the most rows of one.
 __global__ void __launch_bounds__(NT)
     plan_fill(int ncell, const int *__restrict__ cptr, int *__restrict__ out) {
@@ -1044,6 +1407,10 @@ MgPlan *build_plan(System &s, const Mesh &m, const int *order, hipStream_t st) {
     HIPCHECK(hipcub::DeviceRadixSort::SortPairs(t.p, tmp, key.p, skey.p, row.p, pl->crow.p, n, 0,
                                                 bits, st));
     plan_cptr<<<nb(ncell + 1, NT), NT, 0, st>>>(n, ncell, skey.p, pl->cptr.p);
+    pl->cfrac.alloc(n);
+    pl->pos.alloc(np);
+    plan_cfrac<<<nb(np, NT), NT, 0, st>>>(n, np, pl->crow.p, pl->cell.p, pl->frac.p,
+                                          pl->cfrac.p, pl->pos.p);
     plan_fill<<<nb(ncell, NT), NT, 0, st>>>(ncell, pl->cptr.p, fill.p);
     HIPCHECK(hipGetLastError());
     std::vector<int> hf(fill.n);
@@ -1065,14 +1432,14 @@ MgPlan *build_plan(System &s, const Mesh &m, const int *order, hipStream_t st) {
       pl->nx[k] = nx;
       pl->ny[k] = ny;
       pl->px[k] = nx + 2 * MG_HALO;
-      pl->pn[k] = (pl->px[k] * (ny + 2 * MG_HALO) + 63) / 64 * 64;
+      pl->pn[k] = mg_pn(nx, ny);
       if (pl->tail < 0 && pl->pn[k] <= MG_TAIL) pl->tail = k;
       if (nx * ny <= MG_DENSE) break;
-      nx = nx / 2 + 1;
-      ny = ny / 2 + 1;
+      nx = mg_next(nx);
+      ny = mg_next(ny);
     }
     pl->nlev = k + 1;
-    if (pl->tail < 0) return pl;
+    if (pl->tail < 0 || pl->nlev - pl->tail > TAIL_LEVELS) return pl;
     pl->ok = true;
     return pl;
   } catch (...) {
@@ -1083,11 +1450,24 @@ MgPlan *build_plan(System &s, const Mesh &m, const int *order, hipStream_t st) {
 
 size_t tail_lds(const MgPlan &pl) {
   size_t t = 0;
-  for (int k = pl.tail; k < pl.nlev; k++) t += pl.pn[k];
-  return 3 * t * sizeof(float);
+  for (int k = pl.tail; k < pl.nlev; k++) {
+    t += 3 * pl.pn[k];
+    if (k > pl.tail) t += 26 * pl.nx[k] * pl.ny[k];
+  }
+  const size_t nn = (size_t)pl.nx[pl.nlev - 1] * pl.ny[pl.nlev - 1];
+  t += nn * nn;
+  if (pl.tail == 0) t += 4 * (size_t)(pl.nx[0] - 1) * (pl.ny[0] - 1);
+  return t * sizeof(float);
 }
 
 }  // namespace
+
+void mg_allow_lds(const MgPlan &pl) {
+  const size_t lds = tail_lds(pl);
+  REQUIRE(lds <= 150 * 1024, ADMFEM_ERR_UNSUPPORTED, "tail grids too large for LDS");
+  HIPCHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(mk_tail),
+                               hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024));
+}
 
 void mg_plan_free(MgPlan *p) { delete p; }
 
@@ -1098,7 +1478,8 @@ const MgPlan *mg_plan(System &s, hipStream_t st) {
 
 size_t mg_grid_floats(const MgPlan &pl) {
   size_t f = 0;
-  for (int k = 0; k < pl.nlev; k++) f += (size_t)29 * pl.pn[k];
+  for (int k = 0; k < pl.nlev; k++)
+    f += (size_t)29 * pl.pn[k] + (k > pl.tail ? (size_t)26 * pl.nx[k] * pl.ny[k] : 0);
   return f + MG_DENSE * MG_DENSE;
 }
 
@@ -1107,6 +1488,8 @@ void mg_grid_layout(const MgPlan &pl, float *base, MgSys &d) {
   d.frac = pl.frac.p;
   d.cptr = pl.cptr.p;
   d.crow = pl.crow.p;
+  d.cfrac = pl.cfrac.p;
+  d.pos = pl.pos.p;
   d.nlev = pl.nlev;
   d.tail = pl.tail;
   for (int k = 0; k < pl.nlev; k++) {
@@ -1123,7 +1506,18 @@ void mg_grid_layout(const MgPlan &pl, float *base, MgSys &d) {
     l.t = l.b + pn;
     base += 29 * pn;
   }
+  d.pack = base;
+  for (int k = pl.tail + 1; k < pl.nlev; k++) base += 26 * (size_t)pl.nx[k] * pl.ny[k];
   d.cinv = base;
+}
+
+void mg_parts(MgSys &d, int nblk, bool reduce, double *part) {
+  d.nblk = nblk;
+  d.part4 = part;
+  d.partz = part + 4 * (size_t)nblk;
+  d.sum4 = d.partz + nblk;
+  d.sumz = d.sum4 + 4;
+  d.gsum = reduce ? 1 : nblk;
 }
 
 struct MgWork {
@@ -1132,8 +1526,9 @@ struct MgWork {
   DevBuf<MgScal> sc;
   MgScal *h_sc = nullptr;        // pinned
   DevBuf<double> x, r, q, p0, p1, dsq, part;
-  DevBuf<float> sv32, sq, minv, z, rs, x0, t, grid;
+  DevBuf<float> sv32, sq, minv, z, rs, x0, t, ts, grid;
   int nblk = 0;
+  int last_it = 14;              // iterations of the last solve
   uint64_t version = 0;          // of the matrix the set-up was made from
   uint64_t rowsum_version = 0;   // of the matrix the row sums were taken of
   double rowsum = 0.0;
@@ -1162,7 +1557,7 @@ MgWork *ensure_work(System &s, const MgPlan &pl, hipStream_t st) {
     w->p0.alloc(np);
     w->p1.alloc(np);
     w->dsq.alloc(np);
-    w->part.alloc((size_t)4 * w->nblk + 1);
+    w->part.alloc((size_t)5 * w->nblk + 5);
     w->sv32.alloc(std::max(1, s.slice_ptr.back()));
     w->sq.alloc(np);
     w->minv.alloc(np);
@@ -1170,6 +1565,7 @@ MgWork *ensure_work(System &s, const MgPlan &pl, hipStream_t st) {
     w->rs.alloc(np);
     w->x0.alloc(np);
     w->t.alloc(np);
+    w->ts.alloc(np);
     w->grid.alloc(mg_grid_floats(pl));
     w->d.alloc(1);
     w->sc.alloc(1);
@@ -1194,13 +1590,14 @@ MgWork *ensure_work(System &s, const MgPlan &pl, hipStream_t st) {
     d.rs = w->rs.p;
     d.x0 = w->x0.p;
     d.t = w->t.p;
-    d.part = w->part.p;
+    d.ts = w->ts.p;
     d.n = s.n;
     d.npad = s.npad;
-    d.nblk = w->nblk;
+    mg_parts(d, w->nblk, w->nblk > MG_SUM, w->part.p);
     mg_grid_layout(pl, w->grid.p, d);
     mk_zero<<<nb(w->grid.n, 256), 256, 0, st>>>(w->grid.p, w->grid.n);
     HIPCHECK(hipGetLastError());
+    mg_allow_lds(pl);
     HIPCHECK(hipMemcpyAsync(w->d.p, &d, sizeof(MgSys), hipMemcpyHostToDevice, st));
     HIPCHECK(hipStreamSynchronize(st));
   } catch (...) {
@@ -1217,44 +1614,40 @@ MgWork *ensure_work(System &s, const MgPlan &pl, hipStream_t st) {
 // matrices and smoothing weights, the last grid's inverse.
 void mg_setup(const MgPlan &pl, int nblk, const MgSys *D, int sys, hipStream_t st) {
   mk_scale<<<nblk, NT, 0, st>>>(nullptr, D, sys);
-  mk_galerkin<<<nb(pl.nx[0] * pl.ny[0], GT), GT, 0, st>>>(nullptr, D, sys);
-  for (int k = 0; k < pl.tail; k++) {
-    gk_weights<<<nb(pl.nx[k] * pl.ny[k], GT), GT, 0, st>>>(nullptr, D, sys, k);
-    gk_galerkin<<<nb(pl.nx[k + 1] * pl.ny[k + 1], GT), GT, 0, st>>>(nullptr, D, sys, k + 1);
-  }
+  mk_galerkin<<<nb(pl.nx[0] * pl.ny[0], GT / 4), GT, 0, st>>>(nullptr, D, sys);
+  for (int k = 0; k < pl.tail; k++)
+    gk_setup<<<nb(pl.nx[k] * pl.ny[k], GT), GT, 0, st>>>(nullptr, D, sys, k);
   mk_tail_setup<<<1, ST, 0, st>>>(D, nullptr, sys);
   HIPCHECK(hipGetLastError());
 }
 
-namespace {
-
-void v_cycle(const MgPlan &pl, MgWork *w, hipStream_t st) {
-  const MgSys *D = w->d.p;
-  MgScal *S = w->sc.p;
-  auto grid = [&](int k) { return nb(pl.nx[k] * pl.ny[k], NT); };
-  mk_res<<<w->nblk, NT, 0, st>>>(nullptr, D, S, 0);
-  mk_restrict<<<grid(0), NT, 0, st>>>(nullptr, D, S, 0);
-  for (int k = 0; k < pl.tail; k++) {
-    gk_res<<<grid(k), NT, 0, st>>>(nullptr, D, S, 0, k);
-    gk_restrict<<<grid(k + 1), NT, 0, st>>>(nullptr, D, S, 0, k + 1);
-  }
-  mk_tail<<<1, RT, tail_lds(pl), st>>>(D, S, nullptr, 0);
-  for (int k = pl.tail - 1; k >= 0; k--) {
-    gk_prolong<<<grid(k), NT, 0, st>>>(nullptr, D, S, 0, k);
-    gk_smooth<<<grid(k), NT, 0, st>>>(nullptr, D, S, 0, k);
-  }
-  mk_prolong<<<w->nblk, NT, 0, st>>>(nullptr, D, S, 0);
-  mk_post<<<w->nblk, NT, 0, st>>>(nullptr, D, S, 0);
-  ms_beta<<<1, RT, 0, st>>>(D, S, nullptr, 0);
+int mg_tiles_down(const MgPlan &pl, int k) {
+  return (int)(nb(pl.nx[k + 1], TC) * nb(pl.ny[k + 1], TC));
 }
+int mg_tiles_up(const MgPlan &pl, int k) {
+  return k ? (int)(nb(pl.nx[k], TF) * nb(pl.ny[k], TF))
+           : (int)(nb(pl.nx[k] - 1, TF) * nb(pl.ny[k] - 1, TF));
+}
+
+namespace {
 
 void iteration(const MgPlan &pl, MgWork *w, hipStream_t st) {
   const MgSys *D = w->d.p;
   MgScal *S = w->sc.p;
+  mk_res<<<w->nblk, NT, 0, st>>>(nullptr, D, S, 0);
+  if (pl.tail > 0)
+    mk_restrict<<<nb(pl.nx[0] * pl.ny[0], NT / 4), NT, 0, st>>>(nullptr, D, S, 0);
+  for (int k = 0; k < pl.tail; k++)
+    gk_down<<<mg_tiles_down(pl, k), TT, 0, st>>>(nullptr, D, S, 0, k);
+  mk_tail<<<1, RT, tail_lds(pl), st>>>(D, S, nullptr, 0);
+  for (int k = pl.tail - 1; k > 0; k--)
+    gk_up<false><<<mg_tiles_up(pl, k), TT, 0, st>>>(nullptr, D, S, 0, k);
+  if (pl.tail > 0) gk_up<true><<<mg_tiles_up(pl, 0), TT, 0, st>>>(nullptr, D, S, 0, 0);
+  mk_post<<<w->nblk, NT, 0, st>>>(nullptr, D, S, 0);
+  if (w->nblk > MG_SUM) ms_reduce<1><<<1, RT, 0, st>>>(D, S, nullptr, 0);
   mk_dir<<<w->nblk, NT, 0, st>>>(nullptr, D, S, 0);
-  ms_alpha<<<1, RT, 0, st>>>(D, S, nullptr, 0);
+  if (w->nblk > MG_SUM) ms_reduce<4><<<1, RT, 0, st>>>(D, S, nullptr, 0);
   mk_update<<<w->nblk, NT, 0, st>>>(nullptr, D, S, 0);
-  v_cycle(pl, w, st);
 }
 
 // Whether the V-cycle pays for the assembled matrix: not when a mass term
@@ -1277,7 +1670,7 @@ bool mg_pays(System &s, MgWork *w, hipStream_t st) {
   return !(w->rowsum > MASS_DOMINANT);
 }
 
-constexpr int GRAPH_ITERS = 2;
+constexpr int GRAPH_ITERS = 4;
 
 // GRAPH_ITERS iterations, captured once per system (every pointer comes from
 // the device descriptor) and replayed.
@@ -1333,54 +1726,38 @@ bool mg_solve(System &s, const double *b, double *x_out, const admfem_solve_opts
     mg_setup(pl, w->nblk, D, 0, st);
     w->version = s.a_version;
   }
-  mk_start<true><<<w->nblk, NT, 0, st>>>(nullptr, D, 0, b);
-  ms_start<<<1, RT, 0, st>>>(D, S, 0, 1, o.rtol * o.rtol, o.max_iter);
-  int it = 0;
-  double true_prev = -1.0, rr_true = 0.0;
-  for (int restarts = 0;; restarts++) {
-    v_cycle(pl, w, st);
-    int chunk = o.check_every > 0 ? o.check_every : restarts ? 2 : 10;
-    for (;;) {
-      const int stop = (int)std::min<int64_t>((int64_t)it + chunk, o.max_iter);
-      while (it < stop) {
-        if (o.check_every != 1 && it + GRAPH_ITERS <= stop) {
-          launch_graph(pl, w, st);
-          it += GRAPH_ITERS;
-        } else {
-          iteration(pl, w, st);
-          it++;
-        }
+  mk_start<<<w->nblk, NT, 0, st>>>(nullptr, D, 0, b);
+  ms_start<<<1, RT, 0, st>>>(D, S, 0, o.rtol * o.rtol, o.max_iter);
+  // Iterations are enqueued in chunks, each followed by the check (a no-op
+  // while CG runs), and the host reads the state between chunks; kernels past
+  // the end return at once.  The first chunk is what the system's last solve
+  // took: the adjoint usually takes what the forward did.
+  int chunk = o.check_every > 0 ? o.check_every : w->last_it;
+  for (;;) {
+    for (int it = 0; it < chunk;) {
+      if (o.check_every != 1 && it + GRAPH_ITERS <= chunk) {
+        launch_graph(pl, w, st);
+        it += GRAPH_ITERS;
+      } else {
+        iteration(pl, w, st);
+        it++;
       }
-      HIPCHECK(hipGetLastError());
-      HIPCHECK(hipMemcpyAsync(w->h_sc, S, sizeof(MgScal), hipMemcpyDeviceToHost, st));
-      HIPCHECK(hipStreamSynchronize(st));
-      if (w->h_sc->status != ST_RUN || it >= o.max_iter) break;
-      if (o.check_every <= 0) chunk = 2;
     }
-    const int status = w->h_sc->status;
-    it = w->h_sc->it;
-    // the residual of the returned x, from the FP64 matrix
-    mk_start<false><<<w->nblk, NT, 0, st>>>(nullptr, D, 0, b);
-    ms_start<<<1, RT, 0, st>>>(D, S, 0, 0, 0.0, 0);
+    mk_check<<<w->nblk, NT, 0, st>>>(nullptr, D, S, 0, b);
+    ms_check<<<1, RT, 0, st>>>(D, S, nullptr, 0, w->h_sc);
     HIPCHECK(hipGetLastError());
-    HIPCHECK(hipMemcpyAsync(w->h_sc, S, sizeof(MgScal), hipMemcpyDeviceToHost, st));
     HIPCHECK(hipStreamSynchronize(st));
-    rr_true = w->h_sc->rr;
-    w->h_sc->status = status;
-    // the recursive residual decides only when the true one agrees;
-    // otherwise CG restarts from the true one, until that no longer helps
-    if (status != ST_CONV || rr_true <= w->h_sc->tol2 || it >= o.max_iter || restarts >= 8 ||
-        (true_prev >= 0.0 && !(rr_true < 0.25 * true_prev)))
-      break;
-    true_prev = rr_true;
+    if (w->h_sc->a.status != ST_RUN) break;
+    if (o.check_every <= 0) chunk = 2;
   }
+  w->last_it = std::min(64, std::max(4, w->h_sc->a.it));
   HIPCHECK(hipMemcpyAsync(x_out, w->x.p, sizeof(double) * s.n, hipMemcpyDeviceToDevice, st));
   HIPCHECK(hipStreamSynchronize(st));
   const MgScal &h = *w->h_sc;
-  stats.iterations = h.it;
-  stats.replacements = h.nrepl - 1;
-  stats.rel_residual = h.bb > 0 ? std::sqrt(rr_true / h.bb) : 0.0;
-  switch (h.status) {
+  stats.iterations = h.a.it;
+  stats.replacements = h.nrepl;
+  stats.rel_residual = h.bb > 0 ? std::sqrt(h.rr_true / h.bb) : 0.0;
+  switch (h.a.status) {
     case ST_CONV: stats.status = ADMFEM_OK; break;
     case ST_NAN: stats.status = ADMFEM_ERR_NAN; break;
     case ST_BREAK: stats.status = ADMFEM_ERR_BREAKDOWN; break;
