@@ -49,6 +49,10 @@ void batch_init(const BSys *D, BScal *S, int sys, int nblk, double rtol2, double
 // pref[k], nmap blocks in all) over gmap >= nmap grid blocks, XCD-aware
 void batch_map(int nsys, const int *slot, const int *pref, int nmap, int gmap, int2 *map,
                hipStream_t st);
+// several maps of one list of systems, packed: map q's prefixes at pref +
+// q (nsys + 1) (the last of them its size), its entries from off[q] on
+void batch_maps(int nsys, int maps, const int *slot, const int *pref, const int *off, int total,
+                int2 *map, hipStream_t st);
 void batch_iterations(const int2 *map, int nmap, const int *list, int nlist, const BSys *D,
                       BScal *S, int iters, hipStream_t st);
 void batch_spmv_repeat(const int2 *map, int nmap, const BSys *D, const BScal *S, int repeat,

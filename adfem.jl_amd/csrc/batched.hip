@@ -448,15 +448,10 @@ __global__ void syn_nodal(int n, const double *__restrict__ x, const double *__r
 // the 8 XCDs) runs one contiguous eighth of it, entry j of its share at grid
 // block 8 j + x, so neighbouring blocks of a system gather from the same
 // L2.  Grid blocks past a share get system -1 (no work).
-__global__ void expand_map(int nsys, const int *__restrict__ slot, const int *__restrict__ pref,
-                           int nmap, int gmap, int2 *__restrict__ map) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= gmap) return;
+__device__ __forceinline__ int2 map_entry(int nsys, const int *__restrict__ slot,
+                                          const int *__restrict__ pref, int nmap, int b) {
   const int x = b & 7, j = b >> 3, base = nmap >> 3, rem = nmap & 7;
-  if (j >= base + (x < rem ? 1 : 0)) {
-    map[b] = make_int2(-1, 0);
-    return;
-  }
+  if (j >= base + (x < rem ? 1 : 0)) return make_int2(-1, 0);
   const int L = x * base + min(x, rem) + j;
   int lo = 0, hi = nsys - 1;  // the last system starting at or before L
   while (lo < hi) {
@@ -464,7 +459,27 @@ __global__ void expand_map(int nsys, const int *__restrict__ slot, const int *__
     if (pref[mid] <= L) lo = mid;
     else hi = mid - 1;
   }
-  map[b] = make_int2(slot[lo], L - pref[lo]);
+  return make_int2(slot[lo], L - pref[lo]);
+}
+
+__global__ void expand_map(int nsys, const int *__restrict__ slot, const int *__restrict__ pref,
+                           int nmap, int gmap, int2 *__restrict__ map) {
+  const int b = blockIdx.x * blockDim.x + threadIdx.x;
+  if (b < gmap) map[b] = map_entry(nsys, slot, pref, nmap, b);
+}
+
+// Several maps of one list of systems: map q (of maps) has its prefixes at
+// pref + q (nsys + 1), of which the last is its size, and its entries at
+// off[q].
+__global__ void expand_maps(int nsys, int maps, const int *__restrict__ slot,
+                            const int *__restrict__ pref, const int *__restrict__ off, int total,
+                            int2 *__restrict__ map) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= total) return;
+  int q = 0;
+  while (q + 1 < maps && off[q + 1] <= t) q++;
+  const int *p = pref + (size_t)q * (nsys + 1);
+  map[t] = map_entry(nsys, slot, p, p[nsys], t - off[q]);
 }
 
 // user-order interleaved coordinates -> internal-order x, y and xy
@@ -493,6 +508,12 @@ void launch_perm_coords(int n, const int *iperm, const double *coords_user, doub
 void batch_map(int nsys, const int *slot, const int *pref, int nmap, int gmap, int2 *map,
                hipStream_t st) {
   expand_map<<<nb(gmap, 256), 256, 0, st>>>(nsys, slot, pref, nmap, gmap, map);
+  HIPCHECK(hipGetLastError());
+}
+
+void batch_maps(int nsys, int maps, const int *slot, const int *pref, const int *off, int total,
+                int2 *map, hipStream_t st) {
+  expand_maps<<<nb(total, 256), 256, 0, st>>>(nsys, maps, slot, pref, off, total, map);
   HIPCHECK(hipGetLastError());
 }
 

@@ -23,6 +23,10 @@ __host__ __device__ inline int mg_at(int px, int x, int y) {
   return (y + MG_HALO) * px + x + MG_HALO;
 }
 
+// Systems below this many rows stay with Jacobi-PCG: alone, and in a batch,
+// where a launch serves every system and the fewer iterations always pay.
+constexpr int MG_MIN_ROWS = 2048, MG_MIN_ROWS_BATCH = 200;
+
 // a grid's nodes along a side on the next one; its padded size
 __host__ __device__ inline int mg_next(int n) { return n / 2 + 1; }
 __host__ __device__ inline int mg_pn(int nx, int ny) {
@@ -94,5 +98,32 @@ const MgPlan *mg_plan(System &s, hipStream_t st);
 void mg_parts(MgSys &d, int nblk, bool reduce, double *part);
 size_t mg_grid_floats(const MgPlan &pl);
 void mg_grid_layout(const MgPlan &pl, float *base, MgSys &d);
+
+// Allows the tail kernel the LDS it needs for this plan; how much that is.
+void mg_allow_lds(const MgPlan &pl);
+size_t mg_tail_lds(const MgPlan &pl);
+
+// A batch of systems (descriptors of D, states of S by slot): the block maps
+// of every kind of wide launch ((slot, block) per grid block), and the slots.
+enum { MGS_ROWS = 0, MGS_GALERKIN, MGS_RESTRICT, MGS_SETUP,
+       MGS_DOWN = MGS_SETUP + MG_MAXLEV, MGS_UP = MGS_DOWN + MG_MAXLEV,
+       MG_STAGES = MGS_UP + MG_MAXLEV };
+struct MgBatch {
+  int nsys = 0, tail = 0;   // systems; most grids above the tail
+  bool reduce = false;      // some system's partials are summed by one block
+  size_t tail_lds = 0;
+  const int *list = nullptr;
+  const int2 *map[MG_STAGES] = {};
+  int nmap[MG_STAGES] = {};
+};
+// the blocks of one system in each of them
+void mg_stages(const MgPlan &pl, int npad, int (&nblk)[MG_STAGES]);
+void mg_batch_setup(const MgBatch &B, const MgSys *D, hipStream_t st);
+void mg_batch_start(const MgBatch &B, const MgSys *D, MgScal *S, double rtol2, int maxit,
+                    hipStream_t st);
+// iterations, then the check of the systems that stopped; host: pinned copy
+// of the states by slot
+void mg_batch_iterations(const MgBatch &B, const MgSys *D, MgScal *S, int iters, MgScal *host,
+                         hipStream_t st);
 
 }  // namespace admfem

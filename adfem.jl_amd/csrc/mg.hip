@@ -323,8 +323,10 @@ __device__ __forceinline__ void weight_node(const MgLevel &l, int x, int y) {
   float v[25], ajj[25];
 #pragma unroll
   for (int o = 0; o < 25; o++) {
+    const int X = x + o % 5 - 2, Y = y + o / 5 - 2;
     v[o] = a[(size_t)o * l.pn + at];
-    ajj[o] = a[(size_t)12 * l.pn + at + (o / 5 - 2) * l.px + o % 5 - 2];
+    ajj[o] = X >= 0 && X < l.nx && Y >= 0 && Y < l.ny
+                 ? a[(size_t)12 * l.pn + mg_at(l.px, X, Y)] : 0.0f;
   }
   float s = 0.0f;
 #pragma unroll
@@ -457,11 +459,6 @@ __global__ void __launch_bounds__(RT) ms_rowsum(int G, double *__restrict__ out)
   }
 }
 
-__global__ void mk_zero(float *__restrict__ a, size_t n) {
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) a[i] = 0.0f;
-}
-
 // ---------------------------------------------------------------- CG kernels
 
 // The scaled residual and the first smoothing step (from zero) of a row.
@@ -509,7 +506,9 @@ __global__ void __launch_bounds__(NT)
 }
 
 __global__ void __launch_bounds__(RT)
-    ms_start(const MgSys *__restrict__ D, MgScal *S_, int sys, double rtol2, int maxit) {
+    ms_start(const MgSys *__restrict__ D, MgScal *S_, const int *__restrict__ list, int sys,
+             double rtol2, int maxit) {
+  if (list) sys = list[blockIdx.x];
   const MgSys &d = D[sys];
   MgScal *S = S_ + sys;
   double t[2];
@@ -1448,7 +1447,7 @@ MgPlan *build_plan(System &s, const Mesh &m, const int *order, hipStream_t st) {
   }
 }
 
-size_t tail_lds(const MgPlan &pl) {
+size_t tail_lds_of(const MgPlan &pl) {
   size_t t = 0;
   for (int k = pl.tail; k < pl.nlev; k++) {
     t += 3 * pl.pn[k];
@@ -1462,8 +1461,10 @@ size_t tail_lds(const MgPlan &pl) {
 
 }  // namespace
 
+size_t mg_tail_lds(const MgPlan &pl) { return tail_lds_of(pl); }
+
 void mg_allow_lds(const MgPlan &pl) {
-  const size_t lds = tail_lds(pl);
+  const size_t lds = mg_tail_lds(pl);
   REQUIRE(lds <= 150 * 1024, ADMFEM_ERR_UNSUPPORTED, "tail grids too large for LDS");
   HIPCHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(mk_tail),
                                hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024));
@@ -1595,8 +1596,6 @@ MgWork *ensure_work(System &s, const MgPlan &pl, hipStream_t st) {
     d.npad = s.npad;
     mg_parts(d, w->nblk, w->nblk > MG_SUM, w->part.p);
     mg_grid_layout(pl, w->grid.p, d);
-    mk_zero<<<nb(w->grid.n, 256), 256, 0, st>>>(w->grid.p, w->grid.n);
-    HIPCHECK(hipGetLastError());
     mg_allow_lds(pl);
     HIPCHECK(hipMemcpyAsync(w->d.p, &d, sizeof(MgSys), hipMemcpyHostToDevice, st));
     HIPCHECK(hipStreamSynchronize(st));
@@ -1610,6 +1609,71 @@ MgWork *ensure_work(System &s, const MgPlan &pl, hipStream_t st) {
 
 }  // namespace
 
+// ----------------------------------------------------------------- batches
+
+static int mg_tiles_down(const MgPlan &pl, int k) {
+  return (int)(nb(pl.nx[k + 1], TC) * nb(pl.ny[k + 1], TC));
+}
+static int mg_tiles_up(const MgPlan &pl, int k) {
+  return k ? (int)(nb(pl.nx[k], TF) * nb(pl.ny[k], TF))
+           : (int)(nb(pl.nx[k] - 1, TF) * nb(pl.ny[k] - 1, TF));
+}
+
+void mg_stages(const MgPlan &pl, int npad, int (&nblk)[MG_STAGES]) {
+  for (int &v : nblk) v = 0;
+  nblk[MGS_ROWS] = (int)nb(npad, NT);
+  nblk[MGS_GALERKIN] = (int)nb((int64_t)pl.nx[0] * pl.ny[0], GT / 4);
+  if (pl.tail > 0) nblk[MGS_RESTRICT] = (int)nb((int64_t)pl.nx[0] * pl.ny[0], NT / 4);
+  for (int k = 0; k < pl.tail; k++) {
+    nblk[MGS_SETUP + k] = (int)nb((int64_t)pl.nx[k] * pl.ny[k], GT);
+    nblk[MGS_DOWN + k] = mg_tiles_down(pl, k);
+    nblk[MGS_UP + k] = mg_tiles_up(pl, k);
+  }
+}
+
+void mg_batch_setup(const MgBatch &B, const MgSys *D, hipStream_t st) {
+  auto n = [&](int q) { return (unsigned)B.nmap[q]; };
+  mk_scale<<<n(MGS_ROWS), NT, 0, st>>>(B.map[MGS_ROWS], D, 0);
+  mk_galerkin<<<n(MGS_GALERKIN), GT, 0, st>>>(B.map[MGS_GALERKIN], D, 0);
+  for (int k = 0; k < B.tail; k++)
+    gk_setup<<<n(MGS_SETUP + k), GT, 0, st>>>(B.map[MGS_SETUP + k], D, 0, k);
+  mk_tail_setup<<<(unsigned)B.nsys, ST, 0, st>>>(D, B.list, 0);
+  HIPCHECK(hipGetLastError());
+}
+
+void mg_batch_start(const MgBatch &B, const MgSys *D, MgScal *S, double rtol2, int maxit,
+                    hipStream_t st) {
+  mk_start<<<(unsigned)B.nmap[MGS_ROWS], NT, 0, st>>>(B.map[MGS_ROWS], D, 0, nullptr);
+  ms_start<<<(unsigned)B.nsys, RT, 0, st>>>(D, S, B.list, 0, rtol2, maxit);
+  HIPCHECK(hipGetLastError());
+}
+
+void mg_batch_iterations(const MgBatch &B, const MgSys *D, MgScal *S, int iters, MgScal *host,
+                         hipStream_t st) {
+  auto n = [&](int q) { return (unsigned)B.nmap[q]; };
+  const int2 *rows = B.map[MGS_ROWS];
+  const unsigned nl = (unsigned)B.nsys, nr = n(MGS_ROWS);
+  for (int it = 0; it < iters; it++) {
+    mk_res<<<nr, NT, 0, st>>>(rows, D, S, 0);
+    if (B.tail > 0)
+      mk_restrict<<<n(MGS_RESTRICT), NT, 0, st>>>(B.map[MGS_RESTRICT], D, S, 0);
+    for (int k = 0; k < B.tail; k++)
+      gk_down<<<n(MGS_DOWN + k), TT, 0, st>>>(B.map[MGS_DOWN + k], D, S, 0, k);
+    mk_tail<<<nl, RT, B.tail_lds, st>>>(D, S, B.list, 0);
+    for (int k = B.tail - 1; k > 0; k--)
+      gk_up<false><<<n(MGS_UP + k), TT, 0, st>>>(B.map[MGS_UP + k], D, S, 0, k);
+    if (B.tail > 0) gk_up<true><<<n(MGS_UP), TT, 0, st>>>(B.map[MGS_UP], D, S, 0, 0);
+    mk_post<<<nr, NT, 0, st>>>(rows, D, S, 0);
+    if (B.reduce) ms_reduce<1><<<nl, RT, 0, st>>>(D, S, B.list, 0);
+    mk_dir<<<nr, NT, 0, st>>>(rows, D, S, 0);
+    if (B.reduce) ms_reduce<4><<<nl, RT, 0, st>>>(D, S, B.list, 0);
+    mk_update<<<nr, NT, 0, st>>>(rows, D, S, 0);
+  }
+  mk_check<<<nr, NT, 0, st>>>(rows, D, S, 0, nullptr);
+  ms_check<<<nl, RT, 0, st>>>(D, S, B.list, 0, host);
+  HIPCHECK(hipGetLastError());
+}
+
 // The set-up of one matrix (descriptor `sys` of D): fine scaling, the grids'
 // matrices and smoothing weights, the last grid's inverse.
 void mg_setup(const MgPlan &pl, int nblk, const MgSys *D, int sys, hipStream_t st) {
@@ -1619,14 +1683,6 @@ void mg_setup(const MgPlan &pl, int nblk, const MgSys *D, int sys, hipStream_t s
     gk_setup<<<nb(pl.nx[k] * pl.ny[k], GT), GT, 0, st>>>(nullptr, D, sys, k);
   mk_tail_setup<<<1, ST, 0, st>>>(D, nullptr, sys);
   HIPCHECK(hipGetLastError());
-}
-
-int mg_tiles_down(const MgPlan &pl, int k) {
-  return (int)(nb(pl.nx[k + 1], TC) * nb(pl.ny[k + 1], TC));
-}
-int mg_tiles_up(const MgPlan &pl, int k) {
-  return k ? (int)(nb(pl.nx[k], TF) * nb(pl.ny[k], TF))
-           : (int)(nb(pl.nx[k] - 1, TF) * nb(pl.ny[k] - 1, TF));
 }
 
 namespace {
@@ -1639,7 +1695,7 @@ void iteration(const MgPlan &pl, MgWork *w, hipStream_t st) {
     mk_restrict<<<nb(pl.nx[0] * pl.ny[0], NT / 4), NT, 0, st>>>(nullptr, D, S, 0);
   for (int k = 0; k < pl.tail; k++)
     gk_down<<<mg_tiles_down(pl, k), TT, 0, st>>>(nullptr, D, S, 0, k);
-  mk_tail<<<1, RT, tail_lds(pl), st>>>(D, S, nullptr, 0);
+  mk_tail<<<1, RT, mg_tail_lds(pl), st>>>(D, S, nullptr, 0);
   for (int k = pl.tail - 1; k > 0; k--)
     gk_up<false><<<mg_tiles_up(pl, k), TT, 0, st>>>(nullptr, D, S, 0, k);
   if (pl.tail > 0) gk_up<true><<<mg_tiles_up(pl, 0), TT, 0, st>>>(nullptr, D, S, 0, 0);
@@ -1692,9 +1748,6 @@ void launch_graph(const MgPlan &pl, MgWork *w, hipStream_t st) {
 
 }  // namespace
 
-// Systems below this many rows stay with Jacobi-PCG.
-constexpr int MG_MIN_ROWS = 4096;
-
 // A sparse system's rows are the dofs of mesh m (m null: unknown, and it is
 // Jacobi-PCG's); its plan is kept for as long as the mesh stays the same one.
 void mg_set_mesh(System &s, const Mesh *m, const int *order, hipStream_t st) {
@@ -1727,7 +1780,7 @@ bool mg_solve(System &s, const double *b, double *x_out, const admfem_solve_opts
     w->version = s.a_version;
   }
   mk_start<<<w->nblk, NT, 0, st>>>(nullptr, D, 0, b);
-  ms_start<<<1, RT, 0, st>>>(D, S, 0, o.rtol * o.rtol, o.max_iter);
+  ms_start<<<1, RT, 0, st>>>(D, S, nullptr, 0, o.rtol * o.rtol, o.max_iter);
   // Iterations are enqueued in chunks, each followed by the check (a no-op
   // while CG runs), and the host reads the state between chunks; kernels past
   // the end return at once.  The first chunk is what the system's last solve

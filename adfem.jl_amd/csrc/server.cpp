@@ -3,12 +3,13 @@
 // A request runs the reference's pipeline for its own coefficients
 // (assemble -> Dirichlet -> u = K^-1 F -> L -> lambda = K^-1 dL/du ->
 // dL/dkappa).  The engine admits arrived requests while their device memory
-// fits the HBM budget (an arena carved once at creation, so admission and
-// release never call hipMalloc/hipFree), advances every admitted system with
+// fits the HBM budget (an arena that grows to the budget by what waits, so
+// admission rarely and release never calls hipMalloc/hipFree), advances every admitted system with
 // one batched launch per CG step (batched.hip), and moves systems that
 // converge to their next phase at the chunk boundaries, where finished
 // requests release their memory to the waiting queue.
 #include <algorithm>
+#include <array>
 #include <chrono>
 #include <cmath>
 #include <map>
@@ -17,6 +18,7 @@
 #include <unordered_set>
 
 #include "batched.h"
+#include "mg.h"
 
 namespace admfem {
 
@@ -25,44 +27,85 @@ namespace {
 constexpr size_t ALIGN = 256;
 inline size_t up(size_t v) { return (v + ALIGN - 1) / ALIGN * ALIGN; }
 
-// Best-fit allocator over one device allocation, coalescing on free.
+// Best-fit allocator over device segments, coalescing on free.  `cap` bounds
+// the segments' total; they are allocated as requests need them (the bytes
+// of every waiting request at once), not all at creation: an arena of the
+// whole budget cost its allocation at every start, and the driver clears what
+// a process gives back: an engine made and closed for 64 requests in a loop,
+// with a budget of 8 GiB, waited 180 ms in hipFree once the card's free memory
+// had gone round.
 struct Arena {
-  char *base = nullptr;
-  size_t cap = 0, used = 0, peak = 0;
-  std::map<size_t, size_t> free_;  // offset -> size
+  size_t cap = 0, used = 0, peak = 0, held = 0;
+  std::map<char *, size_t> segs;   // segment -> size
+  std::map<char *, size_t> free_;  // block -> size
   void init(size_t bytes) {
     cap = up(bytes);
-    HIPCHECK(hipMalloc(&base, cap));
-    free_.clear();
-    free_[0] = cap;
+    size_t avail = 0, total = 0;
+    HIPCHECK(hipMemGetInfo(&avail, &total));
+    REQUIRE(cap <= avail, ADMFEM_ERR_HIP, "the HBM budget exceeds the free device memory");
   }
   ~Arena() {
-    if (base) (void)hipFree(base);
+    for (auto &s : segs) (void)hipFree(s.first);
   }
-  bool alloc(size_t bytes, size_t &off) {
-    bytes = up(bytes);
-    auto best = free_.end();
-    for (auto it = free_.begin(); it != free_.end(); ++it)
-      if (it->second >= bytes && (best == free_.end() || it->second < best->second)) best = it;
-    if (best == free_.end()) return false;
-    off = best->first;
-    size_t rest = best->second - bytes;
-    free_.erase(best);
-    if (rest) free_[off + bytes] = rest;
-    used += bytes;
-    peak = std::max(peak, used);
+  // A new segment of `want` bytes if the budget has room, else of `bytes`,
+  // after giving back unused segments when it must.  False: no room now.
+  bool grow(size_t bytes, size_t want) {
+    if (held + bytes > cap)
+      for (auto it = segs.begin(); it != segs.end();) {
+        auto f = free_.find(it->first);
+        if (f == free_.end() || f->second != it->second) {
+          ++it;
+          continue;
+        }
+        (void)hipFree(it->first);
+        held -= it->second;
+        free_.erase(f);
+        it = segs.erase(it);
+      }
+    if (held + bytes > cap) return false;
+    const size_t size = std::max(bytes, std::min(want, cap - held));
+    char *p = nullptr;
+    if (hipMalloc(&p, size) != hipSuccess) {
+      (void)hipGetLastError();
+      return false;
+    }
+    segs[p] = size;
+    free_[p] = size;
+    held += size;
     return true;
   }
-  void release(size_t off, size_t bytes) {
+  // (want 0: only from the segments there are)
+  bool alloc(size_t bytes, size_t want, char *&out) {
+    bytes = up(bytes);
+    for (int tries = 0; tries < 2; tries++) {
+      auto best = free_.end();
+      for (auto it = free_.begin(); it != free_.end(); ++it)
+        if (it->second >= bytes && (best == free_.end() || it->second < best->second)) best = it;
+      if (best == free_.end()) {
+        if (tries || !want || !grow(bytes, up(want))) return false;
+        continue;
+      }
+      out = best->first;
+      const size_t rest = best->second - bytes;
+      free_.erase(best);
+      if (rest) free_[out + bytes] = rest;
+      used += bytes;
+      peak = std::max(peak, used);
+      return true;
+    }
+    return false;
+  }
+  void release(char *p, size_t bytes) {
     bytes = up(bytes);
     used -= bytes;
-    auto it = free_.emplace(off, bytes).first;
+    auto it = free_.emplace(p, bytes).first;
     auto nx = std::next(it);
-    if (nx != free_.end() && it->first + it->second == nx->first) {
+    // (a segment's first block never joins the block before it)
+    if (nx != free_.end() && it->first + it->second == nx->first && !segs.count(nx->first)) {
       it->second += nx->second;
       free_.erase(nx);
     }
-    if (it != free_.begin()) {
+    if (it != free_.begin() && !segs.count(it->first)) {
       auto pv = std::prev(it);
       if (pv->first + pv->second == it->first) {
         pv->second += it->second;
@@ -74,9 +117,9 @@ struct Arena {
 
 struct Topo {
   System *sys;
+  const MgPlan *plan;        // multigrid CG's grids, or null: Jacobi-PCG
   double jitter;
   int nblk;                  // batched blocks of 256 rows
-  size_t bytes;              // device bytes of one request on it
   std::vector<int> interior; // user ids of interior nodes
 };
 
@@ -86,13 +129,17 @@ struct Req {
   admfem_request r;
   admfem_result res{};
   int state = Q_WAIT;
+  bool mg = false;           // multigrid CG (else Jacobi-PCG)
   int slot = -1;
-  size_t off = 0;
+  char *mem = nullptr;       // its memory in the arena
   // device buffers (inside the arena)
   double2 *xy;
   double *x, *y, *kappa, *f, *uprev, *b, *sv64, *diag64, *dsq, *xa, *xb, *u64, *lam64,
       *grad, *obsv, *loss2, *part, *stage;
   float *sv32, *ysa, *ysb, *ra, *rb, *pa, *pb, *qa, *qb;
+  // multigrid CG: FP64 x, r, q, two directions; FP32 vectors; the grids
+  double *mgx, *mgr, *mgq, *mgp0, *mgp1;
+  float *sq, *minv, *z, *rs, *x0, *t, *ts, *grid;
   int *obsi;
   int nobs = 0;
   std::vector<int> h_obs;  // synthetic observation indices, kept until the request is done
@@ -121,6 +168,14 @@ struct Server {
   BScal *h_scal = nullptr;       // pinned mirror
   double *h_loss = nullptr;      // pinned, per slot: loss and bad-index flag
   BSys *h_desc = nullptr;        // pinned staging of the descriptors
+  // multigrid requests: descriptors and states by slot, their pinned staging
+  // and mirror, and the maps of the batch, of the set-ups and of the starts
+  DevBuf<MgSys> d_mg;
+  DevBuf<MgScal> d_mgs;
+  MgSys *h_mg = nullptr;
+  MgScal *h_mgs = nullptr;
+  std::vector<int> starts;       // multigrid requests whose solve is to start
+  static constexpr int MG_BATCH_SUM = 128;  // partials summed by the wide kernels
   int *h_list = nullptr;         // pinned staging: the batch's slots, then
                                  // their first logical blocks (list_cap each)
   size_t map_cap = 0, list_cap = 0;
@@ -139,12 +194,15 @@ struct Server {
     if (h_scal) (void)hipHostFree(h_scal);
     if (h_loss) (void)hipHostFree(h_loss);
     if (h_desc) (void)hipHostFree(h_desc);
+    if (h_mg) (void)hipHostFree(h_mg);
+    if (h_mgs) (void)hipHostFree(h_mgs);
     if (h_list) (void)hipHostFree(h_list);
     if (st) (void)hipStreamDestroy(st);
   }
 
   // ------------------------------------------------------------ layout
-  static size_t layout(const System &s, Req *q, char *base, int nobs) {
+  // (pl: the plan of a request that runs on multigrid CG, else null)
+  static size_t layout(const System &s, const MgPlan *pl, Req *q, char *base, int nobs) {
     const Mesh &m = *s.mesh;
     const size_t np = s.npad, ng = m.ngauss, ns = std::max<size_t>(1, s.slice_ptr.back());
     const size_t nblk = (np + BATCH_NT - 1) / BATCH_NT;
@@ -158,21 +216,45 @@ struct Server {
     auto D = [&](size_t n) { return (double *)take(n * sizeof(double)); };
     auto F = [&](size_t n) { return (float *)take(n * sizeof(float)); };
     double *x = D(nv), *y = D(nv), *kappa = D(ng), *f = D(ng), *uprev = D(np), *b = D(np),
-           *sv64 = D(ns), *diag64 = D(np), *dsq = D(np), *xa = D(np), *xb = D(np),
+           *sv64 = D(ns), *diag64 = D(np), *dsq = D(np),
            *u64 = D(np), *lam64 = D(np), *grad = D(ng), *obsv = D(nobs + 1), *loss2 = D(2),
-           *part = D(4 * nblk), *stage = D(2 * np);
+           *part = D(5 * nblk + 5), *stage = D(2 * np);
     double2 *xy = (double2 *)take(nv * sizeof(double2));
-    float *sv32 = F(ns), *ysa = F(np), *ysb = F(np), *ra = F(np), *rb = F(np), *pa = F(np),
-          *pb = F(np), *qa = F(np), *qb = F(np);
+    float *sv32 = F(ns);
+    if (pl) {
+      double *mgx = D(np), *mgr = D(np), *mgq = D(np), *mgp0 = D(np), *mgp1 = D(np);
+      float *sq = F(np), *minv = F(np), *z = F(np), *rs = F(np), *x0 = F(np), *t = F(np),
+            *ts = F(np), *grid = F(mg_grid_floats(*pl));
+      if (q) {
+        q->mgx = mgx; q->mgr = mgr; q->mgq = mgq; q->mgp0 = mgp0; q->mgp1 = mgp1;
+        q->sq = sq; q->minv = minv; q->z = z; q->rs = rs; q->x0 = x0; q->t = t; q->ts = ts;
+        q->grid = grid;
+      }
+    } else {
+      double *xa = D(np), *xb = D(np);
+      float *ysa = F(np), *ysb = F(np), *ra = F(np), *rb = F(np), *pa = F(np), *pb = F(np),
+            *qa = F(np), *qb = F(np);
+      if (q) {
+        q->xa = xa; q->xb = xb; q->ysa = ysa; q->ysb = ysb;
+        q->ra = ra; q->rb = rb; q->pa = pa; q->pb = pb; q->qa = qa; q->qb = qb;
+      }
+    }
     int *obsi = (int *)take((nobs + 1) * sizeof(int));
     if (q) {
       q->x = x; q->y = y; q->xy = xy; q->kappa = kappa; q->f = f; q->uprev = uprev; q->b = b;
-      q->sv64 = sv64; q->diag64 = diag64; q->dsq = dsq; q->xa = xa; q->xb = xb;
+      q->sv64 = sv64; q->diag64 = diag64; q->dsq = dsq;
       q->u64 = u64; q->lam64 = lam64; q->grad = grad; q->obsv = obsv; q->loss2 = loss2;
-      q->part = part; q->stage = stage; q->sv32 = sv32; q->ysa = ysa; q->ysb = ysb;
-      q->ra = ra; q->rb = rb; q->pa = pa; q->pb = pb; q->qa = qa; q->qb = qb; q->obsi = obsi;
+      q->part = part; q->stage = stage; q->sv32 = sv32; q->obsi = obsi;
     }
     return off;
+  }
+  void size_up(Req &q, bool jacobi) {
+    q.nobs = nobs_of(q);
+    q.mg = topos[q.r.topo].plan && o.mode == ADMFEM_MODE_BATCHED && !jacobi;
+  }
+  size_t bytes_of(const Req &q) const {
+    const Topo &T = topos[q.r.topo];
+    return layout(*T.sys, q.mg ? T.plan : nullptr, nullptr, nullptr, q.nobs);
   }
 
   int nobs_of(const Req &q) const {
@@ -212,6 +294,109 @@ struct Server {
     d.npad = s.npad;
     d.nblk = topos[q.r.topo].nblk;
     HIPCHECK(hipMemcpyAsync(d_desc.p + q.slot, &d, sizeof(BSys), hipMemcpyHostToDevice, st));
+  }
+
+  void write_mg_desc(Req &q) {
+    const Topo &T = topos[q.r.topo];
+    const System &s = *T.sys;
+    MgSys &d = h_mg[q.slot];
+    d = MgSys{};
+    d.sp = s.d_slice_ptr.p;
+    d.sc = s.d_sell_col.p;
+    d.sd = s.d_sell_d16.p;
+    d.row_bd = s.d_row_bd.p;
+    d.sv64 = q.sv64;
+    d.diag = q.diag64;
+    d.sv32 = q.sv32;
+    d.dsq = q.dsq;
+    d.sq = q.sq;
+    d.minv = q.minv;
+    d.b = q.b;
+    d.x = q.mgx;
+    d.r = q.mgr;
+    d.q = q.mgq;
+    d.p[0] = q.mgp0;
+    d.p[1] = q.mgp1;
+    d.z = q.z;
+    d.rs = q.rs;
+    d.x0 = q.x0;
+    d.t = q.t;
+    d.ts = q.ts;
+    d.n = s.n;
+    d.npad = s.npad;
+    mg_parts(d, T.nblk, T.nblk > MG_BATCH_SUM, q.part);
+    mg_grid_layout(*T.plan, q.grid, d);
+    HIPCHECK(hipMemcpyAsync(d_mg.p + q.slot, &d, sizeof(MgSys), hipMemcpyHostToDevice, st));
+  }
+
+  // The block maps of a set of multigrid requests, in buffers of the set's own
+  // (rewritten only after the stream has passed their last use).
+  struct MgSet {
+    int *h = nullptr;          // pinned: slots, offsets, prefixes
+    size_t h_cap = 0;
+    DevBuf<int> d;
+    DevBuf<int2> map;
+    MgBatch batch;
+    std::vector<std::pair<int, int>> slots;  // (slot, topology): what the maps
+                                             // were made for
+    ~MgSet() {
+      if (h) (void)hipHostFree(h);
+    }
+  };
+  void build_set(MgSet &B, const std::vector<int> &reqs_) {
+    std::vector<std::pair<int, int>> slots;
+    for (int i : reqs_) slots.emplace_back(reqs[i].slot, reqs[i].r.topo);
+    if (slots == B.slots) return;
+    const int ns = (int)reqs_.size();
+    std::vector<std::array<int, MG_STAGES>> nblk(ns);
+    MgBatch b;
+    b.nsys = ns;
+    for (int a = 0; a < ns; a++) {
+      const Topo &T = topos[reqs[reqs_[a]].r.topo];
+      int v[MG_STAGES];
+      mg_stages(*T.plan, T.sys->npad, v);
+      std::copy(v, v + MG_STAGES, nblk[a].begin());
+      b.tail = std::max(b.tail, T.plan->tail);
+      b.tail_lds = std::max(b.tail_lds, mg_tail_lds(*T.plan));
+      b.reduce = b.reduce || T.nblk > MG_BATCH_SUM;
+    }
+    std::vector<int> used;
+    for (int q = 0; q < MG_STAGES; q++)
+      for (int a = 0; a < ns; a++)
+        if (nblk[a][q]) {
+          used.push_back(q);
+          break;
+        }
+    const int nu = (int)used.size();
+    const size_t need = (size_t)ns + nu + (size_t)nu * (ns + 1);
+    if (need > B.h_cap) {
+      if (B.h) HIPCHECK(hipHostFree(B.h));
+      B.h = nullptr;
+      B.h_cap = std::max(need, 2 * B.h_cap);
+      HIPCHECK(hipHostMalloc((void **)&B.h, sizeof(int) * B.h_cap, hipHostMallocDefault));
+      B.d.alloc(B.h_cap);
+    }
+    int total = 0;
+    for (int a = 0; a < ns; a++) B.h[a] = reqs[reqs_[a]].slot;
+    for (int u = 0; u < nu; u++) {
+      int *pref = B.h + ns + nu + (size_t)u * (ns + 1);
+      int acc = 0;
+      for (int a = 0; a < ns; a++) {
+        pref[a] = acc;
+        acc += nblk[a][used[u]];
+      }
+      pref[ns] = acc;
+      B.h[ns + u] = total;
+      b.nmap[used[u]] = acc;
+      total += acc;
+    }
+    if ((size_t)total > B.map.n) B.map.alloc(std::max((size_t)total, 2 * B.map.n));
+    for (int u = 0; u < nu; u++) b.map[used[u]] = B.map.p + B.h[ns + u];
+    b.list = B.d.p;
+    HIPCHECK(hipMemcpyAsync(B.d.p, B.h, sizeof(int) * need, hipMemcpyHostToDevice, st));
+    batch_maps(ns, nu, B.d.p, B.d.p + ns + nu, B.d.p + ns, total, B.map.p, st);
+    B.batch = b;
+    B.slots = slots;
   }
 
   void inputs(Req &q) {
@@ -297,7 +482,7 @@ struct Server {
     admfem_problem p = problem(q);
     // FP64 matrix and rhs; the FP32 scaled matrix of the inner iteration
     launch_assemble_to(s, q.xy, p, SellOut{q.sv64, q.diag64, q.b}, st);
-    batch_scale(s, q.sv64, q.diag64, q.dsq, q.sv32, st);
+    if (!q.mg) batch_scale(s, q.sv64, q.diag64, q.dsq, q.sv32, st);
   }
 
   void start_cg(Req &q) {
@@ -306,11 +491,13 @@ struct Server {
                o.max_iter, st);
   }
 
-  bool admit(Req &q, double t) {
+  // waiting: bytes of the requests waiting with this one, which a new segment
+  // is made for (0: make none)
+  bool admit(Req &q, double t, size_t waiting, bool jacobi = false) {
     const Topo &T = topos[q.r.topo];
     if (free_slots.empty()) return false;
-    q.nobs = nobs_of(q);
-    size_t bytes = layout(*T.sys, nullptr, nullptr, q.nobs);
+    size_up(q, jacobi);
+    size_t bytes = bytes_of(q);
     if (bytes > arena.cap) {
       q.state = Q_DONE;
       q.res.done = 1;
@@ -318,18 +505,29 @@ struct Server {
       q.res.t_done = t;
       return true;
     }
-    size_t off;
-    if (!arena.alloc(bytes, off)) return false;
-    q.off = off;
+    char *mem;
+    if (!arena.alloc(bytes, waiting ? std::max(bytes, waiting) : 0, mem)) {
+      if (!waiting || arena.used) return false;  // when some request has finished
+      q.state = Q_DONE;              // the card's memory is gone
+      q.res.done = 1;
+      q.res.status = ADMFEM_ERR_BUDGET;
+      q.res.t_done = t;
+      return true;
+    }
+    q.mem = mem;
     q.res.device_bytes = (double)bytes;
-    layout(*T.sys, &q, arena.base + off, q.nobs);
+    layout(*T.sys, q.mg ? T.plan : nullptr, &q, mem, q.nobs);
     q.slot = free_slots.back();
     free_slots.pop_back();
     q.res.t_admit = t;
     try {
       assemble(q);
-      write_desc(q, q.b);
-      start_cg(q);
+      if (q.mg) {
+        write_mg_desc(q);  // set up and started with the batch's others
+      } else {
+        write_desc(q, q.b);
+        start_cg(q);
+      }
     } catch (const Error &e) {
       // the request fails alone: its memory and slot go back to the queue,
       // the requests behind it are admitted as usual
@@ -343,30 +541,39 @@ struct Server {
   }
 
   void release(Req &q) {
-    arena.release(q.off, layout(*topos[q.r.topo].sys, nullptr, nullptr, q.nobs));
+    arena.release(q.mem, bytes_of(q));
     free_slots.push_back(q.slot);
     q.slot = -1;
   }
 
   // forward solve finished: u, loss, dL/du; start the adjoint solve
-  void to_adjoint(Req &q, const BScal &sc) {
+  void to_adjoint(Req &q, int it) {
     const System &s = *topos[q.r.topo].sys;
-    q.res.iters_fwd = sc.it;
-    batch_final(d_desc.p, d_scal.p, q.slot, s.npad, q.u64, st);
+    q.res.iters_fwd = it;
+    solution(q, q.u64);
     launch_loss(s, q.u64, q.obsi, q.obsv, q.nobs, q.b, q.loss2, st);  // g overwrites b
-    start_cg(q);
+    if (!q.mg) start_cg(q);
     q.state = Q_ADJ;
+  }
+
+  // the finished solve's solution
+  void solution(Req &q, double *out) {
+    const System &s = *topos[q.r.topo].sys;
+    if (q.mg)
+      HIPCHECK(hipMemcpyAsync(out, q.mgx, sizeof(double) * s.npad, hipMemcpyDeviceToDevice, st));
+    else
+      batch_final(d_desc.p, d_scal.p, q.slot, s.npad, out, st);
   }
 
   // adjoint solve finished: the gradient and the outputs are enqueued, the
   // loss goes to the slot's pinned staging; complete() finishes the request
   // once the stream has drained (one synchronisation for every request that
   // finished at the same chunk boundary)
-  void finish(Req &q, const BScal &sc) {
+  void finish(Req &q, int it) {
     const System &s = *topos[q.r.topo].sys;
     const Mesh &m = *s.mesh;
-    q.res.iters_adj = sc.it;
-    batch_final(d_desc.p, d_scal.p, q.slot, s.npad, q.lam64, st);
+    q.res.iters_adj = it;
+    solution(q, q.lam64);
     admfem_problem p = problem(q);
     launch_kappa_gradient_to(s, q.xy, q.u64, q.lam64, p.lap_coef, q.grad, st);
     if (q.r.u_out) {
@@ -489,9 +696,12 @@ struct Server {
     });
     size_t next = 0;  // first request (in arrival order) not yet admitted
     while (next < order.size() && reqs[order[next]].state != Q_WAIT) next++;
+    const int mg_chunk = o.chunk > 0 ? o.chunk : 4;
     std::vector<int> active;
     for (size_t i = 0; i < reqs.size(); i++)
       if (reqs[i].state == Q_FWD || reqs[i].state == Q_ADJ) active.push_back((int)i);
+    std::vector<int> fresh, jac, mgr;  // fresh: multigrid requests to be set up
+    MgSet set_fresh, set_starts, set_mg;
     // requests whose last work (outputs, loss) is enqueued, and an event
     // behind that work: they complete once it has passed -- waited for
     // while the next chunk runs, so the host bookkeeping overlaps it
@@ -529,8 +739,24 @@ struct Server {
       while (next < order.size() && (o.max_active <= 0 || (int)active.size() < o.max_active)) {
         Req &q = reqs[order[next]];
         if (q.r.arrival > t) break;
-        if (!admit(q, t)) break;
-        if (q.state != Q_DONE) active.push_back(order[next]);
+        if (!admit(q, t, 0)) {
+          size_t waiting = 0;  // of the arrived requests that there is a slot for
+          for (size_t k = next, n = 0; k < order.size() && n < free_slots.size(); k++, n++) {
+            Req &w = reqs[order[k]];
+            if (w.r.arrival > t) break;
+            size_up(w, false);
+            const size_t bytes = bytes_of(w);
+            if (bytes <= arena.cap) waiting += up(bytes);
+          }
+          if (!waiting || !admit(q, t, waiting)) break;
+        }
+        if (q.state != Q_DONE) {
+          active.push_back(order[next]);
+          if (q.mg) {
+            fresh.push_back(order[next]);
+            starts.push_back(order[next]);
+          }
+        }
         next++;
       }
       peak_active = std::max(peak_active, (int)active.size());
@@ -544,30 +770,49 @@ struct Server {
         if (wait > 0) std::this_thread::sleep_for(std::chrono::duration<double>(std::min(wait, 0.01)));
         continue;
       }
-      // block map over the active systems; with graphs, both grids are padded
-      // to power-of-two buckets with entries that do no work (map: system -1,
-      // list: the never-running dummy slot)
-      size_t nmap = 0;
-      for (int i : active) nmap += topos[reqs[i].r.topo].nblk;
-      const size_t gmap = use_graph ? (size_t)bucket(nmap) : nmap;
-      const size_t glist = use_graph ? (size_t)bucket(active.size()) : active.size();
-      ensure_map(gmap, glist);
-      std::vector<std::pair<int, int>> slots(active.size());
-      for (size_t a = 0; a < active.size(); a++) {
-        const Req &q = reqs[active[a]];
-        slots[a] = std::make_pair(q.slot, topos[q.r.topo].nblk);
+      jac.clear();
+      mgr.clear();
+      for (int i : active) (reqs[i].mg ? mgr : jac).push_back(i);
+      if (!fresh.empty()) {
+        build_set(set_fresh, fresh);
+        mg_batch_setup(set_fresh.batch, d_mg.p, st);
+        fresh.clear();
       }
-      upload_batch(slots, glist, max_slots, nmap, gmap);  // padding: the dummy slot
-      if (use_graph)
-        launch_chunk((int)gmap, (int)glist, chunk);
-      else
-        batch_iterations(d_map.p, (int)nmap, d_list.p, (int)active.size(), d_desc.p, d_scal.p,
-                         chunk, st);
+      if (!starts.empty()) {
+        build_set(set_starts, starts);
+        mg_batch_start(set_starts.batch, d_mg.p, d_mgs.p, o.rtol * o.rtol, o.max_iter, st);
+        starts.clear();
+      }
+      if (!mgr.empty()) {
+        build_set(set_mg, mgr);
+        mg_batch_iterations(set_mg.batch, d_mg.p, d_mgs.p, mg_chunk, h_mgs, st);
+      }
+      if (!jac.empty()) {
+        // block map over the Jacobi-PCG systems; with graphs, both grids are
+        // padded to power-of-two buckets with entries that do no work (map:
+        // system -1, list: the never-running dummy slot)
+        size_t nmap = 0;
+        for (int i : jac) nmap += topos[reqs[i].r.topo].nblk;
+        const size_t gmap = use_graph ? (size_t)bucket(nmap) : nmap;
+        const size_t glist = use_graph ? (size_t)bucket(jac.size()) : jac.size();
+        ensure_map(gmap, glist);
+        std::vector<std::pair<int, int>> slots(jac.size());
+        for (size_t a = 0; a < jac.size(); a++) {
+          const Req &q = reqs[jac[a]];
+          slots[a] = std::make_pair(q.slot, topos[q.r.topo].nblk);
+        }
+        upload_batch(slots, glist, max_slots, nmap, gmap);  // padding: the dummy slot
+        if (use_graph)
+          launch_chunk((int)gmap, (int)glist, chunk);
+        else
+          batch_iterations(d_map.p, (int)nmap, d_list.p, (int)jac.size(), d_desc.p, d_scal.p,
+                           chunk, st);
+        HIPCHECK(hipMemcpyAsync(h_scal, d_scal.p, sizeof(BScal) * max_slots,
+                                hipMemcpyDeviceToHost, st));
+      }
       steps += 1;
-      iters += chunk;
+      iters += jac.empty() ? mg_chunk : chunk;
       batch_sum += (int64_t)active.size();
-      HIPCHECK(hipMemcpyAsync(h_scal, d_scal.p, sizeof(BScal) * max_slots,
-                              hipMemcpyDeviceToHost, st));
       flush();  // the previous chunk's finished requests, while this one runs
       HIPCHECK(hipStreamSynchronize(st));
       // phase changes; requests that finished or failed complete once their
@@ -575,7 +820,16 @@ struct Server {
       std::vector<int> still;
       for (int i : active) {
         Req &q = reqs[i];
-        const BScal sc = h_scal[q.slot];
+        // where the solve stands: status (0 run, 1 converged, else failed),
+        // iterations, true residual and right-hand side norms squared
+        struct { int status, it; double rr, bb; } sc;
+        if (q.mg) {
+          const MgScal &v = h_mgs[q.slot];
+          sc = {v.checked ? v.a.status : 0, v.a.it, v.rr_true, v.bb};
+        } else {
+          const BScal &v = h_scal[q.slot];
+          sc = {v.status, v.it, v.rr, v.bb};
+        }
         if (sc.status == 0) {
           still.push_back(i);
           continue;
@@ -589,11 +843,12 @@ struct Server {
         }
         if (q.state == Q_FWD) {
           q.res.relres_fwd = sc.bb > 0 ? std::sqrt(sc.rr / sc.bb) : 0.0;
-          to_adjoint(q, sc);
+          to_adjoint(q, sc.it);
+          if (q.mg) starts.push_back(i);
           still.push_back(i);
         } else {
           q.res.relres_adj = sc.bb > 0 ? std::sqrt(sc.rr / sc.bb) : 0.0;
-          finish(q, sc);
+          finish(q, sc.it);
           done.push_back(i);
         }
       }
@@ -621,17 +876,17 @@ struct Server {
       t = now_s(t0);
       System &s = *topos[q.r.topo].sys;
       q.nobs = nobs_of(q);
-      size_t bytes = layout(s, nullptr, nullptr, q.nobs);
-      size_t off;
-      if (bytes > arena.cap || !arena.alloc(bytes, off)) {
+      size_t bytes = bytes_of(q);
+      char *mem;
+      if (bytes > arena.cap || !arena.alloc(bytes, bytes, mem)) {
         q.res.status = ADMFEM_ERR_BUDGET;
         q.res.done = 1;
         q.state = Q_DONE;
         continue;
       }
-      q.off = off;
+      q.mem = mem;
       q.res.device_bytes = (double)bytes;
-      layout(s, &q, arena.base + off, q.nobs);
+      layout(s, nullptr, &q, mem, q.nobs);
       q.slot = 0;
       q.res.t_admit = t;
       peak_active = std::max(peak_active, 1);
@@ -645,7 +900,7 @@ struct Server {
       q.res.t_done = now_s(t0);
       q.res.done = 1;
       q.state = Q_DONE;
-      arena.release(q.off, bytes);
+      arena.release(q.mem, bytes);
     }
     wall = now_s(t0);
   }
@@ -723,7 +978,7 @@ double server_spmv_repeat(Server *sv, const int *topos, int nsys, int repeat,
       q.r.topo = topos[i];
       q.r.source = ADMFEM_SRC_SYNTH;
       q.r.seed = (unsigned long long)i;
-      const bool ok = sv->admit(q, 0.0);
+      const bool ok = sv->admit(q, 0.0, (size_t)1 << 30, true);
       REQUIRE(ok && q.state == Q_FWD, ADMFEM_ERR_BUDGET, "batch does not fit the budget");
       admitted++;
       nmap += sv->topos[q.r.topo].nblk;
@@ -775,6 +1030,12 @@ Server *server_create(const admfem_server_opts &o) {
     sv->d_scal.alloc(sv->max_slots + 1);
     HIPCHECK(hipMemset(sv->d_desc.p, 0, sv->d_desc.bytes()));
     HIPCHECK(hipMemset(sv->d_scal.p, 0, sv->d_scal.bytes()));
+    sv->d_mg.alloc(sv->max_slots);
+    sv->d_mgs.alloc(sv->max_slots);
+    HIPCHECK(hipHostMalloc((void **)&sv->h_mg, sizeof(MgSys) * sv->max_slots,
+                           hipHostMallocDefault));
+    HIPCHECK(hipHostMalloc((void **)&sv->h_mgs, sizeof(MgScal) * sv->max_slots,
+                           hipHostMallocDefault));
     BScal dummy{};
     dummy.status = 99;
     HIPCHECK(hipMemcpy(sv->d_scal.p + sv->max_slots, &dummy, sizeof(BScal),
@@ -799,7 +1060,11 @@ int server_add_topology(Server *sv, System *s, double jitter) {
   T.sys = s;
   T.jitter = jitter;
   T.nblk = (s->npad + BATCH_NT - 1) / BATCH_NT;
-  T.bytes = Server::layout(*s, nullptr, nullptr, std::max(1, s->n / 100));
+  T.plan = nullptr;
+  if (s->n >= MG_MIN_ROWS_BATCH && sv->o.mode == ADMFEM_MODE_BATCHED) {
+    T.plan = mg_plan(*s, sv->st);
+    if (T.plan) mg_allow_lds(*T.plan);
+  }
   for (int u = 0; u < s->n; u++)
     if (s->row_bd[s->uperm()[u]] < 0) T.interior.push_back(u);
   REQUIRE(!T.interior.empty(), ADMFEM_ERR_ARG, "topology has no interior node");

@@ -154,3 +154,66 @@ def test_operator_chain_with_grids_matches_oracle(degree, m):
                 d = np.linalg.norm(a.cpu().numpy() - b) / np.linalg.norm(b)
                 print(degree, m, seed, with_mesh, d, flush=True)
                 assert d < 1e-9
+
+
+def test_serving_batches_multigrid_and_jacobi_requests():
+    """Requests on meshes on both sides of the multigrid path's smallest size
+    and with one, two and three grids above the tail, Poisson and heat, host
+    inputs with other coordinates than the topology's, and P2, all in one
+    batch: each against the oracle, and bit-identical when served alone or in
+    rounds cut short by a timeout."""
+    from admfem.server import Server
+    rng = np.random.default_rng(0)
+    topos = []
+    for m, degree in ((30, 1), (63, 1), (64, 1), (130, 1), (260, 1), (40, 2)):
+        c, e = meshgen.jittered_square(m, seed=m)
+        om = O.OracleMesh(c, e) if degree == 1 else O.OracleMesh(c, e, degree=2)
+        gm = admfem.Mesh(c, e, degree=degree, zero_based=True)
+        topos.append((m, c, e, om, admfem.DirichletSystem(gm, admfem.bcnode(gm))))
+    reqs = []
+    for k, (m, c, e, om, S) in enumerate(topos):
+        for heat in (False, True):
+            c2 = c + rng.uniform(-0.02 / m, 0.02 / m, c.shape) if not heat else None
+            o2 = O.OracleMesh(c2, e) if c2 is not None and om.ndof == om.nnode else om
+            if o2 is om:
+                c2 = None
+            bd = om.bcnode()
+            obs = rng.choice(np.setdiff1d(np.arange(S.n), bd - 1), 30, replace=False)
+            P = dict(kappa=np.exp(0.3 * rng.standard_normal(om.ngauss)),
+                     f=rng.uniform(-1, 1, om.ngauss), obs_idx=obs.astype(np.int32),
+                     obs_val=np.zeros(30))
+            kw = dict(kind="poisson")
+            if heat:
+                P["u_prev"] = rng.standard_normal(S.n)
+                kw = dict(kind="heat", dt=1e-3)
+
+            def dl(u, obs=obs):
+                g = np.zeros_like(u)
+                g[obs] = 2 * u[obs]
+                return g
+            ref = O.forward_adjoint(o2, P["kappa"], P["f"], bd, np.zeros(bd.size), dl,
+                                    **(dict(dt=1e-3, u_prev=P["u_prev"]) if heat else {}))
+            reqs.append((k, dict(P, coords=c2, **kw), ref))
+
+    def serve(which, slices=None):
+        sv = Server(2 << 30, rtol=1e-11)
+        t = [sv.add_topology(S) for *_, S in topos]
+        ids = [sv.submit(t[reqs[i][0]], **reqs[i][1]) for i in which]
+        if slices:
+            for k in range(200):
+                sv.run(timeout=slices * (k + 1))
+        sv.run()
+        return [sv.result(i) for i in ids]
+    mix = serve(range(len(reqs)))
+    for r, (k, P, ref) in zip(mix, reqs):
+        assert r["status"] == 0
+        eu = np.linalg.norm(r["u"] - ref["u"]) / np.linalg.norm(ref["u"])
+        eg = np.linalg.norm(r["grad"] - ref["grad_kappa"]) / np.linalg.norm(ref["grad_kappa"])
+        print(topos[k][0], P["kind"], r["iters_fwd"], r["iters_adj"], eu, eg, flush=True)
+        assert eu < 1e-8 and eg < 1e-8
+    cut = serve(range(len(reqs)), slices=2e-4)
+    alone = [serve([i])[0] for i in (2, 7, 8)]
+    for a, b in list(zip(cut, mix)) + list(zip(alone, [mix[2], mix[7], mix[8]])):
+        assert a["status"] == 0
+        np.testing.assert_array_equal(a["u"], b["u"])
+        np.testing.assert_array_equal(a["grad"], b["grad"])
