@@ -23,9 +23,11 @@ __host__ __device__ inline int mg_at(int px, int x, int y) {
   return (y + MG_HALO) * px + x + MG_HALO;
 }
 
-// Systems below this many rows stay with Jacobi-PCG: alone, and in a batch,
-// where a launch serves every system and the fewer iterations always pay.
-constexpr int MG_MIN_ROWS = 2048, MG_MIN_ROWS_BATCH = 200;
+// Systems below this many rows stay with Jacobi-PCG.  One Poisson forward +
+// adjoint, FP64, Jacobi-PCG -> multigrid CG: 50^2 5.6 -> 1.1 ms, 32^2 4.7 -> 1.0
+// ms, 20^2 2.6 -> 0.93 ms, 14^2 1.6 -> 0.83 ms; at 12^2 and below the two are
+// even.
+constexpr int MG_MIN_ROWS = 200;
 
 // a grid's nodes along a side on the next one; its padded size
 __host__ __device__ inline int mg_next(int n) { return n / 2 + 1; }

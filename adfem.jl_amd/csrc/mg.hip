@@ -1728,6 +1728,11 @@ bool mg_pays(System &s, MgWork *w, hipStream_t st) {
 
 constexpr int GRAPH_ITERS = 4;
 
+// Products with the system's matrix in an iteration (mk_res, mk_post,
+// mk_dir): what max_iter bounds and the stats report, as for Jacobi-PCG, whose
+// iterations are one product each.
+constexpr int MG_PRODUCTS = 3;
+
 // GRAPH_ITERS iterations, captured once per system (every pointer comes from
 // the device descriptor) and replayed.
 void launch_graph(const MgPlan &pl, MgWork *w, hipStream_t st) {
@@ -1780,7 +1785,8 @@ bool mg_solve(System &s, const double *b, double *x_out, const admfem_solve_opts
     w->version = s.a_version;
   }
   mk_start<<<w->nblk, NT, 0, st>>>(nullptr, D, 0, b);
-  ms_start<<<1, RT, 0, st>>>(D, S, nullptr, 0, o.rtol * o.rtol, o.max_iter);
+  ms_start<<<1, RT, 0, st>>>(D, S, nullptr, 0, o.rtol * o.rtol,
+                             std::max(1, o.max_iter / MG_PRODUCTS));
   // Iterations are enqueued in chunks, each followed by the check (a no-op
   // while CG runs), and the host reads the state between chunks; kernels past
   // the end return at once.  The first chunk is what the system's last solve
@@ -1807,7 +1813,7 @@ bool mg_solve(System &s, const double *b, double *x_out, const admfem_solve_opts
   HIPCHECK(hipMemcpyAsync(x_out, w->x.p, sizeof(double) * s.n, hipMemcpyDeviceToDevice, st));
   HIPCHECK(hipStreamSynchronize(st));
   const MgScal &h = *w->h_sc;
-  stats.iterations = h.a.it;
+  stats.iterations = MG_PRODUCTS * h.a.it;
   stats.replacements = h.nrepl;
   stats.rel_residual = h.bb > 0 ? std::sqrt(h.rr_true / h.bb) : 0.0;
   switch (h.a.status) {

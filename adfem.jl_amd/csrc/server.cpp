@@ -1061,7 +1061,7 @@ int server_add_topology(Server *sv, System *s, double jitter) {
   T.jitter = jitter;
   T.nblk = (s->npad + BATCH_NT - 1) / BATCH_NT;
   T.plan = nullptr;
-  if (s->n >= MG_MIN_ROWS_BATCH && sv->o.mode == ADMFEM_MODE_BATCHED) {
+  if (s->n >= MG_MIN_ROWS && sv->o.mode == ADMFEM_MODE_BATCHED) {
     T.plan = mg_plan(*s, sv->st);
     if (T.plan) mg_allow_lds(*T.plan);
   }

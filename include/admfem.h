@@ -290,7 +290,8 @@ int admfem_system_csr(admfem_system s, int *row_ptr, int *col, double *val,
 #define ADMFEM_PREC_MIXED 1  /* FP32 Jacobi-PCG, FP64 residual replacement */
 typedef struct {
   int precision;      /* ADMFEM_PREC_* */
-  int max_iter;       /* total inner iterations */
+  int max_iter;       /* total inner iterations, counted in products with A (a
+                         multigrid iteration takes three) */
   double rtol;        /* ||b - A x||_2 <= rtol * ||b||_2 (true residual) */
   int check_every;    /* iterations between host convergence checks (0: auto) */
   double replace_delta; /* mixed: FP64 residual replacement when the inner
