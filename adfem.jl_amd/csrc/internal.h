@@ -266,7 +266,10 @@ void system_host_pattern(System &s);
 void csr_row_ptr(const int *srow, int m, int n, int *rp, hipStream_t st);  // rows sorted
 int64_t device_bandwidth(int n, const int *rp, const int *col, const int *inv, hipStream_t st);
 int device_first_coupled(int n, const int *rp, const int *col, hipStream_t st);
-int64_t device_bfs_max_level(int n, const int *rp, const int *col, int s, hipStream_t st);
+bool device_banded(int64_t bw, int n, const int *rp, const int *col, int s, hipStream_t st);
+// the dofs of a mesh in its banded order: order[k] = dof at position k (P1:
+// iperm), inv its inverse
+void mesh_dof_order(const Mesh &m, DevBuf<int> &order, DevBuf<int> &inv, hipStream_t st);
 void rcm(int n, const int *rp, const int *col, DevBuf<int> &order, DevBuf<int> &inv,
          hipStream_t st);
 

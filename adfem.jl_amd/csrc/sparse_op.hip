@@ -149,14 +149,21 @@ struct CooPattern {
 // row 0: after Dirichlet elimination that is usually a boundary node holding
 // only its diagonal, whose one-node "level" would make every order look
 // unbanded.
-void reorder(CooPattern &p, int n, int nslot, const int *srow, DevBuf<int> &rp,
+// A matrix on a mesh's dofs needs no search: the mesh has a banded order,
+// taken unless the caller's is as good (within a factor of two).
+void reorder(CooPattern &p, const Mesh *m, int n, int nslot, const int *srow, DevBuf<int> &rp,
              DevBuf<int> &col, hipStream_t st) {
   const int64_t bw_id = device_bandwidth(n, rp.p, col.p, nullptr, st);
-  const int start = device_first_coupled(n, rp.p, col.p, st);
-  if (bw_id <= 5 * device_bfs_max_level(n, rp.p, col.p, start, st)) return;
   DevBuf<int> order, inv;
-  rcm(n, rp.p, col.p, order, inv, st);
-  if (device_bandwidth(n, rp.p, col.p, inv.p, st) >= bw_id) return;
+  if (m && m->ndof == n) {
+    mesh_dof_order(*m, order, inv, st);
+    if (bw_id <= 2 * device_bandwidth(n, rp.p, col.p, inv.p, st)) return;
+  } else {
+    const int start = device_first_coupled(n, rp.p, col.p, st);
+    if (device_banded(bw_id, n, rp.p, col.p, start, st)) return;
+    rcm(n, rp.p, col.p, order, inv, st);
+    if (device_bandwidth(n, rp.p, col.p, inv.p, st) >= bw_id) return;
+  }
   DevBuf<unsigned long long> key(nslot), skey(nslot);
   DevBuf<int> val(nslot), sval(nslot), nrow(nslot), ncol(nslot);
   p.pos.alloc(nslot);
@@ -199,16 +206,16 @@ bool same_pattern(CooPattern &p, const long long *ind, int64_t nnz, int n, int d
   return h == 0;
 }
 
-void build_pattern(CooPattern &p, const long long *ind, int64_t nnz, int n, int dev,
+void build_pattern(CooPattern &p, const Mesh *m, const long long *ind, int64_t nnz, int n, int dev,
                    hipStream_t st) {
   p.device = dev;
   p.n = n;
   p.nnz = nnz;
   p.flag.alloc(1);
-  const int64_t m = std::max<int64_t>(nnz, 1);
-  DevBuf<unsigned long long> key(m), skey(m);
-  DevBuf<int> val(m), fresh(m), pos(m), err(1);
-  p.trip.alloc(m);
+  const int64_t nt = std::max<int64_t>(nnz, 1);
+  DevBuf<unsigned long long> key(nt), skey(nt);
+  DevBuf<int> val(nt), fresh(nt), pos(nt), err(1);
+  p.trip.alloc(nt);
   set_int<<<1, 1, 0, st>>>(err.p, 0);
   int nslot = 0;
   DevBuf<int> rp(n + 1), col;
@@ -249,7 +256,7 @@ void build_pattern(CooPattern &p, const long long *ind, int64_t nnz, int n, int 
     csr_row_ptr(srow.p, nslot, n, rp.p, st);
     col.swap(scol);
     p.nslot = nslot;
-    reorder(p, n, nslot, srow.p, rp, col, st);
+    reorder(p, m, n, nslot, srow.p, rp, col, st);
   } else {
     p.start.alloc(1);
     const int zero = 0;
@@ -280,7 +287,7 @@ System &pattern_with_values(const Mesh *m, const long long *ind, const double *v
     }
     CooPattern *p = new CooPattern();
     try {
-      build_pattern(*p, ind, nnz, n, dev, st);
+      build_pattern(*p, m, ind, nnz, n, dev, st);
     } catch (...) {
       system_free(p->s);
       delete p;

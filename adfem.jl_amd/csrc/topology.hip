@@ -784,7 +784,10 @@ struct BfsRun {
   std::vector<int> size;  // nodes per level, levels 0 .. nlev - 1
 };
 
-void run_bfs(int n, const int *rp, const int *col, int s, BfsRun &b, hipStream_t st) {
+// (stop: the search ends once some level has that many nodes, 0: never; then
+// b.size holds the levels searched so far)
+void run_bfs(int n, const int *rp, const int *col, int s, BfsRun &b, hipStream_t st,
+             int64_t stop = 0) {
   b.level.alloc(n);
   b.q.alloc(n);
   b.off.alloc(n + 2);
@@ -799,24 +802,26 @@ void run_bfs(int n, const int *rp, const int *col, int s, BfsRun &b, hipStream_t
   // levels in batches: a level with no nodes ends the search (every later
   // launch sees an empty frontier)
   constexpr int BATCH = 64;
-  int L = 0;
-  for (;;) {
-    const int end = std::min(L + BATCH, n);
+  int L = 0, h[BATCH];
+  b.size.assign(1, 1);
+  for (bool more = true; more;) {
+    const int L0 = L, end = std::min(L + (stop && L < BATCH ? 16 : BATCH), n);
     for (; L < end; L++)
       bfs_level_kernel<<<BFS_BLOCKS, BFS_NT, 0, st>>>(L, rp, col, b.level.p, b.q.p, b.off.p,
                                                       b.cnt.p);
     HIPCHECK(hipGetLastError());
-    int last = 0;
-    HIPCHECK(hipMemcpyAsync(&last, b.cnt.p + L, sizeof(int), hipMemcpyDeviceToHost, st));
+    HIPCHECK(hipMemcpyAsync(h, b.cnt.p + L0 + 1, sizeof(int) * (L - L0), hipMemcpyDeviceToHost,
+                            st));
     HIPCHECK(hipStreamSynchronize(st));
-    if (last == 0 || L >= n) break;
-  }
-  std::vector<int> h(L + 1);
-  HIPCHECK(hipMemcpy(h.data(), b.cnt.p, sizeof(int) * (L + 1), hipMemcpyDeviceToHost));
-  b.size.clear();
-  for (int v : h) {
-    if (v == 0) break;
-    b.size.push_back(v);
+    more = L < n;
+    for (int k = 0; k < L - L0; k++) {
+      if (h[k] == 0) {
+        more = false;
+        break;
+      }
+      b.size.push_back(h[k]);
+      if (stop && h[k] >= stop) more = false;
+    }
   }
 }
 
@@ -833,12 +838,58 @@ unsigned long long min_degree(int m, const int *list, const int *deg, hipStream_
 
 }  // namespace
 
-int64_t device_bfs_max_level(int n, const int *rp, const int *col, int s, hipStream_t st) {
+// Whether an order of bandwidth bw is banded: bw at most 5x the widest level
+// of a breadth-first search from s.  The search stops at the first level
+// that shows it -- a fifth of the levels for a row-ordered grid, where the
+// whole search was 640 launches of 5 us at 300^2; only an order that is not
+// banded is searched to the end.
+bool device_banded(int64_t bw, int n, const int *rp, const int *col, int s, hipStream_t st) {
+  const int64_t width = (bw + 4) / 5;
+  if (width <= 1) return true;  // (the first level)
   BfsRun b;
-  run_bfs(n, rp, col, s, b, st);
-  int64_t w = 0;
-  for (int v : b.size) w = std::max<int64_t>(w, v);
-  return w;
+  run_bfs(n, rp, col, s, b, st, width);
+  for (int v : b.size)
+    if (v >= width) return true;
+  return false;
+}
+
+namespace {
+// each dof's sort key: vertices at their node's position, each followed by
+// the edge dofs whose lower end it is, by their other end
+__global__ void dof_key_kernel(int ndof, int nn, const int *__restrict__ perm,
+                               const long long *__restrict__ edges, long long nedges,
+                               unsigned long long *__restrict__ key, int *__restrict__ id) {
+  const int u = blockIdx.x * blockDim.x + threadIdx.x;
+  if (u >= ndof) return;
+  unsigned long long k;
+  if (u < nn) {
+    k = (unsigned long long)perm[u] * (nn + 1);
+  } else {
+    const int a = perm[edges[u - nn] - 1], b = perm[edges[nedges + u - nn] - 1];
+    k = (unsigned long long)min(a, b) * (nn + 1) + 1 + max(a, b);
+  }
+  key[u] = k;
+  id[u] = u;
+}
+}  // namespace
+
+void mesh_dof_order(const Mesh &m, DevBuf<int> &order, DevBuf<int> &inv, hipStream_t st) {
+  const int nd = (int)m.ndof, nn = m.nnode;
+  order.alloc(nd);
+  inv.alloc(nd);
+  if (m.degree == 1) {
+    HIPCHECK(hipMemcpyAsync(order.p, m.d_iperm.p, sizeof(int) * nd, hipMemcpyDeviceToDevice, st));
+    HIPCHECK(hipMemcpyAsync(inv.p, m.d_perm.p, sizeof(int) * nd, hipMemcpyDeviceToDevice, st));
+    return;
+  }
+  DevBuf<unsigned long long> key(nd), skey(nd);
+  DevBuf<int> id(nd);
+  dof_key_kernel<<<nb(nd, 256), 256, 0, st>>>(nd, nn, m.d_perm.p, m.d_edges.p, m.nedges, key.p,
+                                              id.p);
+  HIPCHECK(hipGetLastError());
+  sort_pairs(key.p, skey.p, id.p, order.p, nd, key_bits((uint64_t)nn * (nn + 1) + nn), st);
+  invert_kernel<<<nb(nd, 256), 256, 0, st>>>(nd, order.p, inv.p);
+  HIPCHECK(hipGetLastError());
 }
 
 // Reverse Cuthill-McKee order of the graph of a symmetric CSR pattern
@@ -942,7 +993,7 @@ void mesh_topology(Mesh &m, const double *coords, hipStream_t st) {
   int s = 0;
   HIPCHECK(hipMemcpy(&s, m.d_perm.p + m.elems[0], sizeof(int), hipMemcpyDeviceToHost));
   const int64_t hbw = device_bandwidth(n, m.d_rp.p, m.d_col.p, nullptr, st);
-  if (hbw > 5 * device_bfs_max_level(n, m.d_rp.p, m.d_col.p, s, st)) {
+  if (!device_banded(hbw, n, m.d_rp.p, m.d_col.p, s, st)) {
     // reverse Cuthill-McKee over the pattern in the element order
     DevBuf<int> ord(n), inv(n), ip(n);
     rcm(n, m.d_rp.p, m.d_col.p, ord, inv, st);
