@@ -48,6 +48,7 @@ class AdmfemError(RuntimeError):
 _SIGS = {
     "admfem_last_error": (ctypes.c_char_p, []),
     "admfem_version": (c_int, []),
+    "admfem_release_memory": (c_int, []),
     "admfem_system_spmv_repeat": (c_int, [c_vp, c_int, c_int, c_vp, c_vp]),
     "admfem_sparse_solve": (c_int, [c_vp, c_vp, c_i64, c_int, c_vp, c_vp,
                                     ctypes.POINTER(SolveOpts), ctypes.POINTER(SolveStats), c_vp]),

@@ -23,7 +23,7 @@ COMMON = [
     "-Wall", "-Wno-unused-function", "-Wno-unused-result",
 ]
 
-SOURCES = ["mesh.cpp", "api.cpp", "geometry.hip", "assemble.hip", "cg.hip", "mg.hip",
+SOURCES = ["memory.cpp", "mesh.cpp", "api.cpp", "geometry.hip", "assemble.hip", "cg.hip", "mg.hip",
            "dirichlet.hip", "batched.hip", "server.cpp", "sparse_op.hip", "fields.hip",
            "p2.hip", "p2_system.hip", "noalloc.hip", "topology.hip"]
 

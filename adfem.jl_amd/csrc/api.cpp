@@ -70,6 +70,10 @@ using namespace admfem;
 extern "C" {
 
 const char *admfem_last_error(void) { return g_err.c_str(); }
+int admfem_release_memory(void) {
+  return guarded([] { release_device_memory(); });
+}
+
 int admfem_version(void) { return 1; }
 
 // ------------------------------------------------------------ B. meshes

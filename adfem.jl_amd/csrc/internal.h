@@ -32,11 +32,17 @@ struct Error {
     if (!(cond)) throw ::admfem::Error{code, msg};                            \
   } while (0)
 
-// Device buffer (RAII over hipMalloc/hipFree).
+// Device memory with a bounded cache of released blocks (memory.cpp).
+void *device_alloc(size_t bytes, int &device);
+void device_free(void *p, size_t bytes, int device);
+void release_device_memory();
+
+// Device buffer (RAII over device_alloc/device_free).
 template <class T>
 struct DevBuf {
   T *p = nullptr;
   size_t n = 0;
+  int device = -1;
   DevBuf() = default;
   explicit DevBuf(size_t count) { alloc(count); }
   DevBuf(const DevBuf &) = delete;
@@ -44,11 +50,11 @@ struct DevBuf {
   ~DevBuf() { release(); }
   void alloc(size_t count) {
     release();
+    if (count) p = (T *)device_alloc(count * sizeof(T), device);
     n = count;
-    if (count) HIPCHECK(hipMalloc(&p, count * sizeof(T)));
   }
   void release() {
-    if (p) (void)hipFree(p);
+    if (p) device_free(p, n * sizeof(T), device);
     p = nullptr;
     n = 0;
   }
@@ -60,6 +66,7 @@ struct DevBuf {
   void swap(DevBuf &o) {
     std::swap(p, o.p);
     std::swap(n, o.n);
+    std::swap(device, o.device);
   }
   size_t bytes() const { return n * sizeof(T); }
 };

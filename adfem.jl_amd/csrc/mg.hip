@@ -1533,11 +1533,7 @@ struct MgWork {
   uint64_t version = 0;          // of the matrix the set-up was made from
   uint64_t rowsum_version = 0;   // of the matrix the row sums were taken of
   double rowsum = 0.0;
-  hipStream_t cap = nullptr;
-  hipGraphExec_t graph = nullptr;
   ~MgWork() {
-    if (graph) (void)hipGraphExecDestroy(graph);
-    if (cap) (void)hipStreamDestroy(cap);
     if (h_sc) (void)hipHostFree(h_sc);
   }
 };
@@ -1726,30 +1722,10 @@ bool mg_pays(System &s, MgWork *w, hipStream_t st) {
   return !(w->rowsum > MASS_DOMINANT);
 }
 
-constexpr int GRAPH_ITERS = 4;
-
 // Products with the system's matrix in an iteration (mk_res, mk_post,
 // mk_dir): what max_iter bounds and the stats report, as for Jacobi-PCG, whose
 // iterations are one product each.
 constexpr int MG_PRODUCTS = 3;
-
-// GRAPH_ITERS iterations, captured once per system (every pointer comes from
-// the device descriptor) and replayed.
-void launch_graph(const MgPlan &pl, MgWork *w, hipStream_t st) {
-  if (!w->graph) {
-    if (!w->cap) HIPCHECK(hipStreamCreateWithFlags(&w->cap, hipStreamNonBlocking));
-    hipGraph_t g;
-    HIPCHECK(hipStreamBeginCapture(w->cap, hipStreamCaptureModeThreadLocal));
-    for (int k = 0; k < GRAPH_ITERS; k++) iteration(pl, w, w->cap);
-    HIPCHECK(hipStreamEndCapture(w->cap, &g));
-    hipGraphExec_t ex;
-    const hipError_t e = hipGraphInstantiate(&ex, g, nullptr, nullptr, 0);
-    (void)hipGraphDestroy(g);
-    HIPCHECK(e);
-    w->graph = ex;
-  }
-  HIPCHECK(hipGraphLaunch(w->graph, st));
-}
 
 }  // namespace
 
@@ -1790,18 +1766,13 @@ bool mg_solve(System &s, const double *b, double *x_out, const admfem_solve_opts
   // Iterations are enqueued in chunks, each followed by the check (a no-op
   // while CG runs), and the host reads the state between chunks; kernels past
   // the end return at once.  The first chunk is what the system's last solve
-  // took: the adjoint usually takes what the forward did.
+  // took: the adjoint usually takes what the forward did.  Plain launches: the
+  // host queues them faster than the device starts them, replayed graphs
+  // measured the same (64^2 1.09 against 1.10 ms, 1024^2 5.02 against 5.06),
+  // and a capture costs a first solve 0.2 - 3 ms and stops other threads' copies.
   int chunk = o.check_every > 0 ? o.check_every : w->last_it;
   for (;;) {
-    for (int it = 0; it < chunk;) {
-      if (o.check_every != 1 && it + GRAPH_ITERS <= chunk) {
-        launch_graph(pl, w, st);
-        it += GRAPH_ITERS;
-      } else {
-        iteration(pl, w, st);
-        it++;
-      }
-    }
+    for (int it = 0; it < chunk; it++) iteration(pl, w, st);
     mk_check<<<w->nblk, NT, 0, st>>>(nullptr, D, S, 0, b);
     ms_check<<<1, RT, 0, st>>>(D, S, nullptr, 0, w->h_sc);
     HIPCHECK(hipGetLastError());

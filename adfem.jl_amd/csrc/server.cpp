@@ -67,7 +67,11 @@ struct Arena {
     char *p = nullptr;
     if (hipMalloc(&p, size) != hipSuccess) {
       (void)hipGetLastError();
-      return false;
+      release_device_memory();
+      if (hipMalloc(&p, size) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+      }
     }
     segs[p] = size;
     free_[p] = size;

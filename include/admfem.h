@@ -42,6 +42,9 @@ extern "C" {
 
 const char *admfem_last_error(void);
 int admfem_version(void);
+/* Gives the device memory the library keeps for its next buffers (at most
+ * 512 MiB of released ones) back to the driver. */
+int admfem_release_memory(void);
 
 typedef struct admfem_mesh_s *admfem_mesh;
 typedef struct admfem_system_s *admfem_system;
@@ -312,11 +315,14 @@ typedef struct {
 
 /* Solves A x = b with the system's assembled A.  b, x: device [n]; b NULL =
  * the assembled rhs.  x is the output (its input value is ignored).  The
- * solver replays its iterations from a HIP graph (8 iterations, kernel nodes
- * only), captured on the first solve of a setting on a stream of its own
- * and replayed on the caller's; the system holds both until it is
- * destroyed.  check_every = 1 launches every iteration by itself (same
- * kernels and order, the same result bit for bit). */
+ * solver is multigrid-preconditioned CG on grids laid over the mesh, or
+ * Jacobi-PCG for the few systems those do not suit (fewer than 200 rows,
+ * strongly graded meshes, matrices dominated by their mass term).  Jacobi-PCG
+ * replays its iterations from a HIP graph (8 iterations, kernel nodes only),
+ * captured on the first solve of a setting on a stream of its own and
+ * replayed on the caller's; the system holds both until it is destroyed.
+ * check_every = 1 launches every iteration by itself (same kernels and order,
+ * the same result bit for bit). */
 int admfem_system_solve(admfem_system s, const double *b, double *x,
                         const admfem_solve_opts *o, admfem_solve_stats *st,
                         void *stream);
