@@ -62,6 +62,7 @@ struct MgSys {
                             // inverse of the last one behind them
   int n, npad, nblk;
   int nlev, tail;           // grid levels, first one of the tail kernel
+  int steps;                // fine smoothing steps before and after (1 or 2)
   MgLevel lv[MG_MAXLEV];
 };
 
@@ -84,7 +85,7 @@ struct MgScal {
 // A topology's grids (made once per system, mg_plan).
 struct MgPlan {
   bool ok = false;          // false: the rows do not suit one uniform grid
-  int nlev = 0, tail = 0;
+  int nlev = 0, tail = 0, steps = 1;
   int nx[MG_MAXLEV], ny[MG_MAXLEV], px[MG_MAXLEV], pn[MG_MAXLEV];
   DevBuf<int> cell, cptr, crow, pos;
   DevBuf<float2> frac, cfrac;
@@ -107,7 +108,7 @@ size_t mg_tail_lds(const MgPlan &pl);
 
 // A batch of systems (descriptors of D, states of S by slot): the block maps
 // of every kind of wide launch ((slot, block) per grid block), and the slots.
-enum { MGS_ROWS = 0, MGS_GALERKIN, MGS_RESTRICT, MGS_SETUP,
+enum { MGS_ROWS = 0, MGS_TWO, MGS_GALERKIN, MGS_RESTRICT, MGS_SETUP,
        MGS_DOWN = MGS_SETUP + MG_MAXLEV, MGS_UP = MGS_DOWN + MG_MAXLEV,
        MG_STAGES = MGS_UP + MG_MAXLEV };
 struct MgBatch {

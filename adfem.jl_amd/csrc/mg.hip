@@ -3,7 +3,7 @@
 // over a hierarchy of uniform grids.
 //
 // Jacobi-PCG takes O(1/h) iterations (4,800 at 1024^2); the V-cycle keeps the
-// count at 13 - 16 for P1 at every size (P2: 16 - 27), so a solve reads the
+// count at 11 - 13 for P1 at every size (P2: 12 - 15), so a solve reads the
 // matrix about 60 times in all.  One forward + adjoint on MI355X, Jacobi-PCG
 // -> this: Poisson 64^2 FP64 9.1 -> 1.7 ms, 511^2 FP64 81 -> 3.6 ms, 1024^2
 // mixed 276 -> 5.9 ms, heat 200^2 16.5 -> 2.4 ms, P2 101^2 43 -> 4.7 ms; the
@@ -28,15 +28,17 @@
 // A solve is converged when the residual recomputed from the FP64 matrix is.
 //
 // One iteration (every kernel returns at once when its system is done):
-//   mk_res       residual of the first smoothing step (taken from zero where
-//                the residual itself is written)
+//   mk_pre       second smoothing step (the first, from zero, is taken where
+//                the residual itself is written); plans with two steps
+//   mk_res       residual after it
 //   mk_restrict  to the first grid, with its first smoothing step
 //   gk_down      the grids down to MG_TAIL nodes: residual and restriction of
 //                a tile in one launch
 //   mk_tail      the remaining grids, one workgroup per system, in LDS
 //   gk_up        and up: prolongation and smoothing of a tile; the first grid
 //                also interpolates its rows
-//   mk_post      the fine level's second smoothing step: z, partials of r.z
+//   mk_mid, mk_post  the fine level's smoothing (mk_mid: plans with two
+//                steps): z, partials of r.z
 //   mk_dir       beta = r.z / previous r.z, p = z + beta p, q = A p; partials
 //                of p.q, r.q, q.q, r.r
 //   mk_update    alpha = r.z / p.q, the new |r|^2 = r.r - 2 alpha r.q +
@@ -53,6 +55,7 @@
 
 #include <chrono>
 #include <cmath>
+#include <mutex>
 
 #include "batched.h"
 #include "geom.h"
@@ -69,6 +72,10 @@ constexpr int ST_RUN = 0, ST_CONV = 1, ST_MAXIT = 2, ST_NAN = 3, ST_BREAK = 4;
 // Smoothing weight: any value below 2 is safe; 1.6 took the fewest
 // iterations over jittered meshes (15 with 4/3, 13 - 14 with 1.5 - 1.7).
 constexpr float OM = 1.6f;
+// Two smoothing steps on the fine level instead (plans with steps = 2): the
+// degree-2 Chebyshev polynomial of M^-1 A for its spectrum's part [1/8, 1],
+// first step x + C0 M^-1 r, second x' + CM (x' - x) + C1 M^-1 r'.
+constexpr float C0 = 16.0f / 9.0f, CM = 0.43369f, C1 = 2.54902f;
 // Partials that the wide kernels' blocks sum themselves, at most.
 constexpr int MG_SUM = 1280;
 
@@ -465,7 +472,12 @@ __global__ void __launch_bounds__(RT) ms_rowsum(int G, double *__restrict__ out)
 __device__ __forceinline__ void first_smooth(const MgSys &d, int i, double ri) {
   const float rs = (float)(ri * global_ptr(d.dsq)[i]);
   global_mut(d.rs)[i] = rs;
-  global_mut(d.x0)[i] = OM * global_ptr(d.minv)[i] * rs;
+  global_mut(d.x0)[i] = (d.steps == 2 ? C0 : OM) * global_ptr(d.minv)[i] * rs;
+}
+
+// Where the smoothing before the correction left its result.
+__device__ __forceinline__ const float *smoothed(const MgSys &d) {
+  return d.steps == 2 ? d.t : d.x0;
 }
 
 // Row i's product with the FP32 scaled off-diagonals.
@@ -679,10 +691,9 @@ __global__ void __launch_bounds__(NT)
   first_smooth(d, i, ri);
 }
 
-// ts = the fine residual after the first smoothing step, in the unscaled
-// form's dual, sqrt(a_ii) (rs - Â x0), in the order of the cells
+// The second smoothing step from zero (steps = 2): t
 __global__ void __launch_bounds__(NT)
-    mk_res(const int2 *__restrict__ map, const MgSys *__restrict__ D, const MgScal *S, int sys) {
+    mk_pre(const int2 *__restrict__ map, const MgSys *__restrict__ D, const MgScal *S, int sys) {
   const int2 m = where(map, sys);
   if (m.x < 0 || S[m.x].a.status != ST_RUN) return;
   const MgSys &d = D[m.x];
@@ -691,6 +702,38 @@ __global__ void __launch_bounds__(NT)
   const gptr<float> x0 = global_ptr(d.x0);
   const double res = (double)global_ptr(d.rs)[i] - (double)x0[i] -
                      dot32(d, i, [&](int c) { return x0[c]; });
+  global_mut(d.t)[i] = (float)((1.0 + (double)CM) * (double)x0[i] +
+                               (double)(C1 * global_ptr(d.minv)[i]) * res);
+}
+
+// The first of two smoothing steps after the correction (steps = 2):
+// x0 = t + C0 M^-1 (rs - Â t)
+__global__ void __launch_bounds__(NT)
+    mk_mid(const int2 *__restrict__ map, const MgSys *__restrict__ D, const MgScal *S, int sys) {
+  const int2 m = where(map, sys);
+  if (m.x < 0 || S[m.x].a.status != ST_RUN) return;
+  const MgSys &d = D[m.x];
+  const int i = m.y * NT + threadIdx.x;
+  if (i >= d.npad) return;
+  const gptr<float> t = global_ptr(d.t);
+  const double res = (double)global_ptr(d.rs)[i] - (double)t[i] -
+                     dot32(d, i, [&](int c) { return t[c]; });
+  global_mut(d.x0)[i] =
+      (float)fma((double)(C0 * global_ptr(d.minv)[i]), res, (double)t[i]);
+}
+
+// ts = the fine residual after the first smoothing step(s), in the unscaled
+// form's dual, sqrt(a_ii) (rs - Â x0), in the order of the cells
+__global__ void __launch_bounds__(NT)
+    mk_res(const int2 *__restrict__ map, const MgSys *__restrict__ D, const MgScal *S, int sys) {
+  const int2 m = where(map, sys);
+  if (m.x < 0 || S[m.x].a.status != ST_RUN) return;
+  const MgSys &d = D[m.x];
+  const int i = m.y * NT + threadIdx.x;
+  if (i >= d.npad) return;
+  const gptr<float> x = global_ptr(smoothed(d));
+  const double res = (double)global_ptr(d.rs)[i] - (double)x[i] -
+                     dot32(d, i, [&](int c) { return x[c]; });
   const int k = global_ptr(d.pos)[i];
   if (k >= 0) global_mut(d.ts)[k] = (float)(res * (double)global_ptr(d.sq)[i]);
 }
@@ -888,6 +931,7 @@ __global__ void __launch_bounds__(TT)
   const int ncx = l.nx - 1, ncy = l.ny - 1;
   const gptr<int> cptr = global_ptr(d.cptr), crow = global_ptr(d.crow);
   const gptr<f2_t> cfrac = frac_ptr(d.cfrac);
+  const gptr<float> x = global_ptr(smoothed(d));
   for (int i = threadIdx.x; i < TF * TF; i += TT) {
     const int ix = i % TF, iy = i / TF, cx = x0 + ix, cy = y0 + iy;
     if (cx >= ncx || cy >= ncy) continue;
@@ -895,7 +939,7 @@ __global__ void __launch_bounds__(TT)
     for (int q = cptr[cl]; q < k1; q++) {
       const int r = crow[q];
       global_mut(d.t)[r] = fmaf(global_ptr(d.sq)[r], bilinear(cfrac[q], xs + iy * W + ix, W),
-                                global_ptr(d.x0)[r]);
+                                x[r]);
     }
   }
 }
@@ -1124,7 +1168,7 @@ __global__ void __launch_bounds__(RT)
   }
   const gptr<int> cell = global_ptr(d.cell);
   const gptr<f2_t> frac = frac_ptr(d.frac);
-  const gptr<float> sq = global_ptr(d.sq), x0 = global_ptr(d.x0);
+  const gptr<float> sq = global_ptr(d.sq), x0 = global_ptr(smoothed(d));
   const float icx = 1.0f / (float)(fx - 1);
   for (int i = tid; i < d.npad; i += 4 * RT) {  // four rows' loads in flight
     int c[4];
@@ -1148,7 +1192,8 @@ __global__ void __launch_bounds__(RT)
   }
 }
 
-// z = S (t + w M^-1 (rs - Â t)); partials of r.z
+// z = S (t + w M^-1 (rs - Â t)), or the second step after mk_mid's; partials
+// of r.z
 __global__ void __launch_bounds__(NT)
     mk_post(const int2 *__restrict__ map, const MgSys *__restrict__ D, const MgScal *S, int sys) {
   const int2 m = where(map, sys);
@@ -1157,13 +1202,22 @@ __global__ void __launch_bounds__(NT)
   const int i = m.y * NT + threadIdx.x;
   double v[1] = {0.0};
   if (i < d.npad) {
-    const gptr<float> t = global_ptr(d.t);
-    // a row outside the grids (Dirichlet, uncoupled) has no t: its value is x0
-    const float ti = global_ptr(d.pos)[i] < 0 ? global_ptr(d.x0)[i] : t[i];
-    const double res = (double)global_ptr(d.rs)[i] - (double)ti -
-                       dot32(d, i, [&](int c) { return t[c]; });
-    const float zi = (float)(fma((double)(OM * global_ptr(d.minv)[i]), res, (double)ti) *
-                             global_ptr(d.dsq)[i]);
+    float zi;
+    if (d.steps == 2) {
+      const gptr<float> x = global_ptr(d.x0);  // mk_mid's step
+      const double xi = (double)x[i], res = (double)global_ptr(d.rs)[i] - xi -
+                                            dot32(d, i, [&](int c) { return x[c]; });
+      zi = (float)((xi + (double)CM * (xi - (double)global_ptr(d.t)[i]) +
+                    (double)(C1 * global_ptr(d.minv)[i]) * res) * global_ptr(d.dsq)[i]);
+    } else {
+      const gptr<float> t = global_ptr(d.t);
+      // a row outside the grids (Dirichlet, uncoupled) has no t: its value is x0
+      const float ti = global_ptr(d.pos)[i] < 0 ? global_ptr(d.x0)[i] : t[i];
+      const double res = (double)global_ptr(d.rs)[i] - (double)ti -
+                         dot32(d, i, [&](int c) { return t[c]; });
+      zi = (float)(fma((double)(OM * global_ptr(d.minv)[i]), res, (double)ti) *
+                   global_ptr(d.dsq)[i]);
+    }
     global_mut(d.z)[i] = zi;
     v[0] = global_ptr(d.r)[i] * (double)zi;
   }
@@ -1424,6 +1478,12 @@ MgPlan *build_plan(System &s, const Mesh &m, const int *order, hipStream_t st) {
     // a graded mesh puts many rows into some cells: the grid is then too
     // coarse there for the smoother, and plain Jacobi-PCG keeps the system
     if (rows > 10.0 * occ || most > 64) return pl;
+    // One fine smoothing step where the cells are wide against the couplings
+    // (a uniform grid: 2; P1 forward + adjoint, one -> two steps: 150^2 1.44 ->
+    // 1.61 ms, 300^2 1.78 -> 1.93, 700^2 even); else two (P1 jittered by a
+    // fifth, 1.43: 100^2 1.55 -> 1.33 ms, 511^2 2.62 -> 2.42, 700^2 3.72 ->
+    // 3.06; P2, 1: 101^2 3.47 -> 2.43 ms, 190^2 5.07 -> 3.44).
+    pl->steps = hx > 1.6 * ex && hy > 1.6 * ey ? 1 : 2;
     int k = 0;
     pl->tail = -1;
     for (;; k++) {
@@ -1473,6 +1533,8 @@ void mg_allow_lds(const MgPlan &pl) {
 void mg_plan_free(MgPlan *p) { delete p; }
 
 const MgPlan *mg_plan(System &s, hipStream_t st) {
+  static std::mutex mu;  // an engine and a solver may share the system
+  std::lock_guard<std::mutex> g(mu);
   if (!s.mg_plan && s.mesh) s.mg_plan = build_plan(s, *s.mesh, nullptr, st);
   return s.mg_plan && s.mg_plan->ok ? s.mg_plan : nullptr;
 }
@@ -1491,6 +1553,7 @@ void mg_grid_layout(const MgPlan &pl, float *base, MgSys &d) {
   d.crow = pl.crow.p;
   d.cfrac = pl.cfrac.p;
   d.pos = pl.pos.p;
+  d.steps = pl.steps;
   d.nlev = pl.nlev;
   d.tail = pl.tail;
   for (int k = 0; k < pl.nlev; k++) {
@@ -1618,6 +1681,7 @@ static int mg_tiles_up(const MgPlan &pl, int k) {
 void mg_stages(const MgPlan &pl, int npad, int (&nblk)[MG_STAGES]) {
   for (int &v : nblk) v = 0;
   nblk[MGS_ROWS] = (int)nb(npad, NT);
+  if (pl.steps == 2) nblk[MGS_TWO] = nblk[MGS_ROWS];
   nblk[MGS_GALERKIN] = (int)nb((int64_t)pl.nx[0] * pl.ny[0], GT / 4);
   if (pl.tail > 0) nblk[MGS_RESTRICT] = (int)nb((int64_t)pl.nx[0] * pl.ny[0], NT / 4);
   for (int k = 0; k < pl.tail; k++) {
@@ -1650,6 +1714,7 @@ void mg_batch_iterations(const MgBatch &B, const MgSys *D, MgScal *S, int iters,
   const int2 *rows = B.map[MGS_ROWS];
   const unsigned nl = (unsigned)B.nsys, nr = n(MGS_ROWS);
   for (int it = 0; it < iters; it++) {
+    if (n(MGS_TWO)) mk_pre<<<n(MGS_TWO), NT, 0, st>>>(B.map[MGS_TWO], D, S, 0);
     mk_res<<<nr, NT, 0, st>>>(rows, D, S, 0);
     if (B.tail > 0)
       mk_restrict<<<n(MGS_RESTRICT), NT, 0, st>>>(B.map[MGS_RESTRICT], D, S, 0);
@@ -1659,6 +1724,7 @@ void mg_batch_iterations(const MgBatch &B, const MgSys *D, MgScal *S, int iters,
     for (int k = B.tail - 1; k > 0; k--)
       gk_up<false><<<n(MGS_UP + k), TT, 0, st>>>(B.map[MGS_UP + k], D, S, 0, k);
     if (B.tail > 0) gk_up<true><<<n(MGS_UP), TT, 0, st>>>(B.map[MGS_UP], D, S, 0, 0);
+    if (n(MGS_TWO)) mk_mid<<<n(MGS_TWO), NT, 0, st>>>(B.map[MGS_TWO], D, S, 0);
     mk_post<<<nr, NT, 0, st>>>(rows, D, S, 0);
     if (B.reduce) ms_reduce<1><<<nl, RT, 0, st>>>(D, S, B.list, 0);
     mk_dir<<<nr, NT, 0, st>>>(rows, D, S, 0);
@@ -1686,6 +1752,7 @@ namespace {
 void iteration(const MgPlan &pl, MgWork *w, hipStream_t st) {
   const MgSys *D = w->d.p;
   MgScal *S = w->sc.p;
+  if (pl.steps == 2) mk_pre<<<w->nblk, NT, 0, st>>>(nullptr, D, S, 0);
   mk_res<<<w->nblk, NT, 0, st>>>(nullptr, D, S, 0);
   if (pl.tail > 0)
     mk_restrict<<<nb(pl.nx[0] * pl.ny[0], NT / 4), NT, 0, st>>>(nullptr, D, S, 0);
@@ -1695,6 +1762,7 @@ void iteration(const MgPlan &pl, MgWork *w, hipStream_t st) {
   for (int k = pl.tail - 1; k > 0; k--)
     gk_up<false><<<mg_tiles_up(pl, k), TT, 0, st>>>(nullptr, D, S, 0, k);
   if (pl.tail > 0) gk_up<true><<<mg_tiles_up(pl, 0), TT, 0, st>>>(nullptr, D, S, 0, 0);
+  if (pl.steps == 2) mk_mid<<<w->nblk, NT, 0, st>>>(nullptr, D, S, 0);
   mk_post<<<w->nblk, NT, 0, st>>>(nullptr, D, S, 0);
   if (w->nblk > MG_SUM) ms_reduce<1><<<1, RT, 0, st>>>(D, S, nullptr, 0);
   mk_dir<<<w->nblk, NT, 0, st>>>(nullptr, D, S, 0);
