@@ -105,8 +105,11 @@ _SIGS = {
     "admfem_dof_to_gauss_points_grad": (c_int, [c_vp, c_vp, c_vp, c_vp]),
     "admfem_fem_grad": (c_int, [c_vp, c_vp, c_vp, c_vp]),
     "admfem_fem_grad_grad": (c_int, [c_vp, c_vp, c_vp, c_vp]),
+    "admfem_fem_grad_grad_on": (c_int, [c_vp, c_vp, c_vp, c_vp, c_vp]),
     "admfem_fem_laplace_term": (c_int, [c_vp, c_vp, c_vp, c_vp, c_vp]),
+    "admfem_fem_laplace_term_on": (c_int, [c_vp, c_vp, c_vp, c_vp, c_vp, c_vp]),
     "admfem_fem_laplace_term_grad": (c_int, [c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp]),
+    "admfem_fem_laplace_term_grad_on": (c_int, [c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp]),
     "admfem_impose_dirichlet": (c_int, [c_vp, c_vp, c_i64, c_vp, c_vp, c_int, c_vp, c_int,
                                         c_vp, c_vp, c_vp, c_vp, c_vp]),
     "admfem_impose_dirichlet_grad": (c_int, [c_vp, c_vp, c_vp, c_vp, c_i64, c_vp, c_vp, c_int,

@@ -211,6 +211,11 @@ def dof_to_gauss_points(u, mesh):
     return out.cpu().numpy() if host else out
 
 
+def _work(mesh):
+    """Scratch for the maps that pass the elements' terms through memory."""
+    return torch.empty(mesh.elem_ndof * mesh.nelem, dtype=torch.float64, device=_DEV)
+
+
 class _FemGrad(torch.autograd.Function):
     @staticmethod
     def forward(ctx, u, mesh):
@@ -225,8 +230,9 @@ class _FemGrad(torch.autograd.Function):
     def backward(ctx, g):
         g = _dev(g)
         gu = torch.empty(ctx.mesh.ndof, dtype=torch.float64, device=_DEV)
-        _lib.check(_lib.lib().admfem_fem_grad_grad(ctx.mesh.handle, _lib.ptr(g), _lib.ptr(gu),
-                                                   _lib.stream_ptr()))
+        work = _work(ctx.mesh)
+        _lib.check(_lib.lib().admfem_fem_grad_grad_on(ctx.mesh.handle, _lib.ptr(g), _lib.ptr(gu),
+                                                      _lib.ptr(work), _lib.stream_ptr()))
         return gu, None
 
 
@@ -243,8 +249,10 @@ class _LaplaceTerm(torch.autograd.Function):
     def forward(ctx, u, nu, mesh):
         uu, nn = _dev(u), _dev(nu)
         out = torch.empty(mesh.ndof, dtype=torch.float64, device=_DEV)
-        _lib.check(_lib.lib().admfem_fem_laplace_term(mesh.handle, _lib.ptr(uu), _lib.ptr(nn),
-                                                      _lib.ptr(out), _lib.stream_ptr()))
+        work = _work(mesh)
+        _lib.check(_lib.lib().admfem_fem_laplace_term_on(
+            mesh.handle, _lib.ptr(uu), _lib.ptr(nn), _lib.ptr(out), _lib.ptr(work),
+            _lib.stream_ptr()))
         ctx.save_for_backward(uu, nn)
         ctx.mesh = mesh
         return out
@@ -255,9 +263,10 @@ class _LaplaceTerm(torch.autograd.Function):
         g = _dev(g)
         gu = torch.empty_like(uu) if ctx.needs_input_grad[0] else None
         gn = torch.empty_like(nn) if ctx.needs_input_grad[1] else None
-        _lib.check(_lib.lib().admfem_fem_laplace_term_grad(
+        work = _work(ctx.mesh) if gu is not None else None
+        _lib.check(_lib.lib().admfem_fem_laplace_term_grad_on(
             ctx.mesh.handle, _lib.ptr(g), _lib.ptr(uu), _lib.ptr(nn), _lib.ptr(gu),
-            _lib.ptr(gn), _lib.stream_ptr()))
+            _lib.ptr(gn), _lib.ptr(work), _lib.stream_ptr()))
         return gu, gn, None
 
 

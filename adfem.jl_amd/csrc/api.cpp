@@ -266,27 +266,43 @@ int admfem_fem_grad(admfem_mesh h, const double *u, double *out, void *stream) {
   });
 }
 
-int admfem_fem_grad_grad(admfem_mesh h, const double *grad_out, double *grad_u, void *stream) {
+int admfem_fem_grad_grad_on(admfem_mesh h, const double *grad_out, double *grad_u, double *work,
+                            void *stream) {
   return guarded([&] {
     REQUIRE(grad_out && grad_u, ADMFEM_ERR_ARG, "null pointer");
-    launch_fem_grad_grad(M(h), grad_out, grad_u, S(stream));
+    launch_fem_grad_grad(M(h), grad_out, grad_u, work, S(stream));
+  });
+}
+
+int admfem_fem_grad_grad(admfem_mesh h, const double *grad_out, double *grad_u, void *stream) {
+  return admfem_fem_grad_grad_on(h, grad_out, grad_u, nullptr, stream);
+}
+
+int admfem_fem_laplace_term_on(admfem_mesh h, const double *u, const double *nu, double *out,
+                               double *work, void *stream) {
+  return guarded([&] {
+    REQUIRE(u && nu && out, ADMFEM_ERR_ARG, "null pointer");
+    launch_laplace_term(M(h), u, nu, out, work, S(stream));
   });
 }
 
 int admfem_fem_laplace_term(admfem_mesh h, const double *u, const double *nu, double *out,
                             void *stream) {
-  return guarded([&] {
-    REQUIRE(u && nu && out, ADMFEM_ERR_ARG, "null pointer");
-    launch_laplace_term(M(h), u, nu, out, S(stream));
-  });
+  return admfem_fem_laplace_term_on(h, u, nu, out, nullptr, stream);
 }
 
 int admfem_fem_laplace_term_grad(admfem_mesh h, const double *grad_out, const double *u,
                                  const double *nu, double *grad_u, double *grad_nu,
                                  void *stream) {
+  return admfem_fem_laplace_term_grad_on(h, grad_out, u, nu, grad_u, grad_nu, nullptr, stream);
+}
+
+int admfem_fem_laplace_term_grad_on(admfem_mesh h, const double *grad_out, const double *u,
+                                    const double *nu, double *grad_u, double *grad_nu,
+                                    double *work, void *stream) {
   return guarded([&] {
     REQUIRE(grad_out && u && nu, ADMFEM_ERR_ARG, "null pointer");
-    if (grad_u) launch_laplace_term(M(h), grad_out, nu, grad_u, S(stream));
+    if (grad_u) launch_laplace_term(M(h), grad_out, nu, grad_u, work, S(stream));
     if (grad_nu) launch_laplace_term_nu_grad(M(h), grad_out, u, grad_nu, S(stream));
   });
 }
@@ -833,7 +849,7 @@ void ComputeLaplaceTermMfem_forward_Julia(double *out, const double *nu, const d
     DevBuf<double> du, dnu, dk(m->ndof);
     du.upload(u, m->ndof);
     dnu.upload(nu, m->ngauss);
-    launch_laplace_term(*m, du.p, dnu.p, dk.p, nullptr);
+    launch_laplace_term(*m, du.p, dnu.p, dk.p, nullptr, nullptr);
     std::vector<double> k(m->ndof);
     d2h(k.data(), dk.p, k.size());
     for (size_t i = 0; i < k.size(); i++) out[i] += k[i];  // accumulates, as the reference

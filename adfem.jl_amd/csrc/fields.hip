@@ -10,9 +10,10 @@
 //     ComputeLaplaceTermMfem.h:4-39): out = K(nu) u without forming K.
 // Fields are in the user's node order, Gauss arrays in the user's element
 // order (g = nq e + k).  Forward maps to Gauss points run one thread per
-// Gauss point; every map to the nodes (the backward ops and the Laplace
-// term) is a per-node gather over the node's incident elements: one writer
-// per output, no atomics.
+// Gauss point.  The maps to the nodes have one writer per output and no
+// atomics: a gather over the node's incident elements, or, where deriving an
+// element's geometry anew at each of its nodes costs more than passing its
+// terms through memory, a pass over the elements and a pass over the nodes.
 #include "geom.h"
 
 namespace admfem {
@@ -67,11 +68,8 @@ __global__ void fem_grad_kernel(int nelem, QuadRule rule, const int *__restrict_
   out[2 * g + 1] = gy;
 }
 
-// Per node: the transposes of the two maps above, and K(nu) u.
-// NODE_LAPLACE reads its field in the internal node order (permuted once by
-// the launcher), so each incidence's three values are local gathers through
-// the element's internal vertex ids instead of random ones in user order.
-enum { NODE_TO_GAUSS_T = 0, NODE_GRAD_T = 1, NODE_LAPLACE = 2 };
+// Per node: the transposes of the two maps above.
+enum { NODE_TO_GAUSS_T = 0, NODE_GRAD_T = 1 };
 
 template <int OP, int NQ>
 __global__ void __launch_bounds__(256) node_gather_kernel(int n, int nelem, QuadRule rule, const int *__restrict__ conn,
@@ -81,9 +79,7 @@ __global__ void __launch_bounds__(256) node_gather_kernel(int n, int nelem, Quad
                                    const int *__restrict__ n2e_elem,
                                    const uint32_t *__restrict__ slots,
                                    const int *__restrict__ iperm,
-                                   const double *__restrict__ gw,   // mesh Gauss weights
-                                   const double *__restrict__ in,   // Gauss array or field
-                                   const double *__restrict__ nu,   // NODE_LAPLACE
+                                   const double *__restrict__ in,   // Gauss array
                                    double *__restrict__ out_user) {
   const int r = blockIdx.x * blockDim.x + threadIdx.x;
   if (r >= n) return;
@@ -102,27 +98,78 @@ __global__ void __launch_bounds__(256) node_gather_kernel(int n, int nelem, Quad
       const Tri tr = load_tri(conn, nelem, e, x, y);
       double gx[3], gy[3];
       elem_grads(tr.x[0], tr.y[0], tr.x[1], tr.y[1], tr.x[2], tr.y[2], gx, gy);
-      if (OP == NODE_GRAD_T) {
 #pragma unroll
-        for (int k = 0; k < NQ; k++) {
-          const size_t g = (size_t)NQ * e + k;
-          acc += in[2 * g] * gx[p] + in[2 * g + 1] * gy[p];
-        }
-      } else {  // K(nu) u: sum_k nu_k w_k grad phi_p . grad u_e
-        double ux = 0.0, uy = 0.0;
-#pragma unroll
-        for (int q = 0; q < 3; q++) {
-          const double uq = in[conn[(size_t)q * nelem + e]];
-          ux += gx[q] * uq;
-          uy += gy[q] * uq;
-        }
-        double cw = 0.0;
-#pragma unroll
-        for (int k = 0; k < NQ; k++) cw += nu[(size_t)NQ * e + k] * gw[(size_t)NQ * e + k];
-        acc += cw * (gx[p] * ux + gy[p] * uy);
+      for (int k = 0; k < NQ; k++) {
+        const size_t g = (size_t)NQ * e + k;
+        acc += in[2 * g] * gx[p] + in[2 * g + 1] * gy[p];
       }
     }
   }
+  out_user[iperm[r]] = acc;
+}
+
+// The two passes of K(nu) u and of fem_grad's transpose.  Element e's term of
+// its vertex p goes to c[p nelem + e]; the node pass sums each node's terms
+// in ascending element order.  Both are bound by memory: the element pass
+// streams the Gauss arrays once (the one-pass gather met each element's
+// values and vertex ids six times, in the nodes' order) and the node pass
+// reads one scattered double per incidence.  K(nu) u: 9.6 -> 6.3 us at 64^2,
+// 64 -> 43 us at 700^2; fem_grad's transpose at 700^2: 55 -> 32 us.
+template <bool LAPLACE, int NQ>
+__global__ void __launch_bounds__(256)
+    elem_terms_kernel(int nelem, const int *__restrict__ conn, const int *__restrict__ conn_user,
+                      const double2 *__restrict__ xy, const double *__restrict__ gw,
+                      const double *__restrict__ in,  // LAPLACE: field, else Gauss array (x, y)
+                      const double *__restrict__ nu, double *__restrict__ c) {
+  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= nelem) return;
+  double2 v[3];
+#pragma unroll
+  for (int q = 0; q < 3; q++) v[q] = xy[conn[(size_t)q * nelem + e]];
+  double gx[3], gy[3], sx = 0.0, sy = 0.0;
+  elem_grads(v[0].x, v[0].y, v[1].x, v[1].y, v[2].x, v[2].y, gx, gy);
+  if (LAPLACE) {  // sum_k nu_k w_k grad phi_p . grad u_e
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+      const double uq = in[conn_user[(size_t)q * nelem + e]];
+      sx += gx[q] * uq;
+      sy += gy[q] * uq;
+    }
+    double cw = 0.0;
+#pragma unroll
+    for (int k = 0; k < NQ; k++) cw += nu[(size_t)NQ * e + k] * gw[(size_t)NQ * e + k];
+    sx *= cw;
+    sy *= cw;
+  } else {
+#pragma unroll
+    for (int k = 0; k < NQ; k++) {
+      const size_t g = (size_t)NQ * e + k;
+      sx += in[2 * g];
+      sy += in[2 * g + 1];
+    }
+  }
+#pragma unroll
+  for (int p = 0; p < 3; p++) c[(size_t)p * nelem + e] = sx * gx[p] + sy * gy[p];
+}
+
+__global__ void __launch_bounds__(256)
+    node_sum_kernel(int n, int nelem, const int *__restrict__ n2e_ptr,
+                    const int *__restrict__ n2e_elem, const uint32_t *__restrict__ slots,
+                    const int *__restrict__ iperm, const double *__restrict__ c,
+                    double *__restrict__ out_user) {
+  const int r = blockIdx.x * blockDim.x + threadIdx.x;
+  if (r >= n) return;
+  const int t1 = n2e_ptr[r + 1];
+  double acc = 0.0;
+  int t = n2e_ptr[r];
+  for (; t + 2 < t1; t += 3) {  // three terms' loads in flight
+    double v[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++) v[k] = c[(size_t)(slots[t + k] & 3u) * nelem + n2e_elem[t + k]];
+#pragma unroll
+    for (int k = 0; k < 3; k++) acc += v[k];
+  }
+  for (; t < t1; t++) acc += c[(size_t)(slots[t] & 3u) * nelem + n2e_elem[t]];
   out_user[iperm[r]] = acc;
 }
 
@@ -154,27 +201,39 @@ __global__ void laplace_term_nu_grad_kernel(int nelem, QuadRule rule, const int 
 
 inline unsigned nb(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 
-// dst[r] = src[iperm[r]]: a user-order field in the internal order
-__global__ void permute_kernel(int n, const int *__restrict__ iperm,
-                               const double *__restrict__ src, double *__restrict__ dst) {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r < n) dst[r] = src[iperm[r]];
-}
-
 template <int OP>
-void node_gather(const Mesh &m, const double *in, const double *nu, double *out_user,
-                 hipStream_t st) {
+void node_gather(const Mesh &m, const double *in, double *out_user, hipStream_t st) {
   auto go = [&](auto kern) {
     kern<<<nb(m.nnode, 256), 256, 0, st>>>(m.nnode, m.nelem, m.rule, m.conn.p, m.conn_user.p,
                                            m.x.p, m.y.p, m.d_n2e_ptr.p, m.d_n2e_elem.p,
-                                           m.d_slots_full.p, m.d_iperm.p, m.gw.p, in, nu,
-                                           out_user);
+                                           m.d_slots_full.p, m.d_iperm.p, in, out_user);
   };
   if (m.rule.nq == 3) go(node_gather_kernel<OP, 3>);
   else if (m.rule.nq == 6) go(node_gather_kernel<OP, 6>);
   else go(node_gather_kernel<OP, 1>);
   HIPCHECK(hipGetLastError());
 }
+
+template <bool LAPLACE>
+void two_pass(const Mesh &m, const double *in, const double *nu, double *out_user, double *c,
+              hipStream_t st) {
+  auto go = [&](auto kern) {
+    kern<<<nb(m.nelem, 256), 256, 0, st>>>(m.nelem, m.conn.p, m.conn_user.p, m.xy.p, m.gw.p, in,
+                                           nu, c);
+  };
+  if (m.rule.nq == 3) go(elem_terms_kernel<LAPLACE, 3>);
+  else if (m.rule.nq == 6) go(elem_terms_kernel<LAPLACE, 6>);
+  else go(elem_terms_kernel<LAPLACE, 1>);
+  node_sum_kernel<<<nb(m.nnode, 256), 256, 0, st>>>(m.nnode, m.nelem, m.d_n2e_ptr.p,
+                                                    m.d_n2e_elem.p, m.d_slots_full.p,
+                                                    m.d_iperm.p, c, out_user);
+  HIPCHECK(hipGetLastError());
+}
+
+// fem_grad's transpose takes the two passes from here on: below, the second
+// launch costs what the passes save (one pass / two: 200^2 7.0 / 7.7 us,
+// 250^2 8.5 / 8.8, 360^2 14.1 / 12.1, 700^2 55 / 32).
+constexpr int GRAD_T_TWO_PASS = 100000;
 
 }  // namespace
 
@@ -185,7 +244,7 @@ void launch_to_gauss(const Mesh &m, const double *u, double *out, hipStream_t st
 
 void launch_to_gauss_grad(const Mesh &m, const double *grad_out, double *grad_u,
                           hipStream_t st) {
-  node_gather<NODE_TO_GAUSS_T>(m, grad_out, nullptr, grad_u, st);
+  node_gather<NODE_TO_GAUSS_T>(m, grad_out, grad_u, st);
 }
 
 void launch_dof_to_gauss(const Mesh &m, const double *u, double *out, hipStream_t st) {
@@ -206,22 +265,25 @@ void launch_fem_grad(const Mesh &m, const double *u, double *out, hipStream_t st
   HIPCHECK(hipGetLastError());
 }
 
-void launch_fem_grad_grad(const Mesh &m, const double *grad_out, double *grad_u,
+void launch_fem_grad_grad(const Mesh &m, const double *grad_out, double *grad_u, double *work,
                           hipStream_t st) {
-  if (m.degree == 2) return launch_p2_fem_grad_grad(m, grad_out, grad_u, st);
-  node_gather<NODE_GRAD_T>(m, grad_out, nullptr, grad_u, st);
+  if (m.degree == 2) return launch_p2_fem_grad_grad(m, grad_out, grad_u, work, st);
+  if (work && m.nnode >= GRAD_T_TWO_PASS)
+    two_pass<false>(m, grad_out, nullptr, grad_u, work, st);
+  else
+    node_gather<NODE_GRAD_T>(m, grad_out, grad_u, st);
 }
 
-// u (user order) -> internal order in a stream-ordered temporary, then the
-// per-node gather
+// A caller without scratch gets a stream-ordered temporary (10 us on the host,
+// 20 to 30 when the stream has drained since the last one).
 void launch_laplace_term(const Mesh &m, const double *u, const double *nu, double *out,
-                         hipStream_t st) {
-  if (m.degree == 2) return launch_p2_laplace_term(m, u, nu, out, st);
-  double *u_int = nullptr;
-  HIPCHECK(hipMallocAsync((void **)&u_int, sizeof(double) * std::max(m.nnode, 1), st));
-  permute_kernel<<<nb(m.nnode, 256), 256, 0, st>>>(m.nnode, m.d_iperm.p, u, u_int);
-  node_gather<NODE_LAPLACE>(m, u_int, nu, out, st);
-  HIPCHECK(hipFreeAsync(u_int, st));
+                         double *work, hipStream_t st) {
+  double *c = work;
+  if (!work)
+    HIPCHECK(hipMallocAsync((void **)&c, sizeof(double) * (m.degree == 2 ? 6 : 3) * m.nelem, st));
+  if (m.degree == 2) launch_p2_laplace_term(m, u, nu, out, c, st);
+  else two_pass<true>(m, u, nu, out, c, st);
+  if (!work) HIPCHECK(hipFreeAsync(c, st));
 }
 
 void launch_laplace_term_nu_grad(const Mesh &m, const double *grad_out, const double *u,

@@ -300,10 +300,11 @@ void launch_to_gauss(const Mesh &m, const double *u, double *out, hipStream_t st
 void launch_to_gauss_grad(const Mesh &m, const double *grad_out, double *grad_u,
                           hipStream_t st);
 void launch_fem_grad(const Mesh &m, const double *u, double *out, hipStream_t st);
-void launch_fem_grad_grad(const Mesh &m, const double *grad_out, double *grad_u,
+// work: elem_ndof * nelem doubles of scratch on the stream, or nullptr
+void launch_fem_grad_grad(const Mesh &m, const double *grad_out, double *grad_u, double *work,
                           hipStream_t st);
 void launch_laplace_term(const Mesh &m, const double *u, const double *nu, double *out,
-                         hipStream_t st);
+                         double *work, hipStream_t st);
 void launch_laplace_term_nu_grad(const Mesh &m, const double *grad_out, const double *u,
                                  double *grad_nu, hipStream_t st);
 // DofToGaussPoints (DofToGaussPointsMfem.h:6-32): the degree's basis (for P1
@@ -322,9 +323,10 @@ void launch_p2_source_grad(const Mesh &m, const double *grhs, double *gf, hipStr
 void launch_p2_dof_to_gauss(const Mesh &m, const double *u, double *out, hipStream_t st);
 void launch_p2_dof_to_gauss_grad(const Mesh &m, const double *g, double *gu, hipStream_t st);
 void launch_p2_fem_grad(const Mesh &m, const double *u, double *out, hipStream_t st);
-void launch_p2_fem_grad_grad(const Mesh &m, const double *g, double *gu, hipStream_t st);
+void launch_p2_fem_grad_grad(const Mesh &m, const double *g, double *gu, double *work,
+                             hipStream_t st);
 void launch_p2_laplace_term(const Mesh &m, const double *u, const double *nu, double *out,
-                            hipStream_t st);
+                            double *work, hipStream_t st);
 void launch_p2_laplace_term_nu_grad(const Mesh &m, const double *go, const double *u,
                                     double *gnu, hipStream_t st);
 // assemble.hip

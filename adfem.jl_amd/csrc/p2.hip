@@ -197,30 +197,24 @@ __global__ void p2_gauss_kernel(int nelem, QuadRule rule, const int *__restrict_
   }
 }
 
-enum { D_SOURCE = 0, D_DOF_TO_GAUSS_T = 1, D_FEM_GRAD_T = 2, D_LAPLACE = 3 };
+enum { D_SOURCE = 0, D_DOF_TO_GAUSS_T = 1, D_FEM_GRAD_T = 2 };
 
 // Per dof, over its incident (element, local dof p) pairs, ascending element:
 //   D_SOURCE          FemSourceScalar_forward: sum_k f[g] h_p(k) w_k
 //   D_DOF_TO_GAUSS_T  DofToGaussPointsMfem_backward: sum_k in[g] h_p(k)
 //   D_FEM_GRAD_T      FemGradMfem_backward: sum_k in[2g] dh_p/dx + in[2g+1] dh_p/dy
-//   D_LAPLACE         ComputeLaplaceTermMfem_forward (= K(nu) u), with u and
-//                     the thread order in the internal dof order (vertex
-//                     dofs permuted like the nodes, edge dofs as they are),
-//                     so an incidence's six values are local gathers:
-//                     sum_k nu_k w_k grad h_p . grad u_e(k)
 template <int OP, int NQ>
-__global__ void __launch_bounds__(256) p2_dof_kernel(int ndof, int nnode, const int *__restrict__ iperm, int nelem,
+__global__ void __launch_bounds__(256) p2_dof_kernel(int ndof, int nelem,
                               QuadRule rule, const int *__restrict__ conn,
-                              const int *__restrict__ conn_dof, const double *__restrict__ x,
+                              const double *__restrict__ x,
                               const double *__restrict__ y, const double *__restrict__ gw,
                               const int *__restrict__ d2e_ptr, const int *__restrict__ d2e,
-                              const double *__restrict__ in, const double *__restrict__ nu,
+                              const double *__restrict__ in,
                               double *__restrict__ out, int accumulate) {
 #pragma clang fp contract(off)
   constexpr bool CHEAP = OP == D_DOF_TO_GAUSS_T || OP == D_SOURCE;
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= ndof) return;
-  const int dof = (OP == D_LAPLACE && r < nnode) ? iperm[r] : r;  // user dof id
+  const int dof = blockIdx.x * blockDim.x + threadIdx.x;  // user dof id
+  if (dof >= ndof) return;
   double acc = accumulate ? out[dof] : 0.0;
   const int t1 = d2e_ptr[dof + 1];
   // the cheap ops are unrolled over incidences so that their loads overlap;
@@ -243,7 +237,7 @@ __global__ void __launch_bounds__(256) p2_dof_kernel(int ndof, int nnode, const 
         const size_t g = (size_t)NQ * e + k;
         acc += in[g] * h[p] * gw[g];
       }
-    } else if (OP == D_FEM_GRAD_T) {
+    } else {
       const ElemGeom G = p2_geom(conn, nelem, e, x, y);
 #pragma unroll
       for (int k = 0; k < NQ; k++) {
@@ -252,39 +246,81 @@ __global__ void __launch_bounds__(256) p2_dof_kernel(int ndof, int nnode, const 
         const size_t g = (size_t)NQ * e + k;
         acc += in[2 * g] * gx[p] + in[2 * g + 1] * gy[p];
       }
-    } else {  // D_LAPLACE
-      const ElemGeom G = p2_geom(conn, nelem, e, x, y);
-      double ue[6];
-#pragma unroll
-      for (int q = 0; q < 6; q++)
-        ue[q] = in[q < 3 ? conn[(size_t)q * nelem + e] : conn_dof[(size_t)q * nelem + e]];
-#pragma unroll
-      for (int k = 0; k < NQ; k++) {
-        double gx[6], gy[6];
-        p2_grad(rule.xi[k], rule.eta[k], G, gx, gy);
-        double ux = 0.0, uy = 0.0;
-#pragma unroll
-        for (int q = 0; q < 6; q++) {
-          ux += gx[q] * ue[q];
-          uy += gy[q] * ue[q];
-        }
-        const size_t g = (size_t)NQ * e + k;
-        acc += nu[g] * gw[g] * (gx[p] * ux + gy[p] * uy);
-      }
     }
   }
   out[dof] = acc;
 }
 
-inline unsigned nb(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs); }
-
-// dst = src in the internal dof order: vertex dof r <- src[iperm[r]], edge
-// dofs unchanged
-__global__ void p2_permute_dofs(int ndof, int nnode, const int *__restrict__ iperm,
-                                const double *__restrict__ src, double *__restrict__ dst) {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r < ndof) dst[r] = src[r < nnode ? iperm[r] : r];
+// K(nu) u (ComputeLaplaceTermMfem_forward) and FemGradMfem_backward in two
+// passes: element e's term of its dof p at c[p nelem + e], with the basis and
+// geometry evaluated once per Gauss point instead of once per (dof, element)
+// pair, six times as often; then each dof's terms in ascending element order,
+// threads in the internal dof order (vertex dofs permuted like the nodes,
+// edge dofs as they are).  Bound by memory at 300^2: K(nu) u 53 -> 20 us,
+// fem_grad's transpose 70 -> 17 us; at 33^2, bound by the launches' latency,
+// 17 -> 7.4 us and 13.5 -> 7.2 us.
+template <bool LAPLACE, int NQ>
+__global__ void __launch_bounds__(256)
+    p2_elem_terms_kernel(int nelem, QuadRule rule, const int *__restrict__ conn,
+                         const int *__restrict__ conn_dof, const double *__restrict__ x,
+                         const double *__restrict__ y, const double *__restrict__ gw,
+                         const double *__restrict__ in,  // LAPLACE: field, else Gauss (x, y)
+                         const double *__restrict__ nu, double *__restrict__ c) {
+  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= nelem) return;
+  double v[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0}, ue[6];
+  if (LAPLACE)
+#pragma unroll
+    for (int q = 0; q < 6; q++) ue[q] = in[conn_dof[(size_t)q * nelem + e]];
+  const ElemGeom G = p2_geom(conn, nelem, e, x, y);
+#pragma unroll 2
+  for (int k = 0; k < NQ; k++) {
+    double gx[6], gy[6], sx, sy;
+    p2_grad(rule.xi[k], rule.eta[k], G, gx, gy);
+    const size_t g = (size_t)NQ * e + k;
+    if (LAPLACE) {  // nu_k w_k grad u_e(k)
+      sx = sy = 0.0;
+#pragma unroll
+      for (int q = 0; q < 6; q++) {
+        sx += gx[q] * ue[q];
+        sy += gy[q] * ue[q];
+      }
+      const double cw = nu[g] * gw[g];
+      sx *= cw;
+      sy *= cw;
+    } else {
+      sx = in[2 * g];
+      sy = in[2 * g + 1];
+    }
+#pragma unroll
+    for (int p = 0; p < 6; p++) v[p] += sx * gx[p] + sy * gy[p];
+  }
+#pragma unroll
+  for (int p = 0; p < 6; p++) c[(size_t)p * nelem + e] = v[p];
 }
+
+__global__ void __launch_bounds__(256)
+    p2_dof_sum_kernel(int ndof, int nnode, const int *__restrict__ iperm, int nelem,
+                      const int *__restrict__ d2e_ptr, const int *__restrict__ d2e,
+                      const double *__restrict__ c, double *__restrict__ out) {
+  const int r = blockIdx.x * blockDim.x + threadIdx.x;
+  if (r >= ndof) return;
+  const int dof = r < nnode ? iperm[r] : r;  // user dof id
+  const int t1 = d2e_ptr[dof + 1];
+  double acc = 0.0;
+  int t = d2e_ptr[dof];
+  for (; t + 1 < t1; t += 2) {  // two terms' loads in flight
+    const int a = d2e[t], b = d2e[t + 1];
+    const double va = c[(size_t)(a & 7) * nelem + (a >> 3)],
+                 vb = c[(size_t)(b & 7) * nelem + (b >> 3)];
+    acc += va;
+    acc += vb;
+  }
+  if (t < t1) acc += c[(size_t)(d2e[t] & 7) * nelem + (d2e[t] >> 3)];
+  out[dof] = acc;
+}
+
+inline unsigned nb(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 
 template <int OP>
 void gauss_op(const Mesh &m, const double *a, const double *b, double *out, hipStream_t st) {
@@ -294,17 +330,30 @@ void gauss_op(const Mesh &m, const double *a, const double *b, double *out, hipS
 }
 
 template <int OP>
-void dof_op(const Mesh &m, const double *in, const double *nu, double *out, bool accumulate,
-            hipStream_t st) {
+void dof_op(const Mesh &m, const double *in, double *out, bool accumulate, hipStream_t st) {
   auto go = [&](auto kern) {
-    kern<<<nb(m.ndof, 256), 256, 0, st>>>((int)m.ndof, m.nnode, m.d_iperm.p, m.nelem, m.rule,
-                                          m.conn.p, m.conn_dof.p,
-                                          m.x.p, m.y.p, m.gw.p, m.d_d2e_ptr.p, m.d_d2e.p, in, nu,
-                                          out, accumulate ? 1 : 0);
+    kern<<<nb(m.ndof, 256), 256, 0, st>>>((int)m.ndof, m.nelem, m.rule, m.conn.p, m.x.p, m.y.p,
+                                          m.gw.p, m.d_d2e_ptr.p, m.d_d2e.p, in, out,
+                                          accumulate ? 1 : 0);
   };
   if (m.rule.nq == 6) go(p2_dof_kernel<OP, 6>);
   else if (m.rule.nq == 3) go(p2_dof_kernel<OP, 3>);
   else go(p2_dof_kernel<OP, 1>);
+  HIPCHECK(hipGetLastError());
+}
+
+template <bool LAPLACE>
+void two_pass(const Mesh &m, const double *in, const double *nu, double *out, double *c,
+              hipStream_t st) {
+  auto go = [&](auto kern) {
+    kern<<<nb(m.nelem, 256), 256, 0, st>>>(m.nelem, m.rule, m.conn.p, m.conn_dof.p, m.x.p, m.y.p,
+                                           m.gw.p, in, nu, c);
+  };
+  if (m.rule.nq == 6) go(p2_elem_terms_kernel<LAPLACE, 6>);
+  else if (m.rule.nq == 3) go(p2_elem_terms_kernel<LAPLACE, 3>);
+  else go(p2_elem_terms_kernel<LAPLACE, 1>);
+  p2_dof_sum_kernel<<<nb(m.ndof, 256), 256, 0, st>>>((int)m.ndof, m.nnode, m.d_iperm.p, m.nelem,
+                                                     m.d_d2e_ptr.p, m.d_d2e.p, c, out);
   HIPCHECK(hipGetLastError());
 }
 
@@ -336,7 +385,7 @@ void launch_p2_coo_grad(const Mesh &m, bool mass, const double *gvv, double *out
 
 void launch_p2_source(const Mesh &m, const double *f, double *rhs, bool accumulate,
                       hipStream_t st) {
-  dof_op<D_SOURCE>(m, f, nullptr, rhs, accumulate, st);
+  dof_op<D_SOURCE>(m, f, rhs, accumulate, st);
 }
 
 void launch_p2_source_grad(const Mesh &m, const double *grhs, double *gf, hipStream_t st) {
@@ -348,24 +397,22 @@ void launch_p2_dof_to_gauss(const Mesh &m, const double *u, double *out, hipStre
 }
 
 void launch_p2_dof_to_gauss_grad(const Mesh &m, const double *g, double *gu, hipStream_t st) {
-  dof_op<D_DOF_TO_GAUSS_T>(m, g, nullptr, gu, false, st);
+  dof_op<D_DOF_TO_GAUSS_T>(m, g, gu, false, st);
 }
 
 void launch_p2_fem_grad(const Mesh &m, const double *u, double *out, hipStream_t st) {
   gauss_op<G_FEM_GRAD>(m, u, nullptr, out, st);
 }
 
-void launch_p2_fem_grad_grad(const Mesh &m, const double *g, double *gu, hipStream_t st) {
-  dof_op<D_FEM_GRAD_T>(m, g, nullptr, gu, false, st);
+void launch_p2_fem_grad_grad(const Mesh &m, const double *g, double *gu, double *work,
+                             hipStream_t st) {
+  if (work) two_pass<false>(m, g, nullptr, gu, work, st);
+  else dof_op<D_FEM_GRAD_T>(m, g, gu, false, st);
 }
 
 void launch_p2_laplace_term(const Mesh &m, const double *u, const double *nu, double *out,
-                            hipStream_t st) {
-  double *u_int = nullptr;  // u in the internal dof order, a stream-ordered temporary
-  HIPCHECK(hipMallocAsync((void **)&u_int, sizeof(double) * m.ndof, st));
-  p2_permute_dofs<<<nb(m.ndof, 256), 256, 0, st>>>((int)m.ndof, m.nnode, m.d_iperm.p, u, u_int);
-  dof_op<D_LAPLACE>(m, u_int, nu, out, false, st);
-  HIPCHECK(hipFreeAsync(u_int, st));
+                            double *work, hipStream_t st) {
+  two_pass<true>(m, u, nu, out, work, st);
 }
 
 void launch_p2_laplace_term_nu_grad(const Mesh &m, const double *go, const double *u,

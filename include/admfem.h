@@ -204,19 +204,31 @@ int admfem_dof_to_gauss_points_grad(admfem_mesh m, const double *grad_out, doubl
 int admfem_fem_grad(admfem_mesh m, const double *u, double *out, void *stream);
 /* FemGradMfemGrad (h:24-41): grad_out [ngauss x 2] -> grad_u [ndof]. */
 int admfem_fem_grad_grad(admfem_mesh m, const double *grad_out, double *grad_u, void *stream);
+/* The same with caller-owned scratch: work [elem_ndof * nelem] on the stream,
+ * contents lost, or NULL.  The elements' terms pass through it instead of
+ * each node deriving all its elements' anew. */
+int admfem_fem_grad_grad_on(admfem_mesh m, const double *grad_out, double *grad_u, double *work,
+                            void *stream);
 /* ComputeLaplaceTermMfem (deps/MFEM/ComputeLaplaceTermMfem/
  * ComputeLaplaceTermMfem.h:4-17), the op behind compute_fem_laplace_term1
  * (src/MFEM/MCore.jl:740-763): out [ndof] = K(nu) u without forming K
  * (overwritten); u [ndof], nu [ngauss].  Takes a stream-ordered temporary
- * of ndof doubles (u in the internal order). */
+ * of elem_ndof * nelem doubles (the elements' terms). */
 int admfem_fem_laplace_term(admfem_mesh m, const double *u, const double *nu, double *out,
                             void *stream);
+/* The same with caller-owned scratch (as admfem_fem_grad_grad_on). */
+int admfem_fem_laplace_term_on(admfem_mesh m, const double *u, const double *nu, double *out,
+                               double *work, void *stream);
 /* ComputeLaplaceTermMfemGrad (h:19-39): grad_u = K(nu) grad_out (K is
  * symmetric), grad_nu[g] = w_g grad(grad_out) . grad(u) on g's element.
  * Either output may be NULL. */
 int admfem_fem_laplace_term_grad(admfem_mesh m, const double *grad_out, const double *u,
                                  const double *nu, double *grad_u, double *grad_nu,
                                  void *stream);
+/* The same with caller-owned scratch (as admfem_fem_grad_grad_on). */
+int admfem_fem_laplace_term_grad_on(admfem_mesh m, const double *grad_out, const double *u,
+                                    const double *nu, double *grad_u, double *grad_nu,
+                                    double *work, void *stream);
 /* ImposeDirichlet (deps/MFEM/ImposeDirichlet/ImposeDirichlet.cpp:14-40,
  * forward ImposeDirichlet.h:27-60).  indices [sN x 2] int64 0-based, vv [sN],
  * bd [bdN] int64 1-based, rhs [N], bdval [bdN].  Outputs: oindices
