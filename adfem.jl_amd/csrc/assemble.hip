@@ -23,6 +23,7 @@
 // Each row's thread then writes its slice lanes: consecutive rows are
 // consecutive addresses.  Every value has one writer and a fixed summation
 // order: no atomics, deterministic.
+#include "batched.h"
 #include "geom.h"
 
 namespace admfem {
@@ -441,11 +442,11 @@ __global__ void kappa_grad_kernel(int nelem, QuadRule rule,
 // observations first claim their rows in g (g[r] = k + 1), and one whose
 // claim did not stick shares its row with another.  (A shared row would
 // need its terms summed; the entry points require distinct indices.)
-__global__ void __launch_bounds__(1024)
-    loss_kernel(int n, const int *__restrict__ perm, const int *__restrict__ idx,
-                const double *__restrict__ obs, int nobs,
-                const double *__restrict__ u, double *__restrict__ g,
-                double *__restrict__ loss) {
+__device__ __forceinline__ void loss_block(int n, const int *__restrict__ perm,
+                                           const int *__restrict__ idx,
+                                           const double *__restrict__ obs, int nobs,
+                                           const double *__restrict__ u, double *__restrict__ g,
+                                           double *__restrict__ loss) {
   __shared__ double sh[16];
   double acc = 0.0, bad = 0.0;
   for (int k = threadIdx.x; k < nobs; k += blockDim.x) {
@@ -476,6 +477,66 @@ __global__ void __launch_bounds__(1024)
     loss[0] = t;
     loss[1] = b;
   }
+}
+
+__global__ void __launch_bounds__(1024)
+    loss_kernel(int n, const int *__restrict__ perm, const int *__restrict__ idx,
+                const double *__restrict__ obs, int nobs, const double *__restrict__ u,
+                double *__restrict__ g, double *__restrict__ loss) {
+  loss_block(n, perm, idx, obs, nobs, u, g, loss);
+}
+
+// The serving engine's transfers, one launch for every request at once (rows
+// of `per` blocks a request).  One request's copies, permutations and loss
+// were up to fourteen commands of about 10 us each on the host, which is what
+// a queue of small requests ran at (64 requests, sides 32-224: inputs 5.5 of
+// the engine's 12.8 ms).
+constexpr int SV_NT = 256;
+__global__ void __launch_bounds__(SV_NT)
+    serve_in_kernel(const ServeIn *__restrict__ jobs, int per) {
+  const ServeIn &q = jobs[blockIdx.x / per];
+  const int t0 = (int)(blockIdx.x % per) * SV_NT + (int)threadIdx.x, step = per * SV_NT;
+#pragma unroll
+  for (int a = 0; a < 4; a++) {
+    const double *__restrict__ src = q.src[a];
+    double *__restrict__ dst = q.dst[a];
+    const int n = q.len[a];
+    if (a < 3) {
+#pragma unroll 4
+      for (int i = t0; i < n; i += step) dst[i] = src[i];
+    } else {
+      const int *__restrict__ perm = q.perm;
+#pragma unroll 4
+      for (int i = t0; i < n; i += step) dst[perm[i]] = src[i];
+    }
+  }
+  for (int i = t0; i < q.ni; i += step) q.idst[i] = q.isrc[i];
+}
+
+__global__ void __launch_bounds__(SV_NT)
+    serve_turn_kernel(const ServeTurn *__restrict__ jobs, int per) {
+  const ServeTurn &q = jobs[blockIdx.x / per];
+  const int t0 = (int)(blockIdx.x % per) * SV_NT + (int)threadIdx.x, step = per * SV_NT;
+  const double *__restrict__ x = q.x;
+  double *__restrict__ u = q.u, *__restrict__ g = q.g;
+  const int n = q.npad;
+  for (int i = t0; i < n; i += step) {
+    if (x) u[i] = x[i];
+    g[i] = 0.0;
+  }
+}
+
+__global__ void __launch_bounds__(1024)
+    serve_loss_kernel(const ServeTurn *__restrict__ jobs) {
+  const ServeTurn &q = jobs[blockIdx.x];
+  loss_block(q.n, q.perm, q.obsi, q.obsv, q.nobs, q.u, q.g, q.loss);
+}
+
+__global__ void __launch_bounds__(SV_NT)
+    serve_out_kernel(const ServeOut *__restrict__ jobs, int per) {
+  const ServeOut &q = jobs[blockIdx.x / per];
+  const int t0 = (int)(blockIdx.x % per) * SV_NT + (int)threadIdx.x, step = per * SV_NT;
+  for (int i = t0; i < q.n; i += step) q.dst[q.perm[i]] = q.src[i];
 }
 
 inline unsigned nblk(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs); }
@@ -593,6 +654,30 @@ void launch_loss(const System &s, const double *u_int, const int *obs_idx,
   fill_zero<<<nblk(s.npad, 256), 256, 0, st>>>(g_int, s.npad);
   loss_kernel<<<1, 1024, 0, st>>>(s.n, s.d_uperm(), obs_idx, obs_val, nobs, u_int, g_int,
                                   loss2);
+  HIPCHECK(hipGetLastError());
+}
+
+// (blocks a request: eight entries a thread of the longest, 256 at most)
+static int serve_per(int longest) {
+  return std::min(256, std::max(1, (int)nblk(longest, 8 * SV_NT)));
+}
+
+void serve_inputs(const ServeIn *jobs, int n, int longest, hipStream_t st) {
+  const int per = serve_per(longest);
+  serve_in_kernel<<<(unsigned)n * per, SV_NT, 0, st>>>(jobs, per);
+  HIPCHECK(hipGetLastError());
+}
+
+void serve_turn(const ServeTurn *jobs, int n, int longest, hipStream_t st) {
+  const int per = serve_per(longest);
+  serve_turn_kernel<<<(unsigned)n * per, SV_NT, 0, st>>>(jobs, per);
+  serve_loss_kernel<<<(unsigned)n, 1024, 0, st>>>(jobs);
+  HIPCHECK(hipGetLastError());
+}
+
+void serve_outputs(const ServeOut *jobs, int n, int longest, hipStream_t st) {
+  const int per = serve_per(longest);
+  serve_out_kernel<<<(unsigned)n * per, SV_NT, 0, st>>>(jobs, per);
   HIPCHECK(hipGetLastError());
 }
 

@@ -43,6 +43,36 @@ struct SynField {
   double wx[32], wy[32], phi[32];
 };
 
+// Requests' inputs in device memory, copied together: four arrays (the last
+// one by perm: dst[perm[i]] = src[i]) and the observed indices; empty arrays
+// have length 0.
+struct ServeIn {
+  const double *src[4];
+  double *dst[4];
+  int len[4];
+  const int *perm, *isrc;
+  int *idst;
+  int ni;
+};
+void serve_inputs(const ServeIn *jobs, int n, int longest, hipStream_t st);
+// Requests between forward and adjoint solve: u = the solution x (null: u
+// holds it), g = dL/du, loss = {L, bad-index flag}.
+struct ServeTurn {
+  const double *x, *obsv;
+  const int *perm, *obsi;
+  double *u, *g, *loss;
+  int n, npad, nobs;
+};
+void serve_turn(const ServeTurn *jobs, int n, int longest, hipStream_t st);
+// Finished requests' solutions in the caller's order: dst[perm[i]] = src[i].
+struct ServeOut {
+  const int *perm;
+  const double *src;
+  double *dst;
+  int n;
+};
+void serve_outputs(const ServeOut *jobs, int n, int longest, hipStream_t st);
+
 void batch_init(const BSys *D, BScal *S, int sys, int nblk, double rtol2, double delta2,
                 int maxit, hipStream_t st);
 // the block map of nsys systems (slots slot[k], first logical block

@@ -179,6 +179,35 @@ struct Server {
   MgSys *h_mg = nullptr;
   MgScal *h_mgs = nullptr;
   std::vector<int> starts;       // multigrid requests whose solve is to start
+  DevBuf<double> d_loss;         // per slot: loss and bad-index flag
+  // the requests whose inputs, turn or outputs go out together: pinned and
+  // device job lists (rewritten only after the stream has passed them)
+  template <class T> struct Jobs {
+    T *h = nullptr;
+    DevBuf<T> d;
+    int n = 0, longest = 0;
+    void alloc(int cap) {
+      HIPCHECK(hipHostMalloc((void **)&h, sizeof(T) * cap, hipHostMallocDefault));
+      d.alloc(cap);
+    }
+    void add(const T &job, int len) {
+      h[n++] = job;
+      longest = std::max(longest, len);
+    }
+    template <class F> void flush(F launch, hipStream_t st) {
+      if (!n) return;
+      HIPCHECK(hipMemcpyAsync(d.p, h, sizeof(T) * n, hipMemcpyHostToDevice, st));
+      launch(d.p, n, longest, st);
+      clear();
+    }
+    void clear() { n = longest = 0; }
+    ~Jobs() {
+      if (h) (void)hipHostFree(h);
+    }
+  };
+  Jobs<ServeIn> jobs_in;
+  Jobs<ServeTurn> jobs_turn;
+  Jobs<ServeOut> jobs_out;
   static constexpr int MG_BATCH_SUM = 128;  // partials summed by the wide kernels
   int *h_list = nullptr;         // pinned staging: the batch's slots, then
                                  // their first logical blocks (list_cap each)
@@ -221,7 +250,7 @@ struct Server {
     auto F = [&](size_t n) { return (float *)take(n * sizeof(float)); };
     double *x = D(nv), *y = D(nv), *kappa = D(ng), *f = D(ng), *uprev = D(np), *b = D(np),
            *sv64 = D(ns), *diag64 = D(np), *dsq = D(np),
-           *u64 = D(np), *lam64 = D(np), *grad = D(ng), *obsv = D(nobs + 1), *loss2 = D(2),
+           *u64 = D(np), *lam64 = D(np), *grad = D(ng), *obsv = D(nobs + 1),
            *part = D(5 * nblk + 5), *stage = D(2 * np);
     double2 *xy = (double2 *)take(nv * sizeof(double2));
     float *sv32 = F(ns);
@@ -247,7 +276,7 @@ struct Server {
     if (q) {
       q->x = x; q->y = y; q->xy = xy; q->kappa = kappa; q->f = f; q->uprev = uprev; q->b = b;
       q->sv64 = sv64; q->diag64 = diag64; q->dsq = dsq;
-      q->u64 = u64; q->lam64 = lam64; q->grad = grad; q->obsv = obsv; q->loss2 = loss2;
+      q->u64 = u64; q->lam64 = lam64; q->grad = grad; q->obsv = obsv;
       q->part = part; q->stage = stage; q->sv32 = sv32; q->obsi = obsi;
     }
     return off;
@@ -330,7 +359,18 @@ struct Server {
     d.npad = s.npad;
     mg_parts(d, T.nblk, T.nblk > MG_BATCH_SUM, q.part);
     mg_grid_layout(*T.plan, q.grid, d);
-    HIPCHECK(hipMemcpyAsync(d_mg.p + q.slot, &d, sizeof(MgSys), hipMemcpyHostToDevice, st));
+  }
+
+  // The descriptors of new requests, in one copy: of the slots between them
+  // too, whose descriptors are what they were (or nobody's).
+  void upload_mg_descs(const std::vector<int> &reqs_) {
+    int lo = max_slots, hi = -1;
+    for (int i : reqs_) {
+      lo = std::min(lo, reqs[i].slot);
+      hi = std::max(hi, reqs[i].slot);
+    }
+    HIPCHECK(hipMemcpyAsync(d_mg.p + lo, h_mg + lo, sizeof(MgSys) * (hi - lo + 1),
+                            hipMemcpyHostToDevice, st));
   }
 
   // The block maps of a set of multigrid requests, in buffers of the set's own
@@ -451,9 +491,15 @@ struct Server {
       HIPCHECK(hipMemcpyAsync(q.stage, r.coords, sizeof(double) * 2 * nn, kind, st));
       launch_perm_coords(nn, m.d_iperm.p, q.stage, q.x, q.y, q.xy, st);
     } else {
-      HIPCHECK(hipMemcpyAsync(q.x, m.x.p, sizeof(double) * nn, hipMemcpyDeviceToDevice, st));
-      HIPCHECK(hipMemcpyAsync(q.y, m.y.p, sizeof(double) * nn, hipMemcpyDeviceToDevice, st));
-      HIPCHECK(hipMemcpyAsync(q.xy, m.xy.p, sizeof(double2) * nn, hipMemcpyDeviceToDevice, st));
+      q.xy = m.xy.p;  // (only read)
+    }
+    if (r.source == ADMFEM_SRC_DEVICE) {  // with the other requests'
+      jobs_in.add(ServeIn{{r.kappa, r.f, r.obs_val, heat ? r.u_prev : nullptr},
+                          {q.kappa, q.f, q.obsv, q.uprev},
+                          {(int)m.ngauss, (int)m.ngauss, r.nobs, heat ? s.n : 0},
+                          s.d_uperm(), r.obs_idx, q.obsi, r.nobs},
+                  std::max({(int)m.ngauss, s.n, r.nobs}));
+      return;
     }
     HIPCHECK(hipMemcpyAsync(q.kappa, r.kappa, sizeof(double) * m.ngauss, kind, st));
     HIPCHECK(hipMemcpyAsync(q.f, r.f, sizeof(double) * m.ngauss, kind, st));
@@ -482,7 +528,6 @@ struct Server {
 
   void assemble(Req &q) {
     const System &s = *topos[q.r.topo].sys;
-    inputs(q);
     admfem_problem p = problem(q);
     // FP64 matrix and rhs; the FP32 scaled matrix of the inner iteration
     launch_assemble_to(s, q.xy, p, SellOut{q.sv64, q.diag64, q.b}, st);
@@ -522,19 +567,19 @@ struct Server {
     q.res.device_bytes = (double)bytes;
     layout(*T.sys, q.mg ? T.plan : nullptr, &q, mem, q.nobs);
     q.slot = free_slots.back();
+    q.loss2 = d_loss.p + 2 * q.slot;
     free_slots.pop_back();
     q.res.t_admit = t;
+    return attempt(q, [&] { inputs(q); });
+  }
+
+  // A step of a request's admission.  When it fails the request fails alone:
+  // its memory and slot go back to the queue, the requests behind it are
+  // admitted as usual.
+  template <class F> bool attempt(Req &q, F step) {
     try {
-      assemble(q);
-      if (q.mg) {
-        write_mg_desc(q);  // set up and started with the batch's others
-      } else {
-        write_desc(q, q.b);
-        start_cg(q);
-      }
+      step();
     } catch (const Error &e) {
-      // the request fails alone: its memory and slot go back to the queue,
-      // the requests behind it are admitted as usual
       (void)hipStreamSynchronize(st);
       set_error(e.msg);
       fail(q, e.code == ADMFEM_ERR_HIP ? ADMFEM_ERR_HIP : ADMFEM_ERR_ARG);
@@ -542,6 +587,22 @@ struct Server {
     }
     q.state = Q_FWD;
     return true;
+  }
+
+  // an admitted request's matrix and start, behind its inputs
+  void prepare(Req &q) {
+    attempt(q, [&] {
+      assemble(q);
+      if (q.mg) {
+        write_mg_desc(q);  // set up and started with the batch's others
+      } else {
+        write_desc(q, q.b);
+        start_cg(q);
+      }
+    });
+  }
+  void flush_inputs() {
+    jobs_in.flush(serve_inputs, st);
   }
 
   void release(Req &q) {
@@ -554,42 +615,45 @@ struct Server {
   void to_adjoint(Req &q, int it) {
     const System &s = *topos[q.r.topo].sys;
     q.res.iters_fwd = it;
-    solution(q, q.u64);
-    launch_loss(s, q.u64, q.obsi, q.obsv, q.nobs, q.b, q.loss2, st);  // g overwrites b
-    if (!q.mg) start_cg(q);
+    if (!q.mg) batch_final(d_desc.p, d_scal.p, q.slot, s.npad, q.u64, st);
+    jobs_turn.add(ServeTurn{q.mg ? q.mgx : nullptr, q.obsv, s.d_uperm(), q.obsi, q.u64, q.b,
+                            q.loss2, s.n, s.npad, q.nobs},  // (g overwrites b)
+                  s.npad);
     q.state = Q_ADJ;
   }
 
-  // the finished solve's solution
-  void solution(Req &q, double *out) {
-    const System &s = *topos[q.r.topo].sys;
-    if (q.mg)
-      HIPCHECK(hipMemcpyAsync(out, q.mgx, sizeof(double) * s.npad, hipMemcpyDeviceToDevice, st));
-    else
-      batch_final(d_desc.p, d_scal.p, q.slot, s.npad, out, st);
-  }
-
-  // adjoint solve finished: the gradient and the outputs are enqueued, the
-  // loss goes to the slot's pinned staging; complete() finishes the request
-  // once the stream has drained (one synchronisation for every request that
-  // finished at the same chunk boundary)
+  // adjoint solve finished: the gradient is enqueued, and the solution's way
+  // to the caller's order with the other requests'
   void finish(Req &q, int it) {
     const System &s = *topos[q.r.topo].sys;
-    const Mesh &m = *s.mesh;
     q.res.iters_adj = it;
-    solution(q, q.lam64);
+    if (!q.mg) batch_final(d_desc.p, d_scal.p, q.slot, s.npad, q.lam64, st);
     admfem_problem p = problem(q);
-    launch_kappa_gradient_to(s, q.xy, q.u64, q.lam64, p.lap_coef, q.grad, st);
-    if (q.r.u_out) {
-      launch_scatter(s.d_uiperm(), q.u64, q.stage, s.n, st);  // user order
-      HIPCHECK(hipMemcpyAsync(q.r.u_out, q.stage, sizeof(double) * s.n, hipMemcpyDeviceToHost,
-                              st));
+    launch_kappa_gradient_to(s, q.xy, q.u64, q.mg ? q.mgx : q.lam64, p.lap_coef, q.grad, st);
+    if (q.r.u_out) jobs_out.add(ServeOut{s.d_uiperm(), q.u64, q.stage, s.n}, s.n);
+  }
+
+  // The outputs of the requests that finished at one chunk boundary, their
+  // losses to the slots' pinned staging in one copy; complete() finishes them
+  // once the stream has drained.
+  void copy_outputs(const std::vector<int> &done) {
+    jobs_out.flush(serve_outputs, st);
+    int lo = max_slots, hi = -1;
+    for (int i : done) {
+      Req &q = reqs[i];
+      const System &s = *topos[q.r.topo].sys;
+      lo = std::min(lo, q.slot);
+      hi = std::max(hi, q.slot);
+      if (q.r.u_out)
+        HIPCHECK(hipMemcpyAsync(q.r.u_out, q.stage, sizeof(double) * s.n, hipMemcpyDeviceToHost,
+                                st));
+      if (q.r.grad_out)
+        HIPCHECK(hipMemcpyAsync(q.r.grad_out, q.grad, sizeof(double) * s.mesh->ngauss,
+                                hipMemcpyDeviceToHost, st));
     }
-    if (q.r.grad_out)
-      HIPCHECK(hipMemcpyAsync(q.r.grad_out, q.grad, sizeof(double) * m.ngauss,
-                              hipMemcpyDeviceToHost, st));
-    HIPCHECK(hipMemcpyAsync(h_loss + 2 * q.slot, q.loss2, 2 * sizeof(double),
-                            hipMemcpyDeviceToHost, st));
+    if (hi >= lo)
+      HIPCHECK(hipMemcpyAsync(h_loss + 2 * lo, d_loss.p + 2 * lo,
+                              2 * sizeof(double) * (hi - lo + 1), hipMemcpyDeviceToHost, st));
   }
 
   // after the stream has drained: a finished request's loss and status, its
@@ -698,13 +762,16 @@ struct Server {
     std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
       return reqs[a].r.arrival < reqs[b].r.arrival;
     });
+    jobs_in.clear();  // (a run that ended in an error may have left some)
+    jobs_turn.clear();
+    jobs_out.clear();
     size_t next = 0;  // first request (in arrival order) not yet admitted
     while (next < order.size() && reqs[order[next]].state != Q_WAIT) next++;
     const int mg_chunk = o.chunk > 0 ? o.chunk : 4;
     std::vector<int> active;
     for (size_t i = 0; i < reqs.size(); i++)
       if (reqs[i].state == Q_FWD || reqs[i].state == Q_ADJ) active.push_back((int)i);
-    std::vector<int> fresh, jac, mgr;  // fresh: multigrid requests to be set up
+    std::vector<int> admitted, fresh, jac, mgr;  // fresh: multigrid requests to be set up
     MgSet set_fresh, set_starts, set_mg;
     // requests whose last work (outputs, loss) is enqueued, and an event
     // behind that work: they complete once it has passed -- waited for
@@ -740,7 +807,9 @@ struct Server {
       double t = now_s(t0);
       if (t > timeout) break;
       // admit arrived requests, FIFO, while memory and slots allow
-      while (next < order.size() && (o.max_active <= 0 || (int)active.size() < o.max_active)) {
+      admitted.clear();
+      while (next < order.size() &&
+             (o.max_active <= 0 || (int)(active.size() + admitted.size()) < o.max_active)) {
         Req &q = reqs[order[next]];
         if (q.r.arrival > t) break;
         if (!admit(q, t, 0)) {
@@ -754,14 +823,18 @@ struct Server {
           }
           if (!waiting || !admit(q, t, waiting)) break;
         }
-        if (q.state != Q_DONE) {
-          active.push_back(order[next]);
-          if (q.mg) {
-            fresh.push_back(order[next]);
-            starts.push_back(order[next]);
-          }
-        }
+        if (q.state != Q_DONE) admitted.push_back(order[next]);
         next++;
+      }
+      flush_inputs();
+      for (int i : admitted) {
+        prepare(reqs[i]);
+        if (reqs[i].state == Q_DONE) continue;
+        active.push_back(i);
+        if (reqs[i].mg) {
+          fresh.push_back(i);
+          starts.push_back(i);
+        }
       }
       peak_active = std::max(peak_active, (int)active.size());
       if (active.empty()) {
@@ -778,6 +851,7 @@ struct Server {
       mgr.clear();
       for (int i : active) (reqs[i].mg ? mgr : jac).push_back(i);
       if (!fresh.empty()) {
+        upload_mg_descs(fresh);
         build_set(set_fresh, fresh);
         mg_batch_setup(set_fresh.batch, d_mg.p, st);
         fresh.clear();
@@ -821,7 +895,7 @@ struct Server {
       HIPCHECK(hipStreamSynchronize(st));
       // phase changes; requests that finished or failed complete once their
       // enqueued work has passed
-      std::vector<int> still;
+      std::vector<int> still, turned;
       for (int i : active) {
         Req &q = reqs[i];
         // where the solve stands: status (0 run, 1 converged, else failed),
@@ -848,7 +922,7 @@ struct Server {
         if (q.state == Q_FWD) {
           q.res.relres_fwd = sc.bb > 0 ? std::sqrt(sc.rr / sc.bb) : 0.0;
           to_adjoint(q, sc.it);
-          if (q.mg) starts.push_back(i);
+          turned.push_back(i);
           still.push_back(i);
         } else {
           q.res.relres_adj = sc.bb > 0 ? std::sqrt(sc.rr / sc.bb) : 0.0;
@@ -856,6 +930,12 @@ struct Server {
           done.push_back(i);
         }
       }
+      jobs_turn.flush(serve_turn, st);
+      for (int i : turned) {
+        if (reqs[i].mg) starts.push_back(i);
+        else start_cg(reqs[i]);
+      }
+      copy_outputs(done);
       if (!done.empty() || !failed.empty()) HIPCHECK(hipEventRecord(ev_done, st));
       active.swap(still);
     }
@@ -892,6 +972,7 @@ struct Server {
       q.res.device_bytes = (double)bytes;
       layout(s, nullptr, &q, mem, q.nobs);
       q.slot = 0;
+      q.loss2 = d_loss.p;
       q.res.t_admit = t;
       peak_active = std::max(peak_active, 1);
       try {
@@ -913,6 +994,7 @@ struct Server {
   // buffers (the request's arena range holds its inputs and outputs).
   void serve_seq(Req &q, System &s) {
     inputs(q);
+    flush_inputs();
     admfem_problem p = problem(q);
     s.a_version++;
     s.mass = p.mass_coef != 0.0;
@@ -983,6 +1065,7 @@ double server_spmv_repeat(Server *sv, const int *topos, int nsys, int repeat,
       q.r.source = ADMFEM_SRC_SYNTH;
       q.r.seed = (unsigned long long)i;
       const bool ok = sv->admit(q, 0.0, (size_t)1 << 30, true);
+      if (ok && q.state == Q_FWD) sv->prepare(q);
       REQUIRE(ok && q.state == Q_FWD, ADMFEM_ERR_BUDGET, "batch does not fit the budget");
       admitted++;
       nmap += sv->topos[q.r.topo].nblk;
@@ -1035,6 +1118,10 @@ Server *server_create(const admfem_server_opts &o) {
     HIPCHECK(hipMemset(sv->d_desc.p, 0, sv->d_desc.bytes()));
     HIPCHECK(hipMemset(sv->d_scal.p, 0, sv->d_scal.bytes()));
     sv->d_mg.alloc(sv->max_slots);
+    sv->d_loss.alloc(2 * (size_t)sv->max_slots);
+    sv->jobs_in.alloc(sv->max_slots);
+    sv->jobs_turn.alloc(sv->max_slots);
+    sv->jobs_out.alloc(sv->max_slots);
     sv->d_mgs.alloc(sv->max_slots);
     HIPCHECK(hipHostMalloc((void **)&sv->h_mg, sizeof(MgSys) * sv->max_slots,
                            hipHostMallocDefault));
