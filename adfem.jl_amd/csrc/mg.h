@@ -58,8 +58,10 @@ struct MgSys {
   double *part4, *partz;    // 4 x nblk and nblk block partials
   double *sum4, *sumz;      // their sums, when one block makes them
   int gsum;                 // values the wide kernels sum: nblk, or 1
-  float *pack, *cinv;       // the tail's grids below its first, the dense
-                            // inverse of the last one behind them
+  // the tail's matrices: its first grid's entries and weights as 7 quads a
+  // node ([7][nodes], entry 25 the weight), then each further grid's [25][nodes]
+  // and [nodes], then the dense inverse of the last
+  float *pack;
   int n, npad, nblk;
   int nlev, tail;           // grid levels, first one of the tail kernel
   int steps;                // fine smoothing steps before and after (1 or 2)
@@ -85,7 +87,7 @@ struct MgScal {
 // A topology's grids (made once per system, mg_plan).
 struct MgPlan {
   bool ok = false;          // false: the rows do not suit one uniform grid
-  int nlev = 0, tail = 0, steps = 1;
+  int n = 0, nlev = 0, tail = 0, steps = 1;
   int nx[MG_MAXLEV], ny[MG_MAXLEV], px[MG_MAXLEV], pn[MG_MAXLEV];
   DevBuf<int> cell, cptr, crow, pos;
   DevBuf<float2> frac, cfrac;
@@ -105,6 +107,7 @@ void mg_grid_layout(const MgPlan &pl, float *base, MgSys &d);
 // Allows the tail kernel the LDS it needs for this plan; how much that is.
 void mg_allow_lds(const MgPlan &pl);
 size_t mg_tail_lds(const MgPlan &pl);
+size_t mg_setup_lds(const MgPlan &pl);
 
 // A batch of systems (descriptors of D, states of S by slot): the block maps
 // of every kind of wide launch ((slot, block) per grid block), and the slots.
@@ -114,7 +117,7 @@ enum { MGS_ROWS = 0, MGS_TWO, MGS_GALERKIN, MGS_RESTRICT, MGS_SETUP,
 struct MgBatch {
   int nsys = 0, tail = 0;   // systems; most grids above the tail
   bool reduce = false;      // some system's partials are summed by one block
-  size_t tail_lds = 0;
+  size_t tail_lds = 0, setup_lds = 0;
   const int *list = nullptr;
   const int2 *map[MG_STAGES] = {};
   int nmap[MG_STAGES] = {};

@@ -89,6 +89,7 @@ __device__ __forceinline__ int2 where(const int2 *map, int sys) {
 }
 
 typedef float f2_t __attribute__((ext_vector_type(2)));
+typedef float f4_t __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ gptr<f2_t> frac_ptr(const float2 *p) {
   return (gptr<f2_t>)reinterpret_cast<const f2_t *>(p);
 }
@@ -226,23 +227,30 @@ __global__ void __launch_bounds__(NT)
   global_mut(d.minv)[i] = aii > 0.0 ? (float)(1.0 / sum) : 0.0f;
 }
 
-// The first grid's matrix P^T A P: four threads per grid node, one for each
-// of its cells, gathering from the cell's rows; a thread's 25 sums live in
-// LDS (they are addressed by the columns' cells).  Bound by the latency of
-// the row -> column -> cell loads: with one thread per node it took 88 us for
-// 4,356 nodes (P1 128^2) and 473 us for 1,000 (P2 40^2).
-constexpr int GT = 128;
+// The first grid's matrix P^T A P: 4 GR threads per grid node, GR for each of
+// its cells, which share the cell's rows; a thread's sums for the 4 x 4 nodes
+// around its cell live in LDS (they are addressed by the columns' cells).
+// Bound by the latency of the row -> column -> cell loads: with four lanes to a
+// cell 33 -> 15 us for the 1,156 nodes of P1 64^2 and 115 -> 47 for P2 101^2.
+// Past GALERKIN_SPLIT nodes (and in batches) the threads fill the chip with one
+// lane each, and the LDS of the sums bounds their waves: 66,000 nodes of P1 1024^2 237
+// -> 201 us (16 sums a thread instead of 25), 331 with four lanes.
+constexpr int GT = 256;
+constexpr int GALERKIN_SPLIT = 20000;
+constexpr int mg_gn(int gr) { return GT / (4 * gr); }  // nodes of a block
+template <int GR>
 __global__ void __launch_bounds__(GT)
     mk_galerkin(const int2 *__restrict__ map, const MgSys *__restrict__ D, int sys) {
-  __shared__ double acc[25][GT];
+  constexpr int GN = mg_gn(GR);
+  __shared__ double acc[16][GT];
   const int2 mb = where(map, sys);
   if (mb.x < 0) return;
   const MgSys &d = D[mb.x];
   const MgLevel &l = d.lv[0];
-  const int tid = threadIdx.x, id = mb.y * (GT / 4) + (tid >> 2), nn = l.nx * l.ny;
+  const int tid = threadIdx.x, id = mb.y * GN + tid / (4 * GR), nn = l.nx * l.ny;
   const int X = id % l.nx, Y = id / l.nx, ncx = l.nx - 1, ncy = l.ny - 1;
 #pragma unroll
-  for (int o = 0; o < 25; o++) acc[o][tid] = 0.0;
+  for (int o = 0; o < 16; o++) acc[o][tid] = 0.0;
   const int cx = X - (tid & 1), cy = Y - ((tid >> 1) & 1);
   if (id < nn && cx >= 0 && cx < ncx && cy >= 0 && cy < ncy) {
     const gptr<int> cptr = global_ptr(d.cptr), crow = global_ptr(d.crow),
@@ -251,7 +259,7 @@ __global__ void __launch_bounds__(GT)
     const gptr<double> sv = global_ptr(d.sv64), dg = global_ptr(d.diag);
     const gptr<f2_t> frac = frac_ptr(d.frac);
     const int c = cy * ncx + cx, k1 = cptr[c + 1];
-    for (int k = cptr[c]; k < k1; k++) {
+    for (int k = cptr[c] + ((tid >> 2) & (GR - 1)); k < k1; k += GR) {
       const int i = crow[k];
       const f2_t f = frac[i];
       const double wi =
@@ -263,168 +271,266 @@ __global__ void __launch_bounds__(GT)
         const double v = wi * (e < 0 ? dg[i] : sv[off + 64 * e]);
         const int cj = cell[j];
         const f2_t g = frac[j];
-        const int jy = cj / ncx, ox = cj - jy * ncx - X + 2, oy = jy - Y + 2;
+        const int jy = cj / ncx, ox = cj - jy * ncx - cx + 1, oy = jy - cy + 1;
         // (cj < 0: no part; the plan excludes cells further off)
-        if (cj < 0 || ox < 0 || ox > 3 || oy < 0 || oy > 3) continue;
-        acc[oy * 5 + ox][tid] += v * ((1.0 - g.x) * (1.0 - g.y));
-        acc[oy * 5 + ox + 1][tid] += v * ((double)g.x * (1.0 - g.y));
-        acc[oy * 5 + ox + 5][tid] += v * ((1.0 - g.x) * (double)g.y);
-        acc[oy * 5 + ox + 6][tid] += v * ((double)g.x * (double)g.y);
+        if (cj < 0 || ox < 0 || ox > 2 || oy < 0 || oy > 2) continue;
+        acc[oy * 4 + ox][tid] += v * ((1.0 - g.x) * (1.0 - g.y));
+        acc[oy * 4 + ox + 1][tid] += v * ((double)g.x * (1.0 - g.y));
+        acc[oy * 4 + ox + 4][tid] += v * ((1.0 - g.x) * (double)g.y);
+        acc[oy * 4 + ox + 5][tid] += v * ((double)g.x * (double)g.y);
       }
     }
   }
   __syncthreads();
-  for (int t = tid; t < 25 * (GT / 4); t += GT) {
-    const int o = t / (GT / 4), q = t % (GT / 4), node = mb.y * (GT / 4) + q;
-    if (node < nn)
-      global_mut(l.a)[(size_t)o * l.pn + mg_at(l.px, node % l.nx, node / l.nx)] =
-          (float)((acc[o][4 * q] + acc[o][4 * q + 1]) + (acc[o][4 * q + 2] + acc[o][4 * q + 3]));
+  for (int t = tid; t < 25 * GN; t += GT) {
+    const int o = t / GN, q = t % GN, node = mb.y * GN + q;
+    if (node >= nn) continue;
+    double sum = 0.0;
+#pragma unroll
+    for (int cl = 0; cl < 4; cl++) {  // the node is (1 - (cl & 1), 1 - (cl >> 1)) of the cell's
+      const int ox = o % 5 - 1 + (cl & 1), oy = o / 5 - 1 + (cl >> 1);
+      if (ox < 0 || ox > 3 || oy < 0 || oy > 3) continue;
+#pragma unroll
+      for (int r = 0; r < GR; r++) sum += acc[oy * 4 + ox][q * 4 * GR + 4 * r + cl];
+    }
+    global_mut(l.a)[(size_t)o * l.pn + mg_at(l.px, node % l.nx, node / l.nx)] = (float)sum;
   }
 }
 
-// One node's entries of the next grid's matrix: P^T A P with the bilinear
-// interpolation of a grid from every second node.
-__device__ __forceinline__ void coarse_node(const MgLevel &f, const MgLevel &c, int X, int Y) {
-  double T[7][7];
+// One node's entries of the next grid's matrix, P^T A P with the bilinear
+// interpolation of a grid from every second node: the part of the finer row
+// 2 Y + dy, dy in -1 .. 1 (else nothing).  a(o, x, y): the finer grid's entries.
+template <class A>
+__device__ __forceinline__ void coarse_part(A a, int nx, int ny, int X, int Y, int dy,
+                                            double (&s)[25]) {
+  double T[5][7];
 #pragma unroll
-  for (int u = 0; u < 7; u++)
+  for (int u = 0; u < 5; u++)
 #pragma unroll
     for (int v = 0; v < 7; v++) T[u][v] = 0.0;
-  const gptr<float> a = global_ptr(f.a);
-#pragma unroll
-  for (int dy = -1; dy <= 1; dy++)
+  const int y = 2 * Y + dy;
+  if (dy <= 1 && y >= 0 && y < ny) {
 #pragma unroll
     for (int dx = -1; dx <= 1; dx++) {
-      const int x = 2 * X + dx, y = 2 * Y + dy;
-      if (x < 0 || y < 0 || x >= f.nx || y >= f.ny) continue;
+      const int x = 2 * X + dx;
+      if (x < 0 || x >= nx) continue;
       const double w = (dx ? 0.5 : 1.0) * (dy ? 0.5 : 1.0);
-      const int at = mg_at(f.px, x, y);
 #pragma unroll
       for (int oy = 0; oy < 5; oy++)
 #pragma unroll
-        for (int ox = 0; ox < 5; ox++)
-          T[dy + oy + 1][dx + ox + 1] += w * (double)a[(size_t)(oy * 5 + ox) * f.pn + at];
+        for (int ox = 0; ox < 5; ox++) T[oy][dx + ox + 1] += w * (double)a(oy * 5 + ox, x, y);
     }
-  const int at = mg_at(c.px, X, Y);
+  }
 #pragma unroll
-  for (int oy = -2; oy <= 2; oy++)
+  for (int o = 0; o < 25; o++) s[o] = 0.0;
 #pragma unroll
-    for (int ox = -2; ox <= 2; ox++) {
-      double s = 0.0;
+  for (int oy = 0; oy < 5; oy++) {
+    double U[5];
 #pragma unroll
-      for (int v = -1; v <= 1; v++)
+    for (int ox = 0; ox < 5; ox++) {
+      // column 2 (ox - 2) + u + 3 of T, weights 1/2, 1, 1/2
+      U[ox] = 0.0;
 #pragma unroll
-        for (int u = -1; u <= 1; u++) {
-          const int ty = 2 * oy + v + 3, tx = 2 * ox + u + 3;
-          if (ty >= 0 && ty < 7 && tx >= 0 && tx < 7)
-            s += (u ? 0.5 : 1.0) * (v ? 0.5 : 1.0) * T[ty][tx];
-        }
-      global_mut(c.a)[(size_t)((oy + 2) * 5 + ox + 2) * c.pn + at] = (float)s;
+      for (int u = -1; u <= 1; u++) {
+        const int tx = 2 * ox - 1 + u;
+        if (tx >= 0 && tx < 7) U[ox] += (u ? 0.5 : 1.0) * T[oy][tx];
+      }
     }
+#pragma unroll
+    for (int cy = 0; cy < 5; cy++) {
+      // finer offset dy + oy - 2 against the coarser 2 (cy - 2)
+      const int v = dy + oy + 2 - 2 * cy;
+      const double w = v == 0 ? 1.0 : v == 1 || v == -1 ? 0.5 : 0.0;
+#pragma unroll
+      for (int ox = 0; ox < 5; ox++) s[cy * 5 + ox] += w * U[ox];
+    }
+  }
 }
 
-// A grid's smoothing weights.
-__device__ __forceinline__ void weight_node(const MgLevel &l, int x, int y) {
-  const gptr<float> a = global_ptr(l.a);
-  const int at = mg_at(l.px, x, y);
+// The same by the four lanes of a quad (one finer row each, one idle); put(o,
+// v) stores, a quarter of the entries by each lane.
+template <class A, class P>
+__device__ __forceinline__ void coarse_node(A a, int nx, int ny, int X, int Y, P put) {
+  const int q = threadIdx.x & 3;
+  double s[25];
+  coarse_part(a, nx, ny, X, Y, q - 1, s);
+#pragma unroll
+  for (int o = 0; o < 25; o++) {
+    s[o] += __shfl_xor(s[o], 1, 64);
+    s[o] += __shfl_xor(s[o], 2, 64);
+    if ((o & 3) == q) put(o, (float)s[o]);
+  }
+}
+
+// A grid's smoothing weight at a node.
+template <class A>
+__device__ __forceinline__ float weight_node(A a, int nx, int ny, int x, int y) {
   float v[25], ajj[25];
 #pragma unroll
   for (int o = 0; o < 25; o++) {
     const int X = x + o % 5 - 2, Y = y + o / 5 - 2;
-    v[o] = a[(size_t)o * l.pn + at];
-    ajj[o] = X >= 0 && X < l.nx && Y >= 0 && Y < l.ny
-                 ? a[(size_t)12 * l.pn + mg_at(l.px, X, Y)] : 0.0f;
+    v[o] = a(o, x, y);
+    ajj[o] = X >= 0 && X < nx && Y >= 0 && Y < ny ? a(12, X, Y) : 0.0f;
   }
   float s = 0.0f;
 #pragma unroll
   for (int o = 0; o < 25; o++)
     if (ajj[o] > 1e-30f) s += fabsf(v[o]) * rsqrtf(ajj[o]);
-  global_mut(l.minv)[at] = ajj[12] > 1e-30f ? rsqrtf(ajj[12]) / s : 0.0f;
+  return ajj[12] > 1e-30f ? rsqrtf(ajj[12]) / s : 0.0f;
 }
 
-// Grid k's weights and the matrix of grid k + 1.
-__global__ void __launch_bounds__(GT)
+// Grid k's weights and the matrix of grid k + 1; for the tail's first grid
+// both in the form mk_tail reads them (mg.h).  Four threads a node of grid
+// k + 1 (a thread's 225 dependent sums took 21 us a grid on average at P1
+// 1024^2; four quarter them, 12 us), and their threads take the nodes of grid k
+// in turn.
+constexpr int GS = 128;
+__global__ void __launch_bounds__(GS)
     gk_setup(const int2 *__restrict__ map, const MgSys *__restrict__ D, int sys, int k) {
   const int2 mb = where(map, sys);
   if (mb.x < 0) return;
-  const MgLevel &f = D[mb.x].lv[k], &c = D[mb.x].lv[k + 1];
-  const int id = mb.y * GT + threadIdx.x;
-  if (id < f.nx * f.ny) weight_node(f, id % f.nx, id / f.nx);
-  if (id < c.nx * c.ny) coarse_node(f, c, id % c.nx, id / c.nx);
+  const MgSys &d = D[mb.x];
+  const MgLevel &f = d.lv[k];
+  const gptr<float> fa = global_ptr(f.a);
+  const int px = f.px, pn = f.pn;
+  auto a = [=](int o, int x, int y) { return fa[(size_t)o * pn + mg_at(px, x, y)]; };
+  const int id = mb.y * GS + threadIdx.x, nf = f.nx * f.ny;
+  const bool tail = k == d.tail;
+  if (id < nf) {
+    const int x = id % f.nx, y = id / f.nx;
+    const float w = weight_node(a, f.nx, f.ny, x, y);
+    global_mut(f.minv)[mg_at(px, x, y)] = w;
+    if (tail) {
+      float v[28];
+#pragma unroll
+      for (int o = 0; o < 25; o++) v[o] = a(o, x, y);
+      v[25] = OM * w;
+      v[26] = v[27] = 0.0f;
+#pragma unroll
+      for (int u = 0; u < 7; u++)
+        ((gmptr<f4_t>)reinterpret_cast<f4_t *>(d.pack))[u * nf + id] =
+            f4_t{v[4 * u], v[4 * u + 1], v[4 * u + 2], v[4 * u + 3]};
+    }
+  }
+  if (k + 1 == d.nlev) return;  // (the tail's only grid)
+  const MgLevel &c = d.lv[k + 1];
+  const int nc = c.nx * c.ny, cid = id >> 2;
+  if (cid >= nc) return;  // (whole quads)
+  float *out = tail ? d.pack + 28 * nf + cid : c.a + mg_at(c.px, cid % c.nx, cid / c.nx);
+  const int step = tail ? nc : c.pn;
+  coarse_node(a, f.nx, f.ny, cid % c.nx, cid / c.nx,
+              [&](int o, float v) { global_mut(out)[(size_t)o * step] = v; });
 }
 
-// The tail's grids (from d.tail on, whose matrix is there) and the dense
-// inverse of the last one by Gauss-Jordan on its scaled form; a node whose
-// pivot vanishes (outside the mesh, or the constant of a singular matrix)
-// is left out.
-constexpr int ST = 512;  // (each thread holds a 7 x 7 patch)
+// The tail's grids below its first two, their weights and the dense inverse
+// of the last one, by Gauss-Jordan on its scaled form, two pivots a barrier; a
+// node whose pivot vanishes (outside the mesh, or the constant of a singular
+// matrix) is left out.  The matrices live in LDS as mk_tail keeps them; one
+// workgroup, so latency is all: 
+constexpr int ST = 512;
 __global__ void __launch_bounds__(ST)
     mk_tail_setup(const MgSys *__restrict__ D, const int *__restrict__ list, int sys) {
   if (list) sys = list[blockIdx.x];
   if (sys < 0) return;
   const MgSys &d = D[sys];
-  for (int k = d.tail; k < d.nlev; k++) {
-    const MgLevel &l = d.lv[k];
-    const int nn = l.nx * l.ny;
-    if (k > d.tail) {
-      for (int id = threadIdx.x; id < nn; id += ST) coarse_node(d.lv[k - 1], l, id % l.nx, id / l.nx);
-      __syncthreads();
+  extern __shared__ __align__(16) float lds[];  // [25][nodes] entries and [nodes] weights a grid
+  __shared__ double A[2][MG_DENSE][MG_DENSE + 1], sc[MG_DENSE];
+  const int tid = threadIdx.x, last = d.nlev - 1;
+  int nx = d.lv[d.tail].nx, ny = d.lv[d.tail].ny;
+  float *const pack = d.pack + 28 * nx * ny;
+  if (d.tail < last) {
+    nx = mg_next(nx);
+    ny = mg_next(ny);
+    const int n0 = 25 * nx * ny;
+    for (int i = tid; i < n0; i += 8 * ST) {
+      float v[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) v[u] = global_ptr(pack)[min(i + u * ST, n0 - 1)];
+#pragma unroll
+      for (int u = 0; u < 8; u++)
+        if (i + u * ST < n0) lds[i + u * ST] = v[u];
     }
-    for (int id = threadIdx.x; id < nn; id += ST) weight_node(l, id % l.nx, id / l.nx);
+  } else {  // one grid: its entries from the quads
+    const int nn = nx * ny;
+    for (int i = tid; i < 25 * nn; i += ST)
+      lds[i] = global_ptr(d.pack)[((i / nn >> 2) * nn + i % nn) * 4 + (i / nn & 3)];
+  }
+  __syncthreads();
+  float *l = lds;
+  for (int k = d.tail + 1; k <= last; k++) {
+    const int nn = nx * ny;
+    const float *la = l;
+    auto a = [=](int o, int x, int y) { return la[o * nn + y * nx + x]; };
+    for (int id = tid; id < nn; id += ST)
+      l[25 * nn + id] = OM * weight_node(a, nx, ny, id % nx, id / nx);
+    if (k < last) {
+      const int mx = mg_next(nx), my = mg_next(ny), mm = mx * my;
+      float *c = l + 26 * nn;
+      for (int t = tid; t < 4 * mm; t += ST) {
+        const int id = t >> 2;
+        coarse_node(a, nx, ny, id % mx, id / mx, [&](int o, float v) { c[o * mm + id] = v; });
+      }
+      l = c;
+      nx = mx;
+      ny = my;
+    }
     __syncthreads();
   }
-  // entries and weights of the grids below the first, node by node, as mk_tail
-  // keeps them in LDS
-  {
-    float *pk = d.pack;
-    for (int k = d.tail + 1; k < d.nlev; k++) {
-      const MgLevel &l = d.lv[k];
-      const int nn = l.nx * l.ny;
-      for (int id = threadIdx.x; id < nn; id += ST) {
-        const int at = mg_at(l.px, id % l.nx, id / l.nx);
-#pragma unroll
-        for (int o = 0; o < 25; o++)
-          global_mut(pk)[o * nn + id] = global_ptr(l.a)[(size_t)o * l.pn + at];
-        global_mut(pk)[25 * nn + id] = OM * global_ptr(l.minv)[at];
-      }
-      pk += 26 * nn;
-    }
-  }
-  __shared__ double A[2][MG_DENSE][MG_DENSE + 1], sc[MG_DENSE];
-  const MgLevel &l = d.lv[d.nlev - 1];
-  const int nn = l.nx * l.ny;
-  const gptr<float> a = global_ptr(l.a);
-  for (int i = threadIdx.x; i < nn; i += ST) {
-    const float aii = a[(size_t)12 * l.pn + mg_at(l.px, i % l.nx, i / l.nx)];
+  const int nn = nx * ny;
+  for (int i = tid; i < nn; i += ST) {
+    const float aii = l[12 * nn + i];
     sc[i] = aii > 1e-30f ? 1.0 / sqrt((double)aii) : 0.0;
   }
   __syncthreads();
-  for (int t = threadIdx.x; t < nn * nn; t += ST) {
+  for (int t = tid; t < nn * nn; t += ST) {
     const int i = t / nn, j = t % nn;
-    const int dx = j % l.nx - i % l.nx, dy = j / l.nx - i / l.nx;
+    const int dx = j % nx - i % nx, dy = j / nx - i / nx;
     double v = 0.0;
-    if (abs(dx) <= 2 && abs(dy) <= 2)
-      v = (double)a[(size_t)((dy + 2) * 5 + dx + 2) * l.pn + mg_at(l.px, i % l.nx, i / l.nx)];
+    if (abs(dx) <= 2 && abs(dy) <= 2) v = (double)l[((dy + 2) * 5 + dx + 2) * nn + i];
     A[0][i][j] = v * sc[i] * sc[j];
   }
+  // (the grids' entries and weights are final: out they go meanwhile)
+  if (d.tail < last) {
+    const int np = (int)(l - lds) + 26 * nn;
+    for (int i = tid; i < np; i += ST) global_mut(pack)[i] = lds[i];
+  }
   __syncthreads();
-  const int gi = threadIdx.x >> 6, gj = threadIdx.x & 63;
-  for (int k = 0; k < nn; k++) {  // step k reads one copy and writes the other
-    const double(*P)[MG_DENSE + 1] = A[k & 1];
-    double(*Q)[MG_DENSE + 1] = A[(k & 1) ^ 1];
-    const double pv = P[k][k];
-    const bool keep = pv > 1e-9;  // else the variable leaves the system
-    const double ip = keep ? 1.0 / pv : 0.0;
-    if (gj < nn)
-      for (int i = gi; i < nn; i += ST / 64) {
-        const double pij = P[i][gj], pik = P[i][k], pkj = P[k][gj] * ip;
-        Q[i][gj] = i == k ? (gj == k ? ip : pkj) : gj == k ? -pik * ip : pij - pik * pkj;
+  // one elimination: the entry (i, j) after pivot k, from its old value, the
+  // pivot row's and column's and the pivot's reciprocal (0: the variable leaves
+  // the system)
+  auto elim = [](int i, int j, int k, double pij, double pik, double pkj, double ip) {
+    const double r = pkj * ip;
+    return i == k ? (j == k ? ip : r) : j == k ? -pik * ip : pij - pik * r;
+  };
+  auto recip = [](double pv) { return pv > 1e-9 ? 1.0 / pv : 0.0; };
+  const int gi = tid >> 6, gj = tid & 63;
+  int cur = 0;
+  for (int k = 0; k < nn; k += 2, cur ^= 1) {  // reads one copy, writes the other
+    const double(*P)[MG_DENSE + 1] = A[cur];
+    double(*Q)[MG_DENSE + 1] = A[cur ^ 1];
+    if (gj < nn) {
+      const int m = k + 1;
+      const double ip = recip(P[k][k]), pkj = P[k][gj];
+      if (m < nn) {
+        const double pkm = P[k][m], pmk = P[m][k];
+        const double im = recip(elim(m, m, k, P[m][m], pmk, pkm, ip));
+        const double pmj = elim(m, gj, k, P[m][gj], pmk, pkj, ip);
+        for (int i = gi; i < nn; i += ST / 64) {
+          const double pik = P[i][k];
+          const double v = elim(i, gj, k, P[i][gj], pik, pkj, ip);
+          Q[i][gj] = elim(i, gj, m, v, elim(i, m, k, P[i][m], pik, pkm, ip), pmj, im);
+        }
+      } else {
+        for (int i = gi; i < nn; i += ST / 64)
+          Q[i][gj] = elim(i, gj, k, P[i][gj], P[i][k], pkj, ip);
       }
+    }
     __syncthreads();
   }
-  for (int t = threadIdx.x; t < nn * nn; t += ST) {
+  float *inv = pack + (d.tail < last ? (int)(l - lds) + 26 * nn : 0);
+  for (int t = tid; t < nn * nn; t += ST) {
     const int i = t / nn, j = t % nn;
-    global_mut(d.cinv)[t] = (float)(A[nn & 1][i][j] * sc[i] * sc[j]);
+    global_mut(inv)[t] = (float)(A[cur][i][j] * sc[i] * sc[j]);
   }
 }
 
@@ -770,33 +876,6 @@ __device__ __forceinline__ double restrict_cell(const MgSys &d, const MgLevel &l
   return s;
 }
 
-// A cell's shares of its four corners' P^T t.
-__device__ __forceinline__ void cell_shares(const MgSys &d, int c, float (&out)[4]) {
-  const gptr<f2_t> cfrac = frac_ptr(d.cfrac);
-  const gptr<float> t = global_ptr(d.ts);
-  const int k0 = global_ptr(d.cptr)[c], k1 = global_ptr(d.cptr)[c + 1];
-  double s[4] = {0.0, 0.0, 0.0, 0.0};
-  for (int k = k0; k < k1; k += 4) {  // four rows' loads in flight
-    f2_t f[4];
-    float v[4];
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-      const int j = min(k + u, k1 - 1);
-      f[u] = cfrac[j];
-      v[u] = k + u < k1 ? t[j] : 0.0f;
-    }
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-      s[0] += (double)((1.0f - f[u].x) * (1.0f - f[u].y)) * (double)v[u];
-      s[1] += (double)(f[u].x * (1.0f - f[u].y)) * (double)v[u];
-      s[2] += (double)((1.0f - f[u].x) * f[u].y) * (double)v[u];
-      s[3] += (double)(f[u].x * f[u].y) * (double)v[u];
-    }
-  }
-#pragma unroll
-  for (int q = 0; q < 4; q++) out[q] = (float)s[q];
-}
-
 // First grid: b = P^T t and the first smoothing step from zero; four threads
 // a node, one for each of its cells.
 __global__ void __launch_bounds__(NT)
@@ -956,20 +1035,25 @@ __device__ __forceinline__ float stencil32(C c, const float *v, int pv) {
 
 // The grids from d.tail on, in one workgroup.  A chain of some fifteen
 // barriers, so latency is all: every stencil entry is requested before the
-// first barrier (the first grid's into registers, TAIL_NODES nodes a thread,
-// the others' into LDS), and the phases then run on LDS alone.  With the
-// entries read in each phase it took 15 us for a first grid of 34 x 34.  When
-// every grid is in the tail it also restricts from the rows and interpolates
-// to them.  LDS: x, b and t of every grid, entries and weights of all but the
-// first, the dense inverse.
+// first barrier, in quads (the first grid's into registers, TAIL_NODES nodes a
+// thread; the others' into registers too, and on to LDS behind the first
+// grid's residual), and the phases then run on LDS alone.  When every grid is
+// in the tail it also restricts from the rows and interpolates to them.  LDS:
+// x, b and t of every grid, entries and weights of all but the first, the
+// dense inverse.  Of its 12.7 us at P2 101^2 (14.1 with the entries read one by
+// one), 3.0 are the loads, 2.7 the first grid's two stencils, the rest phases of
+// 0.25 - 0.7 us between barriers; P1 1024^2 13.7 -> 11.7 us.
 constexpr int TAIL_NODES = MG_TAIL / RT;
+constexpr int TAIL_PACK = 5;     // quads of the pack in flight, a thread
+constexpr int TAIL_ROWS = 5;     // rows in flight, a thread
+constexpr int TAIL_STAGE = 7000; // rows staged in LDS (12 bytes each), at most
 constexpr int TAIL_LEVELS = 10;  // grids of a tail, at most
 static_assert(TAIL_NODES * RT == MG_TAIL, "a thread owns whole nodes");
 __global__ void __launch_bounds__(RT)
     mk_tail(const MgSys *__restrict__ D, const MgScal *S, const int *__restrict__ list, int sys) {
   if (list) sys = list[blockIdx.x];
   if (sys < 0 || S[sys].a.status != ST_RUN) return;
-  extern __shared__ float lds[];
+  extern __shared__ __align__(16) float lds[];
   __shared__ float part[RT / 64][64];
   const MgSys &d = D[sys];
   const int tid = threadIdx.x, first = d.tail, last = d.nlev - 1;
@@ -1005,49 +1089,102 @@ __global__ void __launch_bounds__(RT)
   int tot = 0;
   for (int u = 0; u <= nu; u++) tot += dims(u).pn;
   float *coef = lds + 3 * tot;
-  float ca[TAIL_NODES][25], ma[TAIL_NODES];
-  int fat[TAIL_NODES];
-#pragma unroll
-  for (int u = 0; u < TAIL_NODES; u++) {
-    int x, y;
-    split(d0, min(tid + u * RT, nf - 1), x, y);
-    fat[u] = mg_at(d0.px, x, y);
-    ma[u] = OM * global_ptr(F.minv)[fat[u]];
-#pragma unroll
-    for (int o = 0; o < 25; o++) ca[u][o] = global_ptr(F.a)[(size_t)o * d0.pn + fat[u]];
-  }
-  for (int i = tid; i < 3 * tot; i += RT) lds[i] = 0.0f;
   int npk = 0;  // the pack: entries and weights of the other grids, the inverse
   for (int u = 1; u <= nu; u++) npk += 26 * dims(u).nn;
   const float *cinv = coef + npk;
-  npk += dims(nu).nn * dims(nu).nn;
-  {
-    const gptr<float> pk = global_ptr(d.pack);
-    int i = tid;
-    for (; i + 7 * RT < npk; i += 8 * RT) {
-      float v[8];
+  npk = (npk + dims(nu).nn * dims(nu).nn + 3) & ~3;
+  const gptr<f4_t> quad = (gptr<f4_t>)reinterpret_cast<const f4_t *>(d.pack);
+  float ca[TAIL_NODES][28];
+  int fat[TAIL_NODES];
 #pragma unroll
-      for (int u = 0; u < 8; u++) v[u] = pk[i + u * RT];
+  for (int u = 0; u < TAIL_NODES; u++) {
+    const int id = min(tid + u * RT, nf - 1);
+    int x, y;
+    split(d0, id, x, y);
+    fat[u] = mg_at(d0.px, x, y);
+    if (__builtin_amdgcn_readfirstlane(tid) + u * RT >= nf) continue;  // none of the wave's
 #pragma unroll
-      for (int u = 0; u < 8; u++) coef[i + u * RT] = v[u];
+    for (int o = 0; o < 7; o++) {
+      const f4_t v = quad[o * nf + id];
+#pragma unroll
+      for (int j = 0; j < 4; j++) ca[u][4 * o + j] = v[j];
     }
-    float v[8];
-#pragma unroll
-    for (int u = 0; u < 8; u++) v[u] = pk[min(i + u * RT, npk - 1)];
-#pragma unroll
-    for (int u = 0; u < 8; u++)
-      if (i + u * RT < npk) coef[i + u * RT] = v[u];
   }
+  const gptr<f4_t> pk = quad + 7 * nf;
+  f4_t pv[TAIL_PACK];
+#pragma unroll
+  for (int u = 0; u < TAIL_PACK; u++) pv[u] = pk[min(tid + u * RT, npk / 4 - 1)];
+  for (int i = tid; i < 3 * tot / 4; i += RT)
+    reinterpret_cast<f4_t *>(lds)[i] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  // (to LDS when the first grid's residual is done: nothing needs it before)
+  auto put_pack = [&]() {
+    f4_t *c4 = reinterpret_cast<f4_t *>(coef);
+#pragma unroll
+    for (int u = 0; u < TAIL_PACK; u++)
+      if (tid + u * RT < npk / 4) c4[tid + u * RT] = pv[u];
+    for (int i = tid + TAIL_PACK * RT; i < npk / 4; i += RT) c4[i] = pk[i];
+  };
   // the first grid's right-hand side and first smoothing step from zero
   if (first == 0) {
-    // each cell's rows once, into its corners' shares; then the nodes' sums
+    // each cell's rows (by way of LDS, where the pack goes later) into its
+    // corners' shares; then the nodes' sums
     const int ncx = fx - 1, nc = ncx * (d0.ny - 1);
-    float *share = coef + npk;  // [4][nc]
-    for (int c = tid; c < nc; c += RT) {
-      float s[4];
-      cell_shares(d, c, s);
+    const bool staged = d.n <= TAIL_STAGE;
+    float *share = coef + (staged ? max(npk, 3 * d.n) : npk);  // [4][nc]
+    float *row = coef;                        // [3][n]: value and position
+    const gptr<f2_t> cfrac = frac_ptr(d.cfrac);
+    const gptr<float> rt = global_ptr(d.ts);
+    const gptr<int> cptr = global_ptr(d.cptr);
+    const int n = d.n, nin = cptr[nc];  // rows that take part
+    int k0[TAIL_NODES], k1[TAIL_NODES];
 #pragma unroll
-      for (int q = 0; q < 4; q++) share[q * nc + c] = s[q];
+    for (int u = 0; u < TAIL_NODES; u++) {
+      const int c = min(tid + u * RT, nc - 1);
+      k0[u] = cptr[c];
+      k1[u] = cptr[c + 1];
+    }
+    for (int i = staged ? tid : nin; i < nin; i += 4 * RT) {
+      f2_t f[4];
+      float v[4];
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const int j = min(i + u * RT, nin - 1);
+        f[u] = cfrac[j];
+        v[u] = rt[j];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; u++)
+        if (i + u * RT < nin) {
+          row[i + u * RT] = v[u];
+          row[n + i + u * RT] = f[u].x;
+          row[2 * n + i + u * RT] = f[u].y;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < TAIL_NODES; u++) {
+      const int c = tid + u * RT;
+      if (c >= nc) continue;
+      double s[4] = {0.0, 0.0, 0.0, 0.0};
+      for (int k = k0[u]; k < k1[u]; k++) {
+        float v, x, y;
+        if (staged) {
+          v = row[k];
+          x = row[n + k];
+          y = row[2 * n + k];
+        } else {
+          const f2_t f = cfrac[k];
+          v = rt[k];
+          x = f.x;
+          y = f.y;
+        }
+        s[0] += (double)((1.0f - x) * (1.0f - y)) * (double)v;
+        s[1] += (double)(x * (1.0f - y)) * (double)v;
+        s[2] += (double)((1.0f - x) * y) * (double)v;
+        s[3] += (double)(x * y) * (double)v;
+      }
+#pragma unroll
+      for (int q = 0; q < 4; q++) share[q * nc + c] = (float)s[q];
     }
     __syncthreads();
 #pragma unroll
@@ -1063,7 +1200,7 @@ __global__ void __launch_bounds__(RT)
         if (cx >= 0 && cx < ncx && cy >= 0 && cy < d0.ny - 1) s += share[q * nc + cy * ncx + cx];
       }
       lds[tot + fat[u]] = s;
-      lds[fat[u]] = ma[u] * s;
+      lds[fat[u]] = ca[u][25] * s;
     }
   } else {
     __syncthreads();
@@ -1077,15 +1214,19 @@ __global__ void __launch_bounds__(RT)
   __syncthreads();
   int off = 0;
   const float *cf = coef;  // entries of the grid below the current one
+  if (nu > 0) {
+    float *x = lds, *b = x + tot, *t = b + tot;
+#pragma unroll
+    for (int v = 0; v < TAIL_NODES; v++)
+      if (tid + v * RT < nf)
+        t[fat[v]] = b[fat[v]] - stencil32([&](int o) { return ca[v][o]; }, x + fat[v], d0.px);
+  }
+  put_pack();
+  __syncthreads();
   for (int u = 0; u < nu; u++) {  // down
     const Dim l = dims(u), c = dims(u + 1);
     float *x = lds + off, *b = x + tot, *t = b + tot;
-    if (u == 0) {
-#pragma unroll
-      for (int v = 0; v < TAIL_NODES; v++)
-        if (tid + v * RT < nf)
-          t[fat[v]] = b[fat[v]] - stencil32([&](int o) { return ca[v][o]; }, x + fat[v], l.px);
-    } else {
+    if (u > 0) {
       const float *cl = cf - 26 * l.nn;
       for (int id = tid; id < l.nn; id += RT) {
         int px, py;
@@ -1093,8 +1234,8 @@ __global__ void __launch_bounds__(RT)
         const int at = mg_at(l.px, px, py);
         t[at] = b[at] - stencil32([&](int o) { return cl[o * l.nn + id]; }, x + at, l.px);
       }
+      __syncthreads();
     }
-    __syncthreads();
     float *xc = x + l.pn, *bc = xc + tot;
     for (int id = tid; id < c.nn; id += RT) {
       int X, Y;
@@ -1140,50 +1281,59 @@ __global__ void __launch_bounds__(RT)
       t[at] = x[at] + prolong_at(xc, c.px, px, py);
     }
     __syncthreads();
-    if (u == 0) {
-#pragma unroll
-      for (int v = 0; v < TAIL_NODES; v++)
-        if (tid + v * RT < nf)
-          x[fat[v]] = fmaf(
-              ma[v],
-              b[fat[v]] - stencil32([&](int o) { return ca[v][o]; }, t + fat[v], l.px), t[fat[v]]);
-    } else {
-      const float *cl = cf - 26 * l.nn;
-      for (int id = tid; id < l.nn; id += RT) {
-        int px, py;
-        split(l, id, px, py);
-        const int at = mg_at(l.px, px, py);
-        x[at] = fmaf(cl[25 * l.nn + id],
-                     b[at] - stencil32([&](int o) { return cl[o * l.nn + id]; }, t + at, l.px),
-                     t[at]);
-      }
+    if (u == 0) break;
+    const float *cl = cf - 26 * l.nn;
+    for (int id = tid; id < l.nn; id += RT) {
+      int px, py;
+      split(l, id, px, py);
+      const int at = mg_at(l.px, px, py);
+      x[at] = fmaf(cl[25 * l.nn + id],
+                   b[at] - stencil32([&](int o) { return cl[o * l.nn + id]; }, t + at, l.px),
+                   t[at]);
     }
     __syncthreads();
   }
+  const float *b0 = lds + tot, *t0 = b0 + tot;
+  // the first grid's smoothing (a single grid has its solution already)
+  auto smooth = [&](int v) {
+    return nu > 0 ? fmaf(ca[v][25],
+                         b0[fat[v]] -
+                             stencil32([&](int o) { return ca[v][o]; }, t0 + fat[v], d0.px),
+                         t0[fat[v]])
+                  : lds[fat[v]];
+  };
   if (first > 0) {
 #pragma unroll
-    for (int u = 0; u < TAIL_NODES; u++)
-      if (tid + u * RT < nf) global_mut(F.t)[fat[u]] = lds[fat[u]];
+    for (int v = 0; v < TAIL_NODES; v++)
+      if (tid + v * RT < nf) global_mut(F.t)[fat[v]] = smooth(v);
     return;
   }
   const gptr<int> cell = global_ptr(d.cell);
   const gptr<f2_t> frac = frac_ptr(d.frac);
   const gptr<float> sq = global_ptr(d.sq), x0 = global_ptr(smoothed(d));
   const float icx = 1.0f / (float)(fx - 1);
-  for (int i = tid; i < d.npad; i += 4 * RT) {  // four rows' loads in flight
-    int c[4];
-    f2_t f[4];
-    float w[4], y[4];
+  int c[TAIL_ROWS];
+  f2_t f[TAIL_ROWS];
+  float w[TAIL_ROWS], y[TAIL_ROWS];
+  auto rows = [&](int i) {  // TAIL_ROWS rows' loads in flight
 #pragma unroll
-    for (int u = 0; u < 4; u++) {
+    for (int u = 0; u < TAIL_ROWS; u++) {
       const int j = min(i + u * RT, d.npad - 1);
       c[u] = cell[j];
       f[u] = frac[j];
       w[u] = sq[j];
       y[u] = x0[j];
     }
+  };
+  rows(tid);
 #pragma unroll
-    for (int u = 0; u < 4; u++) {
+  for (int v = 0; v < TAIL_NODES; v++)
+    if (nu > 0 && tid + v * RT < nf) lds[fat[v]] = smooth(v);
+  __syncthreads();
+  for (int i = tid; i < d.npad; i += TAIL_ROWS * RT) {
+    if (i != tid) rows(i);
+#pragma unroll
+    for (int u = 0; u < TAIL_ROWS; u++) {
       if (i + u * RT >= d.npad || c[u] < 0) continue;
       const int cy = (int)(((float)c[u] + 0.5f) * icx);
       global_mut(d.t)[i + u * RT] =
@@ -1411,6 +1561,7 @@ MgPlan *build_plan(System &s, const Mesh &m, const int *order, hipStream_t st) {
   try {
     const int n = s.n, np = s.npad;
     const bool own = s.mesh != nullptr;
+    pl->n = n;
     const unsigned g = nb(n, NT);
     DevBuf<double> ext((size_t)7 * g), ar(256);
     DevBuf<double2> pt(n);
@@ -1508,26 +1659,36 @@ MgPlan *build_plan(System &s, const Mesh &m, const int *order, hipStream_t st) {
 }
 
 size_t tail_lds_of(const MgPlan &pl) {
-  size_t t = 0;
+  size_t t = 0, pack = 3;  // (whole quads)
   for (int k = pl.tail; k < pl.nlev; k++) {
     t += 3 * pl.pn[k];
-    if (k > pl.tail) t += 26 * pl.nx[k] * pl.ny[k];
+    if (k > pl.tail) pack += (size_t)26 * pl.nx[k] * pl.ny[k];
   }
   const size_t nn = (size_t)pl.nx[pl.nlev - 1] * pl.ny[pl.nlev - 1];
-  t += nn * nn;
-  if (pl.tail == 0) t += 4 * (size_t)(pl.nx[0] - 1) * (pl.ny[0] - 1);
-  return t * sizeof(float);
+  pack += nn * nn;
+  if (pl.tail == 0)
+    pack = std::max(pack, pl.n <= TAIL_STAGE ? (size_t)3 * pl.n : 0) + 4 * (size_t)(pl.nx[0] - 1) * (pl.ny[0] - 1);
+  return (t + pack) * sizeof(float);
 }
 
 }  // namespace
 
 size_t mg_tail_lds(const MgPlan &pl) { return tail_lds_of(pl); }
 
+size_t mg_setup_lds(const MgPlan &pl) {
+  size_t t = pl.tail + 1 == pl.nlev ? (size_t)25 * pl.nx[pl.tail] * pl.ny[pl.tail] : 0;
+  for (int k = pl.tail + 1; k < pl.nlev; k++) t += (size_t)26 * pl.nx[k] * pl.ny[k];
+  return t * sizeof(float);
+}
+
 void mg_allow_lds(const MgPlan &pl) {
   const size_t lds = mg_tail_lds(pl);
   REQUIRE(lds <= 150 * 1024, ADMFEM_ERR_UNSUPPORTED, "tail grids too large for LDS");
+  REQUIRE(mg_setup_lds(pl) <= 110 * 1024, ADMFEM_ERR_UNSUPPORTED, "tail grids too large for LDS");
   HIPCHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(mk_tail),
                                hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024));
+  HIPCHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(mk_tail_setup),
+                               hipFuncAttributeMaxDynamicSharedMemorySize, 110 * 1024));
 }
 
 void mg_plan_free(MgPlan *p) { delete p; }
@@ -1542,8 +1703,10 @@ const MgPlan *mg_plan(System &s, hipStream_t st) {
 size_t mg_grid_floats(const MgPlan &pl) {
   size_t f = 0;
   for (int k = 0; k < pl.nlev; k++)
-    f += (size_t)29 * pl.pn[k] + (k > pl.tail ? (size_t)26 * pl.nx[k] * pl.ny[k] : 0);
-  return f + MG_DENSE * MG_DENSE;
+    f += (size_t)29 * pl.pn[k] +
+         (k > pl.tail ? (size_t)26 * pl.nx[k] * pl.ny[k]
+                      : k == pl.tail ? (size_t)28 * pl.nx[k] * pl.ny[k] : 0);
+  return f + MG_DENSE * MG_DENSE + 3;
 }
 
 void mg_grid_layout(const MgPlan &pl, float *base, MgSys &d) {
@@ -1571,8 +1734,6 @@ void mg_grid_layout(const MgPlan &pl, float *base, MgSys &d) {
     base += 29 * pn;
   }
   d.pack = base;
-  for (int k = pl.tail + 1; k < pl.nlev; k++) base += 26 * (size_t)pl.nx[k] * pl.ny[k];
-  d.cinv = base;
 }
 
 void mg_parts(MgSys &d, int nblk, bool reduce, double *part) {
@@ -1673,6 +1834,10 @@ MgWork *ensure_work(System &s, const MgPlan &pl, hipStream_t st) {
 static int mg_tiles_down(const MgPlan &pl, int k) {
   return (int)(nb(pl.nx[k + 1], TC) * nb(pl.ny[k + 1], TC));
 }
+static int mg_blocks_setup(const MgPlan &pl, int k) {
+  const int64_t nf = (int64_t)pl.nx[k] * pl.ny[k];
+  return (int)nb(k + 1 < pl.nlev ? std::max(nf, 4 * (int64_t)pl.nx[k + 1] * pl.ny[k + 1]) : nf, GS);
+}
 static int mg_tiles_up(const MgPlan &pl, int k) {
   return k ? (int)(nb(pl.nx[k], TF) * nb(pl.ny[k], TF))
            : (int)(nb(pl.nx[k] - 1, TF) * nb(pl.ny[k] - 1, TF));
@@ -1682,10 +1847,10 @@ void mg_stages(const MgPlan &pl, int npad, int (&nblk)[MG_STAGES]) {
   for (int &v : nblk) v = 0;
   nblk[MGS_ROWS] = (int)nb(npad, NT);
   if (pl.steps == 2) nblk[MGS_TWO] = nblk[MGS_ROWS];
-  nblk[MGS_GALERKIN] = (int)nb((int64_t)pl.nx[0] * pl.ny[0], GT / 4);
+  nblk[MGS_GALERKIN] = (int)nb((int64_t)pl.nx[0] * pl.ny[0], mg_gn(1));
   if (pl.tail > 0) nblk[MGS_RESTRICT] = (int)nb((int64_t)pl.nx[0] * pl.ny[0], NT / 4);
+  for (int k = 0; k <= pl.tail; k++) nblk[MGS_SETUP + k] = mg_blocks_setup(pl, k);
   for (int k = 0; k < pl.tail; k++) {
-    nblk[MGS_SETUP + k] = (int)nb((int64_t)pl.nx[k] * pl.ny[k], GT);
     nblk[MGS_DOWN + k] = mg_tiles_down(pl, k);
     nblk[MGS_UP + k] = mg_tiles_up(pl, k);
   }
@@ -1694,10 +1859,10 @@ void mg_stages(const MgPlan &pl, int npad, int (&nblk)[MG_STAGES]) {
 void mg_batch_setup(const MgBatch &B, const MgSys *D, hipStream_t st) {
   auto n = [&](int q) { return (unsigned)B.nmap[q]; };
   mk_scale<<<n(MGS_ROWS), NT, 0, st>>>(B.map[MGS_ROWS], D, 0);
-  mk_galerkin<<<n(MGS_GALERKIN), GT, 0, st>>>(B.map[MGS_GALERKIN], D, 0);
-  for (int k = 0; k < B.tail; k++)
-    gk_setup<<<n(MGS_SETUP + k), GT, 0, st>>>(B.map[MGS_SETUP + k], D, 0, k);
-  mk_tail_setup<<<(unsigned)B.nsys, ST, 0, st>>>(D, B.list, 0);
+  mk_galerkin<1><<<n(MGS_GALERKIN), GT, 0, st>>>(B.map[MGS_GALERKIN], D, 0);
+  for (int k = 0; k <= B.tail; k++)
+    gk_setup<<<n(MGS_SETUP + k), GS, 0, st>>>(B.map[MGS_SETUP + k], D, 0, k);
+  mk_tail_setup<<<(unsigned)B.nsys, ST, B.setup_lds, st>>>(D, B.list, 0);
   HIPCHECK(hipGetLastError());
 }
 
@@ -1740,10 +1905,12 @@ void mg_batch_iterations(const MgBatch &B, const MgSys *D, MgScal *S, int iters,
 // matrices and smoothing weights, the last grid's inverse.
 void mg_setup(const MgPlan &pl, int nblk, const MgSys *D, int sys, hipStream_t st) {
   mk_scale<<<nblk, NT, 0, st>>>(nullptr, D, sys);
-  mk_galerkin<<<nb(pl.nx[0] * pl.ny[0], GT / 4), GT, 0, st>>>(nullptr, D, sys);
-  for (int k = 0; k < pl.tail; k++)
-    gk_setup<<<nb(pl.nx[k] * pl.ny[k], GT), GT, 0, st>>>(nullptr, D, sys, k);
-  mk_tail_setup<<<1, ST, 0, st>>>(D, nullptr, sys);
+  const int64_t nodes = (int64_t)pl.nx[0] * pl.ny[0];
+  if (nodes <= GALERKIN_SPLIT) mk_galerkin<4><<<nb(nodes, mg_gn(4)), GT, 0, st>>>(nullptr, D, sys);
+  else mk_galerkin<1><<<nb(nodes, mg_gn(1)), GT, 0, st>>>(nullptr, D, sys);
+  for (int k = 0; k <= pl.tail; k++)
+    gk_setup<<<mg_blocks_setup(pl, k), GS, 0, st>>>(nullptr, D, sys, k);
+  mk_tail_setup<<<1, ST, mg_setup_lds(pl), st>>>(D, nullptr, sys);
   HIPCHECK(hipGetLastError());
 }
 

@@ -402,6 +402,7 @@ struct Server {
       std::copy(v, v + MG_STAGES, nblk[a].begin());
       b.tail = std::max(b.tail, T.plan->tail);
       b.tail_lds = std::max(b.tail_lds, mg_tail_lds(*T.plan));
+      b.setup_lds = std::max(b.setup_lds, mg_setup_lds(*T.plan));
       b.reduce = b.reduce || T.nblk > MG_BATCH_SUM;
     }
     std::vector<int> used;
