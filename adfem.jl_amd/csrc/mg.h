@@ -51,9 +51,11 @@ struct MgSys {
   const float2 *cfrac;      // frac in that order
   const int *pos;           // each row's place in it (-1: none)
   const double *b;          // right-hand side
-  double *x, *r, *q, *p[2];
+  double *x, *r[2], *q, *p[2];  // (r, p: iteration it reads one and writes the
+                            // other; r[it & 1] is the residual after it)
   float *z, *rs, *x0, *t;   // preconditioned residual, scaled residual,
                             // smoothed correction, corrected
+  float2 *wrq;              // r and q times the first smoothing step's weight
   float *ts;                // the restriction's input, in the cells' order
   double *part4, *partz;    // 4 x nblk and nblk block partials
   double *sum4, *sumz;      // their sums, when one block makes them
@@ -69,7 +71,7 @@ struct MgSys {
 };
 
 // One system's solve: the state, in two copies (mk_dir reads a and writes b,
-// mk_update reads b and writes a, every other kernel reads a).
+// mk_step reads b and writes a, every other kernel reads a).
 struct MgState {
   double rz, rr;
   int status;               // as in cg.hip: 0 run, 1 converged, 2 iterations

@@ -27,10 +27,10 @@
 // form S A S of cg.hip) with FP64 sums; it only shapes the search direction.
 // A solve is converged when the residual recomputed from the FP64 matrix is.
 //
-// One iteration (every kernel returns at once when its system is done):
-//   mk_pre       second smoothing step (the first, from zero, is taken where
-//                the residual itself is written); plans with two steps
-//   mk_res       residual after it
+// One iteration (every kernel returns at once when its system is done), from
+// the fine residual after the first smoothing step (mk_step; mk_lead when CG
+// starts):
+//   mk_res       residual after the second one; plans with two steps
 //   mk_restrict  to the first grid, with its first smoothing step
 //   gk_down      the grids down to MG_TAIL nodes: residual and restriction of
 //                a tile in one launch
@@ -41,11 +41,12 @@
 //                steps): z, partials of r.z
 //   mk_dir       beta = r.z / previous r.z, p = z + beta p, q = A p; partials
 //                of p.q, r.q, q.q, r.r
-//   mk_update    alpha = r.z / p.q, the new |r|^2 = r.r - 2 alpha r.q +
-//                alpha^2 q.q, x += alpha p, r -= alpha q, first smoothing
-// When every grid fits the tail, mk_tail also restricts and interpolates: five
+//   mk_step      alpha = r.z / p.q, the new |r|^2 = r.r - 2 alpha r.q +
+//                alpha^2 q.q, x += alpha p, r -= alpha q, first smoothing step
+//                and the residual after it (two steps: the second step)
+// When every grid fits the tail, mk_tail also restricts and interpolates: four
 // launches an iteration.  The scalars need no launch of their own: every
-// block of mk_dir and mk_update sums the partials itself, in one order, and
+// block of mk_dir and mk_step sums the partials itself, in one order, and
 // block 0 keeps the result for the next kernel (two copies of the state, each
 // kernel reading one and writing the other).  Above MG_SUM partials one
 // block sums them first (ms_reduce): 1,032 blocks reading 1,032 x 4 partials
@@ -581,17 +582,35 @@ __device__ __forceinline__ void first_smooth(const MgSys &d, int i, double ri) {
   global_mut(d.x0)[i] = (d.steps == 2 ? C0 : OM) * global_ptr(d.minv)[i] * rs;
 }
 
+// A row's residual after the first smoothing step, x0 - rs its negative
+// without the off-diagonal part `dot`: with one step the input of the
+// restriction, in the unscaled form's dual, sqrt(a_ii) (rs - Â x0), in the
+// order of the cells; with two, the second step.
+__device__ __forceinline__ void smooth_on(const MgSys &d, int i, float x0, float rs, double dot) {
+  const double res = (double)rs - (double)x0 - dot;
+  if (d.steps == 2) {
+    global_mut(d.t)[i] = (float)((1.0 + (double)CM) * (double)x0 +
+                                 (double)(C1 * global_ptr(d.minv)[i]) * res);
+  } else {
+    const int k = global_ptr(d.pos)[i];
+    if (k >= 0) global_mut(d.ts)[k] = (float)(res * (double)global_ptr(d.sq)[i]);
+  }
+}
+
 // Where the smoothing before the correction left its result.
 __device__ __forceinline__ const float *smoothed(const MgSys &d) {
   return d.steps == 2 ? d.t : d.x0;
 }
 
 // Row i's product with the FP32 scaled off-diagonals.
+template <class L, class F>
+__device__ __forceinline__ double dot32(const MgSys &d, int i, L load, F comb) {
+  return d.sd ? sell_dot16<float>(i, d.sp, d.sd, d.sv32, load, comb)
+              : sell_dot<float>(i, d.sp, d.sc, d.sv32, load, comb);
+}
 template <class L>
 __device__ __forceinline__ double dot32(const MgSys &d, int i, L load) {
-  auto dbl = [](float v) { return (double)v; };
-  return d.sd ? sell_dot16<float>(i, d.sp, d.sd, d.sv32, load, dbl)
-              : sell_dot<float>(i, d.sp, d.sc, d.sv32, load, dbl);
+  return dot32(d, i, load, [](float v) { return (double)v; });
 }
 
 // Start: x = b on identity rows and 0 elsewhere, r = b - A x (0 on those
@@ -615,7 +634,7 @@ __global__ void __launch_bounds__(NT)
     // never written for a row outside the grids, but read (times zero) through
     // its padding entries
     if (global_ptr(d.pos)[i] < 0) global_mut(d.t)[i] = 0.0f;
-    global_mut(d.r)[i] = ri;
+    global_mut(d.r[0])[i] = ri;
     first_smooth(d, i, ri);
     t[0] = ri * ri;
     t[1] = bi * bi;
@@ -661,7 +680,7 @@ __global__ void __launch_bounds__(NT)
     const double ax = global_ptr(d.diag)[i] * x[i] +
                       sell_dot<double>(i, d.sp, d.sc, d.sv64, [&](int c) { return x[c]; });
     const double ri = bi - ax;
-    global_mut(d.r)[i] = ri;
+    global_mut(d.r[S[m.x].a.it & 1])[i] = ri;
     first_smooth(d, i, ri);
     t[0] = ri * ri;
   }
@@ -715,8 +734,8 @@ __global__ void __launch_bounds__(RT)
     for (int j = 0; j < NV; j++) global_mut(NV == 1 ? d.sumz : d.sum4)[j] = t[j];
 }
 
-// p = z + beta p (into the other buffer), q = A p; partials of p.q, r.q,
-// q.q, r.r.  A neighbour's p is formed on the fly by the same fused
+// p = z + beta p (into the other buffer), q = A p, and r and q with the first
+// smoothing step's weight for mk_step; partials of p.q, r.q, q.q, r.r.  A neighbour's p is formed on the fly by the same fused
 // multiply-add as its own row forms it.
 __global__ void __launch_bounds__(NT)
     mk_dir(const int2 *__restrict__ map, const MgSys *__restrict__ D, MgScal *S_, int sys) {
@@ -746,11 +765,14 @@ __global__ void __launch_bounds__(NT)
     struct zp { float z; double p; };
     auto load = [&](int c) { return zp{z[c], p[c]}; };
     auto comb = [&](zp v) { return fma(beta, v.p, (double)v.z); };
-    const double pi = comb(load(i)), ri = global_ptr(d.r)[i];
+    const double pi = comb(load(i)), ri = global_ptr(d.r[odd])[i];
     const double qi =
         global_ptr(d.diag)[i] * pi + sell_dot<double>(i, d.sp, d.sc, d.sv64, load, comb);
     global_mut(d.p[!odd])[i] = pi;
     global_mut(d.q)[i] = qi;
+    const double w =
+        (double)((d.steps == 2 ? C0 : OM) * global_ptr(d.minv)[i]) * global_ptr(d.dsq)[i];
+    ((gmptr<f2_t>)reinterpret_cast<f2_t *>(d.wrq))[i] = f2_t{(float)(w * ri), (float)(w * qi)};
     t[0] = pi * qi;
     t[1] = ri * qi;
     t[2] = qi * qi;
@@ -759,10 +781,15 @@ __global__ void __launch_bounds__(NT)
   put_partials<4>(t, d.part4, d.nblk, m.y);
 }
 
-// x += alpha p, r -= alpha q (p: the buffer mk_dir wrote), first smoothing
-// step of the next V-cycle
+// x += alpha p, r -= alpha q (p: the buffer mk_dir wrote; r into the other
+// buffer), and the next V-cycle's first smoothing step and residual.  The step
+// of row and neighbours alike is w r - alpha w q from mk_dir's pair (w the
+// step's weight), one 8-byte gather: against an update and a residual of their
+// own it saves a launch, one pass of P1 64^2 1.11 -> 1.06 ms, heat 200^2 1.39 ->
+// 1.35, even at 1024^2; with the neighbours' r, q and weights gathered (28
+// bytes) 1024^2 was 1.3% slower.
 __global__ void __launch_bounds__(NT)
-    mk_update(const int2 *__restrict__ map, const MgSys *__restrict__ D, MgScal *S_, int sys) {
+    mk_step(const int2 *__restrict__ map, const MgSys *__restrict__ D, MgScal *S_, int sys) {
   const int2 m = where(map, sys);
   if (m.x < 0) return;
   const MgSys &d = D[m.x];
@@ -789,27 +816,30 @@ __global__ void __launch_bounds__(NT)
   if (lead) S->a = st;
   const int i = m.y * NT + threadIdx.x;
   if (!ok || i >= d.npad) return;
-  const double pi = global_ptr(d.p[st.it & 1])[i];
-  const double xi = fma(alpha, pi, global_ptr(d.x)[i]);
-  const double ri = fma(-alpha, global_ptr(d.q)[i], global_ptr(d.r)[i]);
-  global_mut(d.x)[i] = xi;
-  global_mut(d.r)[i] = ri;
-  first_smooth(d, i, ri);
+  const double ri = fma(-alpha, global_ptr(d.q)[i], global_ptr(d.r[(st.it & 1) ^ 1])[i]);
+  global_mut(d.x)[i] = fma(alpha, global_ptr(d.p[st.it & 1])[i], global_ptr(d.x)[i]);
+  global_mut(d.r[st.it & 1])[i] = ri;
+  if (st.status != ST_RUN) return;
+  const gptr<f2_t> w = frac_ptr(d.wrq);
+  auto load = [&](int c) { return w[c]; };
+  auto first = [&](f2_t v) { return (float)fma(-alpha, (double)v.y, (double)v.x); };
+  const float rs = (float)(ri * global_ptr(d.dsq)[i]), x0 = first(load(i));
+  global_mut(d.rs)[i] = rs;
+  global_mut(d.x0)[i] = x0;
+  smooth_on(d, i, x0, rs, dot32(d, i, load, [&](f2_t v) { return (double)first(v); }));
 }
 
-// The second smoothing step from zero (steps = 2): t
+// The same from the first smoothing step that mk_start or mk_check took, when
+// CG starts.
 __global__ void __launch_bounds__(NT)
-    mk_pre(const int2 *__restrict__ map, const MgSys *__restrict__ D, const MgScal *S, int sys) {
+    mk_lead(const int2 *__restrict__ map, const MgSys *__restrict__ D, const MgScal *S, int sys) {
   const int2 m = where(map, sys);
-  if (m.x < 0 || S[m.x].a.status != ST_RUN) return;
+  if (m.x < 0 || S[m.x].a.status != ST_RUN || !S[m.x].a.first) return;
   const MgSys &d = D[m.x];
   const int i = m.y * NT + threadIdx.x;
   if (i >= d.npad) return;
   const gptr<float> x0 = global_ptr(d.x0);
-  const double res = (double)global_ptr(d.rs)[i] - (double)x0[i] -
-                     dot32(d, i, [&](int c) { return x0[c]; });
-  global_mut(d.t)[i] = (float)((1.0 + (double)CM) * (double)x0[i] +
-                               (double)(C1 * global_ptr(d.minv)[i]) * res);
+  smooth_on(d, i, x0[i], global_ptr(d.rs)[i], dot32(d, i, [&](int c) { return x0[c]; }));
 }
 
 // The first of two smoothing steps after the correction (steps = 2):
@@ -828,8 +858,7 @@ __global__ void __launch_bounds__(NT)
       (float)fma((double)(C0 * global_ptr(d.minv)[i]), res, (double)t[i]);
 }
 
-// ts = the fine residual after the first smoothing step(s), in the unscaled
-// form's dual, sqrt(a_ii) (rs - Â x0), in the order of the cells
+// ts = the fine residual after the second smoothing step (steps = 2)
 __global__ void __launch_bounds__(NT)
     mk_res(const int2 *__restrict__ map, const MgSys *__restrict__ D, const MgScal *S, int sys) {
   const int2 m = where(map, sys);
@@ -837,7 +866,7 @@ __global__ void __launch_bounds__(NT)
   const MgSys &d = D[m.x];
   const int i = m.y * NT + threadIdx.x;
   if (i >= d.npad) return;
-  const gptr<float> x = global_ptr(smoothed(d));
+  const gptr<float> x = global_ptr(d.t);
   const double res = (double)global_ptr(d.rs)[i] - (double)x[i] -
                      dot32(d, i, [&](int c) { return x[c]; });
   const int k = global_ptr(d.pos)[i];
@@ -1369,7 +1398,7 @@ __global__ void __launch_bounds__(NT)
                    global_ptr(d.dsq)[i]);
     }
     global_mut(d.z)[i] = zi;
-    v[0] = global_ptr(d.r)[i] * (double)zi;
+    v[0] = global_ptr(d.r[S[m.x].a.it & 1])[i] * (double)zi;
   }
   put_partials<1>(v, d.partz, d.nblk, m.y);
 }
@@ -1750,7 +1779,8 @@ struct MgWork {
   DevBuf<MgSys> d;
   DevBuf<MgScal> sc;
   MgScal *h_sc = nullptr;        // pinned
-  DevBuf<double> x, r, q, p0, p1, dsq, part;
+  DevBuf<double> x, r, r1, q, p0, p1, dsq, part;
+  DevBuf<float2> wrq;
   DevBuf<float> sv32, sq, minv, z, rs, x0, t, ts, grid;
   int nblk = 0;
   int last_it = 14;              // iterations of the last solve
@@ -1774,6 +1804,7 @@ MgWork *ensure_work(System &s, const MgPlan &pl, hipStream_t st) {
     w->nblk = (int)(nb(np, NT) + 7) / 8 * 8;  // a multiple of 8: the XCD deal
     w->x.alloc(np);
     w->r.alloc(np);
+    w->r1.alloc(np);
     w->q.alloc(np);
     w->p0.alloc(np);
     w->p1.alloc(np);
@@ -1787,6 +1818,7 @@ MgWork *ensure_work(System &s, const MgPlan &pl, hipStream_t st) {
     w->x0.alloc(np);
     w->t.alloc(np);
     w->ts.alloc(np);
+    w->wrq.alloc(np);
     w->grid.alloc(mg_grid_floats(pl));
     w->d.alloc(1);
     w->sc.alloc(1);
@@ -1803,7 +1835,8 @@ MgWork *ensure_work(System &s, const MgPlan &pl, hipStream_t st) {
     d.sq = w->sq.p;
     d.minv = w->minv.p;
     d.x = w->x.p;
-    d.r = w->r.p;
+    d.r[0] = w->r.p;
+    d.r[1] = w->r1.p;
     d.q = w->q.p;
     d.p[0] = w->p0.p;
     d.p[1] = w->p1.p;
@@ -1812,6 +1845,7 @@ MgWork *ensure_work(System &s, const MgPlan &pl, hipStream_t st) {
     d.x0 = w->x0.p;
     d.t = w->t.p;
     d.ts = w->ts.p;
+    d.wrq = w->wrq.p;
     d.n = s.n;
     d.npad = s.npad;
     mg_parts(d, w->nblk, w->nblk > MG_SUM, w->part.p);
@@ -1878,9 +1912,9 @@ void mg_batch_iterations(const MgBatch &B, const MgSys *D, MgScal *S, int iters,
   auto n = [&](int q) { return (unsigned)B.nmap[q]; };
   const int2 *rows = B.map[MGS_ROWS];
   const unsigned nl = (unsigned)B.nsys, nr = n(MGS_ROWS);
+  mk_lead<<<nr, NT, 0, st>>>(rows, D, S, 0);
   for (int it = 0; it < iters; it++) {
-    if (n(MGS_TWO)) mk_pre<<<n(MGS_TWO), NT, 0, st>>>(B.map[MGS_TWO], D, S, 0);
-    mk_res<<<nr, NT, 0, st>>>(rows, D, S, 0);
+    if (n(MGS_TWO)) mk_res<<<n(MGS_TWO), NT, 0, st>>>(B.map[MGS_TWO], D, S, 0);
     if (B.tail > 0)
       mk_restrict<<<n(MGS_RESTRICT), NT, 0, st>>>(B.map[MGS_RESTRICT], D, S, 0);
     for (int k = 0; k < B.tail; k++)
@@ -1894,7 +1928,7 @@ void mg_batch_iterations(const MgBatch &B, const MgSys *D, MgScal *S, int iters,
     if (B.reduce) ms_reduce<1><<<nl, RT, 0, st>>>(D, S, B.list, 0);
     mk_dir<<<nr, NT, 0, st>>>(rows, D, S, 0);
     if (B.reduce) ms_reduce<4><<<nl, RT, 0, st>>>(D, S, B.list, 0);
-    mk_update<<<nr, NT, 0, st>>>(rows, D, S, 0);
+    mk_step<<<nr, NT, 0, st>>>(rows, D, S, 0);
   }
   mk_check<<<nr, NT, 0, st>>>(rows, D, S, 0, nullptr);
   ms_check<<<nl, RT, 0, st>>>(D, S, B.list, 0, host);
@@ -1919,8 +1953,7 @@ namespace {
 void iteration(const MgPlan &pl, MgWork *w, hipStream_t st) {
   const MgSys *D = w->d.p;
   MgScal *S = w->sc.p;
-  if (pl.steps == 2) mk_pre<<<w->nblk, NT, 0, st>>>(nullptr, D, S, 0);
-  mk_res<<<w->nblk, NT, 0, st>>>(nullptr, D, S, 0);
+  if (pl.steps == 2) mk_res<<<w->nblk, NT, 0, st>>>(nullptr, D, S, 0);
   if (pl.tail > 0)
     mk_restrict<<<nb(pl.nx[0] * pl.ny[0], NT / 4), NT, 0, st>>>(nullptr, D, S, 0);
   for (int k = 0; k < pl.tail; k++)
@@ -1934,7 +1967,7 @@ void iteration(const MgPlan &pl, MgWork *w, hipStream_t st) {
   if (w->nblk > MG_SUM) ms_reduce<1><<<1, RT, 0, st>>>(D, S, nullptr, 0);
   mk_dir<<<w->nblk, NT, 0, st>>>(nullptr, D, S, 0);
   if (w->nblk > MG_SUM) ms_reduce<4><<<1, RT, 0, st>>>(D, S, nullptr, 0);
-  mk_update<<<w->nblk, NT, 0, st>>>(nullptr, D, S, 0);
+  mk_step<<<w->nblk, NT, 0, st>>>(nullptr, D, S, 0);
 }
 
 // Whether the V-cycle pays for the assembled matrix: not when a mass term
@@ -1957,7 +1990,7 @@ bool mg_pays(System &s, MgWork *w, hipStream_t st) {
   return !(w->rowsum > MASS_DOMINANT);
 }
 
-// Products with the system's matrix in an iteration (mk_res, mk_post,
+// Products with the system's matrix in an iteration (mk_step, mk_post,
 // mk_dir): what max_iter bounds and the stats report, as for Jacobi-PCG, whose
 // iterations are one product each.
 constexpr int MG_PRODUCTS = 3;
@@ -2007,6 +2040,7 @@ bool mg_solve(System &s, const double *b, double *x_out, const admfem_solve_opts
   // and a capture costs a first solve 0.2 - 3 ms and stops other threads' copies.
   int chunk = o.check_every > 0 ? o.check_every : w->last_it;
   for (;;) {
+    mk_lead<<<w->nblk, NT, 0, st>>>(nullptr, D, S, 0);
     for (int it = 0; it < chunk; it++) iteration(pl, w, st);
     mk_check<<<w->nblk, NT, 0, st>>>(nullptr, D, S, 0, b);
     ms_check<<<1, RT, 0, st>>>(D, S, nullptr, 0, w->h_sc);

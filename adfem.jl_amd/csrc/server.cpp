@@ -142,8 +142,9 @@ struct Req {
       *grad, *obsv, *loss2, *part, *stage;
   float *sv32, *ysa, *ysb, *ra, *rb, *pa, *pb, *qa, *qb;
   // multigrid CG: FP64 x, r, q, two directions; FP32 vectors; the grids
-  double *mgx, *mgr, *mgq, *mgp0, *mgp1;
+  double *mgx, *mgr, *mgr1, *mgq, *mgp0, *mgp1;
   float *sq, *minv, *z, *rs, *x0, *t, *ts, *grid;
+  float2 *wrq;
   int *obsi;
   int nobs = 0;
   std::vector<int> h_obs;  // synthetic observation indices, kept until the request is done
@@ -255,11 +256,13 @@ struct Server {
     double2 *xy = (double2 *)take(nv * sizeof(double2));
     float *sv32 = F(ns);
     if (pl) {
-      double *mgx = D(np), *mgr = D(np), *mgq = D(np), *mgp0 = D(np), *mgp1 = D(np);
+      double *mgx = D(np), *mgr = D(np), *mgr1 = D(np), *mgq = D(np), *mgp0 = D(np), *mgp1 = D(np);
       float *sq = F(np), *minv = F(np), *z = F(np), *rs = F(np), *x0 = F(np), *t = F(np),
             *ts = F(np), *grid = F(mg_grid_floats(*pl));
+      float2 *wrq = (float2 *)take(np * sizeof(float2));
       if (q) {
-        q->mgx = mgx; q->mgr = mgr; q->mgq = mgq; q->mgp0 = mgp0; q->mgp1 = mgp1;
+        q->wrq = wrq;
+        q->mgx = mgx; q->mgr = mgr; q->mgr1 = mgr1; q->mgq = mgq; q->mgp0 = mgp0; q->mgp1 = mgp1;
         q->sq = sq; q->minv = minv; q->z = z; q->rs = rs; q->x0 = x0; q->t = t; q->ts = ts;
         q->grid = grid;
       }
@@ -346,7 +349,8 @@ struct Server {
     d.minv = q.minv;
     d.b = q.b;
     d.x = q.mgx;
-    d.r = q.mgr;
+    d.r[0] = q.mgr;
+    d.r[1] = q.mgr1;
     d.q = q.mgq;
     d.p[0] = q.mgp0;
     d.p[1] = q.mgp1;
@@ -355,6 +359,7 @@ struct Server {
     d.x0 = q.x0;
     d.t = q.t;
     d.ts = q.ts;
+    d.wrq = q.wrq;
     d.n = s.n;
     d.npad = s.npad;
     mg_parts(d, T.nblk, T.nblk > MG_BATCH_SUM, q.part);
