@@ -302,8 +302,7 @@ int admfem_fem_laplace_term_grad_on(admfem_mesh h, const double *grad_out, const
                                     double *work, void *stream) {
   return guarded([&] {
     REQUIRE(grad_out && u && nu, ADMFEM_ERR_ARG, "null pointer");
-    if (grad_u) launch_laplace_term(M(h), grad_out, nu, grad_u, work, S(stream));
-    if (grad_nu) launch_laplace_term_nu_grad(M(h), grad_out, u, grad_nu, S(stream));
+    launch_laplace_term_grad(M(h), grad_out, u, nu, grad_u, grad_nu, work, S(stream));
   });
 }
 

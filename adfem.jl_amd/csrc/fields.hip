@@ -10,10 +10,12 @@
 //     ComputeLaplaceTermMfem.h:4-39): out = K(nu) u without forming K.
 // Fields are in the user's node order, Gauss arrays in the user's element
 // order (g = nq e + k).  Forward maps to Gauss points run one thread per
-// Gauss point.  The maps to the nodes have one writer per output and no
+// element.  The maps to the nodes have one writer per output and no
 // atomics: a gather over the node's incident elements, or, where deriving an
 // element's geometry anew at each of its nodes costs more than passing its
 // terms through memory, a pass over the elements and a pass over the nodes.
+#include <type_traits>
+
 #include "geom.h"
 
 namespace admfem {
@@ -37,35 +39,83 @@ __device__ __forceinline__ Tri load_tri(const int *__restrict__ conn, int nelem,
   return t;
 }
 
-__global__ void to_gauss_kernel(int nelem, QuadRule rule, const int *__restrict__ conn_user,
-                                const double *__restrict__ u, double *__restrict__ out) {
+// Forward maps: one thread per element and an XCD's blocks one range of
+// elements; the values leave by way of LDS, in consecutive stores.  With one
+// thread per Gauss point the three of an element fetched its vertices and ids
+// three times, and every XCD all of the vertices (700^2, 3 points: to the Gauss
+// points 15.4 -> 14.1 us, gradients 23.7 -> 19.9; 29 with each element's
+// thread storing its own).
+template <int NQ>
+__global__ void __launch_bounds__(256)
+    to_gauss_kernel(int nelem, QuadRule rule, const int *__restrict__ conn_user,
+                    const double *__restrict__ u, double *__restrict__ out) {
 #pragma clang fp contract(off)
-  const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= (int64_t)rule.nq * nelem) return;
-  const int e = (int)(g / rule.nq), k = (int)(g - (int64_t)rule.nq * e);
-  const double xi = rule.xi[k], eta = rule.eta[k];
-  out[g] = u[conn_user[e]] * shape(0, xi, eta) +
-           u[conn_user[(size_t)nelem + e]] * shape(1, xi, eta) +
-           u[conn_user[2 * (size_t)nelem + e]] * shape(2, xi, eta);
+  __shared__ double sh[256 * NQ];
+  const int e0 = xcd_block(blockIdx.x, gridDim.x) * 256, e = e0 + threadIdx.x;
+  if (e < nelem) {
+    const double u0 = u[conn_user[e]], u1 = u[conn_user[(size_t)nelem + e]],
+                 u2 = u[conn_user[2 * (size_t)nelem + e]];
+#pragma unroll
+    for (int k = 0; k < NQ; k++)
+      sh[NQ * threadIdx.x + k] = u0 * shape(0, rule.xi[k], rule.eta[k]) +
+                                 u1 * shape(1, rule.xi[k], rule.eta[k]) +
+                                 u2 * shape(2, rule.xi[k], rule.eta[k]);
+  }
+  __syncthreads();
+  const int ng = NQ * min(256, nelem - e0);
+  double *o = out + (size_t)NQ * e0;
+#pragma unroll
+  for (int k = 0; k < NQ; k++) {
+    const int g = k * 256 + threadIdx.x;
+    if (g < ng) o[g] = sh[g];
+  }
 }
 
-__global__ void fem_grad_kernel(int nelem, QuadRule rule, const int *__restrict__ conn,
-                                const int *__restrict__ conn_user, const double *__restrict__ x,
-                                const double *__restrict__ y, const double *__restrict__ u,
-                                double *__restrict__ out) {
+// Vertices of element e (xy: internal order).
+__device__ __forceinline__ void load_xy(const int *__restrict__ conn, int nelem, int e,
+                                        const double2 *__restrict__ xy, double2 (&v)[3]) {
+#pragma unroll
+  for (int q = 0; q < 3; q++) v[q] = xy[conn[(size_t)q * nelem + e]];
+}
+
+// out16: out is 16-byte aligned (one store per Gauss point)
+template <int NQ>
+__global__ void __launch_bounds__(256)
+    fem_grad_kernel(int nelem, const int *__restrict__ conn, const int *__restrict__ conn_user,
+                    const double2 *__restrict__ xy, const double *__restrict__ u,
+                    double *__restrict__ out, bool out16) {
 #pragma clang fp contract(off)
-  const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= (int64_t)rule.nq * nelem) return;
-  const int e = (int)(g / rule.nq);
-  const Tri t = load_tri(conn, nelem, e, x, y);
-  const ElemGeom G = elem_geom(t.x[0], t.y[0], t.x[1], t.y[1], t.x[2], t.y[2]);
-  double gx = 0.0, gy = 0.0;
+  __shared__ double sx[256], sy[256];
+  const int e0 = xcd_block(blockIdx.x, gridDim.x) * 256, e = e0 + threadIdx.x;
+  if (e < nelem) {
+    double2 v[3];
+    load_xy(conn, nelem, e, xy, v);
+    double hx[3], hy[3], gx = 0.0, gy = 0.0;
+    elem_grads(v[0].x, v[0].y, v[1].x, v[1].y, v[2].x, v[2].y, hx, hy);
 #pragma unroll
-  for (int r = 0; r < 3; r++) gx += u[conn_user[(size_t)r * nelem + e]] * G.gx[r];
+    for (int r = 0; r < 3; r++) {
+      const double ur = u[conn_user[(size_t)r * nelem + e]];
+      gx += ur * hx[r];
+      gy += ur * hy[r];
+    }
+    sx[threadIdx.x] = gx;
+    sy[threadIdx.x] = gy;
+  }
+  __syncthreads();
+  const int ng = NQ * min(256, nelem - e0);
+  double *o = out + 2 * (size_t)NQ * e0;
 #pragma unroll
-  for (int r = 0; r < 3; r++) gy += u[conn_user[(size_t)r * nelem + e]] * G.gy[r];
-  out[2 * g] = gx;
-  out[2 * g + 1] = gy;
+  for (int k = 0; k < NQ; k++) {
+    const int g = k * 256 + threadIdx.x;
+    if (g >= ng) continue;
+    const double gx = sx[g / NQ], gy = sy[g / NQ];
+    if (out16) {
+      reinterpret_cast<double2 *>(o)[g] = make_double2(gx, gy);
+    } else {
+      o[2 * g] = gx;
+      o[2 * g + 1] = gy;
+    }
+  }
 }
 
 // Per node: the transposes of the two maps above.
@@ -81,7 +131,7 @@ __global__ void __launch_bounds__(256) node_gather_kernel(int n, int nelem, Quad
                                    const int *__restrict__ iperm,
                                    const double *__restrict__ in,   // Gauss array
                                    double *__restrict__ out_user) {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
+  const int r = xcd_block(blockIdx.x, gridDim.x) * 256 + threadIdx.x;
   if (r >= n) return;
   double acc = 0.0;
   const int t1 = n2e_ptr[r + 1];
@@ -114,30 +164,51 @@ __global__ void __launch_bounds__(256) node_gather_kernel(int n, int nelem, Quad
 // streams the Gauss arrays once (the one-pass gather met each element's
 // values and vertex ids six times, in the nodes' order) and the node pass
 // reads one scattered double per incidence.  K(nu) u: 9.6 -> 6.3 us at 64^2,
-// 64 -> 43 us at 700^2; fem_grad's transpose at 700^2: 55 -> 32 us.
-template <bool LAPLACE, int NQ>
+// 64 -> 37 us at 700^2; fem_grad's transpose at 700^2: 55 -> 30 us.
+// K(nu)'s transpose for the gradient (KIND 2) also takes the gradient in nu,
+// w_g grad(in) . grad(u) (ComputeLaplaceTermMfemGrad; the term is linear in nu),
+// from the element's vertices in hand: 55 -> 33 us at 700^2 for the two.  The
+// weights come from the area (8 bytes an element instead of 24; K(nu) u's element
+// pass 26 -> 22 us).
+enum { TERM_GRAD_T = 0, TERM_LAPLACE = 1, TERM_LAPLACE_GRAD = 2 };
+template <int KIND, int NQ>
 __global__ void __launch_bounds__(256)
-    elem_terms_kernel(int nelem, const int *__restrict__ conn, const int *__restrict__ conn_user,
-                      const double2 *__restrict__ xy, const double *__restrict__ gw,
-                      const double *__restrict__ in,  // LAPLACE: field, else Gauss array (x, y)
-                      const double *__restrict__ nu, double *__restrict__ c) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+    elem_terms_kernel(int nelem, QuadRule rule, const int *__restrict__ conn,
+                      const int *__restrict__ conn_user, const double2 *__restrict__ xy,
+                      const double *__restrict__ area,
+                      const double *__restrict__ in,  // field, or (TERM_GRAD_T) Gauss array (x, y)
+                      const double *nu, double *__restrict__ c, const double *__restrict__ u,
+                      double *gnu) {  // (gnu may be nu)
+  const int e = xcd_block(blockIdx.x, gridDim.x) * 256 + threadIdx.x;
   if (e >= nelem) return;
   double2 v[3];
-#pragma unroll
-  for (int q = 0; q < 3; q++) v[q] = xy[conn[(size_t)q * nelem + e]];
+  load_xy(conn, nelem, e, xy, v);
   double gx[3], gy[3], sx = 0.0, sy = 0.0;
   elem_grads(v[0].x, v[0].y, v[1].x, v[1].y, v[2].x, v[2].y, gx, gy);
-  if (LAPLACE) {  // sum_k nu_k w_k grad phi_p . grad u_e
+  if (KIND != TERM_GRAD_T) {  // sum_k nu_k w_k grad phi_p . grad u_e
+    double ux = 0.0, uy = 0.0;
 #pragma unroll
     for (int q = 0; q < 3; q++) {
-      const double uq = in[conn_user[(size_t)q * nelem + e]];
+      const int w = conn_user[(size_t)q * nelem + e];
+      const double uq = in[w];
       sx += gx[q] * uq;
       sy += gy[q] * uq;
+      if (KIND == TERM_LAPLACE_GRAD) {
+        const double vq = u[w];
+        ux += gx[q] * vq;
+        uy += gy[q] * vq;
+      }
     }
-    double cw = 0.0;
+    const double a = area[e];
+    double cw = 0.0, nk[NQ];
 #pragma unroll
-    for (int k = 0; k < NQ; k++) cw += nu[(size_t)NQ * e + k] * gw[(size_t)NQ * e + k];
+    for (int k = 0; k < NQ; k++) nk[k] = nu[(size_t)NQ * e + k];
+#pragma unroll
+    for (int k = 0; k < NQ; k++) {
+      const double wk = gauss_weight(rule.w[k], a);
+      cw += nk[k] * wk;
+      if (KIND == TERM_LAPLACE_GRAD) gnu[(size_t)NQ * e + k] = wk * (sx * ux + sy * uy);
+    }
     sx *= cw;
     sy *= cw;
   } else {
@@ -157,7 +228,7 @@ __global__ void __launch_bounds__(256)
                     const int *__restrict__ n2e_elem, const uint32_t *__restrict__ slots,
                     const int *__restrict__ iperm, const double *__restrict__ c,
                     double *__restrict__ out_user) {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
+  const int r = xcd_block(blockIdx.x, gridDim.x) * 256 + threadIdx.x;
   if (r >= n) return;
   const int t1 = n2e_ptr[r + 1];
   double acc = 0.0;
@@ -173,57 +244,61 @@ __global__ void __launch_bounds__(256)
   out_user[iperm[r]] = acc;
 }
 
-// ComputeLaplaceTermMfemGrad, nu part: w_g grad(grad_out) . grad(u) per Gauss
-// point (the term is linear in nu).
-__global__ void laplace_term_nu_grad_kernel(int nelem, QuadRule rule, const int *__restrict__ conn,
-                                            const int *__restrict__ conn_user,
-                                            const double *__restrict__ x,
-                                            const double *__restrict__ y,
-                                            const double *__restrict__ go,
-                                            const double *__restrict__ u,
-                                            double *__restrict__ gnu) {
-  const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= (int64_t)rule.nq * nelem) return;
-  const int e = (int)(g / rule.nq), k = (int)(g - (int64_t)rule.nq * e);
-  const Tri t = load_tri(conn, nelem, e, x, y);
-  const ElemGeom G = elem_geom(t.x[0], t.y[0], t.x[1], t.y[1], t.x[2], t.y[2]);
-  double ax = 0.0, ay = 0.0, bx = 0.0, by = 0.0;
+// ComputeLaplaceTermMfemGrad's nu part alone.
+template <int NQ>
+__global__ void __launch_bounds__(256)
+    laplace_term_nu_grad_kernel(int nelem, QuadRule rule, const int *__restrict__ conn,
+                                const int *__restrict__ conn_user,
+                                const double2 *__restrict__ xy, const double *__restrict__ area,
+                                const double *__restrict__ go, const double *__restrict__ u,
+                                double *__restrict__ gnu) {
+  const int e = xcd_block(blockIdx.x, gridDim.x) * 256 + threadIdx.x;
+  if (e >= nelem) return;
+  double2 v[3];
+  load_xy(conn, nelem, e, xy, v);
+  double gx[3], gy[3], ax = 0.0, ay = 0.0, bx = 0.0, by = 0.0;
+  elem_grads(v[0].x, v[0].y, v[1].x, v[1].y, v[2].x, v[2].y, gx, gy);
 #pragma unroll
   for (int q = 0; q < 3; q++) {
-    const int v = conn_user[(size_t)q * nelem + e];
-    ax += G.gx[q] * go[v];
-    ay += G.gy[q] * go[v];
-    bx += G.gx[q] * u[v];
-    by += G.gy[q] * u[v];
+    const int w = conn_user[(size_t)q * nelem + e];
+    ax += gx[q] * go[w];
+    ay += gy[q] * go[w];
+    bx += gx[q] * u[w];
+    by += gy[q] * u[w];
   }
-  gnu[g] = gauss_weight(rule.w[k], G.area) * (ax * bx + ay * by);
+  const double a = area[e];
+#pragma unroll
+  for (int k = 0; k < NQ; k++)
+    gnu[(size_t)NQ * e + k] = gauss_weight(rule.w[k], a) * (ax * bx + ay * by);
 }
 
 inline unsigned nb(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 
-template <int OP>
-void node_gather(const Mesh &m, const double *in, double *out_user, hipStream_t st) {
-  auto go = [&](auto kern) {
-    kern<<<nb(m.nnode, 256), 256, 0, st>>>(m.nnode, m.nelem, m.rule, m.conn.p, m.conn_user.p,
-                                           m.x.p, m.y.p, m.d_n2e_ptr.p, m.d_n2e_elem.p,
-                                           m.d_slots_full.p, m.d_iperm.p, in, out_user);
-  };
-  if (m.rule.nq == 3) go(node_gather_kernel<OP, 3>);
-  else if (m.rule.nq == 6) go(node_gather_kernel<OP, 6>);
-  else go(node_gather_kernel<OP, 1>);
+// go(Gauss points of the rule, a compile-time constant)
+template <class F>
+void by_rule(const Mesh &m, F go) {
+  if (m.rule.nq == 3) go(std::integral_constant<int, 3>{});
+  else if (m.rule.nq == 6) go(std::integral_constant<int, 6>{});
+  else go(std::integral_constant<int, 1>{});
   HIPCHECK(hipGetLastError());
 }
 
-template <bool LAPLACE>
+template <int OP>
+void node_gather(const Mesh &m, const double *in, double *out_user, hipStream_t st) {
+  by_rule(m, [&](auto nq) {
+    node_gather_kernel<OP, nq()><<<nb(m.nnode, 256), 256, 0, st>>>(
+        m.nnode, m.nelem, m.rule, m.conn.p, m.conn_user.p, m.x.p, m.y.p, m.d_n2e_ptr.p,
+        m.d_n2e_elem.p, m.d_slots_full.p, m.d_iperm.p, in, out_user);
+  });
+}
+
+template <int KIND>
 void two_pass(const Mesh &m, const double *in, const double *nu, double *out_user, double *c,
-              hipStream_t st) {
-  auto go = [&](auto kern) {
-    kern<<<nb(m.nelem, 256), 256, 0, st>>>(m.nelem, m.conn.p, m.conn_user.p, m.xy.p, m.gw.p, in,
-                                           nu, c);
-  };
-  if (m.rule.nq == 3) go(elem_terms_kernel<LAPLACE, 3>);
-  else if (m.rule.nq == 6) go(elem_terms_kernel<LAPLACE, 6>);
-  else go(elem_terms_kernel<LAPLACE, 1>);
+              const double *u, double *gnu, hipStream_t st) {
+  by_rule(m, [&](auto nq) {
+    elem_terms_kernel<KIND, nq()><<<nb(m.nelem, 256), 256, 0, st>>>(
+        m.nelem, m.rule, m.conn.p, m.conn_user.p, m.xy.p, m.area.p, in, nu, c, u, gnu);
+  });
   node_sum_kernel<<<nb(m.nnode, 256), 256, 0, st>>>(m.nnode, m.nelem, m.d_n2e_ptr.p,
                                                     m.d_n2e_elem.p, m.d_slots_full.p,
                                                     m.d_iperm.p, c, out_user);
@@ -238,8 +313,10 @@ constexpr int GRAD_T_TWO_PASS = 100000;
 }  // namespace
 
 void launch_to_gauss(const Mesh &m, const double *u, double *out, hipStream_t st) {
-  to_gauss_kernel<<<nb(m.ngauss, 256), 256, 0, st>>>(m.nelem, m.rule, m.conn_user.p, u, out);
-  HIPCHECK(hipGetLastError());
+  by_rule(m, [&](auto nq) {
+    to_gauss_kernel<nq()><<<nb(m.nelem, 256), 256, 0, st>>>(m.nelem, m.rule, m.conn_user.p, u,
+                                                            out);
+  });
 }
 
 void launch_to_gauss_grad(const Mesh &m, const double *grad_out, double *grad_u,
@@ -260,38 +337,54 @@ void launch_dof_to_gauss_grad(const Mesh &m, const double *grad_out, double *gra
 
 void launch_fem_grad(const Mesh &m, const double *u, double *out, hipStream_t st) {
   if (m.degree == 2) return launch_p2_fem_grad(m, u, out, st);
-  fem_grad_kernel<<<nb(m.ngauss, 256), 256, 0, st>>>(m.nelem, m.rule, m.conn.p, m.conn_user.p,
-                                                     m.x.p, m.y.p, u, out);
-  HIPCHECK(hipGetLastError());
+  by_rule(m, [&](auto nq) {
+    fem_grad_kernel<nq()><<<nb(m.nelem, 256), 256, 0, st>>>(
+        m.nelem, m.conn.p, m.conn_user.p, m.xy.p, u, out, ((uintptr_t)out & 15) == 0);
+  });
 }
 
 void launch_fem_grad_grad(const Mesh &m, const double *grad_out, double *grad_u, double *work,
                           hipStream_t st) {
   if (m.degree == 2) return launch_p2_fem_grad_grad(m, grad_out, grad_u, work, st);
   if (work && m.nnode >= GRAD_T_TWO_PASS)
-    two_pass<false>(m, grad_out, nullptr, grad_u, work, st);
+    two_pass<TERM_GRAD_T>(m, grad_out, nullptr, grad_u, work, nullptr, nullptr, st);
   else
     node_gather<NODE_GRAD_T>(m, grad_out, grad_u, st);
 }
 
 // A caller without scratch gets a stream-ordered temporary (10 us on the host,
 // 20 to 30 when the stream has drained since the last one).
-void launch_laplace_term(const Mesh &m, const double *u, const double *nu, double *out,
-                         double *work, hipStream_t st) {
+static void laplace_term(const Mesh &m, const double *v, const double *nu, double *out,
+                         double *work, const double *u, double *gnu, hipStream_t st) {
   double *c = work;
   if (!work)
     HIPCHECK(hipMallocAsync((void **)&c, sizeof(double) * (m.degree == 2 ? 6 : 3) * m.nelem, st));
-  if (m.degree == 2) launch_p2_laplace_term(m, u, nu, out, c, st);
-  else two_pass<true>(m, u, nu, out, c, st);
+  if (m.degree == 2) {
+    launch_p2_laplace_term(m, v, nu, out, c, st);
+    if (gnu) launch_p2_laplace_term_nu_grad(m, v, u, gnu, st);
+  } else if (gnu) {
+    two_pass<TERM_LAPLACE_GRAD>(m, v, nu, out, c, u, gnu, st);
+  } else {
+    two_pass<TERM_LAPLACE>(m, v, nu, out, c, nullptr, nullptr, st);
+  }
   if (!work) HIPCHECK(hipFreeAsync(c, st));
 }
 
-void launch_laplace_term_nu_grad(const Mesh &m, const double *grad_out, const double *u,
-                                 double *grad_nu, hipStream_t st) {
+void launch_laplace_term(const Mesh &m, const double *u, const double *nu, double *out,
+                         double *work, hipStream_t st) {
+  laplace_term(m, u, nu, out, work, nullptr, nullptr, st);
+}
+
+void launch_laplace_term_grad(const Mesh &m, const double *grad_out, const double *u,
+                              const double *nu, double *grad_u, double *grad_nu, double *work,
+                              hipStream_t st) {
+  if (grad_u) return laplace_term(m, grad_out, nu, grad_u, work, u, grad_nu, st);
+  if (!grad_nu) return;
   if (m.degree == 2) return launch_p2_laplace_term_nu_grad(m, grad_out, u, grad_nu, st);
-  laplace_term_nu_grad_kernel<<<nb(m.ngauss, 256), 256, 0, st>>>(
-      m.nelem, m.rule, m.conn.p, m.conn_user.p, m.x.p, m.y.p, grad_out, u, grad_nu);
-  HIPCHECK(hipGetLastError());
+  by_rule(m, [&](auto nq) {
+    laplace_term_nu_grad_kernel<nq()><<<nb(m.nelem, 256), 256, 0, st>>>(
+        m.nelem, m.rule, m.conn.p, m.conn_user.p, m.xy.p, m.area.p, grad_out, u, grad_nu);
+  });
 }
 
 }  // namespace admfem

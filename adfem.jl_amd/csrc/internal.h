@@ -305,8 +305,10 @@ void launch_fem_grad_grad(const Mesh &m, const double *grad_out, double *grad_u,
                           hipStream_t st);
 void launch_laplace_term(const Mesh &m, const double *u, const double *nu, double *out,
                          double *work, hipStream_t st);
-void launch_laplace_term_nu_grad(const Mesh &m, const double *grad_out, const double *u,
-                                 double *grad_nu, hipStream_t st);
+// its gradients (either may be null)
+void launch_laplace_term_grad(const Mesh &m, const double *grad_out, const double *u,
+                              const double *nu, double *grad_u, double *grad_nu, double *work,
+                              hipStream_t st);
 // DofToGaussPoints (DofToGaussPointsMfem.h:6-32): the degree's basis (for P1
 // the vertex functions, as launch_to_gauss).
 void launch_dof_to_gauss(const Mesh &m, const double *u, double *out, hipStream_t st);
