@@ -500,9 +500,17 @@ int admfem_system_forward_adjoint(admfem_system h, const admfem_problem *p,
     assemble_impl(h, p, str);
     admfem_solve_stats s0{}, s1{};
     cg_solve(s, s.rhs.p, h->u_int.p, *o, s0, str);
-    double L = loss_and_grad(s, h->u_int.p, obs_idx, obs_val, nobs, h->g_int.p, h->loss2.p,
-                             str);
+    // the loss and its check of the indices (none is followed unchecked) come
+    // to the host with the adjoint solve's state
+    launch_loss(s, h->u_int.p, obs_idx, obs_val, nobs, h->g_int.p, h->loss2.p, str);
+    HostSlot hs(str);
+    hs.read(0, h->loss2.p);
+    hs.read(8, h->loss2.p + 1);
     cg_solve(s, h->g_int.p, h->lam_int.p, *o, s1, str);
+    hs.wait();
+    const double L = hs.get<double>(0);
+    REQUIRE(hs.get<double>(8) == 0.0, ADMFEM_ERR_ARG,
+            "observation index out of range [0, n) or repeated");
     if (grad_kappa)
       launch_kappa_gradient(s, h->u_int.p, h->lam_int.p, p->lap_coef, grad_kappa, str);
     if (u) launch_scatter(s.d_uiperm(), h->u_int.p, u, s.n, str);

@@ -695,16 +695,4 @@ void launch_scatter(const int *idx, const double *src, double *dst, int n, hipSt
   HIPCHECK(hipGetLastError());
 }
 
-double loss_and_grad(const System &s, const double *u_int, const int *obs_idx,
-                     const double *obs_val, int nobs, double *g_int, double *loss2,
-                     hipStream_t st) {
-  launch_loss(s, u_int, obs_idx, obs_val, nobs, g_int, loss2, st);
-  double h[2] = {0.0, 0.0};
-  HIPCHECK(hipMemcpyAsync(h, loss2, 2 * sizeof(double), hipMemcpyDeviceToHost, st));
-  HIPCHECK(hipStreamSynchronize(st));
-  REQUIRE(h[1] == 0.0, ADMFEM_ERR_ARG,
-          "observation index out of range [0, n) or repeated");
-  return h[0];
-}
-
 }  // namespace admfem

@@ -405,12 +405,14 @@ void prepare(DirPrep &d, const long long *ind, int64_t sN, const long long *bd, 
   HIPCHECK(hipGetLastError());
   exclusive_scan(w, w.tkeep.p, w.tkpos.p, nt + 1, st);
   exclusive_scan(w, w.tlift.p, w.tlpos.p, nt + 1, st);
-  int herr = 0;
-  HIPCHECK(hipMemcpyAsync(&herr, w.err.p, sizeof(int), hipMemcpyDeviceToHost, st));
-  HIPCHECK(hipMemcpyAsync(&d.nkept, w.tkpos.p + nt, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-  HIPCHECK(hipMemcpyAsync(&d.nlift, w.tlpos.p + nt, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-  HIPCHECK(hipStreamSynchronize(st));
-  REQUIRE(!herr, ADMFEM_ERR_ARG, "triplet index out of range [0, N)");
+  HostSlot h(st);
+  h.read(0, w.tkpos.p + nt);
+  h.read(8, w.tlpos.p + nt);
+  h.read(16, w.err.p);
+  h.wait();
+  d.nkept = h.get<int64_t>(0);
+  d.nlift = h.get<int64_t>(8);
+  REQUIRE(!h.get<int>(16), ADMFEM_ERR_ARG, "triplet index out of range [0, N)");
 }
 
 // room for the lift list (written by tile_place / tile_grad into w.lkey /

@@ -37,6 +37,31 @@ void *device_alloc(size_t bytes, int &device);
 void device_free(void *p, size_t bytes, int device);
 void release_device_memory();
 
+// 64 bytes of pinned host memory for a call's results (memory.cpp): read()
+// enqueues a copy from the device, wait() makes what was read visible.  A copy
+// to ordinary memory instead blocks the host by itself, 10 - 15 us each.
+class HostSlot {
+ public:
+  explicit HostSlot(hipStream_t stream);
+  ~HostSlot();
+  HostSlot(const HostSlot &) = delete;
+  HostSlot &operator=(const HostSlot &) = delete;
+  template <class T> void read(int at, const T *dev) {
+    HIPCHECK(hipMemcpyAsync((char *)p + at, dev, sizeof(T), hipMemcpyDeviceToHost, st));
+    pending = true;
+  }
+  void wait() {
+    HIPCHECK(hipStreamSynchronize(st));
+    pending = false;
+  }
+  template <class T> T get(int at) const { return *(const T *)((const char *)p + at); }
+
+ private:
+  void *p;
+  hipStream_t st;
+  bool pending = false;
+};
+
 // Device buffer (RAII over device_alloc/device_free).
 template <class T>
 struct DevBuf {
@@ -420,9 +445,5 @@ void server_stats(Server *sv, double *stats);
 double server_spmv_repeat(Server *sv, const int *topos, int nsys, int repeat,
                           hipStream_t st, double *seconds);
 // loss gradient: g_int = 0; g[perm[idx]] = 2 (u - obs); returns loss on host
-// (loss2: 2 device doubles of the caller's, loss and an index-error flag)
-double loss_and_grad(const System &s, const double *u_int, const int *obs_idx,
-                     const double *obs_val, int nobs, double *g_int, double *loss2,
-                     hipStream_t st);
 
 }  // namespace admfem

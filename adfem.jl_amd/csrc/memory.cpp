@@ -13,6 +13,7 @@
 // fails, and by admfem_release_memory.
 #include <map>
 #include <mutex>
+#include <vector>
 
 #include "internal.h"
 
@@ -94,6 +95,39 @@ void device_free(void *p, size_t bytes, int device) {
   }
   (void)hipGetLastError();
   (void)hipFree(p);
+}
+
+// ------------------------------------------------------------- host slots
+
+namespace {
+struct Slots {
+  std::mutex mu;
+  std::vector<void *> free_;  // at most as many as calls ever ran at once
+};
+Slots &slots() {
+  static Slots *s = new Slots();  // lives until the process ends
+  return *s;
+}
+}  // namespace
+
+HostSlot::HostSlot(hipStream_t stream) : p(nullptr), st(stream) {
+  {
+    Slots &s = slots();
+    std::lock_guard<std::mutex> g(s.mu);
+    if (!s.free_.empty()) {
+      p = s.free_.back();
+      s.free_.pop_back();
+      return;
+    }
+  }
+  HIPCHECK(hipHostMalloc(&p, 64, hipHostMallocPortable));
+}
+
+HostSlot::~HostSlot() {
+  if (pending) (void)hipStreamSynchronize(st);  // (an error between read and wait)
+  Slots &s = slots();
+  std::lock_guard<std::mutex> g(s.mu);
+  s.free_.push_back(p);
 }
 
 }  // namespace admfem

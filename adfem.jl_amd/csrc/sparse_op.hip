@@ -200,10 +200,10 @@ bool same_pattern(CooPattern &p, const long long *ind, int64_t nnz, int n, int d
   set_int<<<1, 1, 0, st>>>(p.flag.p, 0);
   coo_differs<<<nb(2 * nnz, 256), 256, 0, st>>>(2 * nnz, ind, p.ind.p, p.flag.p);
   HIPCHECK(hipGetLastError());
-  int h = 1;
-  HIPCHECK(hipMemcpyAsync(&h, p.flag.p, sizeof(int), hipMemcpyDeviceToHost, st));
-  HIPCHECK(hipStreamSynchronize(st));
-  return h == 0;
+  HostSlot h(st);
+  h.read(0, p.flag.p);
+  h.wait();
+  return h.get<int>(0) == 0;
 }
 
 void build_pattern(CooPattern &p, const Mesh *m, const long long *ind, int64_t nnz, int n, int dev,
