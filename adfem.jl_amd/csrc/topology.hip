@@ -255,6 +255,42 @@ __global__ void __launch_bounds__(BFS_NT)
   }
 }
 
+// Levels L0 .. end - 1 of the same search by one workgroup, sixteen lanes a
+// node: while a level holds at most BFS_NARROW nodes, its chain of dependent
+// loads is all there is (3.5 us a level; 5.5 and a gap as a launch: the search
+// for P1 300^2 0.70 -> 0.28 ms).  Wider levels need the other CUs.  *done: the
+// level reached, below `end` when a level was wider.
+constexpr int BFS_NARROW = 1024, BFS_LANES = 16, BFS_WG = 1024;
+__global__ void __launch_bounds__(BFS_WG)
+    bfs_narrow_kernel(int L0, int end, const int *__restrict__ rp, const int *__restrict__ col,
+                      int *level, int *q, int *off, int *cnt, int *done) {
+  __shared__ int next[2];
+  const int tid = threadIdx.x;
+  int o = off[L0], c = cnt[L0], L = L0;
+  if (tid < 2) next[tid] = 0;
+  __syncthreads();
+  for (; L < end && c > 0 && c <= BFS_NARROW; L++) {  // (uniform)
+    int *const n = &next[L & 1];
+    for (int i = tid / BFS_LANES; i < c; i += BFS_WG / BFS_LANES) {
+      const int u = q[o + i], k1 = rp[u + 1];
+      for (int k = rp[u] + tid % BFS_LANES; k < k1; k += BFS_LANES) {
+        const int v = col[k];
+        if (atomicCAS(&level[v], -1, L + 1) == -1) q[o + c + atomicAdd(n, 1)] = v;
+      }
+    }
+    __syncthreads();
+    o += c;
+    c = *n;
+    if (tid == 0) {
+      off[L + 1] = o;
+      cnt[L + 1] = c;
+      next[(L & 1) ^ 1] = 0;
+    }
+    __syncthreads();
+  }
+  if (tid == 0) *done = c > 0 ? L : end;  // (an empty level: the search is over)
+}
+
 // Cuthill-McKee positions level by level, in one workgroup: a node of level
 // L + 1 follows its parent -- its neighbour of level L placed first -- and
 // the parent's children are placed in (degree, id) order, which is the
@@ -536,19 +572,19 @@ __global__ void post_fill_kernel(int n, const int *__restrict__ rp, const int *_
     if (row_bd[col[k]] < 0) pcol[o++] = col[k];
 }
 
-// SELL-64: slice size = 64 x the widest row's off-diagonal count
+// SELL-64: slice size = 64 x the widest row's off-diagonal count; a wave per
+// slice (with a thread per slice the 64 rows in turn took 82 us at P1 300^2
+// and 206 at P2 50^2)
 __global__ void slice_size_kernel(int n, int nslices, const int *__restrict__ rp,
                                   const int *__restrict__ col, int *__restrict__ size) {
-  const int sl = blockIdx.x * blockDim.x + threadIdx.x;
-  if (sl > nslices) return;
+  const int r = blockIdx.x * blockDim.x + threadIdx.x, sl = r >> 6;
+  if (sl > nslices) return;  // (whole waves)
   int w = 0;
-  if (sl < nslices)
-    for (int r = sl * 64; r < min(sl * 64 + 64, n); r++) {
-      int c = 0;
-      for (int k = rp[r]; k < rp[r + 1]; k++) c += col[k] != r;
-      w = max(w, c);
-    }
-  size[sl] = 64 * w;
+  if (r < n)
+    for (int k = rp[r]; k < rp[r + 1]; k++) w += col[k] != r;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) w = max(w, __shfl_xor(w, o, 64));
+  if ((r & 63) == 0) size[sl] = 64 * w;
 }
 
 // off-diagonal columns, column-major inside the slice; padding points at the
@@ -803,16 +839,25 @@ void run_bfs(int n, const int *rp, const int *col, int s, BfsRun &b, hipStream_t
   // launch sees an empty frontier)
   constexpr int BATCH = 64;
   int L = 0, h[BATCH];
+  int *const done = b.cnt.p + n + 1;  // (beyond the last level's count)
   b.size.assign(1, 1);
   for (bool more = true; more;) {
     const int L0 = L, end = std::min(L + (stop && L < BATCH ? 16 : BATCH), n);
-    for (; L < end; L++)
-      bfs_level_kernel<<<BFS_BLOCKS, BFS_NT, 0, st>>>(L, rp, col, b.level.p, b.q.p, b.off.p,
-                                                      b.cnt.p);
+    int reached = end;
+    if (b.size.back() <= BFS_NARROW) {
+      bfs_narrow_kernel<<<1, BFS_WG, 0, st>>>(L, end, rp, col, b.level.p, b.q.p, b.off.p, b.cnt.p,
+                                              done);
+      HIPCHECK(hipMemcpyAsync(&reached, done, sizeof(int), hipMemcpyDeviceToHost, st));
+    } else {
+      for (int l = L; l < end; l++)
+        bfs_level_kernel<<<BFS_BLOCKS, BFS_NT, 0, st>>>(l, rp, col, b.level.p, b.q.p, b.off.p,
+                                                        b.cnt.p);
+    }
     HIPCHECK(hipGetLastError());
-    HIPCHECK(hipMemcpyAsync(h, b.cnt.p + L0 + 1, sizeof(int) * (L - L0), hipMemcpyDeviceToHost,
+    HIPCHECK(hipMemcpyAsync(h, b.cnt.p + L0 + 1, sizeof(int) * (end - L0), hipMemcpyDeviceToHost,
                             st));
     HIPCHECK(hipStreamSynchronize(st));
+    L = reached;
     more = L < n;
     for (int k = 0; k < L - L0; k++) {
       if (h[k] == 0) {
@@ -1087,7 +1132,7 @@ void solver_layout(System *s) {
   const int n = s->n;
   s->nslices = s->npad / 64;
   DevBuf<int> size(s->nslices + 1);
-  slice_size_kernel<<<nb(s->nslices + 1, 256), 256, 0, st>>>(n, s->nslices, s->d_rp.p,
+  slice_size_kernel<<<nb(64 * ((int64_t)s->nslices + 1), 256), 256, 0, st>>>(n, s->nslices, s->d_rp.p,
                                                              s->d_col.p, size.p);
   HIPCHECK(hipGetLastError());
   s->d_slice_ptr.alloc(s->nslices + 1);
