@@ -105,14 +105,23 @@ __global__ void coo_differs(int64_t m, const long long *__restrict__ a,
 __global__ void set_int(int *__restrict__ a, int v) { *a = v; }
 
 // val[pos[slot]] (pos null: val[slot]) = sum of vv over the slot's
-// triplets, in triplet order
+// triplets, in triplet order, eight requested together (a slot of a P2 vertex
+// has up to 72: 30 -> 16 us for K + M of P2 40^2)
 __global__ void coo_sum(int nslot, const int *__restrict__ start, const int *__restrict__ trip,
                         const int *__restrict__ pos, const double *__restrict__ vv,
                         double *__restrict__ val) {
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= nslot) return;
   double a = 0.0;
-  for (int t = start[s]; t < start[s + 1]; t++) a += vv[trip[t]];
+  const int t1 = start[s + 1];
+  for (int t = start[s]; t < t1; t += 8) {
+    double v[8];
+#pragma unroll
+    for (int q = 0; q < 8; q++) v[q] = vv[trip[min(t + q, t1 - 1)]];
+#pragma unroll
+    for (int q = 0; q < 8; q++)
+      if (t + q < t1) a += v[q];
+  }
   val[pos ? pos[s] : s] = a;
 }
 
