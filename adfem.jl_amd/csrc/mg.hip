@@ -2047,13 +2047,19 @@ bool mg_solve(System &s, const double *b, double *x_out, const admfem_solve_opts
     mk_check<<<w->nblk, NT, 0, st>>>(nullptr, D, S, 0, b);
     ms_check<<<1, RT, 0, st>>>(D, S, nullptr, 0, w->h_sc);
     HIPCHECK(hipGetLastError());
-    // (the solution as far as it is: no second wait for the final one)
-    HIPCHECK(hipMemcpyAsync(x_out, w->x.p, sizeof(double) * s.n, hipMemcpyDeviceToDevice, st));
+    // (the solution as far as it is: no second wait for the final one, unless
+    // it goes where the right-hand side still is)
+    if (x_out != b)
+      HIPCHECK(hipMemcpyAsync(x_out, w->x.p, sizeof(double) * s.n, hipMemcpyDeviceToDevice, st));
     HIPCHECK(hipStreamSynchronize(st));
     if (w->h_sc->a.status != ST_RUN) break;
     if (o.check_every <= 0) chunk = 2;
   }
   w->last_it = std::min(64, std::max(4, w->h_sc->a.it));
+  if (x_out == b) {
+    HIPCHECK(hipMemcpyAsync(x_out, w->x.p, sizeof(double) * s.n, hipMemcpyDeviceToDevice, st));
+    HIPCHECK(hipStreamSynchronize(st));
+  }
   const MgScal &h = *w->h_sc;
   stats.iterations = MG_PRODUCTS * h.a.it;
   stats.replacements = h.nrepl;
