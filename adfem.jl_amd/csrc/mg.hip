@@ -535,41 +535,66 @@ __global__ void __launch_bounds__(ST)
   }
 }
 
-// The smallest row sum over diagonal of the interior rows (per block, then
-// over the blocks): what the mass term leaves of the constant's energy.
+// Over the coupled rows: the smallest row sum over diagonal, how many rows
+// there are, and how many whose row sum over diagonal exceeds `heavy` (per
+// block, then over the blocks, into out[0 .. 2]): what the mass term leaves of
+// the constant's energy.
 __global__ void __launch_bounds__(NT)
     mk_rowsum(int n, const int *__restrict__ row_bd, const int *__restrict__ sp,
-              const double *__restrict__ sv, const double *__restrict__ diag,
+              const double *__restrict__ sv, const double *__restrict__ diag, double heavy,
               double *__restrict__ out) {
   const int i = blockIdx.x * NT + threadIdx.x;
-  double v = 1.0;
+  double v = 1.0, cnt[2] = {0.0, 0.0};
   if (i < n && row_bd[i] < 0) {
     const int s0 = sp[i >> 6], w = (sp[(i >> 6) + 1] - s0) >> 6, off = s0 + (i & 63);
     double sum = diag[i];
-    for (int k = 0; k < w; k++) sum += sv[off + 64 * k];
+    bool coupled = false;
+    for (int k = 0; k < w; k++) {
+      const double a = sv[off + 64 * k];
+      sum += a;
+      coupled = coupled || a != 0.0;
+    }
     v = sum / diag[i];
+    cnt[0] = coupled;
+    cnt[1] = coupled && v > heavy;
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v = fmin(v, __shfl_xor(v, o, 64));
-  __shared__ double sh[NT / 64];
-  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+  __shared__ double sh[NT / 64], sc[2][NT / 64];
+  const int wv = threadIdx.x >> 6;
+#pragma unroll
+  for (int j = 0; j < 2; j++) cnt[j] = wave_sum(cnt[j]);
+  if ((threadIdx.x & 63) == 0) {
+    sh[wv] = v;
+    sc[0][wv] = cnt[0];
+    sc[1][wv] = cnt[1];
+  }
   __syncthreads();
   if (threadIdx.x == 0) {
-    for (int k = 1; k < NT / 64; k++) v = fmin(v, sh[k]);
-    out[1 + blockIdx.x] = v;
+    for (int k = 1; k < NT / 64; k++) {
+      v = fmin(v, sh[k]);
+      cnt[0] += sc[0][k];
+      cnt[1] += sc[1][k];
+    }
+    out[3 + blockIdx.x] = v;
+    out[3 + gridDim.x + blockIdx.x] = cnt[0];
+    out[3 + 2 * gridDim.x + blockIdx.x] = cnt[1];
   }
 }
 __global__ void __launch_bounds__(RT) ms_rowsum(int G, double *__restrict__ out) {
   double v = 1.0;
-  for (int k = threadIdx.x; k < G; k += RT) v = fmin(v, out[1 + k]);
+  for (int k = threadIdx.x; k < G; k += RT) v = fmin(v, out[3 + k]);
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v = fmin(v, __shfl_xor(v, o, 64));
   __shared__ double sh[RT / 64];
   if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
-  __syncthreads();
+  double cnt[2];
+  sum_partials<2>(out + 3 + G, G, cnt);  // (its barrier covers sh)
   if (threadIdx.x == 0) {
     for (int k = 1; k < RT / 64; k++) v = fmin(v, sh[k]);
     out[0] = v;
+    out[1] = cnt[0];
+    out[2] = cnt[1];
   }
 }
 
@@ -1786,7 +1811,7 @@ struct MgWork {
   int last_it = 14;              // iterations of the last solve
   uint64_t version = 0;          // of the matrix the set-up was made from
   uint64_t rowsum_version = 0;   // of the matrix the row sums were taken of
-  double rowsum = 0.0;
+  bool pays = true;              // ... and what they say
   ~MgWork() {
     if (h_sc) (void)hipHostFree(h_sc);
   }
@@ -1970,26 +1995,36 @@ void iteration(const MgPlan &pl, MgWork *w, hipStream_t st) {
   mk_step<<<w->nblk, NT, 0, st>>>(nullptr, D, S, 0);
 }
 
-// Whether the V-cycle pays for the assembled matrix: not when a mass term
+// Whether the V-cycle suits the assembled matrix: not when a mass term
 // dominates it.  Jacobi-PCG's condition number is about 2 over the smallest
 // row sum over diagonal (1 for a lumped mass matrix, O(h^2) for a stiffness
 // matrix); at 0.2 it needs about as many launches as the V-cycles do.
-constexpr double MASS_DOMINANT = 0.2;
+// A caller's matrix stays with Jacobi-PCG also where half its coupled rows
+// have a row sum over diagonal above MASS_HEAVY / rows: mass outweighs
+// stiffness even at the scale of the whole domain (0.25 / (dt kappa) for a heat
+// step on P1, 0.19 on P2: dt below 4e-3 or 3e-3).  Such a step moves its field
+// little, and gradients in the density and the coefficient are differences of
+// nearly equal fields: at rtol 1e-12 with boundary values of order 1 two
+// solvers' gradients differ by 1e-9 at dt 1e-3 (P1 160^2) and 2e-8 at 1e-4, by
+// 6e-10 at most from 4e-3 on.
+constexpr double MASS_DOMINANT = 0.2, MASS_HEAVY = 60.0;
 bool mg_pays(System &s, MgWork *w, hipStream_t st) {
   if (!s.mass) return true;
   if (w->rowsum_version != s.a_version) {
     const unsigned g = nb(s.n, NT);
     mk_rowsum<<<g, NT, 0, st>>>(s.n, s.d_row_bd.p, s.d_slice_ptr.p, s.d_sell_val.p, s.d_diag.p,
-                                w->part.p);
+                                MASS_HEAVY / s.n, w->part.p);
     ms_rowsum<<<1, RT, 0, st>>>((int)g, w->part.p);
     HIPCHECK(hipGetLastError());
     HostSlot h(st);
-    h.read(0, w->part.p);
+    for (int j = 0; j < 3; j++) h.read(8 * j, w->part.p + j);
     h.wait();
-    w->rowsum = h.get<double>(0);
+    const bool callers = s.mesh == nullptr;
+    w->pays = !(h.get<double>(0) > MASS_DOMINANT) &&
+              !(callers && 2.0 * h.get<double>(16) > h.get<double>(8));
     w->rowsum_version = s.a_version;
   }
-  return !(w->rowsum > MASS_DOMINANT);
+  return w->pays;
 }
 
 // Products with the system's matrix in an iteration (mk_step, mk_post,
