@@ -277,6 +277,11 @@ struct System {
   uint64_t a_version = 1;
   bool mg_off = false;      // sparse systems whose mesh is not known
   uint64_t mg_serial = 0;   // sparse systems: the mesh the grids were laid over
+  const Mesh *mg_mesh = nullptr;  // sparse systems: the call's mesh and row order
+  const int *mg_order = nullptr;
+  DevBuf<double> mg_rows;   // row sums (mg_pays), of which matrix, what they say
+  uint64_t mg_pays_version = 0;
+  bool mg_pays = true;
   bool mass = false;  // the assembled matrix has a mass term
   size_t device_bytes() const;
   // user node / dof id -> internal row, and back (mesh systems)
@@ -420,7 +425,7 @@ void cg_work_free(CGWork *w);
 // mg.hip
 void mg_plan_free(MgPlan *p);
 void mg_work_free(MgWork *w);
-void mg_set_mesh(System &s, const Mesh *m, const int *order, hipStream_t st);
+void mg_set_mesh(System &s, const Mesh *m, const int *order);
 bool mg_solve(System &s, const double *b_int, double *x_int, const admfem_solve_opts &o,
               admfem_solve_stats &stats, hipStream_t st);
 void spmv_repeat(System &s, int precision, int repeat, hipStream_t st);

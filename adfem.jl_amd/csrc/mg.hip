@@ -1747,11 +1747,19 @@ void mg_allow_lds(const MgPlan &pl) {
 
 void mg_plan_free(MgPlan *p) { delete p; }
 
+static std::mutex g_plan;  // an engine and a solver may share the system
+
 const MgPlan *mg_plan(System &s, hipStream_t st) {
-  static std::mutex mu;  // an engine and a solver may share the system
-  std::lock_guard<std::mutex> g(mu);
+  std::lock_guard<std::mutex> g(g_plan);
   if (!s.mg_plan && s.mesh) s.mg_plan = build_plan(s, *s.mesh, nullptr, st);
+  else if (!s.mg_plan && s.mg_mesh) s.mg_plan = build_plan(s, *s.mg_mesh, s.mg_order, st);
   return s.mg_plan && s.mg_plan->ok ? s.mg_plan : nullptr;
+}
+
+// (false: a plan was made and does not suit the rows)
+static bool mg_may_suit(const System &s) {
+  std::lock_guard<std::mutex> g(g_plan);
+  return !s.mg_plan || s.mg_plan->ok;
 }
 
 size_t mg_grid_floats(const MgPlan &pl) {
@@ -1810,8 +1818,6 @@ struct MgWork {
   int nblk = 0;
   int last_it = 14;              // iterations of the last solve
   uint64_t version = 0;          // of the matrix the set-up was made from
-  uint64_t rowsum_version = 0;   // of the matrix the row sums were taken of
-  bool pays = true;              // ... and what they say
   ~MgWork() {
     if (h_sc) (void)hipHostFree(h_sc);
   }
@@ -2008,23 +2014,26 @@ void iteration(const MgPlan &pl, MgWork *w, hipStream_t st) {
 // solvers' gradients differ by 1e-9 at dt 1e-3 (P1 160^2) and 2e-8 at 1e-4, by
 // 6e-10 at most from 4e-3 on.
 constexpr double MASS_DOMINANT = 0.2, MASS_HEAVY = 60.0;
-bool mg_pays(System &s, MgWork *w, hipStream_t st) {
+// (Looked at before the plan, which a matrix that stays with Jacobi-PCG never
+// needs: 0.3 ms on every new mesh.)
+bool mg_pays(System &s, hipStream_t st) {
   if (!s.mass) return true;
-  if (w->rowsum_version != s.a_version) {
+  if (s.mg_pays_version != s.a_version) {
     const unsigned g = nb(s.n, NT);
+    if (!s.mg_rows.p) s.mg_rows.alloc(3 + 3 * (size_t)g);
     mk_rowsum<<<g, NT, 0, st>>>(s.n, s.d_row_bd.p, s.d_slice_ptr.p, s.d_sell_val.p, s.d_diag.p,
-                                MASS_HEAVY / s.n, w->part.p);
-    ms_rowsum<<<1, RT, 0, st>>>((int)g, w->part.p);
+                                MASS_HEAVY / s.n, s.mg_rows.p);
+    ms_rowsum<<<1, RT, 0, st>>>((int)g, s.mg_rows.p);
     HIPCHECK(hipGetLastError());
     HostSlot h(st);
-    for (int j = 0; j < 3; j++) h.read(8 * j, w->part.p + j);
+    for (int j = 0; j < 3; j++) h.read(8 * j, s.mg_rows.p + j);
     h.wait();
     const bool callers = s.mesh == nullptr;
-    w->pays = !(h.get<double>(0) > MASS_DOMINANT) &&
+    s.mg_pays = !(h.get<double>(0) > MASS_DOMINANT) &&
               !(callers && 2.0 * h.get<double>(16) > h.get<double>(8));
-    w->rowsum_version = s.a_version;
+    s.mg_pays_version = s.a_version;
   }
-  return w->pays;
+  return s.mg_pays;
 }
 
 // Products with the system's matrix in an iteration (mk_step, mk_post,
@@ -2035,17 +2044,21 @@ constexpr int MG_PRODUCTS = 3;
 }  // namespace
 
 // A sparse system's rows are the dofs of mesh m (m null: unknown, and it is
-// Jacobi-PCG's); its plan is kept for as long as the mesh stays the same one.
-void mg_set_mesh(System &s, const Mesh *m, const int *order, hipStream_t st) {
+// Jacobi-PCG's), row i the caller's order[i]; both are only looked at in the
+// solve that follows.  Its plan is kept for as long as the mesh stays the same
+// one.
+void mg_set_mesh(System &s, const Mesh *m, const int *order) {
   s.mg_off = !m || m->ndof != s.n || s.n < MG_MIN_ROWS;
-  if (s.mg_off || (s.mg_plan && s.mg_serial == m->serial)) return;
+  if (s.mg_off) return;
+  s.mass = true;  // the matrix is the caller's: look before using the grids
+  s.mg_mesh = m;
+  s.mg_order = order;
+  if (s.mg_serial == m->serial) return;
   if (s.mg_work) mg_work_free(s.mg_work);
   if (s.mg_plan) mg_plan_free(s.mg_plan);
   s.mg_work = nullptr;
   s.mg_plan = nullptr;
-  s.mg_plan = build_plan(s, *m, order, st);
   s.mg_serial = m->serial;
-  s.mass = true;  // the matrix is the caller's: look before using the grids
 }
 
 // Solves by multigrid CG when that suits the system; false when it is
@@ -2054,11 +2067,12 @@ bool mg_solve(System &s, const double *b, double *x_out, const admfem_solve_opts
               admfem_solve_stats &stats, hipStream_t st) {
   if (s.mg_off || s.n < MG_MIN_ROWS) return false;
   auto t0 = std::chrono::steady_clock::now();
+  if (!mg_may_suit(s)) return false;
+  if (!mg_pays(s, st)) return false;
   const MgPlan *plan = mg_plan(s, st);
   if (!plan) return false;
   const MgPlan &pl = *plan;
   MgWork *w = ensure_work(s, pl, st);
-  if (!mg_pays(s, w, st)) return false;
   const MgSys *D = w->d.p;
   MgScal *S = w->sc.p;
   if (w->version != s.a_version) {  // a new matrix

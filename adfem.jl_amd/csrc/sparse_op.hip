@@ -311,7 +311,7 @@ System &pattern_with_values(const Mesh *m, const long long *ind, const double *v
   HIPCHECK(hipGetLastError());
   launch_to_sell(*p.s, st);
   p.s->a_version++;
-  mg_set_mesh(*p.s, m, p.reordered ? p.order.p : nullptr, st);
+  mg_set_mesh(*p.s, m, p.reordered ? p.order.p : nullptr);
   return *p.s;
 }
 
