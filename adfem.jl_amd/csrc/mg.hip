@@ -5,15 +5,17 @@
 // Jacobi-PCG takes O(1/h) iterations (4,800 at 1024^2); the V-cycle keeps the
 // count at 11 - 13 for P1 at every size (P2: 12 - 15), so a solve reads the
 // matrix about 60 times in all.  One forward + adjoint on MI355X, Jacobi-PCG
-// -> this: Poisson 64^2 FP64 9.1 -> 1.7 ms, 511^2 FP64 81 -> 3.6 ms, 1024^2
-// mixed 276 -> 5.9 ms, heat 200^2 16.5 -> 2.4 ms, P2 101^2 43 -> 4.7 ms; the
-// small ones are bound by launches (about 5 us each), the large ones by the
-// fine level's passes over memory.  The grids are laid over the mesh's bounding box (cells of about
-// four rows) and know nothing of the triangles: a row takes part through the
-// bilinear interpolation P from the four nodes of its cell, and every coarse
-// matrix is the Galerkin product P^T A P of the assembled matrix, a 25-point
-// stencil on each grid, so boundary conditions, holes, coefficients and mass
-// terms need no special case.  Rows of Dirichlet nodes are not interpolated.
+// -> this: Poisson 64^2 FP64 9.0 -> 1.0 ms, 511^2 FP64 79 -> 2.3 ms, 1024^2
+// mixed 265 -> 4.5 ms, heat 200^2 15.6 -> 1.4 ms, P2 101^2 40 -> 2.1 ms; the
+// small ones are bound by launches that depend on each other (4 - 5 us each,
+// the tail 12 - 15), the large ones by the fine level's passes over memory.
+//
+// The grids are laid over the mesh's bounding box (cells of about four rows)
+// and know nothing of the triangles: a row takes part through the bilinear
+// interpolation P from the four nodes of its cell, and every coarse matrix is
+// the Galerkin product P^T A P of the assembled matrix, a 25-point stencil on
+// each grid, so boundary conditions, holes, coefficients and mass terms need no
+// special case.  Rows of Dirichlet nodes are not interpolated.
 //
 // Smoother: x += w M^-1 (b - A x) with M_ii = a_ii sum_j |a_ij| /
 // sqrt(a_ii a_jj) (the l1 row sums of the diagonally scaled matrix): M - A/1
