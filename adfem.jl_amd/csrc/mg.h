@@ -43,8 +43,9 @@ struct MgSys {
   const int *row_bd;
   const double *sv64, *diag;  // FP64 matrix
   float *sv32;              // scaled off-diagonals a_ij / sqrt(a_ii a_jj)
-  double *dsq;              // 1 / sqrt(a_ii)
-  float *sq, *minv;         // sqrt(a_ii), smoother's weights
+  double *unit;             // s: the V-cycle works on s^2 A, a power of two
+  double *dsq;              // 1 / (s sqrt(a_ii))
+  float *sq, *minv;         // s sqrt(a_ii), smoother's weights
   const int *cell;          // grid cell of each row (-1: not interpolated)
   const float2 *frac;       // position inside the cell
   const int *cptr, *crow;   // rows by cell
@@ -81,6 +82,7 @@ struct MgState {
 struct MgScal {
   double bb, tol2;
   double rr_true, true_prev;  // |b - A x|^2 when CG last stopped, and before
+  double sc, back;          // the V-cycle takes sc r and leaves z / back
   int maxit, nrepl;
   int checked;              // the final residual is known
   MgState a, b;
@@ -101,7 +103,8 @@ const MgPlan *mg_plan(System &s, hipStream_t st);
 
 // Device floats of the grid levels of one system, and the level pointers of
 // a descriptor laid out from `base`.
-// (and the partials' pointers: nblk blocks, summed by one block or not)
+// (and the partials' pointers, into 5 nblk + 6 doubles: nblk blocks, summed by
+// one block or not)
 void mg_parts(MgSys &d, int nblk, bool reduce, double *part);
 size_t mg_grid_floats(const MgPlan &pl);
 void mg_grid_layout(const MgPlan &pl, float *base, MgSys &d);

@@ -27,6 +27,10 @@
 // Precision: the matrix, residual, direction, solution and every dot product
 // of CG are FP64.  The V-cycle works on FP32 copies (fine level: the scaled
 // form S A S of cg.hip) with FP64 sums; it only shapes the search direction.
+// FP32's range is no limit on A or b: the V-cycle sees s^2 A and sc r, with s
+// from the diagonal (matrix_unit) and sc from the first residual (ms_start),
+// and mk_dir takes z back by s^2 / sc.  Both are powers of two, so the
+// mantissas, and with them the iterates, are those of the unscaled numbers.
 // A solve is converged when the residual recomputed from the FP64 matrix is.
 //
 // One iteration (every kernel returns at once when its system is done), from
@@ -202,8 +206,21 @@ __device__ __forceinline__ void sum_partials(const double *part_, int G, double 
 
 // ------------------------------------------------------ per-matrix set-up
 
-// dsq = 1/sqrt(a_ii), sq = sqrt(a_ii), the FP32 scaled off-diagonals and the
-// smoother's weights.  A row without a positive diagonal (an isolated node,
+// The power of two s with s sqrt(a_ii) in [1, 2) for the largest of 64 diagonal
+// entries, of rows spread evenly over the cells (by one wave: a row a lane, which
+// every wave reads anew rather than wait for another launch).
+__device__ __forceinline__ double matrix_unit(const MgSys &d) {
+  const gptr<int> cptr = global_ptr(d.cptr), crow = global_ptr(d.crow);
+  const int rows = cptr[(d.lv[0].nx - 1) * (d.lv[0].ny - 1)];
+  double v = global_ptr(d.diag)[crow[(int)((int64_t)(threadIdx.x & 63) * rows >> 6)]];
+  if (!(v > 0.0 && isfinite(v))) v = 0.0;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
+  return v > 0.0 ? ldexp(1.0, -(ilogb(v) >> 1)) : 1.0;
+}
+
+// dsq = 1/(s sqrt(a_ii)), sq = s sqrt(a_ii), the FP32 scaled off-diagonals and
+// the smoother's weights.  A row without a positive diagonal (an isolated node,
 // or a matrix that is not SPD) gets weight 0: the preconditioner skips it.
 __global__ void __launch_bounds__(NT)
     mk_scale(const int2 *__restrict__ map, const MgSys *__restrict__ D, int sys) {
@@ -214,10 +231,11 @@ __global__ void __launch_bounds__(NT)
   if (i >= d.npad) return;
   const gptr<double> dg = global_ptr(d.diag), sv = global_ptr(d.sv64);
   const gptr<int> sc = global_ptr(d.sc), sp = global_ptr(d.sp);
-  const double aii = dg[i];
+  const double aii = dg[i], s = matrix_unit(d);
   const double si = aii > 0.0 ? 1.0 / sqrt(aii) : 0.0;
-  global_mut(d.dsq)[i] = si;
-  global_mut(d.sq)[i] = aii > 0.0 ? (float)sqrt(aii) : 0.0f;
+  if (m.y == 0 && threadIdx.x == 0) *global_mut(d.unit) = s;
+  global_mut(d.dsq)[i] = si / s;
+  global_mut(d.sq)[i] = aii > 0.0 ? (float)(sqrt(aii) * s) : 0.0f;
   const int s0 = sp[i >> 6], w = (sp[(i >> 6) + 1] - s0) >> 6, off = s0 + (i & 63);
   double sum = 1.0;
   for (int k = 0; k < w; k++) {
@@ -230,7 +248,7 @@ __global__ void __launch_bounds__(NT)
   global_mut(d.minv)[i] = aii > 0.0 ? (float)(1.0 / sum) : 0.0f;
 }
 
-// The first grid's matrix P^T A P: 4 GR threads per grid node, GR for each of
+// The first grid's matrix s^2 P^T A P: 4 GR threads per grid node, GR for each of
 // its cells, which share the cell's rows; a thread's sums for the 4 x 4 nodes
 // around its cell live in LDS (they are addressed by the columns' cells).
 // Bound by the latency of the row -> column -> cell loads: with four lanes to a
@@ -284,6 +302,7 @@ __global__ void __launch_bounds__(GT)
       }
     }
   }
+  const double s = *global_ptr(d.unit), s2 = s * s;
   __syncthreads();
   for (int t = tid; t < 25 * GN; t += GT) {
     const int o = t / GN, q = t % GN, node = mb.y * GN + q;
@@ -296,7 +315,8 @@ __global__ void __launch_bounds__(GT)
 #pragma unroll
       for (int r = 0; r < GR; r++) sum += acc[oy * 4 + ox][q * 4 * GR + 4 * r + cl];
     }
-    global_mut(l.a)[(size_t)o * l.pn + mg_at(l.px, node % l.nx, node / l.nx)] = (float)sum;
+    global_mut(l.a)[(size_t)o * l.pn + mg_at(l.px, node % l.nx, node / l.nx)] =
+        (float)(sum * s2);
   }
 }
 
@@ -602,11 +622,10 @@ __global__ void __launch_bounds__(RT) ms_rowsum(int G, double *__restrict__ out)
 
 // ---------------------------------------------------------------- CG kernels
 
-// The scaled residual and the first smoothing step (from zero) of a row.
-__device__ __forceinline__ void first_smooth(const MgSys &d, int i, double ri) {
-  const float rs = (float)(ri * global_ptr(d.dsq)[i]);
-  global_mut(d.rs)[i] = rs;
-  global_mut(d.x0)[i] = (d.steps == 2 ? C0 : OM) * global_ptr(d.minv)[i] * rs;
+// A row's scaled residual for mk_lead, in FP64 and without the factor sc, which
+// ms_start takes from all of them (in q, which mk_dir is the first to need).
+__device__ __forceinline__ void leave_residual(const MgSys &d, int i, double ri) {
+  global_mut(d.q)[i] = ri * global_ptr(d.dsq)[i];
 }
 
 // A row's residual after the first smoothing step, x0 - rs its negative
@@ -662,7 +681,7 @@ __global__ void __launch_bounds__(NT)
     // its padding entries
     if (global_ptr(d.pos)[i] < 0) global_mut(d.t)[i] = 0.0f;
     global_mut(d.r[0])[i] = ri;
-    first_smooth(d, i, ri);
+    leave_residual(d, i, ri);
     t[0] = ri * ri;
     t[1] = bi * bi;
   }
@@ -683,6 +702,11 @@ __global__ void __launch_bounds__(RT)
   s.tol2 = rtol2 * t[1];
   s.maxit = maxit;
   s.true_prev = -1.0;
+  // |sc r| in [1, 2) at the start; what is left of it at the end, 1e-16 of it at
+  // the least, is far above FP32's smallest numbers
+  const double s1 = *global_ptr(d.unit);
+  s.sc = t[0] > 0.0 && isfinite(t[0]) ? ldexp(1.0, -ilogb(sqrt(t[0]))) : 1.0;
+  s.back = s1 * s1 / s.sc;
   s.a.rr = t[0];
   s.a.first = 1;
   s.a.status = (!(t[0] == t[0]) || !isfinite(t[0])) ? ST_NAN
@@ -708,7 +732,7 @@ __global__ void __launch_bounds__(NT)
                       sell_dot<double>(i, d.sp, d.sc, d.sv64, [&](int c) { return x[c]; });
     const double ri = bi - ax;
     global_mut(d.r[S[m.x].a.it & 1])[i] = ri;
-    first_smooth(d, i, ri);
+    leave_residual(d, i, ri);
     t[0] = ri * ri;
   }
   put_partials<1>(t, d.part4, d.nblk, m.y);
@@ -762,8 +786,9 @@ __global__ void __launch_bounds__(RT)
 }
 
 // p = z + beta p (into the other buffer), q = A p, and r and q with the first
-// smoothing step's weight for mk_step; partials of p.q, r.q, q.q, r.r.  A neighbour's p is formed on the fly by the same fused
-// multiply-add as its own row forms it.
+// smoothing step's weight for mk_step; partials of p.q, r.q, q.q, r.r.  A
+// neighbour's p is formed on the fly by the same fused multiply-add as its own
+// row forms it.
 __global__ void __launch_bounds__(NT)
     mk_dir(const int2 *__restrict__ map, const MgSys *__restrict__ D, MgScal *S_, int sys) {
   const int2 m = where(map, sys);
@@ -778,6 +803,8 @@ __global__ void __launch_bounds__(NT)
   }
   double rz[1];
   sum_small<1>(d.gsum == d.nblk ? d.partz : d.sumz, d.gsum, rz);
+  const double back = S->back;  // z as the V-cycle left it -> z
+  rz[0] *= back;
   st.status = rz[0] != rz[0] || !isfinite(rz[0]) ? ST_NAN : !(rz[0] > 0.0) ? ST_BREAK : ST_RUN;
   const double beta = st.first ? 0.0 : rz[0] / st.rz;
   st.rz = rz[0];
@@ -791,14 +818,14 @@ __global__ void __launch_bounds__(NT)
   if (i < d.npad) {
     struct zp { float z; double p; };
     auto load = [&](int c) { return zp{z[c], p[c]}; };
-    auto comb = [&](zp v) { return fma(beta, v.p, (double)v.z); };
+    auto comb = [&](zp v) { return fma(beta, v.p, (double)v.z * back); };
     const double pi = comb(load(i)), ri = global_ptr(d.r[odd])[i];
     const double qi =
         global_ptr(d.diag)[i] * pi + sell_dot<double>(i, d.sp, d.sc, d.sv64, load, comb);
     global_mut(d.p[!odd])[i] = pi;
     global_mut(d.q)[i] = qi;
-    const double w =
-        (double)((d.steps == 2 ? C0 : OM) * global_ptr(d.minv)[i]) * global_ptr(d.dsq)[i];
+    const double w = (double)((d.steps == 2 ? C0 : OM) * global_ptr(d.minv)[i]) *
+                     global_ptr(d.dsq)[i] * S->sc;
     ((gmptr<f2_t>)reinterpret_cast<f2_t *>(d.wrq))[i] = f2_t{(float)(w * ri), (float)(w * qi)};
     t[0] = pi * qi;
     t[1] = ri * qi;
@@ -850,14 +877,14 @@ __global__ void __launch_bounds__(NT)
   const gptr<f2_t> w = frac_ptr(d.wrq);
   auto load = [&](int c) { return w[c]; };
   auto first = [&](f2_t v) { return (float)fma(-alpha, (double)v.y, (double)v.x); };
-  const float rs = (float)(ri * global_ptr(d.dsq)[i]), x0 = first(load(i));
+  const float rs = (float)(ri * global_ptr(d.dsq)[i] * S->sc), x0 = first(load(i));
   global_mut(d.rs)[i] = rs;
   global_mut(d.x0)[i] = x0;
   smooth_on(d, i, x0, rs, dot32(d, i, load, [&](f2_t v) { return (double)first(v); }));
 }
 
-// The same from the first smoothing step that mk_start or mk_check took, when
-// CG starts.
+// The scaled residual, the first smoothing step and the residual after it from
+// what mk_start or mk_check left, when CG starts.
 __global__ void __launch_bounds__(NT)
     mk_lead(const int2 *__restrict__ map, const MgSys *__restrict__ D, const MgScal *S, int sys) {
   const int2 m = where(map, sys);
@@ -865,8 +892,18 @@ __global__ void __launch_bounds__(NT)
   const MgSys &d = D[m.x];
   const int i = m.y * NT + threadIdx.x;
   if (i >= d.npad) return;
-  const gptr<float> x0 = global_ptr(d.x0);
-  smooth_on(d, i, x0[i], global_ptr(d.rs)[i], dot32(d, i, [&](int c) { return x0[c]; }));
+  const gptr<double> q = global_ptr(d.q);
+  const gptr<float> w = global_ptr(d.minv);
+  const double sc = S[m.x].sc;
+  const float om = d.steps == 2 ? C0 : OM;
+  struct qw { double q; float w; };
+  auto load = [&](int c) { return qw{q[c], w[c]}; };
+  auto first = [&](qw v) { return om * v.w * (float)(v.q * sc); };
+  const qw own = load(i);
+  const float x0 = first(own), rs = (float)(own.q * sc);
+  global_mut(d.rs)[i] = rs;
+  global_mut(d.x0)[i] = x0;
+  smooth_on(d, i, x0, rs, dot32(d, i, load, [&](qw v) { return (double)first(v); }));
 }
 
 // The first of two smoothing steps after the correction (steps = 2):
@@ -1806,6 +1843,7 @@ void mg_parts(MgSys &d, int nblk, bool reduce, double *part) {
   d.partz = part + 4 * (size_t)nblk;
   d.sum4 = d.partz + nblk;
   d.sumz = d.sum4 + 4;
+  d.unit = d.sumz + 1;
   d.gsum = reduce ? 1 : nblk;
 }
 
@@ -1842,7 +1880,7 @@ MgWork *ensure_work(System &s, const MgPlan &pl, hipStream_t st) {
     w->p0.alloc(np);
     w->p1.alloc(np);
     w->dsq.alloc(np);
-    w->part.alloc((size_t)5 * w->nblk + 5);
+    w->part.alloc((size_t)5 * w->nblk + 6);
     w->sv32.alloc(std::max(1, s.slice_ptr.back()));
     w->sq.alloc(np);
     w->minv.alloc(np);

@@ -252,7 +252,7 @@ struct Server {
     double *x = D(nv), *y = D(nv), *kappa = D(ng), *f = D(ng), *uprev = D(np), *b = D(np),
            *sv64 = D(ns), *diag64 = D(np), *dsq = D(np),
            *u64 = D(np), *lam64 = D(np), *grad = D(ng), *obsv = D(nobs + 1),
-           *part = D(5 * nblk + 5), *stage = D(2 * np);
+           *part = D(5 * nblk + 6), *stage = D(2 * np);
     double2 *xy = (double2 *)take(nv * sizeof(double2));
     float *sv32 = F(ns);
     if (pl) {
