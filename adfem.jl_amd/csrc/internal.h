@@ -276,6 +276,7 @@ struct System {
   MgWork *mg_work = nullptr;
   uint64_t a_version = 1;
   bool mg_off = false;      // sparse systems whose mesh is not known
+  uint64_t mg_failed = 0;   // the matrix that multigrid CG could not solve with
   uint64_t mg_serial = 0;   // sparse systems: the mesh the grids were laid over
   const Mesh *mg_mesh = nullptr;  // sparse systems: the call's mesh and row order
   const int *mg_order = nullptr;

@@ -2081,6 +2081,12 @@ bool mg_pays(System &s, hipStream_t st) {
 // iterations are one product each.
 constexpr int MG_PRODUCTS = 3;
 
+// Iterations after which a solve is Jacobi-PCG's after all.  Coefficients or
+// elements that the grids know nothing of slow both down, Jacobi-PCG more (P1
+// 64^2 with white noise of deviation 5 in log kappa: 406 against 5,243; elements
+// of 100 : 1: 110 against 740), so the line only ends what does not converge.
+constexpr int MG_GIVE_UP = 2000;
+
 }  // namespace
 
 // A sparse system's rows are the dofs of mesh m (m null: unknown, and it is
@@ -2102,10 +2108,11 @@ void mg_set_mesh(System &s, const Mesh *m, const int *order) {
 }
 
 // Solves by multigrid CG when that suits the system; false when it is
-// Jacobi-PCG's.
+// Jacobi-PCG's: also when multigrid CG broke down, met a NaN or ran out of
+// iterations, which Jacobi-PCG need not (and if it does, the status is its own).
 bool mg_solve(System &s, const double *b, double *x_out, const admfem_solve_opts &o,
               admfem_solve_stats &stats, hipStream_t st) {
-  if (s.mg_off || s.n < MG_MIN_ROWS) return false;
+  if (s.mg_off || s.n < MG_MIN_ROWS || s.mg_failed == s.a_version) return false;
   auto t0 = std::chrono::steady_clock::now();
   if (!mg_may_suit(s)) return false;
   if (!mg_pays(s, st)) return false;
@@ -2121,7 +2128,7 @@ bool mg_solve(System &s, const double *b, double *x_out, const admfem_solve_opts
   }
   mk_start<<<w->nblk, NT, 0, st>>>(nullptr, D, 0, b);
   ms_start<<<1, RT, 0, st>>>(D, S, nullptr, 0, o.rtol * o.rtol,
-                             std::max(1, o.max_iter / MG_PRODUCTS));
+                             std::min(MG_GIVE_UP, std::max(1, o.max_iter / MG_PRODUCTS)));
   // Iterations are enqueued in chunks, each followed by the check (a no-op
   // while CG runs), and the host reads the state between chunks; kernels past
   // the end return at once.  The first chunk is what the system's last solve
@@ -2144,6 +2151,10 @@ bool mg_solve(System &s, const double *b, double *x_out, const admfem_solve_opts
     if (w->h_sc->a.status != ST_RUN) break;
     if (o.check_every <= 0) chunk = 2;
   }
+  if (w->h_sc->a.status != ST_CONV) {
+    s.mg_failed = s.a_version;
+    return false;
+  }
   w->last_it = std::min(64, std::max(4, w->h_sc->a.it));
   if (x_out == b) {
     HIPCHECK(hipMemcpyAsync(x_out, w->x.p, sizeof(double) * s.n, hipMemcpyDeviceToDevice, st));
@@ -2153,12 +2164,7 @@ bool mg_solve(System &s, const double *b, double *x_out, const admfem_solve_opts
   stats.iterations = MG_PRODUCTS * h.a.it;
   stats.replacements = h.nrepl;
   stats.rel_residual = h.bb > 0 ? std::sqrt(h.rr_true / h.bb) : 0.0;
-  switch (h.a.status) {
-    case ST_CONV: stats.status = ADMFEM_OK; break;
-    case ST_NAN: stats.status = ADMFEM_ERR_NAN; break;
-    case ST_BREAK: stats.status = ADMFEM_ERR_BREAKDOWN; break;
-    default: stats.status = ADMFEM_ERR_NOT_CONVERGED; break;
-  }
+  stats.status = ADMFEM_OK;
   stats.seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
   return true;
 }

@@ -329,7 +329,9 @@ typedef struct {
  * the assembled rhs.  x is the output (its input value is ignored).  The
  * solver is multigrid-preconditioned CG on grids laid over the mesh, or
  * Jacobi-PCG for the few systems those do not suit (fewer than 200 rows,
- * strongly graded meshes, matrices dominated by their mass term).  Jacobi-PCG
+ * strongly graded meshes, matrices dominated by their mass term) and for a
+ * matrix that multigrid CG breaks down on or does not converge for (the stats
+ * are then Jacobi-PCG's alone).  Jacobi-PCG
  * replays its iterations from a HIP graph (8 iterations, kernel nodes only),
  * captured on the first solve of a setting on a stream of its own and
  * replayed on the caller's; the system holds both until it is destroyed.
