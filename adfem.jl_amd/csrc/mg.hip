@@ -2081,12 +2081,6 @@ bool mg_pays(System &s, hipStream_t st) {
 // iterations are one product each.
 constexpr int MG_PRODUCTS = 3;
 
-// Iterations after which a solve is Jacobi-PCG's after all.  Coefficients or
-// elements that the grids know nothing of slow both down, Jacobi-PCG more (P1
-// 64^2 with white noise of deviation 5 in log kappa: 406 against 5,243; elements
-// of 100 : 1: 110 against 740), so the line only ends what does not converge.
-constexpr int MG_GIVE_UP = 2000;
-
 }  // namespace
 
 // A sparse system's rows are the dofs of mesh m (m null: unknown, and it is

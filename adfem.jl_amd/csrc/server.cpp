@@ -136,6 +136,7 @@ struct Req {
   bool mg = false;           // multigrid CG (else Jacobi-PCG)
   int slot = -1;
   char *mem = nullptr;       // its memory in the arena
+  size_t bytes = 0;          // how much (of the layout it was admitted with)
   // device buffers (inside the arena)
   double2 *xy;
   double *x, *y, *kappa, *f, *uprev, *b, *sv64, *diag64, *dsq, *xa, *xb, *u64, *lam64,
@@ -570,6 +571,7 @@ struct Server {
       return true;
     }
     q.mem = mem;
+    q.bytes = bytes;
     q.res.device_bytes = (double)bytes;
     layout(*T.sys, q.mg ? T.plan : nullptr, &q, mem, q.nobs);
     q.slot = free_slots.back();
@@ -611,8 +613,27 @@ struct Server {
     jobs_in.flush(serve_inputs, st);
   }
 
+  // A solve that multigrid CG ended without a solution starts over with
+  // Jacobi-PCG, which need not fail (and if it does, the status is its own), and
+  // the request stays there.  The matrix and the right-hand side are where they
+  // were (the caller's inputs may be gone by now); Jacobi-PCG's vectors take the
+  // place of the others.
+  void to_jacobi(Req &q) {
+    const System &s = *topos[q.r.topo].sys;
+    const size_t np = s.npad;
+    q.mg = false;
+    q.xa = q.mgx;
+    q.xb = q.mgr;
+    float **const v[] = {&q.ysa, &q.ysb, &q.ra, &q.rb, &q.pa, &q.pb, &q.qa, &q.qb};
+    float *const at[] = {q.sq, q.minv, q.z, q.rs, q.x0, q.t, (float *)q.wrq, (float *)q.wrq + np};
+    for (int k = 0; k < 8; k++) *v[k] = at[k];
+    batch_scale(s, q.sv64, q.diag64, q.dsq, q.sv32, st);
+    write_desc(q, q.b);
+    start_cg(q);
+  }
+
   void release(Req &q) {
-    arena.release(q.mem, bytes_of(q));
+    arena.release(q.mem, q.bytes);
     free_slots.push_back(q.slot);
     q.slot = -1;
   }
@@ -864,7 +885,8 @@ struct Server {
       }
       if (!starts.empty()) {
         build_set(set_starts, starts);
-        mg_batch_start(set_starts.batch, d_mg.p, d_mgs.p, o.rtol * o.rtol, o.max_iter, st);
+        mg_batch_start(set_starts.batch, d_mg.p, d_mgs.p, o.rtol * o.rtol,
+                       std::min(MG_GIVE_UP, o.max_iter), st);
         starts.clear();
       }
       if (!mgr.empty()) {
@@ -915,6 +937,11 @@ struct Server {
           sc = {v.status, v.it, v.rr, v.bb};
         }
         if (sc.status == 0) {
+          still.push_back(i);
+          continue;
+        }
+        if (sc.status != 1 && q.mg) {
+          to_jacobi(q);
           still.push_back(i);
           continue;
         }

@@ -4,10 +4,13 @@ FP32 grids hold.  The diagonally scaled matrix is harmless, and Jacobi-PCG takes
 many iterations as for any such pattern."""
 import numpy as np
 import pytest
+import scipy.sparse as sp
+import scipy.sparse.linalg as spla
 import torch
 
 import admfem
 from admfem import meshgen
+from admfem.server import Server
 
 pytestmark = pytest.mark.gpu
 
@@ -47,3 +50,37 @@ def test_operators():
     plain = admfem.solve(admfem.SparseTensor(B.indices, B.values, B.n), r, rtol=1e-10,
                          max_iter=5000)
     assert ((x - plain).norm() / plain.norm()).item() < 1e-8
+
+
+def test_serving_requests():
+    """Among requests that multigrid CG serves, and with the same results for those
+    whatever else is in the batch."""
+    mesh, kap, f, bd = board(64)
+    S = admfem.DirichletSystem(mesh, bd)
+    obs = np.setdiff1d(np.arange(mesh.ndof), bd - 1)[::40].astype(np.int32)
+    out = {}
+    for which in ((0, 1, 2, 3), (0, 2), (1, 3)):
+        print("fallback, serving", which, flush=True)
+        sv = Server(1 << 30, rtol=1e-8)
+        t = sv.add_topology(S)
+        ids = {}
+        for k in which:
+            one = torch.ones_like(kap)
+            ids[k] = sv.submit(t, kappa=(kap, one, kap * 2, one * 2)[k], f=f,
+                               obs_idx=torch.tensor(obs), obs_val=torch.zeros(obs.size))
+        sv.run(timeout=60)
+        for k, i in ids.items():
+            r = sv.result(i)
+            assert r["status"] == 0 and r["relres_fwd"] <= 1e-8 and r["relres_adj"] <= 1e-8
+            if k in out:
+                np.testing.assert_array_equal(r["u"], out[k]["u"])
+                np.testing.assert_array_equal(r["grad"], out[k]["grad"])
+            out[k] = r
+        sv.close()
+    # the direct solve of the diagonally scaled matrix, whose condition is a
+    # Laplacian's on 64^2, some 4,000: 1e-8 times that
+    S.assemble(kappa=kap, f=f)
+    A, b = S.csr()
+    s = 1 / np.sqrt(A.diagonal())
+    y = spla.spsolve(sp.diags(s) @ A @ sp.diags(s), s * b)
+    assert np.linalg.norm(out[0]["u"] / s - y) <= 1e-4 * np.linalg.norm(y)
