@@ -29,6 +29,11 @@ __host__ __device__ inline int mg_at(int px, int x, int y) {
 // even.
 constexpr int MG_MIN_ROWS = 200;
 
+// Products with the system's matrix in an iteration (mk_step, mk_post,
+// mk_dir): what max_iter bounds and the stats report, as for Jacobi-PCG, whose
+// iterations are one product each.
+constexpr int MG_PRODUCTS = 3;
+
 // Iterations after which a solve is Jacobi-PCG's after all.  Coefficients or
 // elements that the grids know nothing of slow both down, Jacobi-PCG more (P1
 // 64^2 with white noise of deviation 5 in log kappa: 406 against 5,243; elements

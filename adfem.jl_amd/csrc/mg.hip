@@ -2076,11 +2076,6 @@ bool mg_pays(System &s, hipStream_t st) {
   return s.mg_pays;
 }
 
-// Products with the system's matrix in an iteration (mk_step, mk_post,
-// mk_dir): what max_iter bounds and the stats report, as for Jacobi-PCG, whose
-// iterations are one product each.
-constexpr int MG_PRODUCTS = 3;
-
 }  // namespace
 
 // A sparse system's rows are the dofs of mesh m (m null: unknown, and it is

@@ -886,7 +886,7 @@ struct Server {
       if (!starts.empty()) {
         build_set(set_starts, starts);
         mg_batch_start(set_starts.batch, d_mg.p, d_mgs.p, o.rtol * o.rtol,
-                       std::min(MG_GIVE_UP, o.max_iter), st);
+                       std::min(MG_GIVE_UP, std::max(1, o.max_iter / MG_PRODUCTS)), st);
         starts.clear();
       }
       if (!mgr.empty()) {
@@ -927,11 +927,11 @@ struct Server {
       for (int i : active) {
         Req &q = reqs[i];
         // where the solve stands: status (0 run, 1 converged, else failed),
-        // iterations, true residual and right-hand side norms squared
+        // products with A, true residual and right-hand side norms squared
         struct { int status, it; double rr, bb; } sc;
         if (q.mg) {
           const MgScal &v = h_mgs[q.slot];
-          sc = {v.checked ? v.a.status : 0, v.a.it, v.rr_true, v.bb};
+          sc = {v.checked ? v.a.status : 0, MG_PRODUCTS * v.a.it, v.rr_true, v.bb};
         } else {
           const BScal &v = h_scal[q.slot];
           sc = {v.status, v.it, v.rr, v.bb};

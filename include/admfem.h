@@ -458,7 +458,8 @@ typedef struct {
   int max_active;          /* cap on concurrently admitted requests */
   int mode;                /* ADMFEM_MODE_* */
   double rtol;             /* true relative residual of every solve */
-  int max_iter;
+  int max_iter;            /* per solve, in products with A (a multigrid
+                              iteration takes three) */
   double replace_delta;    /* mixed: residual replacement factor (0: 0.3) */
   int chunk;               /* CG iterations between host checks (0: 16;
                               rounded up to a multiple of 8) */
@@ -504,7 +505,7 @@ typedef struct {
   int done;
   double t_arrival, t_admit, t_done; /* seconds after run start */
   double loss;
-  int iters_fwd, iters_adj;
+  int iters_fwd, iters_adj;          /* in products with A */
   double relres_fwd, relres_adj;     /* true FP64 relative residuals */
   double device_bytes;
 } admfem_result;

@@ -1,0 +1,41 @@
+"""What the serving engine's limits count."""
+import numpy as np
+import pytest
+
+import admfem
+from admfem import meshgen
+from admfem.server import Server
+
+pytestmark = pytest.mark.gpu
+
+
+def topology(m):
+    c, e = meshgen.jittered_square(m, seed=m)
+    mesh = admfem.Mesh(c, e, zero_based=True)
+    return admfem.DirichletSystem(mesh, admfem.bcnode(mesh))
+
+
+def serve(S, mode="batched", n=1, budget=1 << 30, **kw):
+    sv = Server(budget, mode=mode, rtol=1e-8, **kw)
+    t = sv.add_topology(S)
+    ids = [sv.submit(t, seed=k + 1) for k in range(n)]
+    sv.run(timeout=60)
+    out = [sv.result(i) for i in ids]
+    sv.close()
+    return out
+
+
+def test_iterations_are_products_with_the_matrix():
+    """The same unit in both modes, and the one that max_iter is given in: three a
+    multigrid iteration.  Grids of either mode differ by rounding only, so their
+    counts differ by an iteration at most.  Twelve products, four iterations, do not
+    solve to 1e-8 (an iteration takes about a factor of ten)."""
+    S = topology(64)
+    a, b = (serve(S, mode)[0] for mode in ("batched", "seq_fp64"))
+    print("serving, iterations", a["iters_fwd"], a["iters_adj"], b["iters_fwd"], flush=True)
+    for k in ("iters_fwd", "iters_adj"):
+        assert a[k] % 3 == 0 and abs(a[k] - b[k]) <= 3
+    for mode in ("batched", "seq_fp64"):
+        assert serve(S, mode, max_iter=12)[0]["status"] == admfem._lib.ERR_NOT_CONVERGED
+        r = serve(S, mode, max_iter=a["iters_fwd"] + 6)[0]
+        assert r["status"] == 0 and r["iters_fwd"] <= a["iters_fwd"] + 6
