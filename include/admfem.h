@@ -307,7 +307,9 @@ typedef struct {
   int precision;      /* ADMFEM_PREC_* */
   int max_iter;       /* total inner iterations, counted in products with A (a
                          multigrid iteration takes three) */
-  double rtol;        /* ||b - A x||_2 <= rtol * ||b||_2 (true residual) */
+  double rtol;        /* ||b - A x||_2 <= rtol * ||b||_2 (true residual);
+                         below what FP64 can reach for A and b, the solve
+                         ends there as ADMFEM_OK and rel_residual says where */
   int check_every;    /* iterations between host convergence checks (0: auto) */
   double replace_delta; /* mixed: FP64 residual replacement when the inner
                            residual fell by this factor since the last one
