@@ -39,3 +39,21 @@ def test_iterations_are_products_with_the_matrix():
         assert serve(S, mode, max_iter=12)[0]["status"] == admfem._lib.ERR_NOT_CONVERGED
         r = serve(S, mode, max_iter=a["iters_fwd"] + 6)[0]
         assert r["status"] == 0 and r["iters_fwd"] <= a["iters_fwd"] + 6
+
+
+@pytest.mark.parametrize("m", [32, 128])
+def test_budget_that_holds_a_request_with_the_smaller_solver(m):
+    """A request needs more memory with multigrid CG than with Jacobi-PCG: where the
+    budget holds it with the latter only, it is served, one at a time; below that it
+    is refused."""
+    S = topology(m)
+    wide = serve(S)[0]
+    small = next(r for r in (serve(S, budget=wide["device_bytes"] * q / 100)[0]
+                             for q in range(60, 100)) if r["status"] == 0)
+    print("serving, budget", m, wide["device_bytes"], small["device_bytes"], flush=True)
+    assert small["iters_fwd"] > 2 * wide["iters_fwd"]
+    for r in serve(S, n=3, budget=small["device_bytes"]):
+        assert r["status"] == 0
+    assert np.linalg.norm(small["grad"] - wide["grad"]) < 1e-6 * np.linalg.norm(wide["grad"])
+    r = serve(S, budget=small["device_bytes"] - 4096)[0]
+    assert r["status"] == admfem._lib.ERR_BUDGET
