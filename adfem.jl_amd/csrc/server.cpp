@@ -42,6 +42,10 @@ struct Arena {
     cap = up(bytes);
     size_t avail = 0, total = 0;
     HIPCHECK(hipMemGetInfo(&avail, &total));
+    if (cap > avail) {  // (what the library keeps for later buffers is free, too)
+      release_device_memory();
+      HIPCHECK(hipMemGetInfo(&avail, &total));
+    }
     REQUIRE(cap <= avail, ADMFEM_ERR_HIP, "the HBM budget exceeds the free device memory");
   }
   ~Arena() {

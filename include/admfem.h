@@ -456,7 +456,13 @@ typedef struct admfem_server_s *admfem_server;
 #define ADMFEM_MODE_SEQ_FP64 1    /* one request at a time, FP64 solver */
 
 typedef struct {
-  double hbm_budget_bytes; /* device memory for admitted requests */
+  double hbm_budget_bytes; /* device memory for admitted requests, at most: free
+                              when the server is created, but taken only as
+                              requests wait for it and not reserved before.
+                              What another allocator takes meanwhile is missing:
+                              requests then wait for each other, and one that
+                              finds no room on the card with no other admitted
+                              ends with ADMFEM_ERR_BUDGET */
   int max_active;          /* cap on concurrently admitted requests */
   int mode;                /* ADMFEM_MODE_* */
   double rtol;             /* true relative residual of every solve */

@@ -1,6 +1,7 @@
 """What the serving engine's limits count."""
 import numpy as np
 import pytest
+import torch
 
 import admfem
 from admfem import meshgen
@@ -57,3 +58,15 @@ def test_budget_that_holds_a_request_with_the_smaller_solver(m):
     assert np.linalg.norm(small["grad"] - wide["grad"]) < 1e-6 * np.linalg.norm(wide["grad"])
     r = serve(S, budget=small["device_bytes"] - 4096)[0]
     assert r["status"] == admfem._lib.ERR_BUDGET
+
+
+def test_a_budget_counts_cached_blocks_as_free():
+    """An engine's budget is compared with the free memory of the card, and blocks
+    that closed meshes left in the library's cache are free."""
+    S = topology(900)
+    S.close()
+    S.mesh.close()
+    before = torch.cuda.mem_get_info()[0]
+    print("serving, budget and cache", before, flush=True)
+    Server(before + (64 << 20)).close()
+    assert torch.cuda.mem_get_info()[0] >= before + (64 << 20)  # (there were as many)
