@@ -803,7 +803,9 @@ struct Server {
     jobs_out.clear();
     size_t next = 0;  // first request (in arrival order) not yet admitted
     while (next < order.size() && reqs[order[next]].state != Q_WAIT) next++;
-    const int mg_chunk = o.chunk > 0 ? o.chunk : 4;
+    // (a solve is 8 to 12 iterations; 64 a chunk on 8 requests of 64^2: 1.7 -> 3.0 ms,
+    // 512: 21.8)
+    const int mg_chunk = o.chunk > 0 ? std::min(o.chunk, 4) : 4;
     std::vector<int> active;
     for (size_t i = 0; i < reqs.size(); i++)
       if (reqs[i].state == Q_FWD || reqs[i].state == Q_ADJ) active.push_back((int)i);

@@ -310,7 +310,8 @@ typedef struct {
   double rtol;        /* ||b - A x||_2 <= rtol * ||b||_2 (true residual);
                          below what FP64 can reach for A and b, the solve
                          ends there as ADMFEM_OK and rel_residual says where */
-  int check_every;    /* iterations between host convergence checks (0: auto) */
+  int check_every;    /* iterations between host convergence checks (0: auto),
+                         multigrid's at most */
   double replace_delta; /* mixed: FP64 residual replacement when the inner
                            residual fell by this factor since the last one
                            (0: 0.3); also forced after 64 iterations without
@@ -469,8 +470,9 @@ typedef struct {
   int max_iter;            /* per solve, in products with A (a multigrid
                               iteration takes three) */
   double replace_delta;    /* mixed: residual replacement factor (0: 0.3) */
-  int chunk;               /* CG iterations between host checks (0: 16;
-                              rounded up to a multiple of 8) */
+  int chunk;               /* Jacobi-PCG iterations between host checks (0: 16;
+                              rounded up to a multiple of 8); multigrid's are
+                              as many, and four at most */
   int use_graph;           /* replay each chunk as a captured HIP graph */
 } admfem_server_opts;
 
