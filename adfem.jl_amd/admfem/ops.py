@@ -16,6 +16,7 @@ numpy inputs take the reference's Array paths (MCore.jl:77-82, 112-120) and
 return numpy / scipy results.  ``loss.backward()`` plays the role of
 ADCME's ``gradients(loss, kappa)``.
 """
+import copy
 import ctypes
 
 import numpy as np
@@ -46,6 +47,23 @@ class SparseTensor:
     @property
     def shape(self):
         return (self.n, self.n)
+
+    # The mesh holds a handle of the library: copies share it, and a pickle, which
+    # may be read by another process, leaves it out.
+    def __getstate__(self):
+        return {k: v for k, v in self.__dict__.items() if k != "mesh"}
+
+    def __copy__(self):
+        B = type(self).__new__(type(self))
+        B.__dict__.update(self.__dict__)
+        return B
+
+    def __deepcopy__(self, memo):
+        B = type(self).__new__(type(self))
+        memo[id(self)] = B
+        for k, v in self.__dict__.items():
+            B.__dict__[k] = v if k == "mesh" else copy.deepcopy(v, memo)
+        return B
 
     def __add__(self, other):
         if not isinstance(other, SparseTensor) or other.n != self.n:
