@@ -23,8 +23,10 @@ namespace {
 
 constexpr size_t CACHE_BLOCK = (size_t)64 << 20, CACHE_TOTAL = (size_t)512 << 20;
 
-// a request's size class: powers of two up to 64 KiB, then eighths of them
+// a request's size class: powers of two up to 64 KiB, then eighths of them;
+// blocks that are never cached have their own size
 size_t size_class(size_t bytes) {
+  if (bytes > CACHE_BLOCK) return bytes;
   size_t p = 256;
   while (p < bytes) p <<= 1;
   if (p <= (size_t)64 << 10) return p;
