@@ -5,7 +5,7 @@ The Python mirror of the reference's Julia operator surface
 Every compute call runs the library's HIP kernels; there is no CPU
 fallback -- a missing library raises.
 """
-from ._lib import AdmfemError, lib  # noqa: F401
+from ._lib import AdmfemError, lib, release_memory  # noqa: F401
 from .mesh import (Mesh, bcedge, bcnode, fem_nodes, gauss_nodes, gauss_weights,  # noqa: F401
                    get_area, get_ngauss)
 from .system import DirichletSystem, solve_opts  # noqa: F401

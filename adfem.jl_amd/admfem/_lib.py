@@ -161,6 +161,13 @@ def check(rc):
     return rc
 
 
+def release_memory():
+    """Gives the device memory that the library keeps for its next buffers (at
+    most 512 MiB of released ones) back, as torch.cuda.empty_cache() does torch's:
+    torch's allocator does not see it."""
+    check(lib().admfem_release_memory())
+
+
 def stream_ptr(stream=None):
     """HIP stream handle of a torch stream (current stream by default)."""
     s = stream if stream is not None else torch.cuda.current_stream()
