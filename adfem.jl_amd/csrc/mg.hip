@@ -1517,22 +1517,38 @@ __device__ __forceinline__ bool takes_part(int i, const int *__restrict__ row_bd
   return false;
 }
 
-// Per block: the interior rows' bounding box, count and largest coupling
-// extents (|dx|, |dy| over the matrix entries).
+// A mesh's dofs and how many others each shares an element with: P1 from the
+// pattern (ptr, by internal node, with the diagonal), P2 from the number of
+// incident elements (ptr, by the caller's dof): 3 for each of a vertex's, 3 and 2
+// more for an edge's.  uid: row -> the caller's dof (null: the same).
+struct DofGraph {
+  const int *uid, *perm, *ptr;
+  int degree, nnode;
+  __device__ int neighbours(int i) const {
+    const int u = uid ? uid[i] : i, v = degree == 1 ? perm[u] : u;
+    const int k = ptr[v + 1] - ptr[v];
+    return degree == 1 ? k - 1 : u < nnode ? 3 * k : 3 * k + 2;
+  }
+};
+
+// Per block: the interior rows' bounding box, count, largest coupling extents
+// (|dx|, |dy| over the matrix entries) and the sum over the rows of the part of
+// their neighbours that the Dirichlet rows are.
 __global__ void __launch_bounds__(NT)
-    plan_extent(int n, const double2 *__restrict__ pt, const int *__restrict__ row_bd, const int *__restrict__ sp,
-                const int *__restrict__ sc, double *__restrict__ out) {
+    plan_extent(int n, const double2 *__restrict__ pt, const int *__restrict__ row_bd,
+                const int *__restrict__ sp, const int *__restrict__ sc, DofGraph graph,
+                double *__restrict__ out) {
   const int i = blockIdx.x * NT + threadIdx.x;
   // min x, min y, -max x, -max y, -max |dx|, -max |dy|
   double v[6] = {1e300, 1e300, 1e300, 1e300, 0.0, 0.0};
-  double cnt = 0.0;
+  double cnt[2] = {0.0, 0.0};
   if (i < n && takes_part(i, row_bd, sp, sc)) {
     const double2 a = pt[i];
+    int coupled = 0;
     v[0] = a.x;
     v[1] = a.y;
     v[2] = -a.x;
     v[3] = -a.y;
-    cnt = 1.0;
     const int s0 = sp[i >> 6], w = (sp[(i >> 6) + 1] - s0) >> 6, off = s0 + (i & 63);
     for (int k = 0; k < w; k++) {
       const int j = sc[off + 64 * k];
@@ -1540,9 +1556,13 @@ __global__ void __launch_bounds__(NT)
       const double2 b = pt[j];
       v[4] = fmin(v[4], -fabs(a.x - b.x));
       v[5] = fmin(v[5], -fabs(a.y - b.y));
+      coupled += j != i;
     }
+    const int all = graph.neighbours(i);
+    cnt[0] = 1.0;
+    cnt[1] = all > coupled ? (double)(all - coupled) / all : 0.0;
   }
-  __shared__ double sh[7][NT / 64];
+  __shared__ double sh[8][NT / 64];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
 #pragma unroll
   for (int j = 0; j < 6; j++) {
@@ -1551,10 +1571,13 @@ __global__ void __launch_bounds__(NT)
     for (int o = 32; o > 0; o >>= 1) t = fmin(t, __shfl_xor(t, o, 64));
     if (lane == 0) sh[j][wv] = t;
   }
-  cnt = wave_sum(cnt);
-  if (lane == 0) sh[6][wv] = cnt;
+#pragma unroll
+  for (int j = 0; j < 2; j++) {
+    const double t = wave_sum(cnt[j]);
+    if (lane == 0) sh[6 + j][wv] = t;
+  }
   __syncthreads();
-  if (threadIdx.x < 7) {
+  if (threadIdx.x < 8) {
     double t = sh[threadIdx.x][0];
     for (int k = 1; k < NT / 64; k++)
       t = threadIdx.x < 6 ? fmin(t, sh[threadIdx.x][k]) : t + sh[threadIdx.x][k];
@@ -1662,20 +1685,23 @@ MgPlan *build_plan(System &s, const Mesh &m, const int *order, hipStream_t st) {
     const bool own = s.mesh != nullptr;
     pl->n = n;
     const unsigned g = nb(n, NT);
-    DevBuf<double> ext((size_t)7 * g), ar(256);
+    DevBuf<double> ext((size_t)8 * g), ar(256);
     DevBuf<double2> pt(n);
     plan_points<<<g, NT, 0, st>>>(n, m.xy.p, own && s.degree == 2 ? s.d_dof_ends.p : nullptr,
                                   order, own ? nullptr : m.d_perm.p, m.nnode, m.d_edges.p,
                                   m.nedges, pt.p);
-    plan_extent<<<g, NT, 0, st>>>(n, pt.p, s.d_row_bd.p, s.d_slice_ptr.p, s.d_sell_col.p, ext.p);
+    const DofGraph graph{own ? s.d_uiperm() : order, m.d_perm.p,
+                         m.degree == 1 ? m.d_rp.p : m.d_d2e_ptr.p, m.degree, m.nnode};
+    plan_extent<<<g, NT, 0, st>>>(n, pt.p, s.d_row_bd.p, s.d_slice_ptr.p, s.d_sell_col.p, graph,
+                                  ext.p);
     plan_area<<<256, NT, 0, st>>>(m.nelem, m.area.p, ar.p);
     HIPCHECK(hipGetLastError());
-    std::vector<double> he((size_t)7 * g), ha(256);
+    std::vector<double> he((size_t)8 * g), ha(256);
     HIPCHECK(hipMemcpyAsync(he.data(), ext.p, ext.bytes(), hipMemcpyDeviceToHost, st));
     HIPCHECK(hipMemcpyAsync(ha.data(), ar.p, ar.bytes(), hipMemcpyDeviceToHost, st));
     HIPCHECK(hipStreamSynchronize(st));
-    double v[7] = {1e300, 1e300, 1e300, 1e300, 0, 0, 0}, area = 0.0;
-    for (int j = 0; j < 7; j++)
+    double v[8] = {1e300, 1e300, 1e300, 1e300, 0, 0, 0, 0}, area = 0.0;
+    for (int j = 0; j < 8; j++)
       for (unsigned b = 0; b < g; b++)
         v[j] = j < 6 ? std::min(v[j], he[(size_t)j * g + b]) : v[j] + he[(size_t)j * g + b];
     for (double a : ha) area += a;
@@ -1749,6 +1775,19 @@ MgPlan *build_plan(System &s, const Mesh &m, const int *order, hipStream_t st) {
     }
     pl->nlev = k + 1;
     if (pl->tail < 0 || pl->nlev - pl->tail > TAIL_LEVELS) return pl;
+    // Where most rows neighbour a Dirichlet row Jacobi-PCG takes some 11 + 7 / F
+    // iterations of 14 us (F: the part of their neighbours that are Dirichlet
+    // rows), and the V-cycles' launches, two more for every grid above the tail,
+    // cost more.  Forward + adjoint, Jacobi-PCG against multigrid CG: strips of
+    // 2000 x 3 quads (F = 0.33, two grids) 1.00 and 1.12 ms, x 4 (0.22) 1.22 and
+    // 1.14; 20000 x 3 (five grids) 1.07 and 1.80, x 6 (0.13) 1.98 and 2.10, x 8
+    // (0.095) 2.57 and 2.18; every third row of 150^2 Dirichlet (one grid) 0.87 and
+    // 1.08, every fourth 1.19 and 1.16.  P2, whose iterations are twice as many:
+    // 5000 x 1 (0.75) 0.75 and 1.37, x 2 (0.35) 1.54 and 1.62, x 3 (0.21) 2.89 and
+    // 2.09.  Without a grid above the tail multigrid CG is faster (200 x 2: 0.74 and
+    // 0.63).
+    const double near = std::max(0.125, 0.3 - 0.035 * pl->tail) * m.degree;
+    if (pl->tail > 0 && v[7] > near * rows) return pl;
     pl->ok = true;
     return pl;
   } catch (...) {
