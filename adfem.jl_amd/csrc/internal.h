@@ -38,8 +38,9 @@ void device_free(void *p, size_t bytes, int device);
 void release_device_memory();
 
 // 64 bytes of pinned host memory for a call's results (memory.cpp): read()
-// enqueues a copy from the device, wait() makes what was read visible.  A copy
-// to ordinary memory instead blocks the host by itself, 10 - 15 us each.
+// enqueues a copy from the device, wait() makes what was read visible, or what a
+// kernel of the stream wrote to written().  A copy to ordinary memory instead
+// blocks the host by itself, 10 - 15 us each.
 class HostSlot {
  public:
   explicit HostSlot(hipStream_t stream);
@@ -49,6 +50,10 @@ class HostSlot {
   template <class T> void read(int at, const T *dev) {
     HIPCHECK(hipMemcpyAsync((char *)p + at, dev, sizeof(T), hipMemcpyDeviceToHost, st));
     pending = true;
+  }
+  double *written() {
+    pending = true;
+    return (double *)p;
   }
   void wait() {
     HIPCHECK(hipStreamSynchronize(st));

@@ -560,65 +560,74 @@ __global__ void __launch_bounds__(ST)
 }
 
 // Over the coupled rows: the smallest row sum over diagonal, how many rows
-// there are, and how many whose row sum over diagonal exceeds `heavy` (per
-// block, then over the blocks, into out[0 .. 2]): what the mass term leaves of
-// the constant's energy.
+// there are, how many whose row sum over diagonal exceeds `heavy`, and the sums of
+// their row sums and diagonals (per block, then over the blocks to host memory):
+// what the mass term leaves of the constant's energy.
+constexpr int ROWSUMS = 5;
 __global__ void __launch_bounds__(NT)
     mk_rowsum(int n, const int *__restrict__ row_bd, const int *__restrict__ sp,
               const double *__restrict__ sv, const double *__restrict__ diag, double heavy,
               double *__restrict__ out) {
-  const int i = blockIdx.x * NT + threadIdx.x;
-  double v = 1.0, cnt[2] = {0.0, 0.0};
+  // the XCDs' rows are the solvers': entries that another XCD had read were slower
+  // for all of the solve (P2 100^2: k_step 7.0 us instead of 5.9)
+  const int i = xcd_block(blockIdx.x, gridDim.x) * NT + threadIdx.x;
+  double v = 1.0, cnt[ROWSUMS - 1] = {};
   if (i < n && row_bd[i] < 0) {
     const int s0 = sp[i >> 6], w = (sp[(i >> 6) + 1] - s0) >> 6, off = s0 + (i & 63);
     double sum = diag[i];
     bool coupled = false;
-    for (int k = 0; k < w; k++) {
-      const double a = sv[off + 64 * k];
-      sum += a;
-      coupled = coupled || a != 0.0;
+    for (int k = 0; k < w; k += 8) {
+      double a[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++)
+        a[u] = __builtin_nontemporal_load(sv + off + 64 * min(k + u, w - 1));
+#pragma unroll
+      for (int u = 0; u < 8; u++)
+        if (k + u < w) {
+          sum += a[u];
+          coupled = coupled || a[u] != 0.0;
+        }
     }
     v = sum / diag[i];
     cnt[0] = coupled;
     cnt[1] = coupled && v > heavy;
+    cnt[2] = coupled ? sum : 0.0;
+    cnt[3] = coupled ? diag[i] : 0.0;
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v = fmin(v, __shfl_xor(v, o, 64));
-  __shared__ double sh[NT / 64], sc[2][NT / 64];
+  __shared__ double sh[ROWSUMS][NT / 64];
   const int wv = threadIdx.x >> 6;
 #pragma unroll
-  for (int j = 0; j < 2; j++) cnt[j] = wave_sum(cnt[j]);
+  for (int j = 0; j < ROWSUMS - 1; j++) cnt[j] = wave_sum(cnt[j]);
   if ((threadIdx.x & 63) == 0) {
-    sh[wv] = v;
-    sc[0][wv] = cnt[0];
-    sc[1][wv] = cnt[1];
+    sh[0][wv] = v;
+#pragma unroll
+    for (int j = 0; j < ROWSUMS - 1; j++) sh[1 + j][wv] = cnt[j];
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int k = 1; k < NT / 64; k++) {
-      v = fmin(v, sh[k]);
-      cnt[0] += sc[0][k];
-      cnt[1] += sc[1][k];
-    }
-    out[3 + blockIdx.x] = v;
-    out[3 + gridDim.x + blockIdx.x] = cnt[0];
-    out[3 + 2 * gridDim.x + blockIdx.x] = cnt[1];
+  if (threadIdx.x < ROWSUMS) {
+    double t = sh[threadIdx.x][0];
+    for (int k = 1; k < NT / 64; k++)
+      t = threadIdx.x ? t + sh[threadIdx.x][k] : fmin(t, sh[0][k]);
+    out[(size_t)threadIdx.x * gridDim.x + blockIdx.x] = t;
   }
 }
-__global__ void __launch_bounds__(RT) ms_rowsum(int G, double *__restrict__ out) {
+__global__ void __launch_bounds__(RT)
+    ms_rowsum(int G, const double *__restrict__ part, double *__restrict__ host) {
   double v = 1.0;
-  for (int k = threadIdx.x; k < G; k += RT) v = fmin(v, out[3 + k]);
+  for (int k = threadIdx.x; k < G; k += RT) v = fmin(v, part[k]);
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v = fmin(v, __shfl_xor(v, o, 64));
   __shared__ double sh[RT / 64];
   if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
-  double cnt[2];
-  sum_partials<2>(out + 3 + G, G, cnt);  // (its barrier covers sh)
+  double cnt[ROWSUMS - 1];
+  sum_partials<ROWSUMS - 1>(part + G, G, cnt);  // (its barrier covers sh)
   if (threadIdx.x == 0) {
     for (int k = 1; k < RT / 64; k++) v = fmin(v, sh[k]);
-    out[0] = v;
-    out[1] = cnt[0];
-    out[2] = cnt[1];
+    host[0] = v;
+#pragma unroll
+    for (int j = 0; j < ROWSUMS - 1; j++) host[1 + j] = cnt[j];
   }
 }
 
@@ -2089,7 +2098,16 @@ void iteration(const MgPlan &pl, MgWork *w, hipStream_t st) {
 // Whether the V-cycle suits the assembled matrix: not when a mass term
 // dominates it.  Jacobi-PCG's condition number is about 2 over the smallest
 // row sum over diagonal (1 for a lumped mass matrix, O(h^2) for a stiffness
-// matrix); at 0.2 it needs about as many launches as the V-cycles do.
+// matrix); at 0.2 it needs about as many launches as the V-cycles do, and at three
+// quarters of that for each grid above the tail, whose launches come on top (of
+// about the number below): forward + adjoint of P1 heat steps, Jacobi-PCG against
+// multigrid CG, 40^2 dt 1e-4 0.84 and 0.73 ms, 128^2 1e-5 1.04 and 1.05, 3e-5 1.43
+// and 1.03, 400^2 1e-6 1.34 and 1.45, 3e-6 2.02 and 1.45.  P2's row sums say
+// nothing one by one (a vertex function's integral is 0); over all rows their sum
+// is 1.6 times the diagonals' for a mass matrix, and at half of that the two are
+// even: 100^2 dt 1e-6 1.02 and 1.28, 3e-6 1.48 and 1.46; 40^2 (6,561 rows) 3e-6 0.95
+// and 1.05, 3e-5 1.42 and 1.17; with few rows multigrid CG is the faster (20^2,
+// 1,681, at any step: 0.96 and 0.90).
 // A caller's matrix stays with Jacobi-PCG also where half its coupled rows
 // have a row sum over diagonal above MASS_HEAVY / rows: mass outweighs
 // stiffness even at the scale of the whole domain (0.25 / (dt kappa) for a heat
@@ -2098,24 +2116,29 @@ void iteration(const MgPlan &pl, MgWork *w, hipStream_t st) {
 // nearly equal fields: at rtol 1e-12 with boundary values of order 1 two
 // solvers' gradients differ by 1e-9 at dt 1e-3 (P1 160^2) and 2e-8 at 1e-4, by
 // 6e-10 at most from 4e-3 on.
-constexpr double MASS_DOMINANT = 0.2, MASS_HEAVY = 60.0;
+constexpr double MASS_DOMINANT = 0.2, MASS_DOMINANT_P2 = 0.8, MASS_HEAVY = 60.0;
+constexpr int MASS_P2_ROWS = 4000;
 // (Looked at before the plan, which a matrix that stays with Jacobi-PCG never
 // needs: 0.3 ms on every new mesh.)
 bool mg_pays(System &s, hipStream_t st) {
   if (!s.mass) return true;
   if (s.mg_pays_version != s.a_version) {
-    const unsigned g = nb(s.n, NT);
-    if (!s.mg_rows.p) s.mg_rows.alloc(3 + 3 * (size_t)g);
+    const unsigned g = (nb(s.n, NT) + 7) / 8 * 8;
+    if (!s.mg_rows.p) s.mg_rows.alloc(ROWSUMS * (size_t)g);
     mk_rowsum<<<g, NT, 0, st>>>(s.n, s.d_row_bd.p, s.d_slice_ptr.p, s.d_sell_val.p, s.d_diag.p,
                                 MASS_HEAVY / s.n, s.mg_rows.p);
-    ms_rowsum<<<1, RT, 0, st>>>((int)g, s.mg_rows.p);
-    HIPCHECK(hipGetLastError());
     HostSlot h(st);
-    for (int j = 0; j < 3; j++) h.read(8 * j, s.mg_rows.p + j);
+    ms_rowsum<<<1, RT, 0, st>>>((int)g, s.mg_rows.p, h.written());
+    HIPCHECK(hipGetLastError());
     h.wait();
     const bool callers = s.mesh == nullptr;
-    s.mg_pays = !(h.get<double>(0) > MASS_DOMINANT) &&
-              !(callers && 2.0 * h.get<double>(16) > h.get<double>(8));
+    const int degree = (callers ? s.mg_mesh : s.mesh)->degree;
+    double least = MASS_DOMINANT;
+    for (double nodes = s.n / 4.0; nodes > MG_TAIL - 350; nodes /= 4) least *= 0.75;
+    const double rows = h.get<double>(8), heavy = h.get<double>(16), sum = h.get<double>(24),
+                 diag = h.get<double>(32);
+    s.mg_pays = !(h.get<double>(0) > least) && !(callers && 2.0 * heavy > rows) &&
+                !(degree == 2 && s.n > MASS_P2_ROWS && sum > MASS_DOMINANT_P2 * diag);
     s.mg_pays_version = s.a_version;
   }
   return s.mg_pays;
