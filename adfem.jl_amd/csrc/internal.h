@@ -33,9 +33,11 @@ struct Error {
   } while (0)
 
 // Device memory with a bounded cache of released blocks (memory.cpp).
+struct OutOfMemory : Error {};
 void *device_alloc(size_t bytes, int &device);
 void device_free(void *p, size_t bytes, int device);
 void release_device_memory();
+size_t device_available();  // free on the current device, or in the cache
 
 // 64 bytes of pinned host memory for a call's results (memory.cpp): read()
 // enqueues a copy from the device, wait() makes what was read visible, or what a

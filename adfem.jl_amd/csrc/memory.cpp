@@ -57,6 +57,18 @@ void release_device_memory() {
   for (auto &b : out) (void)hipFree(b.second);
 }
 
+size_t device_available() {
+  size_t avail = 0, total = 0;
+  int dev = -1;
+  HIPCHECK(hipMemGetInfo(&avail, &total));
+  HIPCHECK(hipGetDevice(&dev));
+  Cache &c = cache();
+  std::lock_guard<std::mutex> g(c.mu);
+  for (auto &b : c.blocks)
+    if (b.first.first == dev) avail += b.first.second;
+  return avail;
+}
+
 void *device_alloc(size_t bytes, int &device) {
   HIPCHECK(hipGetDevice(&device));
   const size_t cls = size_class(bytes);
@@ -75,7 +87,11 @@ void *device_alloc(size_t bytes, int &device) {
   if (hipMalloc(&p, cls) != hipSuccess) {
     (void)hipGetLastError();
     release_device_memory();
-    HIPCHECK(hipMalloc(&p, cls));
+    if (hipMalloc(&p, cls) != hipSuccess) {
+      (void)hipGetLastError();
+      throw OutOfMemory{{ADMFEM_ERR_HIP, "out of device memory: " + std::to_string(cls) +
+                                             " bytes"}};
+    }
   }
   return p;
 }

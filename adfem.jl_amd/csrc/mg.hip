@@ -2146,6 +2146,9 @@ bool mg_pays(System &s, hipStream_t st) {
 
 }  // namespace
 
+// Device memory of a plan and its work, about, per row (P1).
+constexpr int MG_ROW_BYTES = 188;
+
 // A sparse system's rows are the dofs of mesh m (m null: unknown, and it is
 // Jacobi-PCG's), row i the caller's order[i]; both are only looked at in the
 // solve that follows.  Its plan is kept for as long as the mesh stays the same
@@ -2166,17 +2169,28 @@ void mg_set_mesh(System &s, const Mesh *m, const int *order) {
 
 // Solves by multigrid CG when that suits the system; false when it is
 // Jacobi-PCG's: also when multigrid CG broke down, met a NaN or ran out of
-// iterations, which Jacobi-PCG need not (and if it does, the status is its own).
+// iterations or memory (MG_ROW_BYTES against 120), which Jacobi-PCG need not (and
+// if it does, the status is its own).
 bool mg_solve(System &s, const double *b, double *x_out, const admfem_solve_opts &o,
               admfem_solve_stats &stats, hipStream_t st) {
   if (s.mg_off || s.n < MG_MIN_ROWS || s.mg_failed == s.a_version) return false;
   auto t0 = std::chrono::steady_clock::now();
   if (!mg_may_suit(s)) return false;
   if (!mg_pays(s, st)) return false;
-  const MgPlan *plan = mg_plan(s, st);
-  if (!plan) return false;
+  // (memory is looked at where it is no small matter)
+  const size_t need = (size_t)MG_ROW_BYTES * s.npad;
+  if (!s.mg_work && need > (size_t)32 << 20 && need > device_available()) return false;
+  const MgPlan *plan = nullptr;
+  MgWork *w = nullptr;
+  try {
+    plan = mg_plan(s, st);
+    if (!plan) return false;
+    w = ensure_work(s, *plan, st);
+  } catch (const OutOfMemory &) {
+    release_device_memory();  // (others may need it as well)
+    return false;
+  }
   const MgPlan &pl = *plan;
-  MgWork *w = ensure_work(s, pl, st);
   const MgSys *D = w->d.p;
   MgScal *S = w->sc.p;
   if (w->version != s.a_version) {  // a new matrix

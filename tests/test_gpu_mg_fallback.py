@@ -84,3 +84,33 @@ def test_serving_requests():
     s = 1 / np.sqrt(A.diagonal())
     y = spla.spsolve(sp.diags(s) @ A @ sp.diags(s), s * b)
     assert np.linalg.norm(out[0]["u"] / s - y) <= 1e-4 * np.linalg.norm(y)
+
+
+def test_memory_for_jacobi_only():
+    """On a card whose free memory holds Jacobi-PCG's arrays (504 MB for 2049^2 nodes)
+    but not multigrid CG's (789 MB) a solve is Jacobi-PCG's."""
+    c, e = meshgen.rectangle(2048, 2048, 1 / 2048)
+    mesh = admfem.Mesh(c, e, zero_based=True)
+    S = admfem.DirichletSystem(mesh, admfem.bcnode(mesh))
+    one = torch.ones(mesh.ngauss, dtype=torch.float64, device="cuda")
+    S.assemble(kappa=one, f=one)
+    torch.cuda.synchronize()
+    admfem._lib.check(admfem._lib.lib().admfem_release_memory())
+    torch.cuda.empty_cache()
+    held = []
+    try:
+        for _ in range(8):  # (what the driver gives back may take a moment to show)
+            free = torch.cuda.mem_get_info()[0]
+            if free > 650 << 20:
+                held.append(torch.empty(free - (640 << 20), dtype=torch.uint8, device="cuda"))
+        print("fallback, memory", torch.cuda.mem_get_info(), flush=True)
+        x, st = S.solve(rtol=0.01, max_iter=20000)
+        print(st, flush=True)
+        assert st["status"] == 0 and st["rel_residual"] <= 0.01 and st["iterations"] > 60
+        y, st = S.solve(rtol=0.01, max_iter=20000)  # with Jacobi-PCG's arrays in place
+        assert torch.equal(x, y)
+    finally:
+        del held
+        torch.cuda.empty_cache()
+    _, st = S.solve(rtol=1e-8)
+    assert st["iterations"] < 60  # multigrid CG, with the memory back
