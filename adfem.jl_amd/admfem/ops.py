@@ -385,8 +385,9 @@ class _Solve(torch.autograd.Function):
         u = torch.empty(n, dtype=torch.float64, device=_DEV)
         st = _lib.SolveStats()
         _lib.check(_lib.lib().admfem_sparse_solve_on(
-            mesh.handle if mesh is not None else None, _lib.ptr(ind), _lib.ptr(vv), ind.shape[0], n, _lib.ptr(rhs), _lib.ptr(u),
-            ctypes.byref(opts), ctypes.byref(st), _lib.stream_ptr()))
+            mesh.handle if mesh is not None else None, _lib.ptr(ind), _lib.ptr(vv),
+            ind.shape[0], n, _lib.ptr(rhs), _lib.ptr(u), ctypes.byref(opts), ctypes.byref(st),
+            _lib.stream_ptr()))
         ctx.save_for_backward(vv, ind, u)
         ctx.n, ctx.opts, ctx.mesh = n, opts, mesh
         return u
@@ -399,9 +400,9 @@ class _Solve(torch.autograd.Function):
         gr = torch.empty(ctx.n, dtype=torch.float64, device=_DEV)
         st = _lib.SolveStats()
         _lib.check(_lib.lib().admfem_sparse_solve_grad_on(
-            ctx.mesh.handle if ctx.mesh is not None else None, _lib.ptr(ind), _lib.ptr(vv), ind.shape[0], ctx.n, _lib.ptr(u), _lib.ptr(g_u),
-            _lib.ptr(gv), _lib.ptr(gr), ctypes.byref(ctx.opts), ctypes.byref(st),
-            _lib.stream_ptr()))
+            ctx.mesh.handle if ctx.mesh is not None else None, _lib.ptr(ind), _lib.ptr(vv),
+            ind.shape[0], ctx.n, _lib.ptr(u), _lib.ptr(g_u), _lib.ptr(gv), _lib.ptr(gr),
+            ctypes.byref(ctx.opts), ctypes.byref(st), _lib.stream_ptr()))
         return gv, gr, None, None, None, None
 
 

@@ -6,8 +6,8 @@ compute_fem_source_term1 -> impose_Dirichlet_boundary_conditions -> K\\F ->
 gradients of L = sum (u[obs] - obs_val)^2 w.r.t. kappa) on one of the
 registered meshes.  The engine (libadmfem, C++) admits requests as they
 arrive and as device memory frees up under an HBM budget, advances all
-admitted systems together with one batched launch per CG step, and reports
-per-request latency.
+admitted systems together, every launch of the solver one for all of them, and
+reports per-request latency.
 """
 import ctypes
 

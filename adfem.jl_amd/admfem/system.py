@@ -5,8 +5,8 @@
 fixed boundary node set, assembles
     A = mass_coef*M(rho) + lap_coef*K(kappa),
     rhs = src_coef*F(f) + M(rho) u_prev   (then Dirichlet lifting)
-straight into it, solves with Jacobi-PCG (FP64 or FP32 + FP64 residual
-replacement) and returns dL/dkappa by the adjoint method.  All vectors are
+straight into it, solves by multigrid-preconditioned CG (Jacobi-PCG where grids
+do not suit the system) and returns dL/dkappa by the adjoint method.  All vectors are
 torch tensors on the GPU (float64); node vectors in the user's node order.
 """
 import ctypes

@@ -438,9 +438,9 @@ bool mg_solve(System &s, const double *b_int, double *x_int, const admfem_solve_
               admfem_solve_stats &stats, hipStream_t st);
 void spmv_repeat(System &s, int precision, int repeat, hipStream_t st);
 // sparse_op.hip (m: the mesh whose dofs the rows are, or null)
-void sparse_solve(const Mesh *m, const long long *ind, const double *vv, int64_t nnz, int n, const double *rhs,
-                  double *u, const admfem_solve_opts &o, admfem_solve_stats &stats,
-                  hipStream_t st);
+void sparse_solve(const Mesh *m, const long long *ind, const double *vv, int64_t nnz, int n,
+                  const double *rhs, double *u, const admfem_solve_opts &o,
+                  admfem_solve_stats &stats, hipStream_t st);
 void sparse_solve_info(int64_t info[4]);
 void sparse_solve_grad(const Mesh *m, const long long *ind, const double *vv, int64_t nnz, int n,
                        const double *u, const double *grad_u, double *grad_vv,
@@ -457,6 +457,5 @@ void server_result(Server *sv, int64_t id, admfem_result &out);
 void server_stats(Server *sv, double *stats);
 double server_spmv_repeat(Server *sv, const int *topos, int nsys, int repeat,
                           hipStream_t st, double *seconds);
-// loss gradient: g_int = 0; g[perm[idx]] = 2 (u - obs); returns loss on host
 
 }  // namespace admfem

@@ -6,12 +6,13 @@
 namespace admfem {
 
 constexpr int MG_MAXLEV = 16;    // grid levels at most
-constexpr int MG_HALO = 2;       // zero nodes around a grid (the stencils reach 2)
+constexpr int MG_HALO = 2;       // nodes around a grid (the stencils reach 2)
 constexpr int MG_TAIL = 2048;    // padded nodes of the first level of the tail kernel
 constexpr int MG_DENSE = 49;     // nodes of the last level at most (dense inverse)
 
-// One grid level: nx x ny nodes stored with a halo of MG_HALO zero nodes on
-// every side (pitch px, pn entries in all), node (x, y) at mg_at.
+// One grid level: nx x ny nodes stored with room for MG_HALO nodes on every side
+// (pitch px, pn entries in all), node (x, y) at mg_at.  In memory that room is
+// neither written nor read; it is zero in the tail kernel's copies in LDS.
 struct MgLevel {
   float *a;     // 25 planes of pn: the stencil entries, offset (dx, dy) at
                 // plane (dy + 2) * 5 + dx + 2

@@ -450,8 +450,8 @@ __global__ void __launch_bounds__(GS)
 // The tail's grids below its first two, their weights and the dense inverse
 // of the last one, by Gauss-Jordan on its scaled form, two pivots a barrier; a
 // node whose pivot vanishes (outside the mesh, or the constant of a singular
-// matrix) is left out.  The matrices live in LDS as mk_tail keeps them; one
-// workgroup, so latency is all: 
+// matrix) is left out.  The matrices live in LDS as mk_tail keeps them: a chain of
+// barriers in one workgroup, bound by latency alone.
 constexpr int ST = 512;
 __global__ void __launch_bounds__(ST)
     mk_tail_setup(const MgSys *__restrict__ D, const int *__restrict__ list, int sys) {
@@ -1607,9 +1607,9 @@ __global__ void __launch_bounds__(NT)
 // the rows that take no part last.
 __global__ void __launch_bounds__(NT)
     plan_cells(int n, int npad, const double2 *__restrict__ pt, const int *__restrict__ row_bd,
-               const int *__restrict__ sp, const int *__restrict__ sc, double x0, double y0, double hx, double hy,
-               int ncx, int ncy, int *__restrict__ cell, float2 *__restrict__ frac,
-               int *__restrict__ key, int *__restrict__ row) {
+               const int *__restrict__ sp, const int *__restrict__ sc, double x0, double y0,
+               double hx, double hy, int ncx, int ncy, int *__restrict__ cell,
+               float2 *__restrict__ frac, int *__restrict__ key, int *__restrict__ row) {
   const int i = blockIdx.x * NT + threadIdx.x;
   if (i >= npad) return;
   int c = -1;
@@ -1734,7 +1734,8 @@ MgPlan *build_plan(System &s, const Mesh &m, const int *order, hipStream_t st) {
     pl->crow.alloc(n);
     pl->cptr.alloc(ncell + 1);
     plan_cells<<<nb(np, NT), NT, 0, st>>>(n, np, pt.p, s.d_row_bd.p, s.d_slice_ptr.p,
-                                          s.d_sell_col.p, x0, y0, hx, hy, ncx, ncy, pl->cell.p, pl->frac.p, key.p, row.p);
+                                          s.d_sell_col.p, x0, y0, hx, hy, ncx, ncy,
+                                          pl->cell.p, pl->frac.p, key.p, row.p);
     HIPCHECK(hipGetLastError());
     int bits = 1;
     while (ncell >> bits) bits++;
@@ -1814,7 +1815,8 @@ size_t tail_lds_of(const MgPlan &pl) {
   const size_t nn = (size_t)pl.nx[pl.nlev - 1] * pl.ny[pl.nlev - 1];
   pack += nn * nn;
   if (pl.tail == 0)
-    pack = std::max(pack, pl.n <= TAIL_STAGE ? (size_t)3 * pl.n : 0) + 4 * (size_t)(pl.nx[0] - 1) * (pl.ny[0] - 1);
+    pack = std::max(pack, pl.n <= TAIL_STAGE ? (size_t)3 * pl.n : 0) +
+           4 * (size_t)(pl.nx[0] - 1) * (pl.ny[0] - 1);
   return (t + pack) * sizeof(float);
 }
 
@@ -2111,11 +2113,17 @@ void iteration(const MgPlan &pl, MgWork *w, hipStream_t st) {
 // A caller's matrix stays with Jacobi-PCG also where half its coupled rows
 // have a row sum over diagonal above MASS_HEAVY / rows: mass outweighs
 // stiffness even at the scale of the whole domain (0.25 / (dt kappa) for a heat
-// step on P1, 0.19 on P2: dt below 4e-3 or 3e-3).  Such a step moves its field
-// little, and gradients in the density and the coefficient are differences of
-// nearly equal fields: at rtol 1e-12 with boundary values of order 1 two
-// solvers' gradients differ by 1e-9 at dt 1e-3 (P1 160^2) and 2e-8 at 1e-4, by
-// 6e-10 at most from 4e-3 on.
+// step on P1, 0.19 on P2: dt below 4e-3 or 3e-3).  Gradients of such a step are
+// differences of nearly equal fields, and their error at a given rtol depends on
+// the solver.  Gradient in kappa against 64 bits, operator chain at rtol 1e-12 with
+// boundary values of order 1, Jacobi-PCG and multigrid CG: dt 1e-4 P1 128^2 4.6e-9
+// and 6.0e-9, 160^2 7.4e-9 and 8.1e-9 (64^2 1.1e-9 and 6.9e-10, P2 40^2 2.2e-9 and
+// 7.2e-10), 3e-4 128^2 2.4e-9 and 4.7e-10, 1e-3 1.3e-9 and 4.1e-10, 3e-3 4.5e-10 and
+// 3.1e-10.  So the line keeps the shortest steps as near as they were, and is wider
+// than that takes: from 3e-4 on multigrid CG is the nearer and the faster (128^2 at
+// 1e-3: 8.3 and 3.0 ms a chain, 160^2 9.2 and 3.0, P2 40^2 8.2 and 3.3).  Systems of
+// the fused path and the engine, whose boundary rows are solved exactly, have no such
+// line.
 constexpr double MASS_DOMINANT = 0.2, MASS_DOMINANT_P2 = 0.8, MASS_HEAVY = 60.0;
 constexpr int MASS_P2_ROWS = 4000;
 // (Looked at before the plan, which a matrix that stays with Jacobi-PCG never

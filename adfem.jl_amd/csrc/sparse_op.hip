@@ -5,7 +5,8 @@
 //
 // Duplicates are summed in triplet order (Eigen's setFromTriplets order);
 // the matrix must be symmetric positive definite, since the solve is the
-// library's Jacobi-PCG (then A^-T = A^-1).
+// library's CG (multigrid CG where the mesh is known, else Jacobi-PCG; then
+// A^-T = A^-1).
 //
 // The pattern is built on the device: a stable radix sort of the keys
 // row * n + col (equal keys keep their triplet order), one slot per run of
@@ -283,8 +284,8 @@ void build_pattern(CooPattern &p, const Mesh *m, const long long *ind, int64_t n
 
 // The kept pattern for these indices (rebuilt when they differ), with the
 // values summed into its solver format.  Caller holds g_lock.
-System &pattern_with_values(const Mesh *m, const long long *ind, const double *vv, int64_t nnz, int n,
-                            hipStream_t st) {
+System &pattern_with_values(const Mesh *m, const long long *ind, const double *vv, int64_t nnz,
+                            int n, hipStream_t st) {
   REQUIRE(n > 0 && nnz >= 0 && nnz < INT32_MAX, ADMFEM_ERR_ARG, "bad sizes");
   int dev = 0;
   HIPCHECK(hipGetDevice(&dev));
@@ -327,9 +328,9 @@ void solve_kept(CooPattern &p, const double *b, double *x, const admfem_solve_op
 
 }  // namespace
 
-void sparse_solve(const Mesh *m, const long long *ind, const double *vv, int64_t nnz, int n, const double *rhs,
-                  double *u, const admfem_solve_opts &o, admfem_solve_stats &stats,
-                  hipStream_t st) {
+void sparse_solve(const Mesh *m, const long long *ind, const double *vv, int64_t nnz, int n,
+                  const double *rhs, double *u, const admfem_solve_opts &o,
+                  admfem_solve_stats &stats, hipStream_t st) {
   std::lock_guard<std::mutex> g(g_lock);
   pattern_with_values(m, ind, vv, nnz, n, st);
   solve_kept(*g_kept, rhs, u, o, stats, st);

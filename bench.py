@@ -9,22 +9,24 @@ nodes jittered by U[-0.2h, 0.2h]^2; kappa = exp(GRF: 32 random Fourier modes,
 sigma 1, length 0.1) and f ~ U[-1, 1] at the Gauss points, homogeneous
 Dirichlet on the boundary, L = sum (u - u_obs)^2 over a seeded 1% of the
 interior nodes; each request returns u, L and dL/dkappa.  Requests are served
-by the continuous-batching engine (FP32-storage Jacobi-PCG with FP64 residual
-replacement, every system's true FP64 relative residual driven below rtol)
-under a 64 GB HBM admission budget.  Inputs are generated on the device from
+by the continuous-batching engine (FP64 CG preconditioned by a multigrid V-cycle
+in FP32, every system's true FP64 relative residual driven below rtol) under a
+64 GB HBM admission budget.  Inputs are generated on the device from
 each request's seed; mesh topologies are resident before timing starts.
 
 One step = one pass of the whole stream through a fresh engine with every
 request queued at t = 0 (throughput at capacity).  After the timed steps:
   * load: the same stream with Poisson arrivals at 80% of the measured
     capacity -> p50 / p99 latency (arrival to result);
-  * fp64_plain: the plain FP64 GPU path (one request at a time, FP64
-    Jacobi-PCG) on the first requests of the stream -> its solves/s and
-    latency; the batched engine on the same subset beside it;
+  * fp64_plain: the plain FP64 GPU path (one request at a time, the
+    single-system solver) on the first requests of the stream -> its solves/s
+    and latency; the batched engine on the same subset beside it;
   * accuracy: requests of the stream with host-side inputs, served by both
     paths and compared with the CPU oracle's direct solve (u and dL/dkappa);
-  * roofline: the batched SpMV kernel over the stream's first batch, timed
-    with HIP events on the stream it runs on;
+  * roofline: the engine's Jacobi-PCG step kernel over the stream's first batch,
+    timed with HIP events on the stream it runs on.  The stream's requests, side
+    32 and up, are multigrid CG's and do not run it; profiles/timed_cases.md has
+    the kernels that they run;
   * precision_form: one 2048x2048-quad system (8.4M triangles), mixed vs plain
     FP64 forward+adjoint, errors against an FP64 CG solve to 1e-13, the
     single-system SpMV kernels and the assembly timed with HIP events;
@@ -115,8 +117,10 @@ def summary(n, wall, rs, st, req_sides=None, systems=None):
     svc = np.array([r["t_done"] - r["t_admit"] for r in rs])
     extra = {}
     if req_sides is not None:
-        # latency per side bucket, and the algorithmic bytes of every CG
-        # iteration the pass ran (FP32 step kernels; replacements not counted)
+        # latency per side bucket, and the algorithmic bytes of every product
+        # with a matrix that the pass ran, each as a CG iteration in FP32 storage
+        # (a multigrid iteration is three products, one of them in FP64; its
+        # grids are not counted)
         extra["p99_ms_by_side"] = {}
         for lo, hi in SIDE_BUCKETS:
             sel = (req_sides >= lo) & (req_sides < hi)
@@ -321,7 +325,9 @@ def batched_spmv_roofline(systems, sides, nsys, repeat=200):
                     "r -= alpha q, y += alpha p, p = r + beta p, q = A p, four dot products",
              bytes_note="canonical CSR CG iteration, nnz*(4+4) + 4(n+1) + 2n*4 for the SpMV "
                         "plus 6n*4 for the vector updates, summed over the systems",
-             spmv_only_bytes=int(spmv))
+             spmv_only_bytes=int(spmv),
+             of="the engine's Jacobi-PCG, which serves what multigrid CG does not suit: none "
+                "of the timed requests")
     t = measured_traffic(nsys)
     if t is not None:
         r["traffic"] = t
@@ -775,8 +781,8 @@ def main():
             "topologies": len(systems),
             "max_active": MAX_ACTIVE,
             "rtol": a.rtol,
-            "precision": "FP32 storage, FP64 arithmetic inner CG; FP64 residual replacement "
-                         "and solution",
+            "precision": "FP64 CG (matrix, vectors, dot products, solution), multigrid "
+                         "V-cycle on FP32 copies",
             "outputs": "timed passes keep u and dL/dkappa on the device (no host copies); "
                        "the accuracy leg copies them back",
         },

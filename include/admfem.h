@@ -301,8 +301,10 @@ int admfem_system_assemble(admfem_system s, const admfem_problem *p,
 int admfem_system_csr(admfem_system s, int *row_ptr, int *col, double *val,
                       double *rhs);
 
-#define ADMFEM_PREC_FP64 0   /* FP64 Jacobi-PCG */
-#define ADMFEM_PREC_MIXED 1  /* FP32 Jacobi-PCG, FP64 residual replacement */
+/* Multigrid CG (admfem_system_solve) has its matrix, vectors and dot products in
+ * FP64 and its V-cycle in FP32 with either; where Jacobi-PCG runs: */
+#define ADMFEM_PREC_FP64 0   /* FP64 */
+#define ADMFEM_PREC_MIXED 1  /* FP32, FP64 residual replacement */
 typedef struct {
   int precision;      /* ADMFEM_PREC_* */
   int max_iter;       /* total inner iterations, counted in products with A (a
@@ -426,7 +428,7 @@ int admfem_sparse_solve_grad_on(admfem_mesh m, const long long *indices, const d
  * kept when it is already banded).  Zeros before the first solve. */
 int admfem_sparse_solve_info(int64_t info[4]);
 
-/* Instrumentation (no reference counterpart): launches the solver's step
+/* Instrumentation (no reference counterpart): launches Jacobi-PCG's step
  * kernel (the SpMV with the iteration's vector updates fused in; FP64 or
  * FP32 matrix per `precision`) `repeat` times back to back on `stream`, on
  * the system's work vectors, for timing the dominant kernel.  *bytes (host,
@@ -444,11 +446,12 @@ int admfem_system_spmv_repeat(admfem_system s, int precision, int repeat,
  *    L = sum_k (u[obs_k] - obs_val_k)^2.
  *
  *    Requests are admitted when they have arrived and their device memory
- *    fits the budget; admitted systems advance together, one batched launch
- *    per CG step for all of them (mixed precision: FP32 inner iterations,
- *    FP64 residual replacement); a system that converges moves on (forward
- *    -> adjoint -> gradient -> done) and frees its memory for the next
- *    arrivals.  Results do not depend on what else is in the batch.
+ *    fits the budget; admitted systems advance together, every launch of the
+ *    solver one for all of them (multigrid CG; Jacobi-PCG with FP32 inner
+ *    iterations and FP64 residual replacement for requests that does not suit,
+ *    or that do not fit the budget with it); a system that converges moves on
+ *    (forward -> adjoint -> gradient -> done) and frees its memory for the
+ *    next arrivals.  Results do not depend on what else is in the batch.
  * ==================================================================== */
 
 typedef struct admfem_server_s *admfem_server;
