@@ -790,7 +790,40 @@ struct Server {
     HIPCHECK(hipGraphLaunch(it->second, st));
   }
 
+  // What an error that ends a run leaves half done (inputs on no list any more,
+  // descriptors not uploaded, systems not set up) is not taken up again: the
+  // admitted requests fail with it, and the next run serves the waiting ones.
+  void abandon(int code) {
+    (void)hipStreamSynchronize(st);
+    (void)hipGetLastError();
+    starts.clear();
+    jobs_in.clear();
+    jobs_turn.clear();
+    jobs_out.clear();
+    for (Req &q : reqs) {
+      if (q.slot < 0) continue;
+      q.res.status = code;
+      q.res.done = 1;
+      q.res.t_done = now_s(t0);
+      q.state = Q_DONE;
+      std::vector<int>().swap(q.h_obs);
+      release(q);
+    }
+  }
+
   void run_batched(double timeout) {
+    try {
+      serve_batched(timeout);
+    } catch (const Error &e) {
+      abandon(e.code);
+      throw;
+    } catch (...) {
+      abandon(ADMFEM_ERR_ARG);
+      throw;
+    }
+  }
+
+  void serve_batched(double timeout) {
     const int chunk = o.chunk > 0 ? (o.chunk + REPLACE_EVERY - 1) / REPLACE_EVERY * REPLACE_EVERY
                                   : 2 * REPLACE_EVERY;
     std::vector<int> order(reqs.size());
@@ -798,9 +831,6 @@ struct Server {
     std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
       return reqs[a].r.arrival < reqs[b].r.arrival;
     });
-    jobs_in.clear();  // (a run that ended in an error may have left some)
-    jobs_turn.clear();
-    jobs_out.clear();
     size_t next = 0;  // first request (in arrival order) not yet admitted
     while (next < order.size() && reqs[order[next]].state != Q_WAIT) next++;
     // (a solve is 8 to 12 iterations; 64 a chunk on 8 requests of 64^2: 1.7 -> 3.0 ms,
@@ -1197,8 +1227,12 @@ int server_add_topology(Server *sv, System *s, double jitter) {
   T.nblk = (s->npad + BATCH_NT - 1) / BATCH_NT;
   T.plan = nullptr;
   if (s->n >= MG_MIN_ROWS && sv->o.mode == ADMFEM_MODE_BATCHED) {
-    T.plan = mg_plan(*s, sv->st);
-    if (T.plan) mg_allow_lds(*T.plan);
+    try {
+      T.plan = mg_plan(*s, sv->st);
+      if (T.plan) mg_allow_lds(*T.plan);
+    } catch (const OutOfMemory &) {  // (Jacobi-PCG needs none)
+      release_device_memory();
+    }
   }
   for (int u = 0; u < s->n; u++)
     if (s->row_bd[s->uperm()[u]] < 0) T.interior.push_back(u);

@@ -533,7 +533,9 @@ int admfem_server_add_topology(admfem_server sv, admfem_system s, double jitter,
 /* Queues a request; *req_id receives its id (0, 1, ...). */
 int admfem_server_submit(admfem_server sv, const admfem_request *r, int64_t *req_id);
 /* Serves every queued request (arrival times are measured from the first
- * call), returns when all are done or after timeout_s seconds. */
+ * call), returns when all are done or after timeout_s seconds.  When the call
+ * itself fails, the requests admitted by then are done with that status, and
+ * those still waiting are served by the next call. */
 int admfem_server_run(admfem_server sv, double timeout_s);
 int admfem_server_result(admfem_server sv, int64_t req_id, admfem_result *out);
 /* stats[0..7] = requests done, wall seconds, peak device bytes, peak
